@@ -18,7 +18,37 @@ namespace {
 template <typename T> struct Acc { typedef float type; };
 template <> struct Acc<double> { typedef double type; };
 
-template <typename T, int N> struct alignas(sizeof(T) * N) Pack { T v[N]; };
+// VEC consecutive elements of a row.  RAG: the rows are not whole vectors (or a base address is not aligned to one), so a
+// vector is only aligned to its elements; the hardware takes such loads and stores as they are, whole (dwordx4).
+template <typename T, int N, bool RAG = false> struct alignas(RAG ? sizeof(T) : sizeof(T) * N) Pack { T v[N]; };
+
+// Rows of `batch` elements are read and written as vectors 0 .. ceil(batch / VEC) - 1.  RAG: the last vector of a row is
+// moved back to end with the row, so it repeats `dup` elements of the vector before it.  Elementwise results are then
+// written twice with the same value; sums over the batch leave the repeated elements out (own_part).  What that buys
+// over one element per lane: half rows of 500 elements on six 64000-wide layers, forward + backward 2.11 -> 0.61 ms.
+template <int VEC> __device__ __forceinline__ int64_t vec_count(int64_t batch) {
+    return (int64_t) ((uint64_t) (batch + VEC - 1) / VEC);
+}
+template <int VEC, bool RAG> __device__ __forceinline__ int64_t vec_at(int64_t col, int64_t batch) {
+    const int64_t at = col * VEC;
+    return RAG && at + VEC > batch ? batch - VEC : at;
+}
+template <int VEC, bool RAG> __device__ __forceinline__ int vec_dup(int64_t col, int64_t batch) {
+    return RAG && col * VEC + VEC > batch ? (int) (col * VEC + VEC - batch) : 0;
+}
+template <bool RAG, typename C> __device__ __forceinline__ C own_part(C g, int e, int dup) {
+    return RAG && e < dup ? (C) 0 : g;
+}
+// Vector `col` of row `row` (whole rows are addressed in vectors: one shift less per access, 2 % of a one-pass backward).
+template <typename P, int VEC, bool RAG, typename T>
+__device__ __forceinline__ const P &row_vec(const T *base, int64_t row, int64_t batch, int64_t ncols, int64_t col) {
+    if constexpr (RAG) return *reinterpret_cast<const P *>(base + row * batch + vec_at<VEC, RAG>(col, batch));
+    else return reinterpret_cast<const P *>(base)[row * ncols + col];
+}
+template <typename P, int VEC, bool RAG, typename T>
+__device__ __forceinline__ P &row_vec(T *base, int64_t row, int64_t batch, int64_t ncols, int64_t col) {
+    return const_cast<P &>(row_vec<P, VEC, RAG>(const_cast<const T *>(base), row, batch, ncols, col));
+}
 
 template <typename T> __device__ __forceinline__ typename Acc<T>::type up(T v) { return (typename Acc<T>::type) v; }
 template <> __device__ __forceinline__ float up<__half>(__half v) { return __half2float(v); }
@@ -214,17 +244,18 @@ __device__ __forceinline__ void corners4(const T *__restrict__ w, const int32_t 
 // ------------------------------------------------------------------------------------------
 // LOGITS: `w` holds the raw gate logits; the kernel applies the softmax itself and (column tile 0
 // only) stores the probabilities to `probs` for the backward pass.
-template <typename T, int VEC, int NPW, bool LOGITS>
+template <typename T, int VEC, int NPW, bool LOGITS, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_kernel(const T *__restrict__ x, const int64_t *__restrict__ a,
                                                            const int64_t *__restrict__ b, const T *__restrict__ w,
                                                            T *__restrict__ y, T *__restrict__ probs, int64_t out_dim,
-                                                           int64_t ncols, bool w32) {
+                                                           int64_t batch, bool w32) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t n0 = ((int64_t) blockIdx.x * 4 + wave) * NPW;
     if (n0 >= out_dim) return;
+    const int64_t ncols = vec_count<VEC>(batch);
 
     static_assert(NPW == 4, "corners4 serves four neurons per wave");
     int64_t ia[NPW], ib[NPW];
@@ -238,14 +269,12 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_kernel(const T *__restrict__
         ids[j] = n0 + j < out_dim ? (int32_t) (n0 + j) : -1;
     }
     corners4<T, LOGITS>(w, ids, lane, blockIdx.y == 0, probs, p00, p10, d0, d1, w32);
-    const P *xv = reinterpret_cast<const P *>(x);
-    P *yv = reinterpret_cast<P *>(y);
     for (int64_t col = (int64_t) blockIdx.y * DL_WAVE + lane; col < ncols; col += (int64_t) gridDim.y * DL_WAVE) {
         P va[NPW], vb[NPW];
 #pragma unroll
         for (int j = 0; j < NPW; ++j) {
-            va[j] = xv[ia[j] * ncols + col];
-            vb[j] = xv[ib[j] * ncols + col];
+            va[j] = row_vec<P, VEC, RAG>(x, ia[j], batch, ncols, col);
+            vb[j] = row_vec<P, VEC, RAG>(x, ib[j], batch, ncols, col);
         }
 #pragma unroll
         for (int j = 0; j < NPW; ++j) {
@@ -255,7 +284,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_kernel(const T *__restrict__
                 for (int e = 0; e < VEC; ++e) {
                     r.v[e] = down<T, C>(mix<C>(up<T>(va[j].v[e]), up<T>(vb[j].v[e]), p00[j], p10[j], d0[j], d1[j]));
                 }
-                yv[(n0 + j) * ncols + col] = r;
+                row_vec<P, VEC, RAG>(y, (n0 + j), batch, ncols, col) = r;
             }
         }
     }
@@ -293,14 +322,15 @@ __device__ __forceinline__ void store_grad_w(int lane, bool neuron_valid, int64_
 // ------------------------------------------------------------------------------------------
 // probs != nullptr: chain the softmax backward, gw[n,i] = p_i * (g_i - sum_j p_j g_j), i.e. the
 // gradient with respect to the logits that `probs` (forward_kernel's LOGITS output) came from.
-template <typename T, int VEC, int NPW, int WPN>
+template <typename T, int VEC, int NPW, int WPN, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_w_kernel(const T *__restrict__ x, const int64_t *__restrict__ a,
                                                               const int64_t *__restrict__ b,
                                                               const T *__restrict__ gy, const T *__restrict__ probs,
-                                                              T *__restrict__ gw, int64_t out_dim, int64_t ncols,
+                                                              T *__restrict__ gw, int64_t out_dim, int64_t batch,
                                                               int64_t gdiv, bool w32) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     __shared__ C partial[4][NPW][4];
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
@@ -320,23 +350,22 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_w_kernel(const T *__restric
             ib[j] = b[n];
             nn[j] = grad_row(n, gdiv);
         }
-        const P *xv = reinterpret_cast<const P *>(x);
-        const P *gv = reinterpret_cast<const P *>(gy);
         for (int64_t base = (int64_t) part * DL_WAVE; base < ncols; base += (int64_t) WPN * DL_WAVE) {
             const int64_t col = base + lane;
             if (col < ncols) {
+                const int dup = vec_dup<VEC, RAG>(col, batch);
                 P va[NPW], vb[NPW], vg[NPW];
 #pragma unroll
                 for (int j = 0; j < NPW; ++j) {
-                    va[j] = xv[ia[j] * ncols + col];
-                    vb[j] = xv[ib[j] * ncols + col];
-                    vg[j] = gv[nn[j] * ncols + col];
+                    va[j] = row_vec<P, VEC, RAG>(x, ia[j], batch, ncols, col);
+                    vb[j] = row_vec<P, VEC, RAG>(x, ib[j], batch, ncols, col);
+                    vg[j] = row_vec<P, VEC, RAG>(gy, nn[j], batch, ncols, col);
                 }
 #pragma unroll
                 for (int j = 0; j < NPW; ++j) {
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) {
-                        const C av = up<T>(va[j].v[e]), bv = up<T>(vb[j].v[e]), g = up<T>(vg[j].v[e]);
+                        const C av = up<T>(va[j].v[e]), bv = up<T>(vb[j].v[e]), g = own_part<RAG>(up<T>(vg[j].v[e]), e, dup);
                         const C ga = g * av, gna = g - ga;       // g*a, g*(1-a)
                         const C t11 = ga * bv, t01 = gna * bv;
                         s11[j] += t11;
@@ -388,24 +417,22 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_w_kernel(const T *__restric
 // A neuron wired twice to this input appears twice in the list; each visit adds half of
 // dy/da + dy/db.
 // ------------------------------------------------------------------------------------------
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_x_kernel(const T *__restrict__ x, const int64_t *__restrict__ a,
                                                               const int64_t *__restrict__ b, const T *__restrict__ w,
                                                               const T *__restrict__ gy,
                                                               const int64_t *__restrict__ start,
                                                               const int64_t *__restrict__ idx, T *__restrict__ gx,
-                                                              int64_t in_dim, int64_t ncols,
+                                                              int64_t in_dim, int64_t batch,
                                                               typename Acc<T>::type scale, int64_t gdiv, bool w32) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t c = (int64_t) blockIdx.x * 4 + wave;
     if (c >= in_dim) return;
     const int64_t e0 = start[c], e1 = start[c + 1];
-    const P *xv = reinterpret_cast<const P *>(x);
-    const P *gv = reinterpret_cast<const P *>(gy);
-    P *ov = reinterpret_cast<P *>(gx);
 
     for (int64_t col = (int64_t) blockIdx.y * DL_WAVE + lane; col < ncols; col += (int64_t) gridDim.y * DL_WAVE) {
         C acc[VEC];
@@ -417,8 +444,8 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_x_kernel(const T *__restric
             const int64_t nA = idx[e], nB = two ? idx[e + 1] : nA;
             const int64_t iaA = a[nA], ibA = b[nA], iaB = a[nB], ibB = b[nB];
             const bool isaA = iaA == c, isaB = iaB == c;
-            const P gA = gv[grad_row(nA, gdiv) * ncols + col], oA = xv[(isaA ? ibA : iaA) * ncols + col];
-            const P gB = gv[grad_row(nB, gdiv) * ncols + col], oB = xv[(isaB ? ibB : iaB) * ncols + col];
+            const P gA = row_vec<P, VEC, RAG>(gy, grad_row(nA, gdiv), batch, ncols, col), oA = row_vec<P, VEC, RAG>(x, (isaA ? ibA : iaA), batch, ncols, col);
+            const P gB = row_vec<P, VEC, RAG>(gy, grad_row(nB, gdiv), batch, ncols, col), oB = row_vec<P, VEC, RAG>(x, (isaB ? ibB : iaB), batch, ncols, col);
             const Corners<C> kA = corners<T>(w, nA, w32), kB = corners<T>(w, nB, w32);
             {
                 const C d0 = kA.p01 - kA.p00, d1 = kA.p11 - kA.p10, dd = d1 - d0, da = kA.p10 - kA.p00;
@@ -436,7 +463,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_x_kernel(const T *__restric
         P r;
 #pragma unroll
         for (int q = 0; q < VEC; ++q) r.v[q] = down<T, C>(acc[q] * scale);
-        ov[c * ncols + col] = r;
+        row_vec<P, VEC, RAG>(gx, c, batch, ncols, col) = r;
     }
 }
 
@@ -449,24 +476,23 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_x_kernel(const T *__restric
 // fp64 results are bit-identical (fp16 outputs can differ in the last bit, where the compiler
 // folds the final conversion into a fused multiply-add in one kernel and not in the other).
 // ------------------------------------------------------------------------------------------
-template <typename T, int VEC, int CHUNK, bool LOGITS>
+template <typename T, int VEC, int CHUNK, bool LOGITS, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__restrict__ x,
                                                                  const int32_t *__restrict__ verts,
                                                                  const int32_t *__restrict__ neuron,
                                                                  const uint8_t *__restrict__ flip,
                                                                  const T *__restrict__ w, T *__restrict__ y,
-                                                                 T *__restrict__ probs, int64_t nchunks, int64_t ncols,
+                                                                 T *__restrict__ probs, int64_t nchunks, int64_t batch,
                                                                  bool w32) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t c = (int64_t) blockIdx.x * 4 + wave;
     if (c >= nchunks) return;
     static_assert(CHUNK % 4 == 0, "neurons are served four at a time");
     const int64_t s0 = c * CHUNK;
-    const P *xv = reinterpret_cast<const P *>(x);
-    P *yv = reinterpret_cast<P *>(y);
 
     for (int64_t ct = blockIdx.y; ct * DL_WAVE < ncols; ct += gridDim.y) {
         const int64_t col = ct * DL_WAVE + lane;
@@ -475,7 +501,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__rest
         // every row of the chunk is requested before the first one is used
         P rows[CHUNK + 1];
 #pragma unroll
-        for (int j = 0; j <= CHUNK; ++j) rows[j] = xv[(int64_t) verts[s0 + j] * ncols + cl];
+        for (int j = 0; j <= CHUNK; ++j) rows[j] = row_vec<P, VEC, RAG>(x, (int64_t) verts[s0 + j], batch, ncols, cl);
 #pragma unroll
         for (int j0 = 0; j0 < CHUNK; j0 += 4) {
             int32_t n[4];
@@ -493,7 +519,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__rest
                     const C u0 = up<T>(rows[j].v[e]), u1 = up<T>(rows[j + 1].v[e]);
                     r.v[e] = down<T, C>(mix<C>(f ? u1 : u0, f ? u0 : u1, p00[i], p10[i], d0[i], d1[i]));
                 }
-                if (live && n[i] >= 0) yv[(int64_t) n[i] * ncols + col] = r;
+                if (live && n[i] >= 0) row_vec<P, VEC, RAG>(y, (int64_t) n[i], batch, ncols, cl) = r;
             }
         }
     }
@@ -505,22 +531,21 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__rest
 // (LOGITS: logits, whose softmax goes to `lprobs`).  Values and rounding are those of forward_kernel
 // on the lower layer, so the result equals running the two layers one after the other bit for bit,
 // but the activation between them is neither written nor read.
-template <typename T, int VEC, int CHUNK, bool LOGITS>
+template <typename T, int VEC, int CHUNK, bool LOGITS, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
     const T *__restrict__ lx, const int64_t *__restrict__ low_a, const int64_t *__restrict__ low_b,
     const T *__restrict__ lw, T *__restrict__ lprobs, const int32_t *__restrict__ verts,
     const int32_t *__restrict__ neuron, const uint8_t *__restrict__ flip, const T *__restrict__ w, T *__restrict__ y,
-    T *__restrict__ probs, int64_t nchunks, int64_t ncols) {
+    T *__restrict__ probs, int64_t nchunks, int64_t batch) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t c = (int64_t) blockIdx.x * 4 + wave;
     if (c >= nchunks) return;
     static_assert(CHUNK % 4 == 0, "neurons are served four at a time");
     const int64_t s0 = c * CHUNK;
-    const P *xv = reinterpret_cast<const P *>(lx);
-    P *yv = reinterpret_cast<P *>(y);
 
     // corner coefficients of the chunk's CHUNK + 1 lower neurons and CHUNK neurons, once for all column tiles
     constexpr int NV = CHUNK + 4;
@@ -562,8 +587,8 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (j0 + i <= CHUNK) {
-                    va[i] = xv[ia[j0 + i] * ncols + cl];
-                    vb[i] = xv[ib[j0 + i] * ncols + cl];
+                    va[i] = row_vec<P, VEC, RAG>(lx, ia[j0 + i], batch, ncols, cl);
+                    vb[i] = row_vec<P, VEC, RAG>(lx, ib[j0 + i], batch, ncols, cl);
                 }
             }
 #pragma unroll
@@ -585,7 +610,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
                 const C u0 = up<T>(rows[j].v[e]), u1 = up<T>(rows[j + 1].v[e]);
                 r.v[e] = down<T, C>(mix<C>(f ? u1 : u0, f ? u0 : u1, p00[j], p10[j], d0[j], d1[j]));
             }
-            if (live && n[j] >= 0) yv[(int64_t) n[j] * ncols + col] = r;
+            if (live && n[j] >= 0) row_vec<P, VEC, RAG>(y, (int64_t) n[j], batch, ncols, cl) = r;
         }
     }
 }
@@ -594,23 +619,22 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
 // CPL * 64 consecutive vectors of the row (blockIdx.y picks the segment; lane l holds its vectors
 // l, l + 64, ...), so every gathered row is one contiguous request of up to 4 KB, and the next
 // step's row is requested before this step's arithmetic.
-template <typename T, int VEC, int CPL, bool LOGITS>
+template <typename T, int VEC, int CPL, bool LOGITS, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *__restrict__ x,
                                                                       const int32_t *__restrict__ verts,
                                                                       const int32_t *__restrict__ neuron,
                                                                       const uint8_t *__restrict__ flip,
                                                                       const T *__restrict__ w, T *__restrict__ y,
                                                                       T *__restrict__ probs, int64_t steps, int chunk,
-                                                                      int64_t ncols, bool w32) {
+                                                                      int64_t batch, bool w32) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t s0 = ((int64_t) blockIdx.x * 4 + wave) * chunk;
     if (s0 >= steps) return;
     const int64_t s1 = s0 + chunk < steps ? s0 + chunk : steps;
-    const P *xv = reinterpret_cast<const P *>(x);
-    P *yv = reinterpret_cast<P *>(y);
     const int64_t col0 = (int64_t) blockIdx.y * (CPL * DL_WAVE);
     P zero;
 #pragma unroll
@@ -619,7 +643,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *_
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
             const int64_t col = col0 + lane + q * DL_WAVE;
-            out[q] = col < ncols ? xv[row * ncols + col] : zero;
+            out[q] = col < ncols ? row_vec<P, VEC, RAG>(x, row, batch, ncols, col) : zero;
         }
     };
     P prev[CPL], cur[CPL], next[CPL];
@@ -647,7 +671,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *_
                         const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]);
                         r.v[e] = down<T, C>(mix<C>(f ? u1 : u0, f ? u0 : u1, p00[i], p10[i], d0[i], d1[i]));
                     }
-                    if (n[i] >= 0 && col < ncols) yv[(int64_t) n[i] * ncols + col] = r;
+                    if (n[i] >= 0 && col < ncols) row_vec<P, VEC, RAG>(y, (int64_t) n[i], batch, ncols, col) = r;
                 }
 #pragma unroll
                 for (int q = 0; q < CPL; ++q) {
@@ -660,49 +684,49 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *_
 }
 
 // One wave owns CHUNK steps and the whole batch: lane l holds vectors l, l + 64, ... (CPL of them).
-template <typename T, int VEC, int CPL, int CHUNK>
+template <typename T, int VEC, int CPL, int CHUNK, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_w_chain_kernel(const T *__restrict__ x,
                                                                     const int32_t *__restrict__ verts,
                                                                     const int32_t *__restrict__ neuron,
                                                                     const uint8_t *__restrict__ flip,
                                                                     const T *__restrict__ gy,
                                                                     const T *__restrict__ probs, T *__restrict__ gw,
-                                                                    int64_t nchunks, int64_t ncols, int64_t gdiv, bool w32) {
+                                                                    int64_t nchunks, int64_t batch, int64_t gdiv, bool w32) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t c = (int64_t) blockIdx.x * 4 + wave;
     if (c >= nchunks) return;
     const int64_t s0 = c * CHUNK;
-    const P *xv = reinterpret_cast<const P *>(x);
-    const P *gv = reinterpret_cast<const P *>(gy);
     P zero;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) zero.v[e] = down<T, C>((C) 0);
 
-    auto load_row = [&](const P *base, int64_t row, P *dst) {
+    auto load_row = [&](const T *base, int64_t row, P *dst) {
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
             const int64_t col = lane + q * DL_WAVE;
-            dst[q] = col < ncols ? base[row * ncols + col] : zero;
+            dst[q] = col < ncols ? row_vec<P, VEC, RAG>(base, row, batch, ncols, col) : zero;
         }
     };
     P prev[CPL];
-    load_row(xv, verts[s0], prev);
+    load_row(x, verts[s0], prev);
 #pragma unroll 1
     for (int j = 0; j < CHUNK; ++j) {
         const int32_t n = neuron[s0 + j];
         const bool f = flip[s0 + j] != 0;
         P cur[CPL], g[CPL];
-        load_row(xv, verts[s0 + j + 1], cur);
-        load_row(gv, grad_row(n >= 0 ? n : 0, gdiv), g);
+        load_row(x, verts[s0 + j + 1], cur);
+        load_row(gy, grad_row(n >= 0 ? n : 0, gdiv), g);
         C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
+            const int dup = vec_dup<VEC, RAG>(lane + q * DL_WAVE, batch);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
-                const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]), gg = up<T>(g[q].v[e]);
+                const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]), gg = own_part<RAG>(up<T>(g[q].v[e]), e, dup);
                 const C av = f ? u1 : u0, bv = f ? u0 : u1;
                 const C ga = gg * av, gna = gg - ga;
                 const C t11 = ga * bv, t01 = gna * bv;
@@ -750,16 +774,17 @@ template <typename T> struct LowerLayer {
     T *gw;                      // [in_dim, 16]
 };
 
-template <typename T, int VEC, int CPL, int LOWER>
+template <typename T, int VEC, int CPL, int LOWER, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const T *__restrict__ x, const int32_t *__restrict__ verts, const int32_t *__restrict__ neuron,
     const uint8_t *__restrict__ flip, const int32_t *__restrict__ dst, const T *__restrict__ w,
     const T *__restrict__ gy, const T *__restrict__ probs, T *__restrict__ gw,
     typename Acc<T>::type *__restrict__ partial, T *__restrict__ gx, T *__restrict__ overflow, int64_t steps, int chunk,
-    int64_t in_dim, int64_t out_dim, int64_t ncols, typename Acc<T>::type scale, int64_t gdiv, LowerLayer<T> low,
+    int64_t in_dim, int64_t out_dim, int64_t batch, typename Acc<T>::type scale, int64_t gdiv, LowerLayer<T> low,
     bool w32) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     constexpr bool RECOMPUTE = LOWER == 2;
     constexpr int LCPL = LOWER ? CPL : 1;                       // registers for lower rows only where they are used
     const int wave = dl_wave_in_block();
@@ -767,28 +792,25 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const int64_t s0 = ((int64_t) blockIdx.x * 4 + wave) * chunk;
     if (s0 >= steps) return;
     const int64_t s1 = s0 + chunk < steps ? s0 + chunk : steps;
-    const P *xv = reinterpret_cast<const P *>(x);
-    const P *gv = reinterpret_cast<const P *>(gy);
-    const P *lx = reinterpret_cast<const P *>(low.x);
     const int64_t col0 = (int64_t) blockIdx.y * (CPL * DL_WAVE);   // this wave's segment of the rows
     const int gate = lane & 15;
     P zero;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) zero.v[e] = down<T, C>((C) 0);
 
-    auto load_row = [&](const P *base, int64_t row, bool valid, P *out) {
+    auto load_row = [&](const T *base, int64_t row, bool valid, P *out) {
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
             const int64_t col = col0 + lane + q * DL_WAVE;
-            out[q] = (valid && col < ncols) ? base[row * ncols + col] : zero;
+            out[q] = (valid && col < ncols) ? row_vec<P, VEC, RAG>(base, row, batch, ncols, col) : zero;
         }
     };
     // the two input rows of neuron v of the layer below (v wave-uniform)
     auto lower_rows = [&](int64_t v, bool valid, P *la, P *lb) {
         if constexpr (LOWER != 0) {
             const int64_t r = valid ? v : 0;
-            load_row(lx, low.a[r], valid, la);
-            load_row(lx, low.b[r], valid, lb);
+            load_row(low.x, low.a[r], valid, la);
+            load_row(low.x, low.b[r], valid, lb);
         }
     };
     // row v of x as the lower layer's forward kernel stored it: lane `gate` of every 16-lane row holds the
@@ -813,9 +835,10 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
             C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
 #pragma unroll
             for (int q = 0; q < CPL; ++q) {
+                const int dup = vec_dup<VEC, RAG>(col0 + lane + q * DL_WAVE, batch);
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
-                    const C g = up<T>(down<T, C>(val[q][e] * scale));
+                    const C g = own_part<RAG>(up<T>(down<T, C>(val[q][e] * scale)), e, dup);
                     const C av = up<T>(la[q].v[e]), bv = up<T>(lb[q].v[e]);
                     const C ga = g * av, gna = g - ga;
                     const C t11 = ga * bv, t01 = gna * bv;
@@ -829,15 +852,15 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
             store_grad_w<T>(lane, true, row, s00, s01, s10, s11, low.probs, low.gw);
             return;
         }
-        P *base = row < in_dim ? reinterpret_cast<P *>(gx) + (int64_t) row * ncols
-                               : reinterpret_cast<P *>(overflow) + ((int64_t) row - in_dim) * ncols;
+        T *base = row < in_dim ? gx : overflow;
+        const int64_t at_row = row < in_dim ? row : (int64_t) row - in_dim;
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
             const int64_t col = col0 + lane + q * DL_WAVE;
             P r;
 #pragma unroll
             for (int e = 0; e < VEC; ++e) r.v[e] = down<T, C>(val[q][e] * scale);
-            if (col < ncols) base[col] = r;
+            if (col < ncols) row_vec<P, VEC, RAG>(base, at_row, batch, ncols, col) = r;
         }
     };
 
@@ -850,7 +873,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
         lower_rows(v0, true, pla, plb);
         lower_forward(pla, plb, up<T>(low.w[v0 * 16 + gate]), prev);
     } else {
-        load_row(xv, verts[s0], true, prev);
+        load_row(x, verts[s0], true, prev);
     }
 #pragma unroll
     for (int q = 0; q < CPL; ++q)
@@ -866,9 +889,9 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
             lower_rows(vb, true, ba, bb);
             lower_forward(ba, bb, up<T>(low.w[vb * 16 + gate]), before);
         } else {
-            load_row(xv, verts[s0 - 1], true, before);
+            load_row(x, verts[s0 - 1], true, before);
         }
-        load_row(gv, grad_row(n, gdiv), true, g);
+        load_row(gy, grad_row(n, gdiv), true, g);
         const Corners<C> k = corners<T>(w, n, w32);
         const C d0 = k.p01 - k.p00, dd = (k.p11 - k.p10) - d0, da = k.p10 - k.p00;
         const C kv = f ? da : d0;
@@ -899,13 +922,13 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
             lower_rows(v, true, la, lb);
             lprob = up<T>(low.w[(int64_t) v * 16 + gate]);
         } else {
-            load_row(xv, v, true, row);
+            load_row(x, v, true, row);
             if constexpr (LOWER == 1) {
                 const int32_t d = __builtin_amdgcn_readlane(sch_d, i);
                 lower_rows(d, d >= 0 && d < in_dim, la, lb);
             }
         }
-        load_row(gv, grad_row(nn, gdiv), valid, grad);
+        load_row(gy, grad_row(nn, gdiv), valid, grad);
         prob = wload<T>(w, nn * 16 + gate, w32);
     };
     P cur[CPL], g[CPL], la[LCPL], lb[LCPL];
@@ -931,11 +954,13 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
         C out[CPL][VEC];
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
+            const int dup = vec_dup<VEC, RAG>(col0 + lane + q * DL_WAVE, batch);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]), gg = up<T>(g[q].v[e]);
                 const C av = f ? u1 : u0, bv = f ? u0 : u1;
-                const C ga = gg * av, gna = gg - ga;
+                const C gs = own_part<RAG>(gg, e, dup);
+                const C ga = gs * av, gna = gs - ga;
                 const C t11 = ga * bv, t01 = gna * bv;
                 s11 += t11;
                 s10 += ga - t11;
@@ -992,60 +1017,60 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
 // fix_vertex[i] is the sum, in slot order, of overflow rows [fix_start[i], fix_start[i + 1])
 // (no rows: the input feeds no neuron and its gradient is zero).
 // compact: row i of gx instead of row fix_vertex[i] (gx then has n_fix rows only).
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_fix_kernel(const T *__restrict__ overflow,
                                                                 const int32_t *__restrict__ fix_vertex,
                                                                 const int32_t *__restrict__ fix_start,
-                                                                T *__restrict__ gx, int64_t n_fix, int64_t ncols,
+                                                                T *__restrict__ gx, int64_t n_fix, int64_t batch,
                                                                 bool compact) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t i = (int64_t) blockIdx.x * 4 + wave;
     if (i >= n_fix) return;
     const int64_t v = compact ? i : (int64_t) fix_vertex[i];
     const int32_t r0 = fix_start[i], r1 = fix_start[i + 1];
-    const P *ov = reinterpret_cast<const P *>(overflow);
-    P *out = reinterpret_cast<P *>(gx);
     for (int64_t col = (int64_t) blockIdx.y * DL_WAVE + lane; col < ncols; col += (int64_t) gridDim.y * DL_WAVE) {
         C acc[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc[e] = (C) 0;
         for (int32_t r = r0; r < r1; ++r) {
-            const P part = ov[(int64_t) r * ncols + col];
+            const P part = row_vec<P, VEC, RAG>(overflow, (int64_t) r, batch, ncols, col);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] += up<T>(part.v[e]);
         }
         P res;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) res.v[e] = down<T, C>(acc[e]);
-        out[v * ncols + col] = res;
+        row_vec<P, VEC, RAG>(gx, v, batch, ncols, col) = res;
     }
 }
 
 // backward_w of the layer below for the few vertices whose grad_x row backward_fix_kernel finished:
 // neuron list[i] of that layer, its grad_y row = row i of `rows`.  One wave per neuron, the sums in
 // the order of backward_w_kernel.
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_w_rows_kernel(LowerLayer<T> low, const int32_t *__restrict__ list,
                                                                    const T *__restrict__ rows, int64_t n_list,
-                                                                   int64_t ncols) {
+                                                                   int64_t batch) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int lane = dl_lane();
     const int64_t i = (int64_t) blockIdx.x * 4 + dl_wave_in_block();
     if (i >= n_list) return;
     const int64_t n = list[i];
-    const P *xv = reinterpret_cast<const P *>(low.x);
-    const P *gv = reinterpret_cast<const P *>(rows) + i * ncols;
     const int64_t ia = low.a[n], ib = low.b[n];
     C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
     for (int64_t col = lane; col < ncols; col += DL_WAVE) {
-        const P va = xv[ia * ncols + col], vb = xv[ib * ncols + col], vg = gv[col];
+        const int dup = vec_dup<VEC, RAG>(col, batch);
+        const P va = row_vec<P, VEC, RAG>(low.x, ia, batch, ncols, col), vb = row_vec<P, VEC, RAG>(low.x, ib, batch, ncols, col);
+        const P vg = row_vec<P, VEC, RAG>(rows, i, batch, ncols, col);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            const C av = up<T>(va.v[e]), bv = up<T>(vb.v[e]), g = up<T>(vg.v[e]);
+            const C av = up<T>(va.v[e]), bv = up<T>(vb.v[e]), g = own_part<RAG>(up<T>(vg.v[e]), e, dup);
             const C ga = g * av, gna = g - ga;
             const C t11 = ga * bv, t01 = gna * bv;
             s11 += t11;
@@ -1089,6 +1114,18 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_w_finish_kernel(const typen
 
 template <typename T> struct Vec16 { static constexpr int n = 16 / (int) sizeof(T); };
 
+// How the rows of a call are read and written: whole aligned 16-byte vectors, vectors of that size of which the last
+// overlaps the one before it (RAG kernels), or one element per lane where a row is shorter than a vector.
+enum class Rows { whole, ragged, single };
+
+template <typename T> Rows rows_kind(int64_t batch, const void *p0, const void *p1 = nullptr, const void *p2 = nullptr,
+                                     const void *p3 = nullptr) {
+    constexpr int V = Vec16<T>::n;
+    if (batch % V == 0 && dl_aligned(p0, 16) && dl_aligned(p1, 16) && dl_aligned(p2, 16) && dl_aligned(p3, 16))
+        return Rows::whole;
+    return batch >= V ? Rows::ragged : Rows::single;
+}
+
 unsigned col_tiles(int64_t ncols) {
     int64_t t = dl_ceil_div(ncols, DL_WAVE);
     return (unsigned) (t > 65535 ? 65535 : t);
@@ -1101,14 +1138,15 @@ int forward_t(const void *x, const int64_t *a, const int64_t *b, const void *w, 
     const int64_t blocks = dl_ceil_div(out_dim, 4 * NPW);
     if (out_dim > 0x7fffffffLL) return DL_ERR_TOO_LARGE;     // neuron ids travel as int32 inside the kernel
     constexpr int V = Vec16<T>::n;
-    if (batch % V == 0 && dl_aligned(x, 16) && dl_aligned(y, 16)) {
-        DL_LAUNCH((forward_kernel<T, V, NPW, LOGITS>), dim3((unsigned) blocks, col_tiles(batch / V)),
-                           dim3(DL_BLOCK), 0, s, (const T *) x, a, b, (const T *) w, (T *) y, (T *) probs, out_dim,
-                           batch / V, w32);
-    } else {
-        DL_LAUNCH((forward_kernel<T, 1, NPW, LOGITS>), dim3((unsigned) blocks, col_tiles(batch)), dim3(DL_BLOCK),
-                           0, s, (const T *) x, a, b, (const T *) w, (T *) y, (T *) probs, out_dim, batch, w32);
-    }
+    const Rows kind = rows_kind<T>(batch, x, y);
+    const dim3 grid((unsigned) blocks, col_tiles(kind == Rows::single ? batch : dl_ceil_div(batch, V)));
+#define DL_LAUNCH_FORWARD(VV, RAG)                                                                                       \
+    DL_LAUNCH((forward_kernel<T, VV, NPW, LOGITS, RAG>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, a, b, (const T *) w, \
+              (T *) y, (T *) probs, out_dim, batch, w32)
+    if (kind == Rows::whole) DL_LAUNCH_FORWARD(V, false);
+    else if (kind == Rows::ragged) DL_LAUNCH_FORWARD(V, true);
+    else DL_LAUNCH_FORWARD(1, false);
+#undef DL_LAUNCH_FORWARD
     return dl_launch_status();
 }
 
@@ -1118,23 +1156,21 @@ int backward_w_t(const void *x, const int64_t *a, const int64_t *b, const void *
     constexpr int NPW = 2;       // neurons per wave when the workgroup's waves split a neuron's batch
     constexpr int NPW1 = 2;      // ... when a wave owns whole rows: short rows, more neurons' loads in flight per wave
     constexpr int V = Vec16<T>::n;
-    const bool vec = batch % V == 0 && dl_aligned(x, 16) && dl_aligned(gy, 16);
-    const int64_t ncols = vec ? batch / V : batch;
+    const Rows kind = rows_kind<T>(batch, x, gy);
+    const int64_t ncols = kind == Rows::single ? batch : dl_ceil_div(batch, V);
     // Split one neuron's batch over the four waves once every wave still gets whole segments.
     const bool split = ncols >= 8 * DL_WAVE;
     const int64_t blocks = split ? dl_ceil_div(out_dim, NPW) : dl_ceil_div(out_dim, 4 * NPW1);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-    const dim3 grid((unsigned) blocks), block(DL_BLOCK);
-    const T *xp = (const T *) x, *gp = (const T *) gy, *pp = (const T *) probs;
-    T *wp = (T *) gw;
-    if (vec && split)
-        DL_LAUNCH((backward_w_kernel<T, V, NPW, 4>), grid, block, 0, s, xp, a, b, gp, pp, wp, out_dim, ncols, gdiv, w32);
-    else if (vec)
-        DL_LAUNCH((backward_w_kernel<T, V, NPW1, 1>), grid, block, 0, s, xp, a, b, gp, pp, wp, out_dim, ncols, gdiv, w32);
-    else if (split)
-        DL_LAUNCH((backward_w_kernel<T, 1, NPW, 4>), grid, block, 0, s, xp, a, b, gp, pp, wp, out_dim, ncols, gdiv, w32);
-    else
-        DL_LAUNCH((backward_w_kernel<T, 1, NPW1, 1>), grid, block, 0, s, xp, a, b, gp, pp, wp, out_dim, ncols, gdiv, w32);
+#define DL_LAUNCH_BACKWARD_W(VV, N, WPN, RAG)                                                                          \
+    DL_LAUNCH((backward_w_kernel<T, VV, N, WPN, RAG>), dim3((unsigned) blocks), dim3(DL_BLOCK), 0, s, (const T *) x, a, \
+              b, (const T *) gy, (const T *) probs, (T *) gw, out_dim, batch, gdiv, w32)
+    if (kind == Rows::whole && split) DL_LAUNCH_BACKWARD_W(V, NPW, 4, false);
+    else if (kind == Rows::whole) DL_LAUNCH_BACKWARD_W(V, NPW1, 1, false);
+    else if (kind == Rows::ragged && split) DL_LAUNCH_BACKWARD_W(V, NPW, 4, true);
+    else if (kind == Rows::ragged) DL_LAUNCH_BACKWARD_W(V, NPW1, 1, true);
+    else DL_LAUNCH_BACKWARD_W(1, NPW1, 1, false);
+#undef DL_LAUNCH_BACKWARD_W
     return dl_launch_status();
 }
 
@@ -1146,15 +1182,15 @@ int backward_x_t(const void *x, const int64_t *a, const int64_t *b, const void *
     constexpr int V = Vec16<T>::n;
     const int64_t blocks = dl_ceil_div(in_dim, 4);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-    if (batch % V == 0 && dl_aligned(x, 16) && dl_aligned(gy, 16) && dl_aligned(gx, 16)) {
-        DL_LAUNCH((backward_x_kernel<T, V>), dim3((unsigned) blocks, col_tiles(batch / V)), dim3(DL_BLOCK), 0, s,
-                           (const T *) x, a, b, (const T *) w, (const T *) gy, start, idx, (T *) gx, in_dim, batch / V,
-                           (C) scale, gdiv, w32);
-    } else {
-        DL_LAUNCH((backward_x_kernel<T, 1>), dim3((unsigned) blocks, col_tiles(batch)), dim3(DL_BLOCK), 0, s,
-                           (const T *) x, a, b, (const T *) w, (const T *) gy, start, idx, (T *) gx, in_dim, batch,
-                           (C) scale, gdiv, w32);
-    }
+    const Rows kind = rows_kind<T>(batch, x, gy, gx);
+    const dim3 grid((unsigned) blocks, col_tiles(kind == Rows::single ? batch : dl_ceil_div(batch, V)));
+#define DL_LAUNCH_BACKWARD_X(VV, RAG)                                                                                    \
+    DL_LAUNCH((backward_x_kernel<T, VV, RAG>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, a, b, (const T *) w,          \
+              (const T *) gy, start, idx, (T *) gx, in_dim, batch, (C) scale, gdiv, w32)
+    if (kind == Rows::whole) DL_LAUNCH_BACKWARD_X(V, false);
+    else if (kind == Rows::ragged) DL_LAUNCH_BACKWARD_X(V, true);
+    else DL_LAUNCH_BACKWARD_X(1, false);
+#undef DL_LAUNCH_BACKWARD_X
     return dl_launch_status();
 }
 
@@ -1166,33 +1202,37 @@ int backward_x_t(const void *x, const int64_t *a, const int64_t *b, const void *
 // class block over the rows (lanes along the batch, the workgroup's four waves interleave
 // rows and combine through LDS) into partial[s, c, r]; pass 2 adds the partials in order.
 // ------------------------------------------------------------------------------------------
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void group_sum_partial_kernel(const T *__restrict__ x,
                                                                      typename Acc<T>::type *__restrict__ partial,
-                                                                     int64_t per_class, int64_t ncols, int64_t k,
+                                                                     int64_t per_class, int64_t batch, int64_t k,
                                                                      int64_t rows_per_split) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     __shared__ C lds[4][DL_WAVE * VEC];
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t col = (int64_t) blockIdx.x * DL_WAVE + lane;
     const int64_t cls = blockIdx.y, split = blockIdx.z;
+    const int64_t at = col < ncols ? vec_at<VEC, RAG>(col, batch) : 0;
     int64_t r0 = split * rows_per_split, r1 = r0 + rows_per_split;
     if (r1 > per_class) r1 = per_class;
     C acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = (C) 0;
     if (col < ncols) {
-        const P *xv = reinterpret_cast<const P *>(x) + (cls * per_class) * ncols + col;
+        const T *xc = x + (cls * per_class) * batch;
         int64_t r = r0 + wave;
         for (; r + 12 < r1; r += 16) {      // four independent row loads in flight per wave
-            const P v0 = xv[r * ncols], v1 = xv[(r + 4) * ncols], v2 = xv[(r + 8) * ncols], v3 = xv[(r + 12) * ncols];
+            P v[4];
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] += (up<T>(v0.v[e]) + up<T>(v1.v[e])) + (up<T>(v2.v[e]) + up<T>(v3.v[e]));
+            for (int i = 0; i < 4; ++i) v[i] = row_vec<P, VEC, RAG>(xc, r + 4 * i, batch, ncols, col);
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) acc[e] += (up<T>(v[0].v[e]) + up<T>(v[1].v[e])) + (up<T>(v[2].v[e]) + up<T>(v[3].v[e]));
         }
         for (; r < r1; r += 4) {
-            const P v = xv[r * ncols];
+            const P v = row_vec<P, VEC, RAG>(xc, r, batch, ncols, col);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] += up<T>(v.v[e]);
         }
@@ -1205,7 +1245,7 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_partial_kernel(const T *__
         for (int e = 0; e < VEC; ++e) {
             const int i = lane * VEC + e;
             const C sum = (lds[0][i] + lds[1][i]) + (lds[2][i] + lds[3][i]);
-            partial[((int64_t) split * k + cls) * (ncols * VEC) + col * VEC + e] = sum;
+            partial[((int64_t) split * k + cls) * batch + at + e] = sum;
         }
     }
 }
@@ -1216,15 +1256,16 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_partial_kernel(const T *__
 // layout as group_sum_partial_kernel; a wave takes four consecutive neurons at a time (their
 // corner coefficients are computed together), the workgroup's waves interleave groups of four.
 // LOGITS: `w` holds logits; the probabilities go to `probs` (column tile 0 only).
-template <typename T, int VEC, bool LOGITS>
+template <typename T, int VEC, bool LOGITS, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__restrict__ x, const int64_t *__restrict__ a,
                                                                      const int64_t *__restrict__ b, const T *__restrict__ w,
                                                                      T *__restrict__ probs,
                                                                      typename Acc<T>::type *__restrict__ partial,
-                                                                     int64_t per_class, int64_t ncols, int64_t k,
+                                                                     int64_t per_class, int64_t batch, int64_t k,
                                                                      int64_t rows_per_split) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     __shared__ C lds[4][DL_WAVE * VEC];
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
@@ -1233,7 +1274,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
     const int64_t cls = blockIdx.y, split = blockIdx.z;
     int64_t r0 = split * rows_per_split, r1 = r0 + rows_per_split;
     if (r1 > per_class) r1 = per_class;
-    const P *xv = reinterpret_cast<const P *>(x) + (live ? col : 0);
+    const int64_t cl = live ? col : 0;
     C acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = (C) 0;
@@ -1253,8 +1294,8 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
         P va[4], vb[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            va[j] = xv[ia[j] * ncols];
-            vb[j] = xv[ib[j] * ncols];
+            va[j] = row_vec<P, VEC, RAG>(x, ia[j], batch, ncols, cl);
+            vb[j] = row_vec<P, VEC, RAG>(x, ib[j], batch, ncols, cl);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1271,11 +1312,12 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
     for (int e = 0; e < VEC; ++e) lds[wave][lane * VEC + e] = acc[e];
     __syncthreads();
     if (wave == 0 && live) {
+        const int64_t at = vec_at<VEC, RAG>(col, batch);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             const int i = lane * VEC + e;
             const C sum = (lds[0][i] + lds[1][i]) + (lds[2][i] + lds[3][i]);
-            partial[((int64_t) split * k + cls) * (ncols * VEC) + col * VEC + e] = sum;
+            partial[((int64_t) split * k + cls) * batch + at + e] = sum;
         }
     }
 }
@@ -1301,30 +1343,31 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typena
         y[r * k + c] = down<T, C>(((lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane])) * inv_tau);
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void group_sum_backward_kernel(const T *__restrict__ g, T *__restrict__ gx,
                                                                       int64_t out_dim, int64_t per_class,
-                                                                      int64_t ncols, int64_t k,
+                                                                      int64_t batch, int64_t k,
                                                                       typename Acc<T>::type inv_tau) {
     typedef typename Acc<T>::type C;
-    typedef Pack<T, VEC> P;
+    typedef Pack<T, VEC, RAG> P;
+    const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t col = (int64_t) blockIdx.x * DL_WAVE + lane;
     if (col >= ncols) return;
+    const int64_t at = vec_at<VEC, RAG>(col, batch);
     constexpr int ROWS = 16;                                              // rows per wave
     const int64_t n0 = ((int64_t) blockIdx.y * 4 + wave) * ROWS;
-    P *ov = reinterpret_cast<P *>(gx);
     int64_t cached_cls = -1;
     P val;
     for (int64_t n = n0; n < n0 + ROWS && n < out_dim; ++n) {
         const int64_t cls = n / per_class;
         if (cls != cached_cls) {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) val.v[e] = down<T, C>(up<T>(g[(col * VEC + e) * k + cls]) * inv_tau);
+            for (int e = 0; e < VEC; ++e) val.v[e] = down<T, C>(up<T>(g[(at + e) * k + cls]) * inv_tau);
             cached_cls = cls;
         }
-        ov[n * ncols + col] = val;
+        row_vec<P, VEC, RAG>(gx, n, batch, ncols, col) = val;
     }
 }
 
@@ -1335,17 +1378,17 @@ int group_sum_forward_t(const void *x, void *y, void *workspace, int64_t out_dim
     constexpr int V = Vec16<T>::n;
     const int64_t per_class = out_dim / k;
     const int64_t rows_per_split = dl_ceil_div(per_class, splits);
-    const bool vec = batch % V == 0 && dl_aligned(x, 16);
-    const int64_t ncols = vec ? batch / V : batch;
-    const int64_t gx = dl_ceil_div(ncols, DL_WAVE);
+    const Rows kind = rows_kind<T>(batch, x);
+    const int64_t gx = dl_ceil_div(kind == Rows::single ? batch : dl_ceil_div(batch, V), DL_WAVE);
     if (gx > 0x7fffffffLL || k > 65535) return DL_ERR_TOO_LARGE;
     const dim3 grid((unsigned) gx, (unsigned) k, (unsigned) splits);
-    if (vec)
-        DL_LAUNCH((group_sum_partial_kernel<T, V>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, (C *) workspace,
-                           per_class, ncols, k, rows_per_split);
-    else
-        DL_LAUNCH((group_sum_partial_kernel<T, 1>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, (C *) workspace,
-                           per_class, ncols, k, rows_per_split);
+#define DL_LAUNCH_PARTIAL(VV, RAG)                                                                                  \
+    DL_LAUNCH((group_sum_partial_kernel<T, VV, RAG>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, (C *) workspace, \
+              per_class, batch, k, rows_per_split)
+    if (kind == Rows::whole) DL_LAUNCH_PARTIAL(V, false);
+    else if (kind == Rows::ragged) DL_LAUNCH_PARTIAL(V, true);
+    else DL_LAUNCH_PARTIAL(1, false);
+#undef DL_LAUNCH_PARTIAL
     int st = dl_launch_status();
     if (st != DL_OK) return st;
     const int64_t blocks = dl_ceil_div(batch, DL_WAVE);
@@ -1359,17 +1402,17 @@ template <typename T>
 int group_sum_backward_t(const void *g, void *gx, int64_t out_dim, int64_t batch, int64_t k, double tau, hipStream_t s) {
     typedef typename Acc<T>::type C;
     constexpr int V = Vec16<T>::n;
-    const bool vec = batch % V == 0 && dl_aligned(gx, 16);
-    const int64_t ncols = vec ? batch / V : batch;
-    const int64_t gxd = dl_ceil_div(ncols, DL_WAVE), gyd = dl_ceil_div(out_dim, 64);
+    const Rows kind = rows_kind<T>(batch, gx);
+    const int64_t gxd = dl_ceil_div(kind == Rows::single ? batch : dl_ceil_div(batch, V), DL_WAVE), gyd = dl_ceil_div(out_dim, 64);
     if (gxd > 0x7fffffffLL || gyd > 65535) return DL_ERR_TOO_LARGE;
     const dim3 grid((unsigned) gxd, (unsigned) gyd);
-    if (vec)
-        DL_LAUNCH((group_sum_backward_kernel<T, V>), grid, dim3(DL_BLOCK), 0, s, (const T *) g, (T *) gx, out_dim,
-                           out_dim / k, ncols, k, (C) (1.0 / tau));
-    else
-        DL_LAUNCH((group_sum_backward_kernel<T, 1>), grid, dim3(DL_BLOCK), 0, s, (const T *) g, (T *) gx, out_dim,
-                           out_dim / k, ncols, k, (C) (1.0 / tau));
+#define DL_LAUNCH_BROADCAST(VV, RAG)                                                                                    \
+    DL_LAUNCH((group_sum_backward_kernel<T, VV, RAG>), grid, dim3(DL_BLOCK), 0, s, (const T *) g, (T *) gx, out_dim,   \
+              out_dim / k, batch, k, (C) (1.0 / tau))
+    if (kind == Rows::whole) DL_LAUNCH_BROADCAST(V, false);
+    else if (kind == Rows::ragged) DL_LAUNCH_BROADCAST(V, true);
+    else DL_LAUNCH_BROADCAST(1, false);
+#undef DL_LAUNCH_BROADCAST
     return dl_launch_status();
 }
 
@@ -1383,18 +1426,22 @@ int forward_group_sum_t(const void *x, const int64_t *a, const int64_t *b, const
     const int splits = group_sum_splits(out_dim, batch, k);
     const int64_t per_class = out_dim / k;
     const int64_t rows_per_split = dl_ceil_div(dl_ceil_div(per_class, splits), 16) * 16;     // whole groups of four per wave
-    const bool vec = batch % V == 0 && dl_aligned(x, 16);
-    const int64_t ncols = vec ? batch / V : batch;
-    const int64_t gx = dl_ceil_div(ncols, DL_WAVE);
+    const Rows kind = rows_kind<T>(batch, x);
+    const int64_t gx = dl_ceil_div(kind == Rows::single ? batch : dl_ceil_div(batch, V), DL_WAVE);
     if (gx > 0x7fffffffLL || k > 65535 || out_dim > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     const dim3 grid((unsigned) gx, (unsigned) k, (unsigned) splits);
     const T *xp = (const T *) x, *wp = (const T *) w;
-#define DL_LAUNCH_FGS(VV, LG)                                                                                               \
-    DL_LAUNCH((forward_group_sum_kernel<T, VV, LG>), grid, dim3(DL_BLOCK), 0, s, xp, a, b, wp, (T *) probs, (C *) workspace, \
-              per_class, ncols, k, rows_per_split)
-    if (vec && probs) DL_LAUNCH_FGS(V, true);
-    else if (vec) DL_LAUNCH_FGS(V, false);
-    else if (probs) DL_LAUNCH_FGS(1, true);
+#define DL_LAUNCH_FGS(VV, RAG)                                                                                              \
+    do {                                                                                                                    \
+        if (probs)                                                                                                          \
+            DL_LAUNCH((forward_group_sum_kernel<T, VV, true, RAG>), grid, dim3(DL_BLOCK), 0, s, xp, a, b, wp, (T *) probs,  \
+                      (C *) workspace, per_class, batch, k, rows_per_split);                                                \
+        else                                                                                                                \
+            DL_LAUNCH((forward_group_sum_kernel<T, VV, false, RAG>), grid, dim3(DL_BLOCK), 0, s, xp, a, b, wp, (T *) probs, \
+                      (C *) workspace, per_class, batch, k, rows_per_split);                                                \
+    } while (0)
+    if (kind == Rows::whole) DL_LAUNCH_FGS(V, false);
+    else if (kind == Rows::ragged) DL_LAUNCH_FGS(V, true);
     else DL_LAUNCH_FGS(1, false);
 #undef DL_LAUNCH_FGS
     int st = dl_launch_status();
@@ -1438,52 +1485,70 @@ template <typename T, bool LOGITS>
 int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps,
                     const void *w, void *y, void *probs, int64_t batch, hipStream_t s, bool w32 = false) {
     constexpr int V = Vec16<T>::n;
-    if (batch % V != 0 || !dl_aligned(x, 16) || !dl_aligned(y, 16)) return DL_ERR_TOO_LARGE;
-    const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = batch / V;
+    const Rows kind = rows_kind<T>(batch, x, y);
+    if (kind == Rows::single) return DL_ERR_TOO_LARGE;
+    const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
     const T *xp = (const T *) x, *wp = (const T *) w;
+    const dim3 block(DL_BLOCK);
     if (ncols > DL_FWD_ROWS_MIN && ncols <= DL_ROWS_MAX_VECTORS) {
         // rows of 2 KB and more: a wave takes whole rows, or segments of 4 KB
         const int segments = row_segments(ncols);
         const int chunk = chain_chunk(steps * segments);
         const int64_t blocks = dl_ceil_div(dl_ceil_div(steps, chunk), 4);
         if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-        const dim3 grid((unsigned) blocks, (unsigned) segments), block(DL_BLOCK);
-        if (ncols <= 2 * DL_WAVE)
-            DL_LAUNCH((forward_chain_rows_kernel<T, V, 2, LOGITS>), grid, block, 0, s, xp, verts, neuron, flip, wp,
-                               (T *) y, (T *) probs, steps, chunk, ncols, w32);
-        else
-            DL_LAUNCH((forward_chain_rows_kernel<T, V, 4, LOGITS>), grid, block, 0, s, xp, verts, neuron, flip, wp,
-                               (T *) y, (T *) probs, steps, chunk, ncols, w32);
+        const dim3 grid((unsigned) blocks, (unsigned) segments);
+#define DL_LAUNCH_ROWS(CPL, RAG)                                                                                        \
+    DL_LAUNCH((forward_chain_rows_kernel<T, V, CPL, LOGITS, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, (T *) y, \
+              (T *) probs, steps, chunk, batch, w32)
+        if (ncols <= 2 * DL_WAVE) {
+            if (kind == Rows::whole) DL_LAUNCH_ROWS(2, false);
+            else DL_LAUNCH_ROWS(2, true);
+        } else {
+            if (kind == Rows::whole) DL_LAUNCH_ROWS(4, false);
+            else DL_LAUNCH_ROWS(4, true);
+        }
+#undef DL_LAUNCH_ROWS
         return dl_launch_status();
     }
     const int64_t blocks = dl_ceil_div(nchunks, 4);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-    if (V >= 2 && ncols <= DL_WAVE / 2) {
-        // short rows: 8-byte vectors put a row on all 64 lanes instead of half of them
-        constexpr int H = V >= 2 ? V / 2 : 1;
-        DL_LAUNCH((forward_chain_kernel<T, H, DL_TRAIN_CHUNK, LOGITS>), dim3((unsigned) blocks, 1), dim3(DL_BLOCK), 0, s, xp,
-                  verts, neuron, flip, wp, (T *) y, (T *) probs, nchunks, 2 * ncols, w32);
-        return dl_launch_status();
+    constexpr int H = V >= 2 ? V / 2 : 1;
+    // short rows: 8-byte vectors put a row on all 64 lanes instead of half of them
+    const bool half = V >= 2 && ncols <= DL_WAVE / 2;
+    const dim3 grid((unsigned) blocks, half ? 1 : col_tiles(ncols));
+#define DL_LAUNCH_CHAIN(VV, RAG)                                                                                       \
+    DL_LAUNCH((forward_chain_kernel<T, VV, DL_TRAIN_CHUNK, LOGITS, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, \
+              (T *) y, (T *) probs, nchunks, batch, w32)
+    if (half) {
+        if (kind == Rows::whole) DL_LAUNCH_CHAIN(H, false);
+        else DL_LAUNCH_CHAIN(H, true);
+    } else {
+        if (kind == Rows::whole) DL_LAUNCH_CHAIN(V, false);
+        else DL_LAUNCH_CHAIN(V, true);
     }
-    DL_LAUNCH((forward_chain_kernel<T, V, DL_TRAIN_CHUNK, LOGITS>), dim3((unsigned) blocks, col_tiles(ncols)),
-                       dim3(DL_BLOCK), 0, s, xp, verts, neuron, flip, wp, (T *) y, (T *) probs, nchunks, ncols, w32);
+#undef DL_LAUNCH_CHAIN
     return dl_launch_status();
 }
 
 template <typename T, bool LOGITS>
 int forward_chain_lower_t(const void *lx, const int64_t *la, const int64_t *lb, const void *lw, void *lprobs,
                           const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps, const void *w,
-                          void *y, void *probs, int64_t batch, hipStream_t s) {
+                          void *y, void *probs, int64_t batch, bool any_rows, hipStream_t s) {
     constexpr int V = Vec16<T>::n;
-    if (batch % V != 0 || !dl_aligned(lx, 16) || !dl_aligned(y, 16)) return DL_ERR_TOO_LARGE;
-    const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = batch / V;
+    const Rows kind = rows_kind<T>(batch, lx, y);
+    if (kind != Rows::whole && !(any_rows && kind == Rows::ragged)) return DL_ERR_TOO_LARGE;
+    const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
     if (ncols > DL_FWD_ROWS_MIN) return DL_ERR_TOO_LARGE;        // rows of at most 2 KB
     const int64_t blocks = dl_ceil_div(nchunks, 4);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     // one wave takes every column tile of its chunk (at most two): the corner coefficients are formed once
-    DL_LAUNCH((forward_chain_lower_kernel<T, V, DL_TRAIN_CHUNK, LOGITS>), dim3((unsigned) blocks, 1),
-              dim3(DL_BLOCK), 0, s, (const T *) lx, la, lb, (const T *) lw, (T *) lprobs, verts, neuron, flip, (const T *) w,
-              (T *) y, (T *) probs, nchunks, ncols);
+#define DL_LAUNCH_LOWER(RAG)                                                                                            \
+    DL_LAUNCH((forward_chain_lower_kernel<T, V, DL_TRAIN_CHUNK, LOGITS, RAG>), dim3((unsigned) blocks), dim3(DL_BLOCK), 0, \
+              s, (const T *) lx, la, lb, (const T *) lw, (T *) lprobs, verts, neuron, flip, (const T *) w, (T *) y,      \
+              (T *) probs, nchunks, batch)
+    if (kind == Rows::whole) DL_LAUNCH_LOWER(false);
+    else DL_LAUNCH_LOWER(true);
+#undef DL_LAUNCH_LOWER
     return dl_launch_status();
 }
 
@@ -1492,27 +1557,32 @@ int backward_w_chain_t(const void *x, const int32_t *verts, const int32_t *neuro
                        const void *gy, const void *probs, void *gw, int64_t batch, hipStream_t s, int64_t gdiv = 0,
                        bool w32 = false) {
     constexpr int V = Vec16<T>::n;
-    if (batch % V != 0 || !dl_aligned(x, 16) || !dl_aligned(gy, 16)) return DL_ERR_TOO_LARGE;
-    const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = batch / V;
+    const Rows kind = rows_kind<T>(batch, x, gy);
+    if (kind == Rows::single) return DL_ERR_TOO_LARGE;
+    const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
     const int64_t blocks = dl_ceil_div(nchunks, 4);
     if (blocks > 0x7fffffffLL || ncols > 4 * DL_WAVE) return DL_ERR_TOO_LARGE;   // a lane holds at most 4 vectors of a row
-    const dim3 grid((unsigned) blocks), block(DL_BLOCK);
-    const T *xp = (const T *) x, *gp = (const T *) gy, *pp = (const T *) probs;
-    if (ncols <= DL_WAVE)
-        DL_LAUNCH((backward_w_chain_kernel<T, V, 1, DL_TRAIN_CHUNK>), grid, block, 0, s, xp, verts, neuron, flip,
-                           gp, pp, (T *) gw, nchunks, ncols, gdiv, w32);
-    else if (ncols <= 2 * DL_WAVE)
-        DL_LAUNCH((backward_w_chain_kernel<T, V, 2, DL_TRAIN_CHUNK>), grid, block, 0, s, xp, verts, neuron, flip,
-                           gp, pp, (T *) gw, nchunks, ncols, gdiv, w32);
-    else
-        DL_LAUNCH((backward_w_chain_kernel<T, V, 4, DL_TRAIN_CHUNK>), grid, block, 0, s, xp, verts, neuron, flip,
-                           gp, pp, (T *) gw, nchunks, ncols, gdiv, w32);
+#define DL_LAUNCH_W_CHAIN(CPL)                                                                                         \
+    do {                                                                                                               \
+        if (kind == Rows::whole)                                                                                       \
+            DL_LAUNCH((backward_w_chain_kernel<T, V, CPL, DL_TRAIN_CHUNK, false>), dim3((unsigned) blocks), dim3(DL_BLOCK), \
+                      0, s, (const T *) x, verts, neuron, flip, (const T *) gy, (const T *) probs, (T *) gw, nchunks,  \
+                      batch, gdiv, w32);                                                                               \
+        else                                                                                                           \
+            DL_LAUNCH((backward_w_chain_kernel<T, V, CPL, DL_TRAIN_CHUNK, true>), dim3((unsigned) blocks), dim3(DL_BLOCK), \
+                      0, s, (const T *) x, verts, neuron, flip, (const T *) gy, (const T *) probs, (T *) gw, nchunks,  \
+                      batch, gdiv, w32);                                                                               \
+    } while (0)
+    if (ncols <= DL_WAVE) DL_LAUNCH_W_CHAIN(1);
+    else if (ncols <= 2 * DL_WAVE) DL_LAUNCH_W_CHAIN(2);
+    else DL_LAUNCH_W_CHAIN(4);
+#undef DL_LAUNCH_W_CHAIN
     return dl_launch_status();
 }
 
 template <typename T> int64_t backward_partial_bytes(int64_t out_dim, int64_t batch) {
     constexpr int V = Vec16<T>::n;
-    const int segments = batch % V == 0 ? row_segments(batch / V) : 1;
+    const int segments = row_segments(dl_ceil_div(batch, V));
     return segments > 1 ? (int64_t) segments * out_dim * 4 * (int64_t) sizeof(typename Acc<T>::type) : 0;
 }
 
@@ -1520,18 +1590,20 @@ template <typename T>
 int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, const int32_t *dst,
                      int64_t steps, const void *w, const void *gy, bool softmax_backward, const int32_t *fix_vertex,
                      const int32_t *fix_start, int64_t n_fix, int64_t overflow_rows, void *gw, void *gx, void *workspace,
-                     int64_t in_dim, int64_t out_dim, int64_t batch, double scale, hipStream_t s, int64_t gdiv = 0,
-                     const LowerLayer<T> *lower = nullptr, bool w32 = false) {
+                     int64_t in_dim, int64_t out_dim, int64_t batch, double scale, bool any_rows, hipStream_t s,
+                     int64_t gdiv = 0, const LowerLayer<T> *lower = nullptr, bool w32 = false) {
     typedef typename Acc<T>::type C;
     constexpr int V = Vec16<T>::n;
-    if (batch % V != 0 || !dl_aligned(x, 16) || !dl_aligned(gy, 16) || !dl_aligned(gx, 16) || !dl_aligned(workspace, 16))
-        return DL_ERR_TOO_LARGE;
+    Rows kind = rows_kind<T>(batch, x, gy, gx, workspace);
+    if (kind == Rows::whole && lower && !dl_aligned(lower->x, 16)) kind = Rows::ragged;
+    if (kind != Rows::whole && !(any_rows && kind == Rows::ragged)) return DL_ERR_TOO_LARGE;
+    if (!dl_aligned(workspace, 16)) return DL_ERR_TOO_LARGE;            // partial sums of whole C values lie at its start
     if (!x && (!lower || !lower->w)) return DL_ERR_INVALID_ARGUMENT;     // x may only be left out for recomputation
-    const int64_t ncols = batch / V;
+    const int64_t ncols = dl_ceil_div(batch, V);
     if (ncols > DL_ROWS_MAX_VECTORS) return DL_ERR_TOO_LARGE;
     const int segments = row_segments(ncols);
     // with `lower`: whole rows per wave only, and gx holds the n_fix rows that finish after the pass
-    if (lower && (segments > 1 || !dl_aligned(lower->x, 16) || w32)) return DL_ERR_TOO_LARGE;
+    if (lower && (segments > 1 || w32)) return DL_ERR_TOO_LARGE;
     const LowerLayer<T> none = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     // workspace: [segments x out x 4 corner sums (only with several segments)] [overflow rows]
     const int64_t partial_bytes = backward_partial_bytes<T>(out_dim, batch);
@@ -1544,29 +1616,31 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
     const dim3 grid((unsigned) blocks, (unsigned) segments), block(DL_BLOCK);
     const T *xp = (const T *) x, *wp = (const T *) w, *gp = (const T *) gy, *pp = softmax_backward ? wp : nullptr;
     constexpr int H = V >= 2 ? V / 2 : 1;
-#define DL_LAUNCH_BACKWARD_CHAIN(VV, CPL, NC)                                                                               \
-    do {                                                                                                                    \
-        if (lower && !x)                                                                                                    \
-            DL_LAUNCH((backward_chain_kernel<T, VV, CPL, 2>), grid, block, 0, s, xp, verts, neuron, flip, dst, wp, gp,     \
-                      pp, (T *) gw, partial, (T *) gx, overflow, steps, chunk, in_dim, out_dim, NC, (C) scale, gdiv, *lower, \
-                      false);                                                                                               \
-        else if (lower)                                                                                                     \
-            DL_LAUNCH((backward_chain_kernel<T, VV, CPL, 1>), grid, block, 0, s, xp, verts, neuron, flip, dst, wp, gp,     \
-                      pp, (T *) gw, partial, (T *) gx, overflow, steps, chunk, in_dim, out_dim, NC, (C) scale, gdiv, *lower, \
-                      false);                                                                                               \
-        else                                                                                                                \
-            DL_LAUNCH((backward_chain_kernel<T, VV, CPL, 0>), grid, block, 0, s, xp, verts, neuron, flip, dst, wp, gp,     \
-                      pp, (T *) gw, partial, (T *) gx, overflow, steps, chunk, in_dim, out_dim, NC, (C) scale, gdiv, none,   \
-                      w32);                                                                                                 \
+#define DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, LOWER, RAG)                                                                 \
+    DL_LAUNCH((backward_chain_kernel<T, VV, CPL, LOWER, RAG>), grid, block, 0, s, xp, verts, neuron, flip, dst, wp, gp, pp, \
+              (T *) gw, partial, (T *) gx, overflow, steps, chunk, in_dim, out_dim, batch, (C) scale, gdiv,             \
+              LOWER ? *lower : none, LOWER ? false : w32)
+#define DL_LAUNCH_BACKWARD_CHAIN(VV, CPL)                                                                                \
+    do {                                                                                                                 \
+        if (kind == Rows::whole) {                                                                                       \
+            if (lower && !x) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, false);                                             \
+            else if (lower) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 1, false);                                              \
+            else DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 0, false);                                                         \
+        } else {                                                                                                         \
+            if (lower && !x) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, true);                                              \
+            else if (lower) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 1, true);                                               \
+            else DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 0, true);                                                          \
+        }                                                                                                                \
     } while (0)
     if (V >= 2 && ncols <= DL_WAVE / 2)
-        DL_LAUNCH_BACKWARD_CHAIN(H, 1, 2 * ncols);   // short rows: 8-byte vectors use all 64 lanes
+        DL_LAUNCH_BACKWARD_CHAIN(H, 1);              // short rows: 8-byte vectors use all 64 lanes
     else if (ncols <= DL_WAVE)
-        DL_LAUNCH_BACKWARD_CHAIN(V, 1, ncols);
+        DL_LAUNCH_BACKWARD_CHAIN(V, 1);
     else if (ncols <= 2 * DL_WAVE)
-        DL_LAUNCH_BACKWARD_CHAIN(V, 2, ncols);
+        DL_LAUNCH_BACKWARD_CHAIN(V, 2);
     else
-        DL_LAUNCH_BACKWARD_CHAIN(V, 4, ncols);
+        DL_LAUNCH_BACKWARD_CHAIN(V, 4);
+#undef DL_LAUNCH_BACKWARD_CHAIN_AS
 #undef DL_LAUNCH_BACKWARD_CHAIN
     int st = dl_launch_status();
     if (st != DL_OK) return st;
@@ -1579,12 +1653,21 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
         if (st != DL_OK) return st;
     }
     if (n_fix == 0) return DL_OK;
-    DL_LAUNCH((backward_fix_kernel<T, V>), dim3((unsigned) fix_blocks, col_tiles(ncols)), block, 0, s,
-              (const T *) overflow, fix_vertex, fix_start, (T *) gx, n_fix, ncols, lower != nullptr);
+    const dim3 fix_grid((unsigned) fix_blocks, col_tiles(ncols));
+    if (kind == Rows::whole)
+        DL_LAUNCH((backward_fix_kernel<T, V, false>), fix_grid, block, 0, s, (const T *) overflow, fix_vertex, fix_start,
+                  (T *) gx, n_fix, batch, lower != nullptr);
+    else
+        DL_LAUNCH((backward_fix_kernel<T, V, true>), fix_grid, block, 0, s, (const T *) overflow, fix_vertex, fix_start,
+                  (T *) gx, n_fix, batch, lower != nullptr);
     st = dl_launch_status();
     if (st != DL_OK || !lower) return st;
-    DL_LAUNCH((backward_w_rows_kernel<T, V>), dim3((unsigned) fix_blocks), block, 0, s, *lower, fix_vertex, (const T *) gx,
-              n_fix, ncols);
+    if (kind == Rows::whole)
+        DL_LAUNCH((backward_w_rows_kernel<T, V, false>), dim3((unsigned) fix_blocks), block, 0, s, *lower, fix_vertex,
+                  (const T *) gx, n_fix, batch);
+    else
+        DL_LAUNCH((backward_w_rows_kernel<T, V, true>), dim3((unsigned) fix_blocks), block, 0, s, *lower, fix_vertex,
+                  (const T *) gx, n_fix, batch);
     return dl_launch_status();
 }
 
@@ -1602,11 +1685,19 @@ bool weights_fp32(int &dtype) {
     return false;
 }
 
+// DL_ROWS_ANY in a dtype code: taken out of it, and returned
+bool takes_any_rows(int &dtype) {
+    const bool any = (dtype & DL_ROWS_ANY) != 0;
+    dtype &= ~DL_ROWS_ANY;
+    return any;
+}
+
 }  // namespace
 
 extern "C" int64_t dl_logic_backward_chained_workspace_bytes(int64_t overflow_rows, int64_t out_dim, int64_t batch,
                                                              int dtype) {
     if (overflow_rows < 0 || out_dim < 0 || batch < 0) return -DL_ERR_INVALID_ARGUMENT;
+    takes_any_rows(dtype);
     weights_fp32(dtype);
     switch (dtype) {
     case DL_F16: return backward_partial_bytes<__half>(out_dim, batch) + overflow_rows * batch * 2;
@@ -1622,7 +1713,7 @@ extern "C" int dl_logic_backward_chained(const void *x, const int32_t *verts, co
                                          int64_t n_fix, int64_t overflow_rows, void *grad_w, void *grad_x,
                                          void *workspace, int64_t in_dim, int64_t out_dim, int64_t batch, double scale,
                                          int dtype, void *stream) {
-    const bool w32 = weights_fp32(dtype);
+    const bool any = takes_any_rows(dtype), w32 = weights_fp32(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim <= 0 || out_dim <= 0 || batch <= 0 || steps < out_dim || n_fix < 0 || n_fix > in_dim || overflow_rows < 0)
         return DL_ERR_INVALID_ARGUMENT;
@@ -1633,14 +1724,14 @@ extern "C" int dl_logic_backward_chained(const void *x, const int32_t *verts, co
     switch (dtype) {
     case DL_F16:
         return backward_chain_t<__half>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, s, 0, nullptr,
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, 0, nullptr,
                                         w32);
     case DL_F32:
         return backward_chain_t<float>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, s);
+                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s);
     default:
         return backward_chain_t<double>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, s, 0, nullptr,
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, 0, nullptr,
                                         w32);
     }
 }
@@ -1653,6 +1744,7 @@ extern "C" int dl_logic_backward_chained_lower(const void *x, const int32_t *ver
                                                const int64_t *a_lower, const int64_t *b_lower, const void *w_lower,
                                                int softmax_backward_lower, void *grad_w_lower, int64_t in_dim,
                                                int64_t out_dim, int64_t batch, double scale, int dtype, void *stream) {
+    const bool any = takes_any_rows(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim <= 0 || out_dim <= 0 || batch <= 0 || steps < out_dim || n_fix < 0 || n_fix > in_dim || overflow_rows < 0)
         return DL_ERR_INVALID_ARGUMENT;
@@ -1670,19 +1762,19 @@ extern "C" int dl_logic_backward_chained_lower(const void *x, const int32_t *ver
         const LowerLayer<__half> low = {(const __half *) x_lower, a_lower, b_lower, (const __half *) w_lower,
                                         softmax_backward_lower ? (const __half *) w_lower : nullptr, (__half *) grad_w_lower};
         return backward_chain_t<__half>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, s, 0, &low);
+                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, s, 0, &low);
     }
     case DL_F32: {
         const LowerLayer<float> low = {(const float *) x_lower, a_lower, b_lower, (const float *) w_lower,
                                        softmax_backward_lower ? (const float *) w_lower : nullptr, (float *) grad_w_lower};
         return backward_chain_t<float>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                       overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, s, 0, &low);
+                                       overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, s, 0, &low);
     }
     default: {
         const LowerLayer<double> low = {(const double *) x_lower, a_lower, b_lower, (const double *) w_lower,
                                         softmax_backward_lower ? (const double *) w_lower : nullptr, (double *) grad_w_lower};
         return backward_chain_t<double>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, s, 0, &low);
+                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, s, 0, &low);
     }
     }
 }
@@ -1716,6 +1808,7 @@ extern "C" int dl_logic_forward_chained_lower(const void *x_lower, const int64_t
                                               const int32_t *neuron, const uint8_t *flip, int64_t steps, const void *w,
                                               void *y, void *probs, int64_t in_dim_lower, int64_t in_dim, int64_t out_dim,
                                               int64_t batch, int dtype, void *stream) {
+    const bool any = takes_any_rows(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim_lower <= 0 || in_dim <= 0 || out_dim < 0 || batch <= 0 || steps < out_dim || steps % DL_TRAIN_CHUNK != 0)
         return DL_ERR_INVALID_ARGUMENT;
@@ -1725,7 +1818,7 @@ extern "C" int dl_logic_forward_chained_lower(const void *x_lower, const int64_t
     hipStream_t s = (hipStream_t) stream;
 #define DL_FCL(TT, LG)                                                                                                  \
     forward_chain_lower_t<TT, LG>(x_lower, a_lower, b_lower, w_lower, probs_lower, verts, neuron, flip, steps, w, y, probs, \
-                                  batch, s)
+                                  batch, any, s)
     if (probs) {
         switch (dtype) {
         case DL_F16: return DL_FCL(__half, true);
@@ -1942,6 +2035,7 @@ extern "C" int dl_logic_backward_chained_grouped(const void *x, const int32_t *v
                                                  void *grad_w, void *grad_x, void *workspace, int64_t in_dim,
                                                  int64_t out_dim, int64_t batch, int64_t k, double scale, int dtype,
                                                  void *stream) {
+    const bool any = takes_any_rows(dtype);
     const int st = grouped_args(in_dim, out_dim, batch, k, dtype);
     if (st != DL_OK) return st;
     if (steps < out_dim || n_fix < 0 || n_fix > in_dim || overflow_rows < 0) return DL_ERR_INVALID_ARGUMENT;
@@ -1953,13 +2047,13 @@ extern "C" int dl_logic_backward_chained_grouped(const void *x, const int32_t *v
     switch (dtype) {
     case DL_F16:
         return backward_chain_t<__half>(x, verts, neuron, flip, dst, steps, w, grad_cls, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, s, per_class);
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, per_class);
     case DL_F32:
         return backward_chain_t<float>(x, verts, neuron, flip, dst, steps, w, grad_cls, sb, fix_vertex, fix_start, n_fix,
-                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, s, per_class);
+                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, per_class);
     default:
         return backward_chain_t<double>(x, verts, neuron, flip, dst, steps, w, grad_cls, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, s, per_class);
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, per_class);
     }
 }
 

@@ -225,7 +225,7 @@ class LogicLayerCudaFunction(torch.autograd.Function):
         grad_w = grad_x = None
         if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is not None:
             # one pass along the schedule yields both gradients
-            both = difflogic_cuda.backward_chained(x, w, grad_y, ctx.schedule, ctx.grad_factor)
+            both = difflogic_cuda.backward_chained(x, w, grad_y, ctx.schedule, ctx.grad_factor, any_rows=True)
             if both is not None:
                 return both[1], None, None, both[0], None, None, None, None
         if ctx.needs_input_grad[0]:
@@ -257,7 +257,7 @@ class LogicLayerLogitsFunction(torch.autograd.Function):
         if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is not None:
             # one pass along the schedule yields both gradients
             both = difflogic_cuda.backward_chained(x, probs, grad_y, ctx.schedule, ctx.grad_factor,
-                                                   softmax_backward=True)
+                                                   softmax_backward=True, any_rows=True)
             if both is not None:
                 return both[1], None, None, both[0], None, None, None, None
         if ctx.needs_input_grad[0]:
@@ -366,7 +366,7 @@ class LogicLayerPairFunction(torch.autograd.Function):
         fused = None
         if (x.dtype in (torch.float32, torch.float64)
                 and x.numel() * x.element_size() <= LogicLayerPairFunction.RECOMPUTE_MAX_INPUT_BYTES):
-            fused = difflogic_cuda.forward_logits_lower(x, a1, b1, l1, l2, schedule2)
+            fused = difflogic_cuda.forward_logits_lower(x, a1, b1, l1, l2, schedule2, any_rows=True)
         if fused is not None:
             y2, probs1, probs2 = fused
             y1 = None
@@ -388,7 +388,7 @@ class LogicLayerPairFunction(torch.autograd.Function):
         g1 = g2 = None
         if want1 and want2:
             both = difflogic_cuda.backward_chained_lower(y1, probs2, grad_y, ctx.schedule2, x, a1, b1, probs1,
-                                                         ctx.grad_factor2, softmax_backward=True)
+                                                         ctx.grad_factor2, softmax_backward=True, any_rows=True)
             if both is not None:
                 g2, g1 = both
                 return None, None, None, g1, None, None, None, g2, None, None, None, None
@@ -397,7 +397,7 @@ class LogicLayerPairFunction(torch.autograd.Function):
             y1 = difflogic_cuda.forward(x, a1, b1, probs1, ctx.schedule1)
         if want1:
             both = difflogic_cuda.backward_chained(y1, probs2, grad_y, ctx.schedule2, ctx.grad_factor2,
-                                                   softmax_backward=True) if want2 else None
+                                                   softmax_backward=True, any_rows=True) if want2 else None
             if both is not None:
                 g2, grad_y1 = both
             else:

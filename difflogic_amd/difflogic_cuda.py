@@ -275,18 +275,19 @@ def backward_logits(x, a, b, grad_y, probs, schedule=None):
     return grad_logits
 
 
-def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False):
+def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, any_rows=False):
     """backward_w (or backward_logits when ``softmax_backward``; ``w`` are then the probabilities
     that forward_logits returned) and backward_x in one pass along ``schedule``.  Returns
     (grad_w [out,16], grad_x [in,B]), or None where the fused pass does not apply (the caller
-    then uses the separate functions).  Not part of the reference's extension."""
+    then uses the separate functions).  ``any_rows``: rows that are not whole 16-byte vectors are taken as well
+    (False: None for them).  Not part of the reference's extension."""
     for t, n in ((x, "x"), (w, "w"), (grad_y, "grad_y")):
         _check_input(t, n)
     if (x.dim() != 2 or grad_y.dim() != 2 or grad_y.shape[1] != x.shape[1] or grad_y.dtype != x.dtype
             or w.shape != (grad_y.shape[0], 16)):
         raise RuntimeError(f"expected x [in,B], w [out,16], grad_y [out,B] of one dtype, got {tuple(x.shape)}, "
                            f"{tuple(w.shape)}, {tuple(grad_y.shape)}")
-    code = _layer_code(x, w, "logic_layer_cuda_backward")
+    code = _layer_code(x, w, "logic_layer_cuda_backward") | (_lib.DL_ROWS_ANY if any_rows else 0)
     dev = _same_device(x, w, grad_y)
     in_dim, batch = x.shape
     out_dim = grad_y.shape[0]
@@ -316,17 +317,17 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False):
     return grad_w, grad_x
 
 
-def forward_logits_lower(x_lower, a_lower, b_lower, logits_lower, logits, schedule):
+def forward_logits_lower(x_lower, a_lower, b_lower, logits_lower, logits, schedule, any_rows=False):
     """``forward_logits(forward_logits(x_lower, ...)[0], a, b, logits, schedule)`` in one kernel that
     recomputes the rows of the intermediate activation instead of writing and reading them
     (``schedule``: the EvalSchedule of the upper layer's (a, b)).  Returns (y [out,B],
     probs_lower [in,16], probs [out,16]) with the values the two calls give, or None where the
-    kernel does not apply (rows longer than 2 KB or not whole 16-byte vectors).  Not part of the
-    reference's extension."""
+    kernel does not apply (rows longer than 2 KB or, without ``any_rows``, not whole 16-byte
+    vectors).  Not part of the reference's extension."""
     for t, n in ((x_lower, "x_lower"), (a_lower, "a_lower"), (b_lower, "b_lower"), (logits_lower, "logits_lower"),
                  (logits, "logits")):
         _check_input(t, n)
-    code = _float_code(x_lower, "logic_layer_cuda_forward")
+    code = _float_code(x_lower, "logic_layer_cuda_forward") | (_lib.DL_ROWS_ANY if any_rows else 0)
     if (x_lower.dim() != 2 or logits_lower.dim() != 2 or logits_lower.shape[1] != 16 or logits.dim() != 2
             or logits.shape[1] != 16 or logits_lower.dtype != x_lower.dtype or logits.dtype != x_lower.dtype
             or x_lower.shape[1] == 0):
@@ -357,7 +358,7 @@ def forward_logits_lower(x_lower, a_lower, b_lower, logits_lower, logits, schedu
 
 
 def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_lower, scale=1.0,
-                           softmax_backward=False, softmax_backward_lower=True):
+                           softmax_backward=False, softmax_backward_lower=True, any_rows=False):
     """backward_chained for a layer whose input ``x`` is the output of a layer that needs no
     input gradient (a model's first layer), with that lower layer's backward_w in the same pass:
     the grad_x rows are consumed where they are finished instead of being written and read
@@ -365,11 +366,11 @@ def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_
     the second result is the gradient of its logits, else of its probabilities.  ``x`` may be
     None (fp32 / fp64): its rows are then recomputed from the lower layer (forward_logits_lower
     never stored them).  Returns (grad_w [out,16], grad_w_lower [in,16]), or None where the fused
-    pass does not apply.  Not part of the reference's extension."""
+    pass does not apply (``any_rows`` as in backward_chained).  Not part of the reference's extension."""
     for t, n in ((w, "w"), (grad_y, "grad_y"), (x_lower, "x_lower"), (a_lower, "a_lower"), (b_lower, "b_lower"),
                  (w_lower, "w_lower")):
         _check_input(t, n)
-    code = _float_code(grad_y, "logic_layer_cuda_backward")
+    code = _float_code(grad_y, "logic_layer_cuda_backward") | (_lib.DL_ROWS_ANY if any_rows else 0)
     dtype = grad_y.dtype
     out_dim, batch = grad_y.shape if grad_y.dim() == 2 else (0, 0)
     in_dim = w_lower.shape[0]
@@ -1172,12 +1173,13 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
     dev = _same_device(x, a, b, probs, grad_cls)
     lib = _lib.load()
     if want_x and want_w and schedule is not None:
+        chained_code = code | _lib.DL_ROWS_ANY
         _check_schedule(schedule, in_dim, out_dim, dev)
         dst, fix_vertex, fix_start, n_fix, rows = schedule.backward_plan()
         if rows <= in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
             grad_w = torch.empty((out_dim, 16), dtype=x.dtype, device=dev)
             grad_x = torch.empty_like(x)
-            ws_bytes = lib.dl_logic_backward_chained_workspace_bytes(rows, out_dim, batch, code)
+            ws_bytes = lib.dl_logic_backward_chained_workspace_bytes(rows, out_dim, batch, chained_code)
             if ws_bytes < 0:
                 _raise(-ws_bytes, "logic_layer_cuda_backward_chained")
             workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
@@ -1186,7 +1188,7 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
                     _p(x), _p(schedule.verts), _p(schedule.neuron), _p(schedule.flip), _p(dst), schedule.steps, _p(probs),
                     _p(grad_cls), 1, _p(fix_vertex) if n_fix else None, _p(fix_start) if n_fix else None, n_fix, rows,
                     _p(grad_w), _p(grad_x), _p(workspace) if ws_bytes else None, in_dim, out_dim, batch, k, float(scale),
-                    code, _stream(dev))
+                    chained_code, _stream(dev))
             if st == _lib.DL_OK:
                 return grad_w, grad_x
             if st != _lib.DL_ERR_TOO_LARGE:

@@ -52,6 +52,12 @@ typedef enum dl_status {
  * entry point answers DL_ERR_DTYPE. */
 typedef enum dl_dtype { DL_F16 = 0, DL_F32 = 1, DL_F64 = 2, DL_F16_W32 = 3, DL_F64_W32 = 4 } dl_dtype;
 
+/* Or'ed into `dtype`: rows that are not whole 16-byte vectors, or whose base address is not 16-byte
+ * aligned, are taken as well, as long as a row holds at least 16 bytes (dl_logic_backward_chained,
+ * its _lower and _grouped forms and its workspace size, dl_logic_forward_chained_lower; without it
+ * these return DL_ERR_TOO_LARGE for such rows).  The workspace stays 16-byte aligned. */
+#define DL_ROWS_ANY 0x100
+
 /* Library version (major*10000 + minor*100 + patch) and a static message per status. */
 int dl_version(void);
 const char *dl_status_string(int status);
@@ -99,8 +105,8 @@ int dl_logic_backward_logits(const void *x, const int64_t *a, const int64_t *b, 
  *                     softmax(w) (as dl_logic_forward_logits);
  *          backward - NULL: plain grad_w; else the softmax backward is chained
  *                     (as dl_logic_backward_logits).
- * Return DL_ERR_TOO_LARGE where the chained kernels do not apply (batch not a multiple of 16
- * bytes of elements, unaligned buffers; backward_w: rows longer than 256 vectors of 16 bytes);
+ * Return DL_ERR_TOO_LARGE where the chained kernels do not apply (rows shorter than 16 bytes;
+ * backward_w: rows longer than 256 vectors of 16 bytes);
  * the caller then uses the unchained entry points. */
 int dl_logic_forward_chained(const void *x, const int32_t *verts, const int32_t *neuron,
                              const uint8_t *flip, int64_t steps, const void *w, void *y, void *probs,

@@ -1,0 +1,107 @@
+"""Training kernels on rows that are not whole 16-byte vectors: the last vector of a row overlaps the one before
+it, so what matters is that every element is written and that sums over the batch count it once.  Against fp64
+arithmetic on the values as rounded to the activations' dtype, with the training path's tolerances."""
+import pytest
+import torch
+
+from oracle import float_oracle as fo
+from tests.helpers import within_budget
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float16, torch.float32, torch.float64]
+RTOL = {torch.float16: 4e-3, torch.float32: 1e-5, torch.float64: 1e-12}
+
+
+@pytest.fixture(scope="module")
+def ext():
+    import difflogic_amd
+    return difflogic_amd.difflogic_cuda
+
+
+def _batches(dtype):
+    """Row lengths around the edges: one vector and one element more, 32 / 64 / 128 / 256 vectors (the lane, register
+    and segment limits of the kernels) less one element and more by one, and a last segment of one partial vector."""
+    v = 16 // dtype.itemsize
+    return [v + 1, 2 * v - 1, 32 * v - 1, 32 * v + 1, 64 * v + 1, 128 * v + 1, 256 * v - 1, 256 * v + 1]
+
+
+CASES = [(d, n) for d in DTYPES for n in _batches(d)]
+
+
+@pytest.mark.parametrize("dtype,batch", CASES)
+def test_layer_kernels_on_rows_of_any_length(ext, monkeypatch, dtype, batch):
+    monkeypatch.setattr(ext, "BACKWARD_CHAIN_MAX_OVERFLOW", 1e9)     # exercise the overflow rows on this wiring
+    in_dim, out_dim, k = 30, 44, 4
+    g = torch.Generator().manual_seed(batch)
+    a = torch.randint(0, in_dim, (out_dim,), generator=g)
+    b = torch.randint(0, in_dim, (out_dim,), generator=g)
+    b[1] = a[1]
+    x = torch.rand(in_dim, batch, generator=g).to(dtype)
+    gy = torch.randn(out_dim, batch, generator=g).to(dtype)
+    logits = torch.randn(out_dim, 16, generator=g).to(dtype)
+    rtol = RTOL[dtype]
+
+    def close(got, want64, ref32=None):
+        assert got.dtype == dtype
+        ok, report = within_budget(got, want64, ref32, rtol)
+        assert ok, report
+
+    l64 = logits.double().requires_grad_()
+    x64 = x.double().t().contiguous().requires_grad_()
+    y64 = fo.layer_forward_sequential(x64, a, b, torch.softmax(l64, -1))           # [B, out]
+    (y64 * gy.double().t()).sum().backward()
+    xd, ad, bd, ld, gd = x.cuda(), a.cuda(), b.cuda(), logits.cuda(), gy.cuda()
+    sched = ext.schedule_for(ad, bd, in_dim)
+    from difflogic_amd.functional import build_reverse_index
+    start, idx = (t.cuda() for t in build_reverse_index(a, b, in_dim))
+    for schedule in (None, sched):
+        y, probs = ext.forward_logits(xd, ad, bd, ld, schedule)
+        close(y, y64.t())
+        close(ext.backward_logits(xd, ad, bd, gd, probs, schedule), l64.grad)
+    close(ext.backward_x(xd, ad, bd, probs, gd, start, idx, 1.5), 1.5 * x64.grad.t())
+    gl, gx = ext.backward_chained(xd, probs, gd, sched, 1.5, softmax_backward=True, any_rows=True)
+    close(gl, l64.grad)
+    close(gx, 1.5 * x64.grad.t())
+
+    # the layer with the GroupSum after it, and the GroupSum alone
+    sums = fo.group_sum(y64.detach().to(dtype).double(), k, 3.0)
+    close(ext.forward_group_sum(xd, ad, bd, ld, k, 3.0)[0], sums)
+    close(ext.group_sum_forward(y, k, 3.0), sums)
+    gc = torch.randn(k, batch, generator=g).to(dtype)
+    l64.grad = x64.grad = None
+    yy = fo.layer_forward_sequential(x64, a, b, torch.softmax(l64, -1))
+    (yy * gc.double().repeat_interleave(out_dim // k, 0).t()).sum().backward()
+    for schedule in (None, sched):
+        gl, gx = ext.backward_group_sum(xd, ad, bd, probs, gc.cuda(), start, idx, schedule, 1.0, True, True)
+        close(gl, l64.grad)
+        close(gx, x64.grad.t())
+    back = ext.group_sum_backward(gc.t().contiguous().cuda(), out_dim, 1.0)
+    assert torch.equal(back.cpu(), gc.repeat_interleave(out_dim // k, 0))
+
+
+@pytest.mark.parametrize("dtype,batch", [c for c in CASES if c[1] * c[0].itemsize <= 2048 + 16])
+def test_two_layers_at_once_on_rows_of_any_length(ext, monkeypatch, dtype, batch):
+    """forward_logits_lower and backward_chained_lower against the two layers run one after the other."""
+    monkeypatch.setattr(ext, "BACKWARD_CHAIN_MAX_OVERFLOW", 1e9)
+    in0, in_dim, out_dim = 20, 30, 44
+    g = torch.Generator().manual_seed(batch)
+    draw = lambda hi, n: torch.randint(0, hi, (n,), generator=g).cuda()  # noqa: E731
+    a0, b0, a, b = draw(in0, in_dim), draw(in0, in_dim), draw(in_dim, out_dim), draw(in_dim, out_dim)
+    x0 = torch.rand(in0, batch, generator=g).to(dtype).cuda()
+    l0 = torch.randn(in_dim, 16, generator=g).to(dtype).cuda()
+    l1 = torch.randn(out_dim, 16, generator=g).to(dtype).cuda()
+    gy = torch.randn(out_dim, batch, generator=g).to(dtype).cuda()
+    sched = ext.schedule_for(a, b, in_dim)
+    y1, p0 = ext.forward_logits(x0, a0, b0, l0)
+    y2, p1 = ext.forward_logits(y1, a, b, l1)
+    rtol = RTOL[dtype]
+    ok = lambda got, want: within_budget(got, want, None, rtol)[0]  # noqa: E731
+    if batch * dtype.itemsize <= 2048:
+        got = ext.forward_logits_lower(x0, a0, b0, l0, l1, sched, any_rows=True)
+        assert ok(got[0], y2) and ok(got[2], p1)
+    gw, gx = ext.backward_chained(y1, p1, gy, sched, softmax_backward=True, any_rows=True)
+    gw0 = ext.backward_logits(x0, a0, b0, gx, p0)
+    for x in (y1, None) if dtype != torch.float16 else (y1,):        # None: the inner rows are recomputed
+        both = ext.backward_chained_lower(x, p1, gy, sched, x0, a0, b0, p0, softmax_backward=True, any_rows=True)
+        assert ok(both[0], gw) and ok(both[1], gw0)
