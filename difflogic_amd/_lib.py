@@ -56,6 +56,7 @@ SIGNATURES = {
     "dl_gate_ids": [_vp, _vp, _i64, _int, _vp],
     "dl_fold_gate_constants": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp],
     "dl_gate_ids_folded": [_vp, _int, _vp, _vp, _vp, _vp, _vp, _i64, _vp],
+    "dl_logic_eval_weights": [_vp, _vp, _vp, _vp, _int, _vp, _i64, _i64, _i64, _vp],
     "dl_mark_live_inputs": [_vp, _vp, _vp, _vp, _vp, _i64, _vp],
     "dl_logic_eval": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp],
     "dl_tensor_packbits": [_vp, _vp, _i64, _i64, _int, ctypes.POINTER(_i64), _vp],

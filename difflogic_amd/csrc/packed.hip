@@ -781,6 +781,38 @@ __global__ __launch_bounds__(DL_BLOCK) void packbits_batch_major_rows_kernel(con
     }
 }
 
+// Variant for batches too short to give the tile kernel a workgroup per CU (it takes 512 samples at a time): a wave takes
+// 64 samples x 16 features, lane = sample, and a ballot per feature is the output word.  Bound by latency: one 16-byte
+// load per lane, each from a line of its own (784 features, batch 1000: 16 -> 4 us).
+template <bool ALIGNED>
+__global__ __launch_bounds__(DL_BLOCK) void packbits_ballot_kernel(const uint8_t *__restrict__ x, uint64_t *__restrict__ out,
+                                                                   int64_t batch, int64_t features, int64_t words) {
+    const int lane = dl_lane();
+    const int64_t f0 = ((int64_t) blockIdx.x * 4 + dl_wave_in_block()) * 16;
+    if (f0 >= features) return;
+    const int64_t word = blockIdx.y, sample = word * 64 + lane;
+    uint32_t v[4] = {0, 0, 0, 0};
+    if (sample < batch) {
+        const uint8_t *src = x + sample * features + f0;
+        if constexpr (ALIGNED) {
+            const dl_u32x4 q = *reinterpret_cast<const dl_u32x4 *>(src);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = q[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (f0 + i < features) v[i / 4] |= (uint32_t) src[i] << (8 * (i % 4));
+        }
+    }
+    uint64_t mine = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint64_t bits = __ballot(((v[i / 4] >> (8 * (i % 4))) & 0xffu) != 0);
+        if (lane == i) mine = bits;
+    }
+    if (lane < 16 && f0 + lane < features) out[(f0 + lane) * words + word] = mine;
+}
+
 // ------------------------------------------------------------------------------------------
 // Vertical bit count (GroupSum on packed words).  For each class (a contiguous block of
 // per_class neuron rows) and each sample bit, the number of rows with that bit set.
@@ -1594,6 +1626,134 @@ __global__ __launch_bounds__(DL_BLOCK) void groupbitsum_generic_kernel(const uin
     }
 }
 
+// ------------------------------------------------------------------------------------------
+// Count over stored rows that are too short for groupbitsum_kernel, whose lanes run along the row: a workgroup of 1024
+// threads takes CP 16-byte columns of one class, thread (row lane, column) adds every (1024 / CP)-th row to bit-sliced
+// counters of its own.  The counters are added across the row lanes of a wave by a butterfly whose first two exchanges
+// split the four dwords between the partners, across the waves by a second one over LDS (lane = wave), and every lane
+// expands two samples.  Bound by latency on the shortest rows (5 us, launch included), by reading the rows beyond
+// (64000 rows of 1264 bytes: 81 MB in 25 us).
+// ------------------------------------------------------------------------------------------
+#define DL_TALL_PLANES 8                     // a thread's own counter: at most 255 rows
+#define DL_TALL_WAVES 16
+
+// (p, n planes) += (o, n planes), a bit-sliced sum of n + 1 planes
+template <int N> __device__ __forceinline__ void planes_add(uint32_t *p, const uint32_t *o) {
+    uint32_t carry = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) csa<uint32_t>(carry, p[i], p[i], o[i], carry);
+    p[N] = carry;
+}
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, CTRL, 0xf, 0xf, true);
+}
+// the same with the counters of the lanes 8, 4, 2, 1 away (M = 8: down to CP), which hold the same columns: row rotations
+// (after the first, the values repeat every 8 lanes), then quad permutations
+template <int N, int M, int CP> __device__ __forceinline__ void planes_add_row(uint32_t *p) {
+    if constexpr (M >= CP) {
+        constexpr int CTRL = M == 8 ? 0x128 : M == 4 ? 0x124 : M == 2 ? 0x4E : 0xB1;
+        uint32_t o[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = dpp_u32<CTRL>(p[i]);
+        planes_add<N>(p, o);
+        planes_add_row<N + 1, M / 2, CP>(p);
+    }
+}
+
+constexpr int dl_log2(int v) { return v <= 1 ? 0 : 1 + dl_log2(v / 2); }
+
+template <int CP>
+__global__ __launch_bounds__(DL_WAVE * DL_TALL_WAVES) void groupbitsum_tall_kernel(const dl_u32x4 *__restrict__ bits,
+                                                                                  int32_t *__restrict__ out, int ncols,
+                                                                                  int per_class, int k, int64_t batch) {
+    constexpr int R = DL_WAVE * DL_TALL_WAVES / CP;                       // row lanes
+    constexpr int NW = DL_TALL_PLANES + 6 - dl_log2(CP);                  // planes of a wave's sums
+    constexpr int NB = NW + 4;                                            // ... of the workgroup's
+    constexpr int DC = 4 * CP;                                            // dword columns
+    __shared__ uint32_t sums[NW][DC][DL_TALL_WAVES];
+    // the 8 / CP workgroups that share the 128-byte lines of a class run on one of the 8 XCDs (workgroups are dealt to them
+    // round-robin by index)
+    constexpr unsigned SHARE = 8 / CP;
+    const unsigned turn = blockIdx.x / 8, unit = turn / SHARE * 8 + blockIdx.x % 8;
+    const int cls = (int) (unit % (unsigned) k), col0 = (int) (unit / (unsigned) k * 8 + turn % SHARE * CP);
+    if (col0 >= ncols) return;
+    const int lane = dl_lane(), wave = dl_wave_in_block();
+    const int col = col0 + lane % CP;
+    const int first = (int) (threadIdx.x / CP);
+    const bool live = col < ncols;
+    const dl_u32x4 *src = bits + (int64_t) cls * per_class * ncols + (live ? col : 0);
+    const dl_u32x4 zero = {0, 0, 0, 0};
+
+    dl_u32x4 plane[DL_TALL_PLANES];
+#pragma unroll
+    for (int p = 0; p < DL_TALL_PLANES; ++p) plane[p] = zero;
+    for (int r = first; r < per_class; r += 8 * R) {                      // eight rows in flight
+        dl_u32x4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = live && r + i * R < per_class ? src[(int64_t) (r + i * R) * ncols] : zero;
+        dl_u32x4 t4a = csa_quad<dl_u32x4>(plane[0], plane[1], v), t4b = csa_quad<dl_u32x4>(plane[0], plane[1], v + 4), t8;
+        csa<dl_u32x4>(t8, plane[2], plane[2], t4a, t4b);
+#pragma unroll
+        for (int p = 3; p < DL_TALL_PLANES; ++p) {
+            const dl_u32x4 old = plane[p];
+            plane[p] = old ^ t8;
+            t8 = old & t8;
+        }
+    }
+
+    // Lanes 32 apart: the lower one keeps dwords 0 and 1, the upper one 2 and 3, and adds the partner's (after the swap one
+    // register holds the lane's own half and the other its partner's).  Lanes 16 apart split the two that are left.  Lane l
+    // then holds dword 2 (l / 32) + (l / 16) % 2 of its column.
+    uint32_t s[NB + 1];
+    {
+        uint32_t d0[DL_TALL_PLANES + 1], d1[DL_TALL_PLANES + 1], o0[DL_TALL_PLANES], o1[DL_TALL_PLANES];
+#pragma unroll
+        for (int p = 0; p < DL_TALL_PLANES; ++p) {
+            const auto r0 = __builtin_amdgcn_permlane32_swap(plane[p][0], plane[p][2], false, false);
+            const auto r1 = __builtin_amdgcn_permlane32_swap(plane[p][1], plane[p][3], false, false);
+            d0[p] = r0[0], o0[p] = r0[1], d1[p] = r1[0], o1[p] = r1[1];
+        }
+        planes_add<DL_TALL_PLANES>(d0, o0);
+        planes_add<DL_TALL_PLANES>(d1, o1);
+        uint32_t o[DL_TALL_PLANES + 1];
+#pragma unroll
+        for (int p = 0; p <= DL_TALL_PLANES; ++p) {
+            const auto r = __builtin_amdgcn_permlane16_swap(d0[p], d1[p], false, false);
+            s[p] = r[0], o[p] = r[1];
+        }
+        planes_add<DL_TALL_PLANES + 1>(s, o);
+    }
+    planes_add_row<DL_TALL_PLANES + 2, 8, CP>(s);                         // the row lanes that are left
+    if ((lane & 15) < CP) {
+        const int dc = 4 * (lane & 15) + (lane >> 4 & 1) + 2 * (lane >> 5);
+#pragma unroll
+        for (int p = 0; p < NW; ++p) sums[p][dc][wave] = s[p];
+    }
+    __syncthreads();
+    if ((int) threadIdx.x >= DC * DL_TALL_WAVES) return;                  // whole waves: DC * 16 is a multiple of 64
+    const int dc = (int) threadIdx.x / DL_TALL_WAVES, part = (int) threadIdx.x % DL_TALL_WAVES;
+#pragma unroll
+    for (int p = 0; p < NW; ++p) s[p] = sums[p][dc][part];
+    planes_add_row<NW, 8, 1>(s);                                          // 16 lanes = the 16 waves
+    if (col0 + dc / 4 >= ncols) return;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int bit = part + 16 * h;
+        int32_t n = 0;
+#pragma unroll
+        for (int p = 0; p < NB; ++p) n += (int32_t) ((s[p] >> bit & 1u) << p);
+        const int64_t sample = (int64_t) (col0 * 4 + dc) * 32 + bit;
+        if (sample < batch) out[sample * k + cls] = n;
+    }
+}
+
+template <int CP> void launch_groupbitsum_tall(const void *bits, int32_t *out, int ncols, int per_class, int k, int64_t batch,
+                                               hipStream_t s) {
+    const int64_t units = dl_ceil_div(dl_ceil_div(ncols, 8) * k, 8) * 8;
+    DL_LAUNCH(groupbitsum_tall_kernel<CP>, dim3((unsigned) (units * (8 / CP))), dim3(DL_WAVE * DL_TALL_WAVES), 0, s,
+              (const dl_u32x4 *) bits, out, ncols, per_class, k, batch);
+}
+
 template <typename V>
 void launch_groupbitsum_v(const void *bits, int32_t *out, int64_t row_bytes, int64_t per_class, int64_t k,
                           int64_t batch, hipStream_t s) {
@@ -1613,7 +1773,24 @@ void launch_groupbitsum_v(const void *bits, int32_t *out, int64_t row_bytes, int
 // Rows of whole 64-bit words, 8-byte aligned: 16-byte lanes where rows and base allow it.
 void launch_groupbitsum(const void *bits, int32_t *out, int64_t row_bytes, int64_t per_class, int64_t k, int64_t batch,
                         hipStream_t s) {
-    if (row_bytes % 16 == 0 && dl_aligned(bits, 16))
+    const bool vectors = row_bytes % 16 == 0 && dl_aligned(bits, 16);
+    const int64_t ncols = row_bytes / 16;
+    // groupbitsum_kernel has one workgroup per class and kilobyte of the row: up to about 200 of them leave most of the
+    // chip idle (64000 rows, 10 classes, 1264-byte rows: 201 us against 25; 16 KB rows = 160 workgroups: 213 against 200;
+    // 100 classes of 600 rows, 1600-byte rows = 200: 41 against 37; 4 KB rows = 400: 61 against 64).
+    if (vectors && k * dl_ceil_div(ncols, DL_WAVE) <= 200 && per_class <= 255 * 1024) {
+        const int nc = (int) ncols, pc = (int) per_class, kk = (int) k;
+        // Columns per workgroup: wide enough for whole lines, narrow enough for about a hundred workgroups (64000 rows, 10
+        // classes, with 1 / 2 / 4 / 8 columns: 7.4 / 7.4 / 8.9 / 12 us on 128-byte rows, 18 / 11 / 12 / 14 on 512,
+        // 32 / 27 / 20 / 23 on 1008, 50 / 29 / 27 / 27 on 2048); a thread's counter holds 255 rows.
+        const int64_t work = ncols * k, most = 255 * 1024 / (per_class > 0 ? per_class : 1);
+        if (work >= 1000 && most >= 8) launch_groupbitsum_tall<8>(bits, out, nc, pc, kk, batch, s);
+        else if (work >= 350 && most >= 4) launch_groupbitsum_tall<4>(bits, out, nc, pc, kk, batch, s);
+        else if (work >= 100 && most >= 2) launch_groupbitsum_tall<2>(bits, out, nc, pc, kk, batch, s);
+        else launch_groupbitsum_tall<1>(bits, out, nc, pc, kk, batch, s);
+        return;
+    }
+    if (vectors)
         launch_groupbitsum_v<dl_u32x4>(bits, out, row_bytes, per_class, k, batch, s);
     else
         launch_groupbitsum_v<uint64_t>(bits, out, row_bytes, per_class, k, batch, s);
@@ -1796,6 +1973,86 @@ __global__ __launch_bounds__(DL_BLOCK) void gate_ids_kernel(const T *__restrict_
     ids[n] = (uint8_t) argmax16<T, C>(w + n * 16);
 }
 
+// ------------------------------------------------------------------------------------------
+// One layer straight from its weights, for short rows: argmax gate and gate evaluation in one launch, no records, no
+// schedule, no liveness.  A wave owns 16 neurons: four lanes take the argmax of a neuron's 16 weights (one coalesced
+// kilobyte of fp32 weights per wave), then P lanes work on one neuron's row, 64 / P neurons at a time.  Such a call is bound by
+// latency and launches, so everything a wave needs is requested at once: the rows do not wait for the gate (P < 64;
+// with a whole wave per row the gate is wave-uniform and an input that it ignores is not fetched).  64000 neurons on
+// 128-byte rows: 9.1 us for 4 MB of weights, 16 MB of gathered and 8 MB of written rows; 8000 on 16-byte rows: 3.7 us.
+// ------------------------------------------------------------------------------------------
+template <typename T> struct alignas(sizeof(T)) Weights4 { T v[4]; };
+
+// (value, index) of the better of two candidates: the larger value, a NaN above every number, the lower index of equals.
+template <typename C> __device__ __forceinline__ void argmax_take(C &v, uint32_t &at, C ov, uint32_t oat) {
+    const bool nan = v != v, onan = ov != ov;
+    const bool tie = (nan && onan) || v == ov;
+    if (tie ? oat < at : (onan || (!nan && ov > v))) v = ov, at = oat;
+}
+__device__ __forceinline__ float lane_xor(float v, int m) { return __shfl_xor(v, m, DL_WAVE); }
+__device__ __forceinline__ double lane_xor(double v, int m) { return __shfl_xor(v, m, DL_WAVE); }
+
+template <typename T, typename C, int P>
+__global__ __launch_bounds__(DL_BLOCK) void eval_weights_kernel(const dl_u32x4 *__restrict__ x, const int64_t *__restrict__ a,
+                                                                const int64_t *__restrict__ b, const T *__restrict__ w,
+                                                                dl_u32x4 *__restrict__ y, int64_t out_dim, int ncols) {
+    const int lane = dl_lane();
+    const int64_t n0 = ((int64_t) blockIdx.x * 4 + dl_wave_in_block()) * 16;
+    if (n0 >= out_dim) return;
+    // neurons past the end repeat the last one: nothing of theirs is stored
+    const int64_t nw = n0 + (lane >> 2) < out_dim ? n0 + (lane >> 2) : out_dim - 1;
+    const Weights4<T> part = *reinterpret_cast<const Weights4<T> *>(w + nw * 16 + 4 * (lane & 3));
+    // lanes 0 .. 15 hold the neurons' `a`, lanes 16 .. 31 their `b`
+    const int64_t ni = n0 + (lane & 15) < out_dim ? n0 + (lane & 15) : out_dim - 1;
+    const int32_t idx = (int32_t) ((lane & 16) ? b[ni] : a[ni]);
+    C best = (C) part.v[0];
+    uint32_t at = 4 * (lane & 3);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) argmax_take<C>(best, at, (C) part.v[i], 4 * (lane & 3) + i);
+#pragma unroll
+    for (int m = 1; m < 4; m <<= 1) argmax_take<C>(best, at, lane_xor(best, m), (uint32_t) __shfl_xor((int) at, m, DL_WAVE));
+
+    constexpr int PER = DL_WAVE / P;                                     // neurons side by side
+    constexpr int PASSES = 16 / PER > 0 ? 16 / PER : 1;
+    constexpr int BATCH = PASSES < 4 ? PASSES : 4;                       // passes whose rows are in flight together
+    // gridDim.y (a power of two up to PASSES / BATCH) waves share the 16 neurons, each with its share of the passes
+    const int share = PASSES / (int) gridDim.y;
+#pragma unroll 1
+    for (int p0 = (int) blockIdx.y * share; p0 < ((int) blockIdx.y + 1) * share; p0 += BATCH) {
+        if (n0 + p0 * PER >= out_dim) break;
+        int64_t ra[BATCH], rb[BATCH];
+        uint32_t op[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            if constexpr (P == DL_WAVE) {
+                const int j = p0 + i;
+                ra[i] = (int64_t) __builtin_amdgcn_readlane(idx, j) * ncols;
+                rb[i] = (int64_t) __builtin_amdgcn_readlane(idx, 16 + j) * ncols;
+                op[i] = (uint32_t) __builtin_amdgcn_readlane((int) at, 4 * j);
+            } else {
+                const int j = ((p0 + i) * PER + lane / P) & 15;
+                ra[i] = (int64_t) __shfl(idx, j, DL_WAVE) * ncols;
+                rb[i] = (int64_t) __shfl(idx, 16 + j, DL_WAVE) * ncols;
+                op[i] = (uint32_t) __shfl((int) at, 4 * j, DL_WAVE);
+            }
+        }
+        for (int col = lane % P; col < ncols; col += P) {
+            dl_u32x4 va[BATCH], vb[BATCH];
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) {
+                const bool skip_a = P == DL_WAVE && !gate_uses_a(op[i]), skip_b = P == DL_WAVE && !gate_uses_b(op[i]);
+                va[i] = skip_a ? dl_u32x4{0, 0, 0, 0} : x[ra[i] + col];
+                vb[i] = skip_b ? dl_u32x4{0, 0, 0, 0} : x[rb[i] + col];
+            }
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) {
+                const int j = (p0 + i) * PER + lane / P;
+                if (j < 16 && n0 + j < out_dim) y[(n0 + j) * ncols + col] = gate_apply<dl_u32x4>(va[i], vb[i], gate_masks(op[i]));
+            }
+        }
+    }
+}
+
 // f'(a, b) = f(a, b) with the inputs that are constant (state 1: all zeros, 2: all ones; 0: varies) put in: the
 // gate the neuron amounts to on the inputs that vary.  Gate ids are (f(0,0) f(0,1) f(1,0) f(1,1)), MSB first.
 __device__ __forceinline__ uint32_t fold_gate(uint32_t op, uint32_t sa, uint32_t sb) {
@@ -1824,6 +2081,41 @@ __global__ __launch_bounds__(DL_BLOCK) void gate_ids_folded_kernel(const T *__re
     const uint32_t op = fold_gate(argmax16<T, C>(w + n * 16), sa, sb);
     ids[n] = (uint8_t) op;
     state_out[n] = op == 0u ? 1 : op == 15u ? 2 : 0;
+}
+
+template <typename T, typename C>
+static void launch_eval_weights(const void *x, const int64_t *a, const int64_t *b, const void *w, void *y, int64_t out_dim,
+                                int ncols, hipStream_t s) {
+    const int64_t blocks = dl_ceil_div(out_dim, 64);
+    unsigned most = ncols <= 16 ? 1 : ncols <= 32 ? 2 : 4, split = 1;     // PASSES / BATCH of the kernel that is launched
+    while (split < most && blocks * split < 512) split *= 2;              // narrow layers: two workgroups per CU
+    const dim3 grid((unsigned) blocks, split), block(DL_BLOCK);
+#define DL_LAUNCH_EVAL_WEIGHTS(P)                                                                                   \
+    DL_LAUNCH((eval_weights_kernel<T, C, P>), grid, block, 0, s, (const dl_u32x4 *) x, a, b, (const T *) w, (dl_u32x4 *) y, \
+              out_dim, ncols)
+    if (ncols <= 4) DL_LAUNCH_EVAL_WEIGHTS(4);
+    else if (ncols <= 8) DL_LAUNCH_EVAL_WEIGHTS(8);
+    else if (ncols <= 16) DL_LAUNCH_EVAL_WEIGHTS(16);
+    else if (ncols <= 32) DL_LAUNCH_EVAL_WEIGHTS(32);
+    else DL_LAUNCH_EVAL_WEIGHTS(64);
+#undef DL_LAUNCH_EVAL_WEIGHTS
+}
+
+extern "C" int dl_logic_eval_weights(const void *x, const int64_t *a, const int64_t *b, const void *w, int dtype, void *y,
+                                     int64_t in_dim, int64_t out_dim, int64_t row_bytes, void *stream) {
+    if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
+    if (in_dim < 0 || out_dim < 0 || row_bytes < 0) return DL_ERR_INVALID_ARGUMENT;
+    if (out_dim == 0 || row_bytes == 0) return DL_OK;
+    if (!x || !a || !b || !w || !y || in_dim == 0) return DL_ERR_INVALID_ARGUMENT;
+    if (row_bytes % 16 || !dl_aligned(x, 16) || !dl_aligned(y, 16)) return DL_ERR_INVALID_ARGUMENT;
+    // row numbers travel as int32 inside the kernel
+    if (in_dim > 0x7fffffffLL || out_dim > 0x7fffffffLL || row_bytes / 16 > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
+    const int ncols = (int) (row_bytes / 16);
+    hipStream_t s = (hipStream_t) stream;
+    if (dtype == DL_F16) launch_eval_weights<__half, float>(x, a, b, w, y, out_dim, ncols, s);
+    else if (dtype == DL_F32) launch_eval_weights<float, float>(x, a, b, w, y, out_dim, ncols, s);
+    else launch_eval_weights<double, double>(x, a, b, w, y, out_dim, ncols, s);
+    return dl_launch_status();
 }
 
 extern "C" int dl_gate_ids(const void *w, uint8_t *ids, int64_t out_dim, int dtype, void *stream) {
@@ -1929,7 +2221,18 @@ static int pack_batch_major_rows(const uint8_t *x, void *out, int64_t batch, int
     const int64_t cols = dl_ceil_div(out_row_bytes, 8);          // 64-sample columns of the output
     const int64_t gx = dl_ceil_div(cols, 16);
     if (gx > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-    if (features % 16 == 0 && dl_aligned(x, 16) && out_row_bytes % 8 == 0) {
+    const bool vectors = features % 16 == 0 && dl_aligned(x, 16);
+    // Up to 192 words per row (batch 12288) the tile kernels have too few workgroups (784 features: 17 us against 4 at batch
+    // 1000, 17 against 5 at 10000, 17 against 9 at 16000, 17 against 16 at 32000; 9216 features: 50 against 36 at 10000, 51
+    // against 55 at 16000; 785 features, byte loads: 45 against 20 at 10000, 39 against 36 at 16000).
+    if (out_row_bytes % 8 == 0 && cols <= 192) {
+        const dim3 grid((unsigned) dl_ceil_div(features, 64), (unsigned) cols);
+        if (dl_ceil_div(features, 64) > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
+        if (vectors) DL_LAUNCH(packbits_ballot_kernel<true>, grid, dim3(DL_BLOCK), 0, s, x, (uint64_t *) out, batch, features, cols);
+        else DL_LAUNCH(packbits_ballot_kernel<false>, grid, dim3(DL_BLOCK), 0, s, x, (uint64_t *) out, batch, features, cols);
+        return dl_launch_status();
+    }
+    if (vectors && out_row_bytes % 8 == 0) {
         // A workgroup takes 8 word columns and a slice of the features, 68 bytes of LDS per feature.  Measured:
         // the longer the contiguous piece of a sample row a workgroup reads the better, down to one workgroup
         // per CU (2352 features); slices are whole 128-byte lines where the rows are.

@@ -135,6 +135,8 @@ class LogicLayer(torch.nn.Module):
         key = (self.weights.data_ptr(), self.weights._version, self.out_dim)
         w = self.weights.detach()
         if w.is_cuda and w.is_contiguous() and w.dtype in (torch.float16, torch.float32, torch.float64):
+            if x.takes_weights(self.out_dim):
+                return x.apply_weights(a, b, w)
             # the argmax gates with the constants among x's rows folded in, in one kernel (x tracks which rows those are)
             ids, state = difflogic_cuda.gate_ids_folded(w, a, b, x.row_state(a.device))
             return x.defer_layer(a, b, ids, key=key, state=state)

@@ -460,6 +460,29 @@ def gate_ids(weights):
     return ids
 
 
+def eval_weights(x, a, b, weights):
+    """``eval(x, a, b, gate_ids(weights))`` in one kernel, on rows ``x`` int64 [in, W] of whole 16-byte vectors (W even).
+    Not part of the reference's extension; PackBitsTensor uses it for short rows."""
+    _check_input(x, "x")
+    _check_input(weights, "weights")
+    code = _float_code(weights, "gate_ids")
+    if x.dim() != 2 or x.dtype != torch.int64 or x.shape[1] % 2 or weights.dim() != 2 or weights.shape[1] != 16:
+        raise RuntimeError(f"expected x [in,W] int64 with W even and weights [out,16], got {tuple(x.shape)} {x.dtype}, "
+                           f"{tuple(weights.shape)}")
+    out_dim = weights.shape[0]
+    _check_index(a, "a", out_dim)
+    _check_index(b, "b", out_dim)
+    dev = _same_device(x, a, b, weights)
+    in_dim, words = x.shape
+    y = torch.empty((out_dim, words), dtype=torch.int64, device=dev)
+    with _on(dev):
+        st = _lib.load().dl_logic_eval_weights(_p(x), _p(a), _p(b), _p(weights), code, _p(y), in_dim, out_dim, words * 8,
+                                               _stream(dev))
+    if st:
+        _raise(st, "logic_eval_weights")
+    return y
+
+
 def gate_ids_folded(weights, a, b, state=None):
     """gate_ids and one step of fold_gate_constants in one kernel: (ids, state_out) for a layer with wiring
     ``a``, ``b`` whose input rows are constant where ``state`` says so (uint8 [in]: 0 varies, 1 all zeros, 2 all

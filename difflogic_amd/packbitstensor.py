@@ -34,6 +34,24 @@ _STREAM_CALL_SECONDS = 6e-5  # per call of the streaming path: constant folding,
 _LAUNCH_SECONDS = 3e-6       # per kernel on the stream; decides between plans for small batches only
 
 
+# Layers evaluated from their weights when they are applied (one launch each, difflogic_cuda.eval_weights) instead of
+# deferred.  A deferred net costs two to three launches per layer and the group kernels, 75 to 240 us whatever the batch; a
+# layer at once costs 4 us and the traffic of its rows.  784 -> 6 x 64000, graph replay, deferred / at once: batch 100
+# 188 / 48 us, 1000 190 / 76, 4000 196 / 135, 8000 200 / 202; 4 x 256000: batch 2000 249 / 166, 3000 252 / 265 (the bytes of
+# a layer's rows decide).  Narrower layers are bound by latency instead: 6 x 16000 at 12000 188 / 118, 4 x 32000 162 / 131
+# there; nets that fit in LDS run in one workgroup per 128 samples, 6 x 8000 at 100 74 / 35, 4000 75 / 62, 6000 75 / 75, 12000 77 / 101.
+_DIRECT_BYTES = 64 << 20         # rows of a layer's output
+_DIRECT_ROW_BYTES = 1536         # ... and one row of them
+_DIRECT_ROW_BYTES_LDS = 768      # one row, for layers that the LDS kernel takes
+_DIRECT_MIN_OUT = 1000           # smaller layers, and the tapering end of a net below 4096, stay with the LDS kernel
+
+
+def _direct(in_dim, out_dim, row_bytes, lds_width):
+    """Whether a layer on rows of ``row_bytes`` is evaluated at once (above)."""
+    return (out_dim >= min(max(in_dim, _DIRECT_MIN_OUT), 4096) and 0 < out_dim * row_bytes <= _DIRECT_BYTES
+            and row_bytes <= (_DIRECT_ROW_BYTES_LDS if max(in_dim, out_dim) <= lds_width else _DIRECT_ROW_BYTES))
+
+
 def _chained(depth):
     """Groups of two or more layers run along the top layer's evaluation schedule."""
     return depth >= 2
@@ -166,7 +184,8 @@ class PackBitsTensor:
     Layers applied to the object are held back (``defer_layer``) until ``.t`` is read or
     ``group_sum`` is called; consecutive layers are then evaluated in fused groups (and the last
     group together with the bit count), so most intermediate activations never reach memory.
-    Reading ``.t`` always returns the up-to-date words, as in the reference.
+    Reading ``.t`` always returns the up-to-date words, as in the reference.  Layers on short rows are evaluated when
+    they are applied, in one launch each (``takes_weights``): there launches cost more than the activations.
 
     Inside, a row is a little-endian bit stream padded with zeros to a multiple of 16 bytes and held
     as int64 words: the same bytes as words of any of the four widths, so every batch size and word
@@ -345,6 +364,17 @@ class PackBitsTensor:
         if state is None:
             self._folded = False
         self._state = state
+        return self
+
+    def takes_weights(self, out_dim):
+        """Whether a layer of ``out_dim`` neurons applied next is best evaluated at once, from its weights (apply_weights)."""
+        return not self._pending and _direct(self._in_features(), out_dim, self._row_bytes(self._batch),
+                                             difflogic_cuda.net_lds_max_width())
+
+    def apply_weights(self, a, b, weights):
+        """Applies the gate layer with wiring ``a``, ``b`` and the argmax gates of ``weights`` [out, 16], now."""
+        self._rows, self._public = difflogic_cuda.eval_weights(self._words(), a, b, weights), None
+        self._state = None
         return self
 
     def group_sum(self, k):

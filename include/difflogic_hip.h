@@ -296,6 +296,12 @@ int dl_fold_gate_constants(const int64_t *a, const int64_t *b, const uint8_t *w,
 int dl_gate_ids_folded(const void *w, int dtype, const int64_t *a, const int64_t *b, const uint8_t *state_in,
                        uint8_t *ids, uint8_t *state_out, int64_t out_dim, void *stream);
 
+/* One layer of packed inference straight from its gate weights: y = eval(x, argmax(w)) with the argmax of dl_gate_ids,
+ * in one kernel.  Rows of `row_bytes` bytes (a multiple of 16), x and y 16-byte aligned.  Meant for short rows, where
+ * launches count; no counterpart in the reference's extension (difflogic/difflogic.py:143-153 takes the argmax in torch). */
+int dl_logic_eval_weights(const void *x, const int64_t *a, const int64_t *b, const void *w, int dtype, void *y,
+                          int64_t in_dim, int64_t out_dim, int64_t row_bytes, void *stream);
+
 /* Which input rows a layer looks at, for packed inference across fused groups (no counterpart in the
  * reference): live_in[r] is set to 1 where some neuron n with live_out[n] != 0 (live_out NULL: every
  * neuron) reads row r through an input its gate does not ignore.  live_in [in_dim] is cleared by the
