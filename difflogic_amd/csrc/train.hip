@@ -205,12 +205,17 @@ __device__ __forceinline__ int64_t grad_row(int64_t n, int64_t gdiv) {
     return gdiv ? (int64_t) ((uint32_t) n / (uint32_t) gdiv) : n;
 }
 
+// What a kernel makes of the [out, 16] weights: gate probabilities as they are (0, false), the softmax of logits (1, true),
+// or all of the argmax gate (the discretised net on float inputs; taken here instead of in four torch launches per layer
+// that make a one-hot matrix: 784 -> 6 x 64000, batch 1000: 834 -> 705 us).
+constexpr int GATES_LOGITS = 1, GATES_ARGMAX = 2;
+
 // Corner coefficients of FOUR neurons at once: the 16-lane row r of the wave works on neuron n[r]
-// (n[r] < 0: none), lane i of the row on gate i.  LOGITS: `w` holds logits, the row computes their
+// (n[r] < 0: none), lane i of the row on gate i.  LOGITS (GATES_LOGITS): `w` holds logits, the row computes their
 // softmax (and stores it to `probs` if asked); otherwise `w` holds the probabilities.  The corner
 // sums are masked row sums whose association order is that of corners_of(), so the results are
 // bit-identical to it.  Returns, per neuron, the wave-uniform P00, P10, P01 - P00, P11 - P10.
-template <typename T, bool LOGITS>
+template <typename T, int GATES>
 __device__ __forceinline__ void corners4(const T *__restrict__ w, const int32_t (&n)[4], int lane, bool store_probs,
                                          T *__restrict__ probs, typename Acc<T>::type (&p00)[4],
                                          typename Acc<T>::type (&p10)[4], typename Acc<T>::type (&d0)[4],
@@ -221,10 +226,15 @@ __device__ __forceinline__ void corners4(const T *__restrict__ w, const int32_t 
     const bool valid = mine >= 0;
     const int64_t at = (int64_t) (valid ? mine : 0) * 16 + gate;
     C p = wload<T>(w, at, w32);
-    if (LOGITS) {
+    if (GATES == GATES_LOGITS) {
         const C e = dl_exp(p - row16_max(p));
         p = e / row16_sum(e);
         if (store_probs && valid) wstore<T>(probs, at, p, w32);
+    } else if (GATES == GATES_ARGMAX) {
+        // as argmax: the first of the largest, a NaN above every number (row16_max passes NaNs over)
+        const uint32_t nans = (uint32_t) (__ballot(p != p) >> (16 * row)) & 0xffffu;
+        const uint32_t tops = (uint32_t) (__ballot(p == row16_max(p)) >> (16 * row)) & 0xffffu;
+        p = gate == __ffs((int) (nans ? nans : tops)) - 1 ? (C) 1 : (C) 0;
     }
     const C zero = (C) 0;
     const C q00 = row16_sum((gate & 8) ? p : zero), q01 = row16_sum((gate & 4) ? p : zero);
@@ -244,7 +254,7 @@ __device__ __forceinline__ void corners4(const T *__restrict__ w, const int32_t 
 // ------------------------------------------------------------------------------------------
 // LOGITS: `w` holds the raw gate logits; the kernel applies the softmax itself and (column tile 0
 // only) stores the probabilities to `probs` for the backward pass.
-template <typename T, int VEC, int NPW, bool LOGITS, bool RAG>
+template <typename T, int VEC, int NPW, int GATES, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_kernel(const T *__restrict__ x, const int64_t *__restrict__ a,
                                                            const int64_t *__restrict__ b, const T *__restrict__ w,
                                                            T *__restrict__ y, T *__restrict__ probs, int64_t out_dim,
@@ -268,7 +278,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_kernel(const T *__restrict__
         ib[j] = b[n];
         ids[j] = n0 + j < out_dim ? (int32_t) (n0 + j) : -1;
     }
-    corners4<T, LOGITS>(w, ids, lane, blockIdx.y == 0, probs, p00, p10, d0, d1, w32);
+    corners4<T, GATES>(w, ids, lane, blockIdx.y == 0, probs, p00, p10, d0, d1, w32);
     for (int64_t col = (int64_t) blockIdx.y * DL_WAVE + lane; col < ncols; col += (int64_t) gridDim.y * DL_WAVE) {
         P va[NPW], vb[NPW];
 #pragma unroll
@@ -476,7 +486,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_x_kernel(const T *__restric
 // fp64 results are bit-identical (fp16 outputs can differ in the last bit, where the compiler
 // folds the final conversion into a fused multiply-add in one kernel and not in the other).
 // ------------------------------------------------------------------------------------------
-template <typename T, int VEC, int CHUNK, bool LOGITS, bool RAG>
+template <typename T, int VEC, int CHUNK, int GATES, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__restrict__ x,
                                                                  const int32_t *__restrict__ verts,
                                                                  const int32_t *__restrict__ neuron,
@@ -508,7 +518,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__rest
 #pragma unroll
             for (int i = 0; i < 4; ++i) n[i] = neuron[s0 + j0 + i];
             C p00[4], p10[4], d0[4], d1[4];
-            corners4<T, LOGITS>(w, n, lane, ct == 0, probs, p00, p10, d0, d1, w32);
+            corners4<T, GATES>(w, n, lane, ct == 0, probs, p00, p10, d0, d1, w32);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int j = j0 + i;
@@ -619,7 +629,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
 // CPL * 64 consecutive vectors of the row (blockIdx.y picks the segment; lane l holds its vectors
 // l, l + 64, ...), so every gathered row is one contiguous request of up to 4 KB, and the next
 // step's row is requested before this step's arithmetic.
-template <typename T, int VEC, int CPL, bool LOGITS, bool RAG>
+template <typename T, int VEC, int CPL, int GATES, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *__restrict__ x,
                                                                       const int32_t *__restrict__ verts,
                                                                       const int32_t *__restrict__ neuron,
@@ -655,7 +665,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *_
 #pragma unroll
         for (int i = 0; i < 4; ++i) n[i] = g + i < s1 ? neuron[g + i] : -1;
         C p00[4], p10[4], d0[4], d1[4];
-        corners4<T, LOGITS>(w, n, lane, col0 == 0, probs, p00, p10, d0, d1, w32);
+        corners4<T, GATES>(w, n, lane, col0 == 0, probs, p00, p10, d0, d1, w32);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int64_t s = g + i;
@@ -1131,7 +1141,7 @@ unsigned col_tiles(int64_t ncols) {
     return (unsigned) (t > 65535 ? 65535 : t);
 }
 
-template <typename T, bool LOGITS>
+template <typename T, int GATES>
 int forward_t(const void *x, const int64_t *a, const int64_t *b, const void *w, void *y, void *probs, int64_t out_dim,
               int64_t batch, hipStream_t s, bool w32 = false) {
     constexpr int NPW = 4;
@@ -1141,7 +1151,7 @@ int forward_t(const void *x, const int64_t *a, const int64_t *b, const void *w, 
     const Rows kind = rows_kind<T>(batch, x, y);
     const dim3 grid((unsigned) blocks, col_tiles(kind == Rows::single ? batch : dl_ceil_div(batch, V)));
 #define DL_LAUNCH_FORWARD(VV, RAG)                                                                                       \
-    DL_LAUNCH((forward_kernel<T, VV, NPW, LOGITS, RAG>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, a, b, (const T *) w, \
+    DL_LAUNCH((forward_kernel<T, VV, NPW, GATES, RAG>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, a, b, (const T *) w, \
               (T *) y, (T *) probs, out_dim, batch, w32)
     if (kind == Rows::whole) DL_LAUNCH_FORWARD(V, false);
     else if (kind == Rows::ragged) DL_LAUNCH_FORWARD(V, true);
@@ -1481,7 +1491,7 @@ int chain_chunk(int64_t steps) {
     return 8;
 }
 
-template <typename T, bool LOGITS>
+template <typename T, int GATES>
 int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps,
                     const void *w, void *y, void *probs, int64_t batch, hipStream_t s, bool w32 = false) {
     constexpr int V = Vec16<T>::n;
@@ -1498,7 +1508,7 @@ int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, 
         if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
         const dim3 grid((unsigned) blocks, (unsigned) segments);
 #define DL_LAUNCH_ROWS(CPL, RAG)                                                                                        \
-    DL_LAUNCH((forward_chain_rows_kernel<T, V, CPL, LOGITS, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, (T *) y, \
+    DL_LAUNCH((forward_chain_rows_kernel<T, V, CPL, GATES, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, (T *) y, \
               (T *) probs, steps, chunk, batch, w32)
         if (ncols <= 2 * DL_WAVE) {
             if (kind == Rows::whole) DL_LAUNCH_ROWS(2, false);
@@ -1517,7 +1527,7 @@ int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, 
     const bool half = V >= 2 && ncols <= DL_WAVE / 2;
     const dim3 grid((unsigned) blocks, half ? 1 : col_tiles(ncols));
 #define DL_LAUNCH_CHAIN(VV, RAG)                                                                                       \
-    DL_LAUNCH((forward_chain_kernel<T, VV, DL_TRAIN_CHUNK, LOGITS, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, \
+    DL_LAUNCH((forward_chain_kernel<T, VV, DL_TRAIN_CHUNK, GATES, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, \
               (T *) y, (T *) probs, nchunks, batch, w32)
     if (half) {
         if (kind == Rows::whole) DL_LAUNCH_CHAIN(H, false);
@@ -1685,6 +1695,13 @@ bool weights_fp32(int &dtype) {
     return false;
 }
 
+// DL_GATES_OF_ARGMAX in a dtype code: taken out of it, and returned
+bool gates_argmax(int &dtype) {
+    const bool argmax = (dtype & DL_GATES_OF_ARGMAX) != 0;
+    dtype &= ~DL_GATES_OF_ARGMAX;
+    return argmax;
+}
+
 // DL_ROWS_ANY in a dtype code: taken out of it, and returned
 bool takes_any_rows(int &dtype) {
     const bool any = (dtype & DL_ROWS_ANY) != 0;
@@ -1782,10 +1799,11 @@ extern "C" int dl_logic_backward_chained_lower(const void *x, const int32_t *ver
 extern "C" int dl_logic_forward_chained(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip,
                                         int64_t steps, const void *w, void *y, void *probs, int64_t in_dim,
                                         int64_t out_dim, int64_t batch, int dtype, void *stream) {
-    const bool w32 = weights_fp32(dtype);
+    const bool argmax = gates_argmax(dtype), w32 = weights_fp32(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim < 0 || out_dim < 0 || batch <= 0 || steps < out_dim || steps % DL_TRAIN_CHUNK != 0)
         return DL_ERR_INVALID_ARGUMENT;
+    if (argmax && probs) return DL_ERR_INVALID_ARGUMENT;
     if (out_dim == 0) return DL_OK;
     if (!x || !verts || !neuron || !flip || !w || !y || in_dim == 0) return DL_ERR_INVALID_ARGUMENT;
     hipStream_t s = (hipStream_t) stream;
@@ -1794,6 +1812,13 @@ extern "C" int dl_logic_forward_chained(const void *x, const int32_t *verts, con
         case DL_F16: return forward_chain_t<__half, true>(x, verts, neuron, flip, steps, w, y, probs, batch, s, w32);
         case DL_F32: return forward_chain_t<float, true>(x, verts, neuron, flip, steps, w, y, probs, batch, s);
         default: return forward_chain_t<double, true>(x, verts, neuron, flip, steps, w, y, probs, batch, s, w32);
+        }
+    }
+    if (argmax) {
+        switch (dtype) {
+        case DL_F16: return forward_chain_t<__half, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s, w32);
+        case DL_F32: return forward_chain_t<float, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s);
+        default: return forward_chain_t<double, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s, w32);
         }
     }
     switch (dtype) {
@@ -1854,12 +1879,19 @@ extern "C" int dl_logic_backward_w_chained(const void *x, const int32_t *verts, 
 
 extern "C" int dl_logic_forward(const void *x, const int64_t *a, const int64_t *b, const void *w, void *y,
                                 int64_t in_dim, int64_t out_dim, int64_t batch, int dtype, void *stream) {
-    const bool w32 = weights_fp32(dtype);
+    const bool argmax = gates_argmax(dtype), w32 = weights_fp32(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim < 0 || out_dim < 0 || batch < 0) return DL_ERR_INVALID_ARGUMENT;
     if (out_dim == 0 || batch == 0) return DL_OK;
     if (!x || !a || !b || !w || !y || in_dim == 0) return DL_ERR_INVALID_ARGUMENT;
     hipStream_t s = (hipStream_t) stream;
+    if (argmax) {
+        switch (dtype) {
+        case DL_F16: return forward_t<__half, GATES_ARGMAX>(x, a, b, w, y, nullptr, out_dim, batch, s, w32);
+        case DL_F32: return forward_t<float, GATES_ARGMAX>(x, a, b, w, y, nullptr, out_dim, batch, s);
+        default: return forward_t<double, GATES_ARGMAX>(x, a, b, w, y, nullptr, out_dim, batch, s, w32);
+        }
+    }
     switch (dtype) {
     case DL_F16: return forward_t<__half, false>(x, a, b, w, y, nullptr, out_dim, batch, s, w32);
     case DL_F32: return forward_t<float, false>(x, a, b, w, y, nullptr, out_dim, batch, s);

@@ -109,9 +109,9 @@ class LogicLayer(torch.nn.Module):
         assert x.shape[0] == self.in_dim, (x.shape, self.in_dim)
         a, b = self.indices
         tail = (self.given_x_indices_of_y_start, self.given_x_indices_of_y, float(self.grad_factor))
+        same = self.weights.dtype == x.dtype and x.dtype in (torch.float16, torch.float32, torch.float64)
+        mixed = self.weights.dtype == torch.float32 and x.dtype in (torch.float16, torch.float64)
         if self.training:
-            same = self.weights.dtype == x.dtype
-            mixed = self.weights.dtype == torch.float32 and x.dtype in (torch.float16, torch.float64)
             if (same or mixed) and x.shape[1] > 0:
                 # softmax and its backward run inside the layer kernels; fp32 weights next to half / double
                 # activations (the reference's --training-bit-count 16 / 64) are read as they are
@@ -120,6 +120,10 @@ class LogicLayer(torch.nn.Module):
             w = torch.nn.functional.softmax(self.weights, dim=-1).to(x.dtype)
             return LogicLayerCudaFunction.apply(x, a, b, w, *tail, self._train_schedule()).transpose(0, 1)
         # eval mode: the discretised net on float inputs (no gradients)
+        if (same or mixed) and self.weights.is_cuda and self.weights.is_contiguous():
+            with torch.no_grad():
+                return difflogic_cuda.forward(x, a, b, self.weights.detach(), self._train_schedule(),
+                                              argmax=True).transpose(0, 1)
         w = torch.nn.functional.one_hot(self.weights.argmax(-1), 16).to(x.dtype)
         with torch.no_grad():
             return difflogic_cuda.forward(x, a, b, w, self._train_schedule()).transpose(0, 1)

@@ -108,8 +108,10 @@ def _p(t):
     return t.data_ptr()
 
 
-def forward(x, a, b, w, schedule=None):
+def forward(x, a, b, w, schedule=None, argmax=False):
     """x [in,B], a/b [out] int64, w [out,16] -> y [out,B]   (difflogic.cpp:46-51).
+    ``argmax`` (not in the reference): ``forward(x, a, b, one_hot(w.argmax(-1), 16).to(x.dtype))``, the argmax taken
+    in the kernel; ``w`` of x's dtype or float32.
     ``schedule`` (an EvalSchedule of (a, b); not in the reference) selects the chained kernel:
     same result, one gathered input row per neuron instead of two."""
     for t, n in ((x, "x"), (a, "a"), (b, "b"), (w, "w")):
@@ -117,7 +119,7 @@ def forward(x, a, b, w, schedule=None):
     if x.dim() != 2 or w.dim() != 2 or w.shape[1] != 16:
         raise RuntimeError(f"expected x [in,B] and w [out,16], got {tuple(x.shape)} {x.dtype}, "
                            f"{tuple(w.shape)} {w.dtype}")
-    code = _layer_code(x, w, "logic_layer_cuda_forward")
+    code = _layer_code(x, w, "logic_layer_cuda_forward") | (_lib.DL_GATES_OF_ARGMAX if argmax else 0)
     out_dim = w.shape[0]
     _check_index(a, "a", out_dim)
     _check_index(b, "b", out_dim)

@@ -58,6 +58,11 @@ typedef enum dl_dtype { DL_F16 = 0, DL_F32 = 1, DL_F64 = 2, DL_F16_W32 = 3, DL_F
  * these return DL_ERR_TOO_LARGE for such rows).  The workspace stays 16-byte aligned. */
 #define DL_ROWS_ANY 0x100
 
+/* Or'ed into `dtype` of dl_logic_forward and dl_logic_forward_chained (probs NULL): `w` holds weights of which
+ * each neuron's argmax gate counts alone, as if w were one_hot(argmax(w)) (the first of equals, a NaN above every
+ * number): the discretised net on float inputs, difflogic/difflogic.py:128-131. */
+#define DL_GATES_OF_ARGMAX 0x200
+
 /* Library version (major*10000 + minor*100 + patch) and a static message per status. */
 int dl_version(void);
 const char *dl_status_string(int status);
