@@ -36,6 +36,7 @@ SIGNATURES = {
     "dl_logic_forward_chained": [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp],
     "dl_logic_backward_w_chained": [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp],
     "dl_logic_backward_x": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _dbl, _int, _vp],
+    "dl_logic_backward_both": [_vp, _vp, _vp, _vp, _vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _dbl, _int, _vp],
     "dl_backward_schedule_build": [_vp, _vp, _i64, _i64, _vp, _vp, _vp, ctypes.POINTER(_i64)],
     "dl_logic_backward_chained": [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _int, _vp, _vp, _i64, _i64, _vp, _vp, _vp,
                                   _i64, _i64, _i64, _dbl, _int, _vp],

@@ -234,6 +234,11 @@ class LogicLayerCudaFunction(torch.autograd.Function):
             both = difflogic_cuda.backward_chained(x, w, grad_y, ctx.schedule, ctx.grad_factor, any_rows=True)
             if both is not None:
                 return both[1], None, None, both[0], None, None, None, None
+        if (ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is None and x.numel() > 0
+                and grad_y.numel() > 0):
+            grad_w, grad_x = difflogic_cuda.backward_both(x, a, b, w, grad_y, given_x_indices_of_y_start,
+                                                          given_x_indices_of_y, ctx.grad_factor)
+            return grad_x, None, None, grad_w, None, None, None, None
         if ctx.needs_input_grad[0]:
             grad_x = difflogic_cuda.backward_x(x, a, b, w, grad_y, given_x_indices_of_y_start,
                                                given_x_indices_of_y, ctx.grad_factor)
@@ -266,6 +271,10 @@ class LogicLayerLogitsFunction(torch.autograd.Function):
                                                    softmax_backward=True, any_rows=True)
             if both is not None:
                 return both[1], None, None, both[0], None, None, None, None
+        if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is None and grad_y.numel() > 0:
+            grad_logits, grad_x = difflogic_cuda.backward_both(x, a, b, probs, grad_y, given_x_indices_of_y_start,
+                                                               given_x_indices_of_y, ctx.grad_factor, softmax_backward=True)
+            return grad_x, None, None, grad_logits, None, None, None, None
         if ctx.needs_input_grad[0]:
             grad_x = difflogic_cuda.backward_x(x, a, b, probs, grad_y, given_x_indices_of_y_start,
                                                given_x_indices_of_y, ctx.grad_factor)

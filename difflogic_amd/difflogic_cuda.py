@@ -201,6 +201,36 @@ def backward_x(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indices_o
     return grad_x
 
 
+def backward_both(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indices_of_y, scale=1.0, softmax_backward=False):
+    """backward_w (or backward_logits when ``softmax_backward``; ``w`` are then the probabilities that forward_logits
+    returned) and backward_x in one launch: (grad_w [out,16] of w's dtype, grad_x [in,B]), the values of the two.  Not
+    part of the reference's extension."""
+    for t, n in ((x, "x"), (a, "a"), (b, "b"), (w, "w"), (grad_y, "grad_y"),
+                 (given_x_indices_of_y_start, "given_x_indices_of_y_start"),
+                 (given_x_indices_of_y, "given_x_indices_of_y")):
+        _check_input(t, n)
+    if (x.dim() != 2 or grad_y.dim() != 2 or grad_y.shape[1] != x.shape[1] or grad_y.dtype != x.dtype
+            or w.dim() != 2 or w.shape != (grad_y.shape[0], 16) or 0 in x.shape or 0 in grad_y.shape):
+        raise RuntimeError(f"expected x [in>0,B>0], w [out,16], grad_y [out>0,B] of one dtype, got {tuple(x.shape)}, "
+                           f"{tuple(w.shape)}, {tuple(grad_y.shape)}")
+    code = _layer_code(x, w, "logic_layer_cuda_backward")
+    in_dim, batch = x.shape
+    out_dim = grad_y.shape[0]
+    _check_index(a, "a", out_dim)
+    _check_index(b, "b", out_dim)
+    _check_index(given_x_indices_of_y_start, "given_x_indices_of_y_start", in_dim + 1)
+    _check_index(given_x_indices_of_y, "given_x_indices_of_y", 2 * out_dim)
+    dev = _same_device(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indices_of_y)
+    grad_w, grad_x = torch.empty_like(w), torch.empty_like(x)
+    with _on(dev):
+        st = _lib.load().dl_logic_backward_both(_p(x), _p(a), _p(b), _p(w), _p(grad_y), 1 if softmax_backward else 0,
+                                                _p(given_x_indices_of_y_start), _p(given_x_indices_of_y), _p(grad_w),
+                                                _p(grad_x), in_dim, out_dim, batch, 0, float(scale), code, _stream(dev))
+    if st:
+        _raise(st, "logic_layer_cuda_backward_both")
+    return grad_w, grad_x
+
+
 def forward_logits(x, a, b, logits, schedule=None):
     """``forward(x, a, b, softmax(logits, -1))`` with the softmax computed inside the kernel.
     Returns (y [out,B], probs [out,16]); ``probs`` feeds backward_x / backward_logits.  Not part of
@@ -1218,6 +1248,16 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
                 return grad_w, grad_x
             if st != _lib.DL_ERR_TOO_LARGE:
                 _raise(st, "logic_layer_cuda_backward_chained_grouped")
+    if want_x and want_w:
+        _check_index(start, "given_x_indices_of_y_start", in_dim + 1)
+        _check_index(idx, "given_x_indices_of_y", 2 * out_dim)
+        grad_w, grad_x = torch.empty_like(probs), torch.empty_like(x)
+        with _on(dev):
+            st = lib.dl_logic_backward_both(_p(x), _p(a), _p(b), _p(probs), _p(grad_cls), 1, _p(start), _p(idx), _p(grad_w),
+                                            _p(grad_x), in_dim, out_dim, batch, k, float(scale), code, _stream(dev))
+        if st:
+            _raise(st, "logic_layer_cuda_backward_both")
+        return grad_w, grad_x
     grad_w = grad_x = None
     with _on(dev):
         if want_x:

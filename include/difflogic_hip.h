@@ -134,6 +134,13 @@ int dl_logic_backward_x(const void *x, const int64_t *a, const int64_t *b, const
                         int64_t in_dim, int64_t out_dim, int64_t batch, double scale, int dtype,
                         void *stream);
 
+/* dl_logic_backward_w (softmax_backward: dl_logic_backward_logits with probs = w) and dl_logic_backward_x in one launch; the
+ * same results.  k > 0: grad_y is the [k, batch] gradient of the class sums above the layer, as
+ * dl_logic_backward_x_grouped takes it; k = 0: grad_y is [out_dim, batch].  in_dim, out_dim, batch >= 1. */
+int dl_logic_backward_both(const void *x, const int64_t *a, const int64_t *b, const void *w, const void *grad_y,
+                           int softmax_backward, const int64_t *start, const int64_t *idx, void *grad_w, void *grad_x,
+                           int64_t in_dim, int64_t out_dim, int64_t batch, int64_t k, double scale, int dtype, void *stream);
+
 /* backward_w and backward_x of one layer in a single pass along the schedule (the pair
  * difflogic/difflogic.py:218,220): every neuron's input rows and grad_y row are read once and
  * serve grad_w and both grad_x contributions.  No counterpart in the reference.

@@ -105,3 +105,30 @@ def test_two_layers_at_once_on_rows_of_any_length(ext, monkeypatch, dtype, batch
     for x in (y1, None) if dtype != torch.float16 else (y1,):        # None: the inner rows are recomputed
         both = ext.backward_chained_lower(x, p1, gy, sched, x0, a0, b0, p0, softmax_backward=True, any_rows=True)
         assert ok(both[0], gw) and ok(both[1], gw0)
+
+
+@pytest.mark.parametrize("dtype,wdtype", [(d, d) for d in DTYPES] + [(torch.float16, torch.float32), (torch.float64, torch.float32)])
+@pytest.mark.parametrize("in_dim,out_dim,batch", [(1, 1, 1), (30, 44, 3), (5, 9, 17), (33, 50, 128), (30, 44, 515), (64, 40, 2048),
+                                                  (20, 24, 4100)])
+def test_both_gradients_in_one_launch(ext, dtype, wdtype, in_dim, out_dim, batch):
+    """backward_both is backward_x and backward_w / backward_logits, bit for bit; rows of every kind, one and several
+    column tiles, the batch split over the workgroup's waves, a layer under a GroupSum."""
+    from difflogic_amd.functional import build_reverse_index
+    g = torch.Generator().manual_seed(batch + out_dim)
+    a, b = (torch.randint(0, in_dim, (out_dim,), generator=g) for _ in range(2))
+    start, idx = (t.cuda() for t in build_reverse_index(a, b, in_dim))
+    a, b = a.cuda(), b.cuda()
+    x = torch.rand(in_dim, batch, generator=g).to(dtype).cuda()
+    gy = torch.randn(out_dim, batch, generator=g).to(dtype).cuda()
+    p = torch.softmax(torch.randn(out_dim, 16, generator=g), -1).to(wdtype).cuda()
+    gx = ext.backward_x(x, a, b, p, gy, start, idx, 1.5)
+    gw, gx2 = ext.backward_both(x, a, b, p, gy, start, idx, 1.5, softmax_backward=True)
+    assert torch.equal(gx2, gx) and torch.equal(gw, ext.backward_logits(x, a, b, gy, p))
+    if wdtype == dtype:
+        gw, gx2 = ext.backward_both(x, a, b, p, gy, start, idx, 1.5)
+        assert torch.equal(gx2, gx) and torch.equal(gw, ext.backward_w(x, a, b, gy))
+        k = 4 if out_dim % 4 == 0 else 1
+        gc = torch.randn(k, batch, generator=g).to(dtype).cuda()
+        gl, gx2 = ext.backward_group_sum(x, a, b, p, gc, start, idx, None, 1.5, True, True)
+        assert torch.equal(gx2, ext.backward_group_sum(x, a, b, p, gc, start, idx, None, 1.5, True, False)[1])
+        assert torch.equal(gl, ext.backward_group_sum(x, a, b, p, gc, start, idx, None, 1.5, False, True)[0])
