@@ -77,6 +77,30 @@ def _stream(dev):
     return torch.cuda.current_stream(dev).cuda_stream
 
 
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)      # a CUDA tensor at hand: initialised
+
+
+def _ready(index, tensors):
+    """Whether all tensors are contiguous CUDA tensors on device ``index``: what the checks below ask one by one, in one
+    loop for the calls that a step makes per layer (which are bound by the host).  Where it says no, they raise."""
+    for t in tensors:
+        if not (t.is_cuda and t.is_contiguous() and t.get_device() == index):
+            return False
+    return True
+
+
+def _is_index(t, numel):
+    return t.dtype is torch.int64 and t.dim() == 1 and t.shape[0] == numel
+
+
+def _launch(index, fn, *args):
+    """``fn(*args, current stream of device index)`` with that device current."""
+    if _current_device() == index:
+        return fn(*args, _raw_stream(index) if _raw_stream is not None else torch.cuda.current_stream(index).cuda_stream)
+    with torch.cuda.device(index):
+        return fn(*args, torch.cuda.current_stream(index).cuda_stream)
+
+
 class _NoGuard:
     def __enter__(self):
         return None
@@ -90,7 +114,7 @@ _NO_GUARD = _NoGuard()
 
 def _on(dev):
     """Device guard for a launch: nothing to do when ``dev`` is already current."""
-    if dev.index is None or torch.cuda.current_device() == dev.index:
+    if dev.index is None or _current_device() == dev.index:
         return _NO_GUARD
     return torch.cuda.device(dev)
 
@@ -205,7 +229,10 @@ def backward_both(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indice
     """backward_w (or backward_logits when ``softmax_backward``; ``w`` are then the probabilities that forward_logits
     returned) and backward_x in one launch: (grad_w [out,16] of w's dtype, grad_x [in,B]), the values of the two.  Not
     part of the reference's extension."""
-    for t, n in ((x, "x"), (a, "a"), (b, "b"), (w, "w"), (grad_y, "grad_y"),
+    start, idx = given_x_indices_of_y_start, given_x_indices_of_y
+    index = x.get_device()
+    ready = _ready(index, (x, a, b, w, grad_y, start, idx))
+    for t, n in () if ready else ((x, "x"), (a, "a"), (b, "b"), (w, "w"), (grad_y, "grad_y"),
                  (given_x_indices_of_y_start, "given_x_indices_of_y_start"),
                  (given_x_indices_of_y, "given_x_indices_of_y")):
         _check_input(t, n)
@@ -216,16 +243,17 @@ def backward_both(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indice
     code = _layer_code(x, w, "logic_layer_cuda_backward")
     in_dim, batch = x.shape
     out_dim = grad_y.shape[0]
-    _check_index(a, "a", out_dim)
-    _check_index(b, "b", out_dim)
-    _check_index(given_x_indices_of_y_start, "given_x_indices_of_y_start", in_dim + 1)
-    _check_index(given_x_indices_of_y, "given_x_indices_of_y", 2 * out_dim)
-    dev = _same_device(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indices_of_y)
+    if not (ready and _is_index(a, out_dim) and _is_index(b, out_dim) and _is_index(start, in_dim + 1)
+            and _is_index(idx, 2 * out_dim)):
+        _check_index(a, "a", out_dim)
+        _check_index(b, "b", out_dim)
+        _check_index(start, "given_x_indices_of_y_start", in_dim + 1)
+        _check_index(idx, "given_x_indices_of_y", 2 * out_dim)
+        _same_device(x, a, b, w, grad_y, start, idx)
     grad_w, grad_x = torch.empty_like(w), torch.empty_like(x)
-    with _on(dev):
-        st = _lib.load().dl_logic_backward_both(_p(x), _p(a), _p(b), _p(w), _p(grad_y), 1 if softmax_backward else 0,
-                                                _p(given_x_indices_of_y_start), _p(given_x_indices_of_y), _p(grad_w),
-                                                _p(grad_x), in_dim, out_dim, batch, 0, float(scale), code, _stream(dev))
+    st = _launch(index, _lib.load().dl_logic_backward_both, x.data_ptr(), a.data_ptr(), b.data_ptr(), w.data_ptr(),
+                 grad_y.data_ptr(), 1 if softmax_backward else 0, start.data_ptr(), idx.data_ptr(), grad_w.data_ptr(),
+                 grad_x.data_ptr(), in_dim, out_dim, batch, 0, float(scale), code)
     if st:
         _raise(st, "logic_layer_cuda_backward_both")
     return grad_w, grad_x
@@ -239,30 +267,32 @@ def forward_logits(x, a, b, logits, schedule=None):
     and so is what backward_logits / backward_chained return for them).
     ``schedule`` (an EvalSchedule of (a, b)) selects the chained kernel: same result, one
     gathered input row per neuron instead of two."""
-    for t, n in ((x, "x"), (a, "a"), (b, "b"), (logits, "logits")):
-        _check_input(t, n)
+    index = x.get_device()
+    ready = _ready(index, (x, a, b, logits))
+    if not ready:
+        for t, n in ((x, "x"), (a, "a"), (b, "b"), (logits, "logits")):
+            _check_input(t, n)
     if x.dim() != 2 or logits.dim() != 2 or logits.shape[1] != 16 or x.shape[1] == 0:
         raise RuntimeError(f"expected x [in,B>0] and logits [out,16], got {tuple(x.shape)} {x.dtype}, "
                            f"{tuple(logits.shape)} {logits.dtype}")
     code = _layer_code(x, logits, "logic_layer_cuda_forward")
     out_dim = logits.shape[0]
-    _check_index(a, "a", out_dim)
-    _check_index(b, "b", out_dim)
-    dev = _same_device(x, a, b, logits)
+    if not (ready and _is_index(a, out_dim) and _is_index(b, out_dim)):
+        _check_index(a, "a", out_dim)
+        _check_index(b, "b", out_dim)
+        _same_device(x, a, b, logits)
     in_dim, batch = x.shape
-    y = torch.empty((out_dim, batch), dtype=x.dtype, device=dev)
-    probs = torch.empty((out_dim, 16), dtype=logits.dtype, device=dev)
+    y, probs = x.new_empty((out_dim, batch)), torch.empty_like(logits)
     lib = _lib.load()
-    with _on(dev):
-        st = _lib.DL_ERR_TOO_LARGE
-        if schedule is not None and out_dim > 0:
-            _check_schedule(schedule, in_dim, out_dim, dev)
-            st = lib.dl_logic_forward_chained(_p(x), _p(schedule.verts), _p(schedule.neuron), _p(schedule.flip),
-                                              schedule.steps, _p(logits), _p(y), _p(probs), in_dim, out_dim, batch, code,
-                                              _stream(dev))
-        if st == _lib.DL_ERR_TOO_LARGE:
-            st = lib.dl_logic_forward_logits(_p(x), _p(a), _p(b), _p(logits), _p(y), _p(probs), in_dim, out_dim, batch,
-                                             code, _stream(dev))
+    st = _lib.DL_ERR_TOO_LARGE
+    if schedule is not None and out_dim > 0:
+        _check_schedule(schedule, in_dim, out_dim, x.device)
+        st = _launch(index, lib.dl_logic_forward_chained, x.data_ptr(), schedule.verts.data_ptr(), schedule.neuron.data_ptr(),
+                     schedule.flip.data_ptr(), schedule.steps, logits.data_ptr(), y.data_ptr(), probs.data_ptr(), in_dim,
+                     out_dim, batch, code)
+    if st == _lib.DL_ERR_TOO_LARGE:
+        st = _launch(index, lib.dl_logic_forward_logits, x.data_ptr(), a.data_ptr(), b.data_ptr(), logits.data_ptr(),
+                     y.data_ptr(), probs.data_ptr(), in_dim, out_dim, batch, code)
     if st:
         _raise(st, "logic_layer_cuda_forward_logits")
     return y, probs
@@ -278,7 +308,9 @@ def backward_logits(x, a, b, grad_y, probs, schedule=None):
     """Gradient with respect to the gate logits: backward_w chained with the softmax backward,
     ``p * (g - (p * g).sum(-1, keepdim=True))`` with ``g = backward_w(x, a, b, grad_y)``.
     ``schedule`` selects the chained kernel (bit-identical result)."""
-    for t, n in ((x, "x"), (a, "a"), (b, "b"), (grad_y, "grad_y"), (probs, "probs")):
+    index = x.get_device()
+    ready = _ready(index, (x, a, b, grad_y, probs))
+    for t, n in () if ready else ((x, "x"), (a, "a"), (b, "b"), (grad_y, "grad_y"), (probs, "probs")):
         _check_input(t, n)
     if (x.dim() != 2 or grad_y.dim() != 2 or grad_y.shape[1] != x.shape[1] or grad_y.dtype != x.dtype
             or probs.shape != (grad_y.shape[0], 16)):
@@ -286,22 +318,22 @@ def backward_logits(x, a, b, grad_y, probs, schedule=None):
                            f"{tuple(grad_y.shape)}, {tuple(probs.shape)}")
     code = _layer_code(x, probs, "logic_layer_cuda_backward_w")
     out_dim = grad_y.shape[0]
-    _check_index(a, "a", out_dim)
-    _check_index(b, "b", out_dim)
-    dev = _same_device(x, a, b, grad_y, probs)
+    if not (ready and _is_index(a, out_dim) and _is_index(b, out_dim)):
+        _check_index(a, "a", out_dim)
+        _check_index(b, "b", out_dim)
+        _same_device(x, a, b, grad_y, probs)
     in_dim, batch = x.shape
-    grad_logits = torch.empty((out_dim, 16), dtype=probs.dtype, device=dev)
+    grad_logits = torch.empty_like(probs)
     lib = _lib.load()
-    with _on(dev):
-        st = _lib.DL_ERR_TOO_LARGE
-        if schedule is not None and out_dim > 0 and batch > 0:
-            _check_schedule(schedule, in_dim, out_dim, dev)
-            st = lib.dl_logic_backward_w_chained(_p(x), _p(schedule.verts), _p(schedule.neuron), _p(schedule.flip),
-                                                 schedule.steps, _p(grad_y), _p(probs), _p(grad_logits), in_dim, out_dim,
-                                                 batch, code, _stream(dev))
-        if st == _lib.DL_ERR_TOO_LARGE:
-            st = lib.dl_logic_backward_logits(_p(x), _p(a), _p(b), _p(grad_y), _p(probs), _p(grad_logits), in_dim,
-                                              out_dim, batch, code, _stream(dev))
+    st = _lib.DL_ERR_TOO_LARGE
+    if schedule is not None and out_dim > 0 and batch > 0:
+        _check_schedule(schedule, in_dim, out_dim, x.device)
+        st = _launch(index, lib.dl_logic_backward_w_chained, x.data_ptr(), schedule.verts.data_ptr(),
+                     schedule.neuron.data_ptr(), schedule.flip.data_ptr(), schedule.steps, grad_y.data_ptr(),
+                     probs.data_ptr(), grad_logits.data_ptr(), in_dim, out_dim, batch, code)
+    if st == _lib.DL_ERR_TOO_LARGE:
+        st = _launch(index, lib.dl_logic_backward_logits, x.data_ptr(), a.data_ptr(), b.data_ptr(), grad_y.data_ptr(),
+                     probs.data_ptr(), grad_logits.data_ptr(), in_dim, out_dim, batch, code)
     if st:
         _raise(st, "logic_layer_cuda_backward_logits")
     return grad_logits
@@ -313,14 +345,17 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
     (grad_w [out,16], grad_x [in,B]), or None where the fused pass does not apply (the caller
     then uses the separate functions).  ``any_rows``: rows that are not whole 16-byte vectors are taken as well
     (False: None for them).  Not part of the reference's extension."""
-    for t, n in ((x, "x"), (w, "w"), (grad_y, "grad_y")):
-        _check_input(t, n)
+    index = x.get_device()
+    ready = _ready(index, (x, w, grad_y))
+    if not ready:
+        for t, n in ((x, "x"), (w, "w"), (grad_y, "grad_y")):
+            _check_input(t, n)
     if (x.dim() != 2 or grad_y.dim() != 2 or grad_y.shape[1] != x.shape[1] or grad_y.dtype != x.dtype
             or w.shape != (grad_y.shape[0], 16)):
         raise RuntimeError(f"expected x [in,B], w [out,16], grad_y [out,B] of one dtype, got {tuple(x.shape)}, "
                            f"{tuple(w.shape)}, {tuple(grad_y.shape)}")
     code = _layer_code(x, w, "logic_layer_cuda_backward") | (_lib.DL_ROWS_ANY if any_rows else 0)
-    dev = _same_device(x, w, grad_y)
+    dev = x.device if ready else _same_device(x, w, grad_y)
     in_dim, batch = x.shape
     out_dim = grad_y.shape[0]
     if in_dim == 0 or out_dim == 0 or batch == 0:
@@ -329,19 +364,18 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
     dst, fix_vertex, fix_start, n_fix, rows = schedule.backward_plan()
     if rows > in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
         return None
-    grad_w = torch.empty((out_dim, 16), dtype=w.dtype, device=dev)
-    grad_x = torch.empty_like(x)
+    grad_w, grad_x = torch.empty_like(w), torch.empty_like(x)
     lib = _lib.load()
     ws_bytes = lib.dl_logic_backward_chained_workspace_bytes(rows, out_dim, batch, code)
     if ws_bytes < 0:
         _raise(-ws_bytes, "logic_layer_cuda_backward_chained")
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    with _on(dev):
-        st = lib.dl_logic_backward_chained(
-            _p(x), _p(schedule.verts), _p(schedule.neuron), _p(schedule.flip), _p(dst), schedule.steps, _p(w),
-            _p(grad_y), 1 if softmax_backward else 0, _p(fix_vertex) if n_fix else None,
-            _p(fix_start) if n_fix else None, n_fix, rows, _p(grad_w), _p(grad_x),
-            _p(workspace) if ws_bytes else None, in_dim, out_dim, batch, float(scale), code, _stream(dev))
+    st = _launch(
+        index, lib.dl_logic_backward_chained, x.data_ptr(), schedule.verts.data_ptr(), schedule.neuron.data_ptr(),
+        schedule.flip.data_ptr(), dst.data_ptr(), schedule.steps, w.data_ptr(), grad_y.data_ptr(),
+        1 if softmax_backward else 0, fix_vertex.data_ptr() if n_fix else None, fix_start.data_ptr() if n_fix else None,
+        n_fix, rows, grad_w.data_ptr(), grad_x.data_ptr(), workspace.data_ptr() if ws_bytes else None, in_dim, out_dim,
+        batch, float(scale), code)
     if st == _lib.DL_ERR_TOO_LARGE:
         return None
     if st:
@@ -495,21 +529,24 @@ def gate_ids(weights):
 def eval_weights(x, a, b, weights):
     """``eval(x, a, b, gate_ids(weights))`` in one kernel, on rows ``x`` int64 [in, W] of whole 16-byte vectors (W even).
     Not part of the reference's extension; PackBitsTensor uses it for short rows."""
-    _check_input(x, "x")
-    _check_input(weights, "weights")
+    index = x.get_device()
+    ready = _ready(index, (x, a, b, weights))
+    if not ready:
+        _check_input(x, "x")
+        _check_input(weights, "weights")
     code = _float_code(weights, "gate_ids")
     if x.dim() != 2 or x.dtype != torch.int64 or x.shape[1] % 2 or weights.dim() != 2 or weights.shape[1] != 16:
         raise RuntimeError(f"expected x [in,W] int64 with W even and weights [out,16], got {tuple(x.shape)} {x.dtype}, "
                            f"{tuple(weights.shape)}")
     out_dim = weights.shape[0]
-    _check_index(a, "a", out_dim)
-    _check_index(b, "b", out_dim)
-    dev = _same_device(x, a, b, weights)
+    if not (ready and _is_index(a, out_dim) and _is_index(b, out_dim)):
+        _check_index(a, "a", out_dim)
+        _check_index(b, "b", out_dim)
+        _same_device(x, a, b, weights)
     in_dim, words = x.shape
-    y = torch.empty((out_dim, words), dtype=torch.int64, device=dev)
-    with _on(dev):
-        st = _lib.load().dl_logic_eval_weights(_p(x), _p(a), _p(b), _p(weights), code, _p(y), in_dim, out_dim, words * 8,
-                                               _stream(dev))
+    y = x.new_empty((out_dim, words))
+    st = _launch(index, _lib.load().dl_logic_eval_weights, x.data_ptr(), a.data_ptr(), b.data_ptr(), weights.data_ptr(), code,
+                 y.data_ptr(), in_dim, out_dim, words * 8)
     if st:
         _raise(st, "logic_eval_weights")
     return y
@@ -520,22 +557,27 @@ def gate_ids_folded(weights, a, b, state=None):
     ``a``, ``b`` whose input rows are constant where ``state`` says so (uint8 [in]: 0 varies, 1 all zeros, 2 all
     ones; None: all vary).  ``ids`` uint8 [out] are the argmax gates with those constants folded in, ``state_out``
     uint8 [out] the constants among the layer's outputs.  Not part of the reference's extension."""
-    _check_input(weights, "weights")
+    index = weights.get_device()
+    ready = _ready(index, (weights, a, b) if state is None else (weights, a, b, state))
+    if not ready:
+        _check_input(weights, "weights")
     code = _float_code(weights, "gate_ids")
     if weights.dim() != 2 or weights.shape[1] != 16:
         raise RuntimeError(f"expected weights [out,16], got {tuple(weights.shape)}")
     out_dim = weights.shape[0]
-    _check_index(a, "a", out_dim)
-    _check_index(b, "b", out_dim)
-    dev = _same_device(weights, a, b) if state is None else _same_device(weights, a, b, state)
+    if not (ready and _is_index(a, out_dim) and _is_index(b, out_dim)):
+        _check_index(a, "a", out_dim)
+        _check_index(b, "b", out_dim)
+        _same_device(weights, a, b) if state is None else _same_device(weights, a, b, state)
     if state is not None:
-        _check_input(state, "state")
+        if not ready:
+            _check_input(state, "state")
         if state.dtype != torch.uint8 or state.dim() != 1:
             raise RuntimeError(f"expected state [in] uint8, got {tuple(state.shape)} {state.dtype}")
-    both = torch.empty((2, out_dim), dtype=torch.uint8, device=dev)
-    with _on(dev):
-        st = _lib.load().dl_gate_ids_folded(_p(weights), code, _p(a), _p(b), _p(state) if state is not None else None,
-                                            _p(both[0]), _p(both[1]), out_dim, _stream(dev))
+    both = torch.empty((2, out_dim), dtype=torch.uint8, device=weights.device)
+    ids = both.data_ptr()
+    st = _launch(index, _lib.load().dl_gate_ids_folded, weights.data_ptr(), code, a.data_ptr(), b.data_ptr(),
+                 state.data_ptr() if state is not None else None, ids, ids + out_dim, out_dim)
     if st:
         _raise(st, "gate_ids_folded")
     return both[0], both[1]
