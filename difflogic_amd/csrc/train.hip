@@ -499,7 +499,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_x_kernel(const T *__restric
 
 // Both gradients of a layer in one launch, the first `x_blocks` workgroups (input rows x column tiles) as
 // backward_x_kernel, the others as backward_w_kernel: the two do not depend on each other, and on the small layers that
-// have no schedule each takes about as long as its launch and one chain of dependent loads. 
+// have no schedule each takes about as long as its launch and one chain of dependent loads.
 // 8000 -> 8000 at batch 128: 6.8 + 3.8 us and a second launch -> 8.0; 30000 -> 30000 at 1024: 91 + 53 -> 138.
 template <typename T, int VEC, int NPW, int WPN, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_both_kernel(
@@ -1397,30 +1397,32 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
 }
 
 // One wave per 64 consecutive samples of one class; the four waves of a workgroup take
-// interleaved splits and are added in wave order, so the summation order is fixed.
+// interleaved splits and are added in wave order, so the summation order is fixed.  The partial sums are added and divided
+// in double and rounded once: a score of 64 is 8e-6 from its neighbours, which is what the gradients of a net with large
+// class sums see.
 template <typename T>
 __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typename Acc<T>::type *__restrict__ partial,
                                                                     T *__restrict__ y, int64_t batch, int64_t k,
-                                                                    int splits, typename Acc<T>::type inv_tau) {
+                                                                    int splits, double tau) {
     typedef typename Acc<T>::type C;
-    __shared__ C lds[4][DL_WAVE];
+    __shared__ double lds[4][DL_WAVE];
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t r = (int64_t) blockIdx.x * DL_WAVE + lane;
     const int64_t c = blockIdx.y;
-    C sum = (C) 0;
+    double sum = 0.0;
     if (r < batch)
         for (int s = wave; s < splits; s += 32) {                // eight partial sums in flight, added in order
             C v[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = s + 4 * i < splits ? partial[((int64_t) (s + 4 * i) * k + c) * batch + r] : (C) 0;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) sum += v[i];
+            for (int i = 0; i < 8; ++i) sum += (double) v[i];
         }
     lds[wave][lane] = sum;
     __syncthreads();
     if (wave == 0 && r < batch)
-        y[r * k + c] = down<T, C>(((lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane])) * inv_tau);
+        y[r * k + c] = down<T, C>((C) (((lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane])) / tau));
 }
 
 template <typename T, int VEC, bool RAG>
@@ -1474,7 +1476,7 @@ int group_sum_forward_t(const void *x, void *y, void *workspace, int64_t out_dim
     const int64_t blocks = dl_ceil_div(batch, DL_WAVE);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     DL_LAUNCH((group_sum_finish_kernel<T>), dim3((unsigned) blocks, (unsigned) k), dim3(DL_BLOCK), 0, s,
-                       (const C *) workspace, (T *) y, batch, k, splits, (C) (1.0 / tau));
+                       (const C *) workspace, (T *) y, batch, k, splits, tau);
     return dl_launch_status();
 }
 
@@ -1529,7 +1531,7 @@ int forward_group_sum_t(const void *x, const int64_t *a, const int64_t *b, const
     const int64_t blocks = dl_ceil_div(batch, DL_WAVE);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     DL_LAUNCH((group_sum_finish_kernel<T>), dim3((unsigned) blocks, (unsigned) k), dim3(DL_BLOCK), 0, s,
-                       (const C *) workspace, (T *) y, batch, k, splits, (C) (1.0 / tau));
+                       (const C *) workspace, (T *) y, batch, k, splits, tau);
     return dl_launch_status();
 }
 
