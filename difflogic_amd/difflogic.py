@@ -116,17 +116,17 @@ class LogicLayer(torch.nn.Module):
                 # softmax and its backward run inside the layer kernels; fp32 weights next to half / double
                 # activations (the reference's --training-bit-count 16 / 64) are read as they are
                 return LogicLayerLogitsFunction.apply(x, a, b, self.weights, *tail,
-                                                      self._train_schedule()).transpose(0, 1)
+                                                      self._train_schedule(x)).transpose(0, 1)
             w = torch.nn.functional.softmax(self.weights, dim=-1).to(x.dtype)
-            return LogicLayerCudaFunction.apply(x, a, b, w, *tail, self._train_schedule()).transpose(0, 1)
+            return LogicLayerCudaFunction.apply(x, a, b, w, *tail, self._train_schedule(x)).transpose(0, 1)
         # eval mode: the discretised net on float inputs (no gradients)
         if (same or mixed) and self.weights.is_cuda and self.weights.is_contiguous():
             with torch.no_grad():
-                return difflogic_cuda.forward(x, a, b, self.weights.detach(), self._train_schedule(),
+                return difflogic_cuda.forward(x, a, b, self.weights.detach(), self._train_schedule(x),
                                               argmax=True).transpose(0, 1)
         w = torch.nn.functional.one_hot(self.weights.argmax(-1), 16).to(x.dtype)
         with torch.no_grad():
-            return difflogic_cuda.forward(x, a, b, w, self._train_schedule()).transpose(0, 1)
+            return difflogic_cuda.forward(x, a, b, w, self._train_schedule(x)).transpose(0, 1)
 
     def forward_cuda_eval(self, x: PackBitsTensor):
         """Packed inference.  Updates ``x`` in place (as the reference rebinds ``x.t``) and
@@ -149,15 +149,29 @@ class LogicLayer(torch.nn.Module):
     # Below this many inputs a 1 KB column tile of the whole input stays in the L2 caches and the
     # second gather of a row hits there; above it the chained kernels halve the gathered rows.
     _CHAIN_MIN_IN_DIM = 4096
-    # Narrower layers are latency-bound; a wave walking 8 neurons in sequence only lengthens that.
-    _CHAIN_MIN_OUT_DIM = 32768
+    # Narrower layers are latency-bound: a wave walking 8 neurons in sequence only lengthens that, unless their rows are
+    # long.  Backward along the schedule / without, square fp32 layers: 16000 wide at batch 32 12.1 / 10.8 us, 100 14.0 /
+    # 13.1, 256 16.7 / 22.1; 30000 at 32 15.1 / 19.6; 8000 at 256 13.4 / 12.1, 512 16.7 / 22.2; 2000 at 2048 22.2 / 21.9.
+    # Forward at 16000: batch 100 6.0 / 6.0, 256 7.7 / 8.9.
+    _CHAIN_MIN_OUT_DIM = 20000
+    _CHAIN_MIN_BYTES = 16_000_000           # ... of output rows: a quarter of the width is enough
 
-    def _train_schedule(self):
-        """Evaluation schedule of this layer's wiring for the chained forward / backward_w
-        kernels (cached per wiring), or None where chaining does not pay."""
-        if self.in_dim < self._CHAIN_MIN_IN_DIM or self.out_dim < self._CHAIN_MIN_OUT_DIM:
+    def _train_schedule(self, x=None):
+        """Evaluation schedule of this layer's wiring for the chained forward / backward kernels (cached per
+        wiring), or None where chaining does not pay on feature-major input like ``x`` (None: of any batch) or the schedule
+        would have to be built while a graph is being captured."""
+        if self.in_dim < self._CHAIN_MIN_IN_DIM:
             return None
-        return difflogic_cuda.schedule_for(self.indices[0], self.indices[1], self.in_dim)
+        if self.out_dim < self._CHAIN_MIN_OUT_DIM and (
+                x is None or 4 * self.out_dim < self._CHAIN_MIN_OUT_DIM
+                or self.out_dim * x.shape[1] * x.element_size() < self._CHAIN_MIN_BYTES):
+            return None
+        a, b = self.indices
+        schedule = difflogic_cuda.built_schedule(a, b, self.in_dim)
+        if schedule is not None and (not self.training or schedule._backward is not None):
+            return schedule
+        # building the schedule and its backward plan copies to and from the host
+        return None if torch.cuda.is_current_stream_capturing() else difflogic_cuda.schedule_for(a, b, self.in_dim)
 
     def _gate_ids(self):
         """uint8 [out_dim] argmax gate per neuron.  Recomputed on every call like the reference
@@ -356,7 +370,7 @@ class FusedLogicLayerGroupSum(torch.nn.Module):
         a, b = layer.indices
         return LogicLayerGroupSumFunction.apply(xt, a, b, layer.weights, layer.given_x_indices_of_y_start,
                                                 layer.given_x_indices_of_y, float(layer.grad_factor),
-                                                layer._train_schedule(), int(gs.k), float(gs.tau))
+                                                layer._train_schedule(xt), int(gs.k), float(gs.tau))
 
     def extra_repr(self):
         return "{}, {}".format(self.layer.extra_repr(), self.group_sum.extra_repr())
@@ -429,7 +443,8 @@ class FusedLogicLayerPair(torch.nn.Module):
     ``weights``; the second layer's ``weights`` stay registered at its own position (_LayerDone),
     so the state_dict keys are those of the unfused model.  Takes the fused path in training mode
     on float inputs that need no gradient when the second layer is wide enough to be walked along
-    its schedule; everything else runs the two layers one after the other."""
+    its schedule on any batch (narrower ones lose by it: 784 -> 4 x 8000 at batch 1024 346 us a step
+    with the layers apart, 393 as a pair); everything else runs the two layers one after the other."""
 
     def __init__(self, layer1: LogicLayer, layer2: LogicLayer):
         super().__init__()
@@ -458,10 +473,10 @@ class FusedLogicLayerPair(torch.nn.Module):
             return l2(l1(x))
         xt = x.transpose(0, 1).contiguous()
         assert xt.shape[0] == l1.in_dim, (xt.shape, l1.in_dim)
-        return LogicLayerPairFunction.apply(xt, l1.indices[0], l1.indices[1], l1.weights, l1._train_schedule(),
+        return LogicLayerPairFunction.apply(xt, l1.indices[0], l1.indices[1], l1.weights, l1._train_schedule(xt),
                                             l2.indices[0], l2.indices[1], l2.weights, l2.given_x_indices_of_y_start,
                                             l2.given_x_indices_of_y, float(l2.grad_factor),
-                                            l2._train_schedule()).transpose(0, 1)
+                                            l2._train_schedule(xt)).transpose(0, 1)
 
     def extra_repr(self):
         return "({}) -> ({})".format(self.layer1.extra_repr(), self.layer2.extra_repr())
@@ -597,6 +612,7 @@ class FusedSequential(torch.nn.Sequential):
     def _stages(self, mods, x):
         """The stages of LogicNetFunction for ``mods`` on feature-major input of x's kind, or None."""
         stages, i, first = [], 0, True
+        xt = x.t()                                           # (for its batch and element size)
         dtype = x.dtype
         while i < len(mods):
             m = mods[i]
@@ -609,18 +625,18 @@ class FusedSequential(torch.nn.Sequential):
                         return None
                 if pair_ok:
                     stages.append((LogicLayerPairFunction,
-                                   (None, l1.indices[0], l1.indices[1], l1.weights, l1._train_schedule(), l2.indices[0],
+                                   (None, l1.indices[0], l1.indices[1], l1.weights, l1._train_schedule(xt), l2.indices[0],
                                     l2.indices[1], l2.weights, l2.given_x_indices_of_y_start, l2.given_x_indices_of_y,
-                                    float(l2.grad_factor), l2._train_schedule()), (3, 7)))
+                                    float(l2.grad_factor), l2._train_schedule(xt)), (3, 7)))
                 else:
                     for layer in (l1, l2):
-                        st = self._layer_stage(layer, dtype)
+                        st = self._layer_stage(layer, dtype, xt)
                         if st is None:
                             return None
                         stages.append(st)
                 i += 2
             elif isinstance(m, LogicLayer):
-                st = self._layer_stage(m, dtype) if m.training and m.implementation == "cuda" else None
+                st = self._layer_stage(m, dtype, xt) if m.training and m.implementation == "cuda" else None
                 if st is None:
                     return None
                 stages.append(st)
@@ -633,12 +649,12 @@ class FusedSequential(torch.nn.Sequential):
                 if dtype == layer.weights.dtype:
                     stages.append((LogicLayerGroupSumFunction,
                                    (None, layer.indices[0], layer.indices[1], layer.weights, layer.given_x_indices_of_y_start,
-                                    layer.given_x_indices_of_y, float(layer.grad_factor), layer._train_schedule(), int(gs.k),
+                                    layer.given_x_indices_of_y, float(layer.grad_factor), layer._train_schedule(xt), int(gs.k),
                                     float(gs.tau)), (3,)))
                 else:
                     # half / double activations over fp32 weights: the layer takes them, the fused kernels of layer +
                     # GroupSum do not; the two run as stages of their own on the feature-major activation
-                    st = self._layer_stage(layer, dtype)
+                    st = self._layer_stage(layer, dtype, xt)
                     if st is None:
                         return None
                     stages += [st, (GroupSumCudaFunction, (None, int(gs.k), float(gs.tau)), ())]
@@ -650,13 +666,13 @@ class FusedSequential(torch.nn.Sequential):
         return stages if stages and stages[-1][0] in (LogicLayerGroupSumFunction, GroupSumCudaFunction) else None
 
     @staticmethod
-    def _layer_stage(layer, dtype):
+    def _layer_stage(layer, dtype, xt):
         w = layer.weights.dtype
         if not (w == dtype or (w == torch.float32 and dtype in (torch.float16, torch.float64))):
             return None
         return (LogicLayerLogitsFunction,
                 (None, layer.indices[0], layer.indices[1], layer.weights, layer.given_x_indices_of_y_start,
-                 layer.given_x_indices_of_y, float(layer.grad_factor), layer._train_schedule()), (3,))
+                 layer.given_x_indices_of_y, float(layer.grad_factor), layer._train_schedule(xt)), (3,))
 
     def forward(self, x):
         mods = list(self)

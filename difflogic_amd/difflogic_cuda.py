@@ -366,9 +366,7 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
         return None
     grad_w, grad_x = torch.empty_like(w), torch.empty_like(x)
     lib = _lib.load()
-    ws_bytes = lib.dl_logic_backward_chained_workspace_bytes(rows, out_dim, batch, code)
-    if ws_bytes < 0:
-        _raise(-ws_bytes, "logic_layer_cuda_backward_chained")
+    ws_bytes = schedule.backward_bytes(rows, batch, code)
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
     st = _launch(
         index, lib.dl_logic_backward_chained, x.data_ptr(), schedule.verts.data_ptr(), schedule.neuron.data_ptr(),
@@ -407,6 +405,8 @@ def forward_logits_lower(x_lower, a_lower, b_lower, logits_lower, logits, schedu
     if in0 == 0 or in_dim == 0 or out_dim == 0:
         return None
     _check_schedule(schedule, in_dim, out_dim, dev)
+    if batch * x_lower.element_size() > 2048:                # the kernel's limit: nothing is allocated or cleared for it
+        return None
     y = torch.empty((out_dim, batch), dtype=x_lower.dtype, device=dev)
     probs = torch.empty((out_dim, 16), dtype=x_lower.dtype, device=dev)
     # rows of lower neurons that feed nothing are never visited: zero probabilities give them a zero gradient
@@ -775,6 +775,7 @@ class EvalSchedule:
         self.flip = torch.from_numpy(flip[:steps].copy()).to(a.device)
         self._host = (verts[:steps + 1].copy(), neuron[:steps].copy())
         self._backward = None
+        self._backward_bytes = (None, 0)
         self._count_plans = {}
 
     def count_plan(self, k):
@@ -801,6 +802,17 @@ class EvalSchedule:
                 self._count_plans[k] = (torch.from_numpy(slot).to(dev), torch.from_numpy(runs.view(np.int16)).to(dev),
                                         int(got), int(blocks.value))
         return self._count_plans[k]
+
+    def backward_bytes(self, rows, batch, code):
+        """Workspace of the one-pass backward for rows of this batch and dtype (the last answer is kept)."""
+        key = (batch, code)
+        kept, nbytes = self._backward_bytes
+        if kept != key:
+            nbytes = _lib.load().dl_logic_backward_chained_workspace_bytes(rows, self.out_dim, batch, code)
+            if nbytes < 0:
+                _raise(-nbytes, "logic_layer_cuda_backward_chained")
+            self._backward_bytes = (key, nbytes)
+        return nbytes
 
     def backward_plan(self):
         """(dst, fix_vertex, fix_start, n_fix, overflow_rows) for backward_chained, built on first
@@ -843,11 +855,10 @@ class _WiringCache:
 
     def get(self, tensors, extra, build):
         import weakref
-        key = tuple((t.data_ptr(), t._version, t.shape[0]) for t in tensors) + tuple(extra)
-        with self._lock:
-            hit = self._entries.get(key)
-            if hit is not None and all(r() is t for r, t in zip(hit[0], tensors)):
-                return hit[1]
+        hit = self.peek(tensors, extra)
+        if hit is not None:
+            return hit
+        key = self._key(tensors, extra)
         value = build()
 
         def drop(_ref, key=key, cache=weakref.ref(self)):
@@ -865,6 +876,20 @@ class _WiringCache:
                 del self._entries[old]
             self._entries[key] = (tuple(weakref.ref(t, drop) for t in tensors), value)
         return value
+
+    @staticmethod
+    def _key(tensors, extra):
+        return tuple([(t.data_ptr(), t._version, t.shape[0]) for t in tensors]) + tuple(extra)
+
+    def peek(self, tensors, extra):
+        """What ``get`` would return without building it, or None.  (A lookup takes no lock: entries are never modified.)"""
+        hit = self._entries.get(self._key(tensors, extra))
+        if hit is not None:
+            for r, t in zip(hit[0], tensors):
+                if r() is not t:
+                    return None
+            return hit[1]
+        return None
 
     def __len__(self):
         return len(self._entries)
@@ -884,6 +909,11 @@ def schedule_for(a, b, in_dim):
     """The cached EvalSchedule of the wiring (a, b): lives as long as the tensors do, rebuilt when
     they are replaced or modified in place."""
     return _SCHEDULES.get((a, b), (int(in_dim),), lambda: EvalSchedule(a, b, in_dim))
+
+
+def built_schedule(a, b, in_dim):
+    """schedule_for if that has been built already, else None."""
+    return _SCHEDULES.peek((a, b), (int(in_dim),))
 
 
 def invalidate_wiring(*tensors):

@@ -132,3 +132,33 @@ def test_both_gradients_in_one_launch(ext, dtype, wdtype, in_dim, out_dim, batch
         gl, gx2 = ext.backward_group_sum(x, a, b, p, gc, start, idx, None, 1.5, True, True)
         assert torch.equal(gx2, ext.backward_group_sum(x, a, b, p, gc, start, idx, None, 1.5, True, False)[1])
         assert torch.equal(gl, ext.backward_group_sum(x, a, b, p, gc, start, idx, None, 1.5, False, True)[0])
+
+
+def test_layers_walk_their_schedule_where_their_rows_are_long(ext, monkeypatch):
+    """A layer too narrow for its schedule takes it on a batch whose rows are long enough; outputs and gradients are those
+    of the other kernels.  A schedule that has not been built is not built under graph capture."""
+    import difflogic_amd as dl
+    torch.manual_seed(2)
+    layer = dl.LogicLayer(5000, 6000, grad_factor=1.5)
+    long, short = torch.rand(668, 5000, device="cuda"), torch.rand(600, 5000, device="cuda")
+    graph, fresh = torch.cuda.CUDAGraph(), dl.LogicLayer(5000, 6000).eval()
+    layer(short), torch.cuda.synchronize()
+    with torch.cuda.graph(graph), torch.no_grad():
+        out = fresh(long)
+    graph.replay()
+    assert ext.built_schedule(*fresh.indices, 5000) is None
+    with torch.no_grad():
+        assert torch.equal(out, fresh(long)) and ext.built_schedule(*fresh.indices, 5000) is not None
+    assert layer._train_schedule(short.t()) is None and layer._train_schedule(long.t()) is not None
+    gy = torch.randn(668, 6000, device="cuda")
+    grads = []
+    for least in (layer._CHAIN_MIN_BYTES, 1 << 60):
+        monkeypatch.setattr(dl.LogicLayer, "_CHAIN_MIN_BYTES", least)
+        x = long.clone().requires_grad_()
+        layer.weights.grad = None
+        y = layer(x)
+        y.backward(gy)
+        grads.append((y.detach(), layer.weights.grad, x.grad))
+    (y0, w0, x0), (y1, w1, x1) = grads
+    assert torch.equal(y0, y1) and torch.equal(w0, w1)
+    assert within_budget(x0, x1, None, 1e-5)[0]
