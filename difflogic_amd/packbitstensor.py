@@ -46,6 +46,16 @@ _DIRECT_ROW_BYTES_LDS = 768      # one row, for layers that the LDS kernel takes
 _DIRECT_MIN_OUT = 1000           # smaller layers, and the tapering end of a net below 4096, stay with the LDS kernel
 
 
+# Deferred nets on rows up to this long write the last layer's rows and count them from memory: the count along the schedule
+# takes one workgroup per 2048 outputs and kilobyte of the row, 32 of them on 64000 outputs and the shortest rows, and its
+# per-call plan and the marks of what nobody looks at (which save little of so short a kernel) cost ten launches.
+# 784 -> 6 x 64000, along the schedule / stored: batch 10000 203 / 157 us (two-input gates only 269 / 178), 20000 217 / 205,
+# 40000 241 / 332; 4 x 128000: 10000 208 / 172; 4 x 256000: 4000 250 / 217, 10000 305 / 336; 6 x 16000: 40000 210 / 159,
+# 80000 216 / 231.
+_STORED_BYTES = 160 << 20        # rows of the last layer
+_STORED_ROW_BYTES = 5120         # ... and one row of them
+
+
 def _direct(in_dim, out_dim, row_bytes, lds_width):
     """Whether a layer on rows of ``row_bytes`` is evaluated at once (above)."""
     return (out_dim >= min(max(in_dim, _DIRECT_MIN_OUT), 4096) and 0 < out_dim * row_bytes <= _DIRECT_BYTES
@@ -401,6 +411,11 @@ class PackBitsTensor:
                                                   folded=self._folded)
                 if out is not None:
                     return out
+            row_bytes = self._words().shape[1] * 8
+            if row_bytes <= _STORED_ROW_BYTES and self.features * row_bytes <= _STORED_BYTES:
+                self._run_groups(plan_groups(self._dims(), False, self._words64(), share))
+                rows = self._words()
+                return difflogic_cuda.groupbitsum(rows, self._pad(rows), k)
             self._fold_pending()
             groups = plan_groups(self._dims(), True, self._words64(), share)
             # output rows of the groups before the last that no gate above them looks at are not computed

@@ -74,9 +74,10 @@ def test_pack_into_rows(ext, F, B):
 
 @pytest.mark.parametrize("widths,B,bits", [
     ([1000, 1200, 2000], 1, 8), ([4096, 2100, 4096], 100, 16), ([6000, 6000], 6144, 32), ([6000, 6000], 6145, 64),
-    ([10250, 11000], 12288, 64), ([10250, 11000], 12289, 64), ([1000, 999, 1900, 1000], 300, 64), ([2000, 4000], 1000, 64)])
+    ([10250, 11000], 12288, 64), ([10250, 11000], 12289, 64), ([10250, 10900], 40960, 32), ([10250, 10900], 40961, 64), ([1000, 999, 1900, 1000], 300, 64), ([2000, 4000], 1000, 64)])
 def test_layers_at_once_and_deferred_agree(monkeypatch, widths, B, bits):
-    """Either side of every limit of the rule, the counts and the words are the oracle's, and those of deferred layers."""
+    """Either side of every limit of the rules (layers at once; counted from stored rows), the counts are the oracle's whatever
+    the route, and so are the words of deferred layers."""
     import difflogic_amd as dl
     from difflogic_amd import packbitstensor as pbt
     rng = np.random.default_rng(B + len(widths))
@@ -86,13 +87,16 @@ def test_layers_at_once_and_deferred_agree(monkeypatch, widths, B, bits):
     model = build_model(F, layers, k).eval()
     want = interp.net_eval(x, layers, k)
     xd = torch.as_tensor(x).cuda()
-    for limit in (pbt._DIRECT_BYTES, 0):
+    for limit, stored in ((pbt._DIRECT_BYTES, pbt._STORED_BYTES), (0, pbt._STORED_BYTES), (0, 0)):
         monkeypatch.setattr(pbt, "_DIRECT_BYTES", limit)
+        monkeypatch.setattr(pbt, "_STORED_BYTES", stored)
         with torch.no_grad():
             assert np.array_equal(model(dl.PackBitsTensor(xd, bit_count=bits)).cpu().numpy(), want)
             p = dl.PackBitsTensor(xd, bit_count=bits)
             for m in list(model)[:-1]:
                 p = m(p)
+            for _ in range(2):                                         # counting leaves the object as it is
+                assert np.array_equal(p.group_sum(k).cpu().numpy(), want)
             words = p.t.cpu().numpy()
         if limit:
             at_once = words
