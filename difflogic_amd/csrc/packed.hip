@@ -1531,6 +1531,10 @@ __global__ __launch_bounds__(DL_BLOCK) void count_finish_kernel(const V *__restr
 // ([column][dword][sample][class], a pad per run so that a wave's stores spread over the banks), which the
 // workgroup writes out in 256-byte pieces.
 #define DL_FINISH_COLS 16
+// Below this many column tiles the four workgroups of each leave most CUs idle and count_finish_kernel, with one per tile and
+// class, is faster (784 -> 6 x 64000, whole step: 4 tiles 235 against 228 us, 15 tiles 401 against 395, 30 tiles 676 against
+// 677, 49 tiles 1062 against 1075).
+#define DL_FINISH_ROWS_TILES 24
 template <int NP>
 __global__ __launch_bounds__(16 * DL_WAVE) void count_finish_rows_kernel(const dl_u32x4 *__restrict__ partial,
                                                                          int32_t *__restrict__ out, int64_t ncols,
@@ -2238,7 +2242,17 @@ static int pack_batch_major_rows(const uint8_t *x, void *out, int64_t batch, int
         // per CU (2352 features); slices are whole 128-byte lines where the rows are.
         const int64_t unit = features % 128 == 0 ? 128 : 16;
         const int64_t want = dl_ceil_div(features, DL_PACK_MAX_SLICE / unit * unit);
-        const int64_t slice = dl_ceil_div(dl_ceil_div(features, want), unit) * unit;
+        auto slice_of = [&](int64_t n) { return dl_ceil_div(dl_ceil_div(features, n), unit) * unit; };
+        int64_t slice = slice_of(want);
+        // Slices this long fill a CU's LDS one or two at a time, so the launch runs in rounds over the 256 CUs: a slice or two
+        // more per row where that fills the last round better (9216 features, batch 100003: 784 workgroups = 3.06 rounds of
+        // 2304 features 220 us, 980 = 3.8 rounds of 1920 202 us), as long as the pieces stay a kilobyte long.
+        auto rounds = [&](int64_t sl) {                          // features a CU goes through, one after the other
+            const int64_t fit = (160 << 10) / (sl * DL_PACK_PITCH);
+            return dl_ceil_div(dl_ceil_div(cols, DL_PACK_WC) * dl_ceil_div(features, sl), 256 * fit) * fit * sl;
+        };
+        for (int64_t n = want + 1; n <= want + 2 && slice_of(n) >= 1024; ++n)
+            if (rounds(slice_of(n)) * 20 < rounds(slice) * 19) slice = slice_of(n);
         const int64_t nslices = dl_ceil_div(features, slice);
         const int64_t blocks = dl_ceil_div(cols, DL_PACK_WC) * nslices;
         if (blocks > 0x3fffffffLL) return DL_ERR_TOO_LARGE;
@@ -2595,7 +2609,7 @@ int launch_count_chain(const void *x, const dl_u32x4 *rec, const uint16_t *runs,
     if constexpr (sizeof(V) == 16) {
         // whole-line stores where a wave per class fits a workgroup
         const size_t lds = (size_t) 64 * (16 * k + 1) * 4;
-        if (k <= 16 && per_class < (1LL << 13)) {              // (tiles <= 65535: the grid fits)
+        if (k <= 16 && per_class < (1LL << 13) && tiles >= DL_FINISH_ROWS_TILES) {     // (tiles <= 65535: the grid fits)
             const dim3 rgrid((unsigned) (dl_ceil_div(tiles, 8) * 8 * 4)), rblock((unsigned) (k * DL_WAVE));
             DL_LAUNCH((count_finish_rows_kernel<13>), rgrid, rblock, lds, s, (const dl_u32x4 *) partial, out, ncols, nwg, (int) k, batch,
                       ones);

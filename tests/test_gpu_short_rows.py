@@ -60,8 +60,9 @@ def test_bit_count_of_short_rows(ext, per_class, k, words, pad):
         assert torch.equal(got[:, c].long(), bits[:words * 64 - pad]), c
 
 
-@pytest.mark.parametrize("F", [1, 15, 16, 17, 63, 65, 80, 784])
-@pytest.mark.parametrize("B", [1, 64, 65, 1000, 12288, 12289, 20000])
+# (the last four: more than one slice of the features per workgroup column, and one or two slices more than fit need)
+@pytest.mark.parametrize("F,B", [(f, b) for f in (1, 15, 16, 17, 63, 65, 80, 784) for b in (1, 64, 65, 1000, 12288, 12289, 20000)]
+                         + [(2368, 13000), (4096, 14000), (9216, 14000), (5008, 15001)])
 def test_pack_into_rows(ext, F, B):
     rng = np.random.default_rng(F * 31 + B)
     raw = torch.as_tensor(rng.choice([0, 0, 1, 2, 255], (B, F)).astype(np.uint8))       # any non-zero byte counts
