@@ -1397,13 +1397,13 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
 }
 
 // One wave per 64 consecutive samples of one class; the four waves of a workgroup take
-// interleaved splits and are added in wave order, so the summation order is fixed.  The partial sums are added and divided
+// interleaved splits and are added in wave order, so the summation order is fixed.  The partial sums are added and scaled
 // in double and rounded once: a score of 64 is 8e-6 from its neighbours, which is what the gradients of a net with large
 // class sums see.
 template <typename T>
 __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typename Acc<T>::type *__restrict__ partial,
                                                                     T *__restrict__ y, int64_t batch, int64_t k,
-                                                                    int splits, double tau) {
+                                                                    int splits, double inv_tau) {
     typedef typename Acc<T>::type C;
     __shared__ double lds[4][DL_WAVE];
     const int wave = dl_wave_in_block();
@@ -1412,17 +1412,17 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typena
     const int64_t c = blockIdx.y;
     double sum = 0.0;
     if (r < batch)
-        for (int s = wave; s < splits; s += 32) {                // eight partial sums in flight, added in order
-            C v[8];
+        for (int s = wave; s < splits; s += 64) {                // sixteen partial sums in flight, added in order
+            C v[16];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = s + 4 * i < splits ? partial[((int64_t) (s + 4 * i) * k + c) * batch + r] : (C) 0;
+            for (int i = 0; i < 16; ++i) v[i] = s + 4 * i < splits ? partial[((int64_t) (s + 4 * i) * k + c) * batch + r] : (C) 0;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) sum += (double) v[i];
+            for (int i = 0; i < 16; ++i) sum += (double) v[i];
         }
     lds[wave][lane] = sum;
     __syncthreads();
     if (wave == 0 && r < batch)
-        y[r * k + c] = down<T, C>((C) (((lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane])) / tau));
+        y[r * k + c] = down<T, C>((C) (((lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane])) * inv_tau));
 }
 
 template <typename T, int VEC, bool RAG>
@@ -1476,7 +1476,7 @@ int group_sum_forward_t(const void *x, void *y, void *workspace, int64_t out_dim
     const int64_t blocks = dl_ceil_div(batch, DL_WAVE);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     DL_LAUNCH((group_sum_finish_kernel<T>), dim3((unsigned) blocks, (unsigned) k), dim3(DL_BLOCK), 0, s,
-                       (const C *) workspace, (T *) y, batch, k, splits, tau);
+                       (const C *) workspace, (T *) y, batch, k, splits, 1.0 / tau);
     return dl_launch_status();
 }
 
@@ -1531,16 +1531,17 @@ int forward_group_sum_t(const void *x, const int64_t *a, const int64_t *b, const
     const int64_t blocks = dl_ceil_div(batch, DL_WAVE);
     if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     DL_LAUNCH((group_sum_finish_kernel<T>), dim3((unsigned) blocks, (unsigned) k), dim3(DL_BLOCK), 0, s,
-                       (const C *) workspace, (T *) y, batch, k, splits, tau);
+                       (const C *) workspace, (T *) y, batch, k, splits, 1.0 / tau);
     return dl_launch_status();
 }
 
-// Number of row splits per class: eight workgroups per CU, at least 32 rows each (four and 64 rows: GroupSum over
-// 128000 rows at batch 1024 97 against 90 us, layer and GroupSum on 8000 rows at 128 9.4 against 7.4).
+// Number of row splits per class: enough workgroups to fill the chip, at least 32 rows each (64: layer and GroupSum on 8000
+// rows at batch 128 9.4 against 7.4 us).  Twice the workgroups: GroupSum over 128000 rows at batch 1024 97 -> 90 us, but
+// the finishing pass over the partial sums of 64000 rows at 512 5.3 -> 9.0.
 int group_sum_splits(int64_t out_dim, int64_t batch, int64_t k) {
     const int64_t per_class = out_dim / k;
     const int64_t col_tiles = dl_ceil_div(batch, 4 * DL_WAVE);
-    int64_t want = dl_ceil_div(2048, col_tiles * k);
+    int64_t want = dl_ceil_div(1024, col_tiles * k);
     const int64_t max_by_rows = per_class / 32 > 0 ? per_class / 32 : 1;
     if (want > max_by_rows) want = max_by_rows;
     if (want < 1) want = 1;
