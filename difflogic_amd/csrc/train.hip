@@ -801,7 +801,8 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_w_chain_kernel(const T *__r
 // A vertex in the middle of a trail collects the share of the neuron before it (kept in
 // `carry`) and of the neuron after it and is written once: position p of the schedule goes to
 // row dst[p] (-1: nothing to write; >= in_dim: row dst[p] - in_dim of `overflow`, for vertices
-// that occur at several positions and are summed afterwards by backward_fix_kernel).  Rows longer
+// that occur at several positions and are summed afterwards by backward_fix_kernel; the parts are kept in the type
+// that sums are taken in, and half results are rounded once, after the sum and the scale).  Rows longer
 // than CPL * 64 vectors are cut into segments (blockIdx.y); the corner sums of the segments then
 // go to `partial` and backward_w_finish_kernel adds them.  A wave
 // owns `chunk` positions [s0, s0 + chunk); it recomputes the last neuron of the chunk before it to get
@@ -823,13 +824,17 @@ template <typename T> struct LowerLayer {
     T *gw;                      // [in_dim, 16]
 };
 
+// A vector of an overflow row.  (Eight floats for half rows: two 16-byte accesses, no 32-byte alignment asked for.)
+template <typename T, int VEC, bool RAG>
+using OverflowPack = Pack<typename Acc<T>::type, VEC, RAG || sizeof(T) != sizeof(typename Acc<T>::type)>;
+
 template <typename T, int VEC, int CPL, int LOWER, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const T *__restrict__ x, const int32_t *__restrict__ verts, const int32_t *__restrict__ neuron,
     const uint8_t *__restrict__ flip, const int32_t *__restrict__ dst, const T *__restrict__ w,
     const T *__restrict__ gy, const T *__restrict__ probs, T *__restrict__ gw,
-    typename Acc<T>::type *__restrict__ partial, T *__restrict__ gx, T *__restrict__ overflow, int64_t steps, int chunk,
-    int64_t in_dim, int64_t out_dim, int64_t batch, typename Acc<T>::type scale, int64_t gdiv, LowerLayer<T> low,
+    typename Acc<T>::type *__restrict__ partial, T *__restrict__ gx, typename Acc<T>::type *__restrict__ overflow,
+    int64_t steps, int chunk, int64_t in_dim, int64_t out_dim, int64_t batch, typename Acc<T>::type scale, int64_t gdiv, LowerLayer<T> low,
     bool w32) {
     typedef typename Acc<T>::type C;
     typedef Pack<T, VEC, RAG> P;
@@ -901,15 +906,25 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
             store_grad_w<T>(lane, true, row, s00, s01, s10, s11, low.probs, low.gw);
             return;
         }
-        T *base = row < in_dim ? gx : overflow;
-        const int64_t at_row = row < in_dim ? row : (int64_t) row - in_dim;
+        if (row >= in_dim) {                                     // a part of a sum: in C, scaled here only if that is T
+            typedef OverflowPack<T, VEC, RAG> O;
+#pragma unroll
+            for (int q = 0; q < CPL; ++q) {
+                const int64_t col = col0 + lane + q * DL_WAVE;
+                O r;
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) r.v[e] = sizeof(T) == sizeof(C) ? val[q][e] * scale : val[q][e];
+                if (col < ncols) row_vec<O, VEC, RAG>(overflow, (int64_t) row - in_dim, batch, ncols, col) = r;
+            }
+            return;
+        }
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
             const int64_t col = col0 + lane + q * DL_WAVE;
             P r;
 #pragma unroll
             for (int e = 0; e < VEC; ++e) r.v[e] = down<T, C>(val[q][e] * scale);
-            if (col < ncols) row_vec<P, VEC, RAG>(base, at_row, batch, ncols, col) = r;
+            if (col < ncols) row_vec<P, VEC, RAG>(gx, row, batch, ncols, col) = r;
         }
     };
 
@@ -1065,15 +1080,17 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
 // grad_x rows of the vertices that backward_chain_kernel could not finish in one write: vertex
 // fix_vertex[i] is the sum, in slot order, of overflow rows [fix_start[i], fix_start[i + 1])
 // (no rows: the input feeds no neuron and its gradient is zero).
-// compact: row i of gx instead of row fix_vertex[i] (gx then has n_fix rows only).
+// compact: row i of gx instead of row fix_vertex[i] (gx then has n_fix rows only).  scale: what the parts still lack
+// (1 where backward_chain_kernel put it in).
 template <typename T, int VEC, bool RAG>
-__global__ __launch_bounds__(DL_BLOCK) void backward_fix_kernel(const T *__restrict__ overflow,
+__global__ __launch_bounds__(DL_BLOCK) void backward_fix_kernel(const typename Acc<T>::type *__restrict__ overflow,
                                                                 const int32_t *__restrict__ fix_vertex,
                                                                 const int32_t *__restrict__ fix_start,
                                                                 T *__restrict__ gx, int64_t n_fix, int64_t batch,
-                                                                bool compact) {
+                                                                typename Acc<T>::type scale, bool compact) {
     typedef typename Acc<T>::type C;
     typedef Pack<T, VEC, RAG> P;
+    typedef OverflowPack<T, VEC, RAG> O;
     const int64_t ncols = vec_count<VEC>(batch);
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
@@ -1086,13 +1103,13 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_fix_kernel(const T *__restr
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc[e] = (C) 0;
         for (int32_t r = r0; r < r1; ++r) {
-            const P part = row_vec<P, VEC, RAG>(overflow, (int64_t) r, batch, ncols, col);
+            const O part = row_vec<O, VEC, RAG>(overflow, (int64_t) r, batch, ncols, col);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] += up<T>(part.v[e]);
+            for (int e = 0; e < VEC; ++e) acc[e] += part.v[e];
         }
         P res;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) res.v[e] = down<T, C>(acc[e]);
+        for (int e = 0; e < VEC; ++e) res.v[e] = down<T, C>(acc[e] * scale);
         row_vec<P, VEC, RAG>(gx, v, batch, ncols, col) = res;
     }
 }
@@ -1693,7 +1710,7 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
     const int64_t partial_bytes = backward_partial_bytes<T>(out_dim, batch);
     if ((partial_bytes > 0 || overflow_rows > 0) && workspace == nullptr) return DL_ERR_INVALID_ARGUMENT;
     C *partial = partial_bytes > 0 ? (C *) workspace : nullptr;
-    T *overflow = (T *) ((char *) workspace + partial_bytes);
+    C *overflow = (C *) ((char *) workspace + partial_bytes);
     const int chunk = chain_chunk(steps * segments);
     const int64_t blocks = dl_ceil_div(dl_ceil_div(steps, chunk), 4), fix_blocks = dl_ceil_div(n_fix, 4);
     if (blocks > 0x7fffffffLL || fix_blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
@@ -1738,12 +1755,13 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
     }
     if (n_fix == 0) return DL_OK;
     const dim3 fix_grid((unsigned) fix_blocks, col_tiles(ncols));
+    const C fix_scale = sizeof(T) == sizeof(C) ? (C) 1 : (C) scale;
     if (kind == Rows::whole)
-        DL_LAUNCH((backward_fix_kernel<T, V, false>), fix_grid, block, 0, s, (const T *) overflow, fix_vertex, fix_start,
-                  (T *) gx, n_fix, batch, lower != nullptr);
+        DL_LAUNCH((backward_fix_kernel<T, V, false>), fix_grid, block, 0, s, (const C *) overflow, fix_vertex, fix_start,
+                  (T *) gx, n_fix, batch, fix_scale, lower != nullptr);
     else
-        DL_LAUNCH((backward_fix_kernel<T, V, true>), fix_grid, block, 0, s, (const T *) overflow, fix_vertex, fix_start,
-                  (T *) gx, n_fix, batch, lower != nullptr);
+        DL_LAUNCH((backward_fix_kernel<T, V, true>), fix_grid, block, 0, s, (const C *) overflow, fix_vertex, fix_start,
+                  (T *) gx, n_fix, batch, fix_scale, lower != nullptr);
     st = dl_launch_status();
     if (st != DL_OK || !lower) return st;
     if (kind == Rows::whole)
@@ -1791,7 +1809,7 @@ extern "C" int64_t dl_logic_backward_chained_workspace_bytes(int64_t overflow_ro
     takes_any_rows(dtype);
     weights_fp32(dtype);
     switch (dtype) {
-    case DL_F16: return backward_partial_bytes<__half>(out_dim, batch) + overflow_rows * batch * 2;
+    case DL_F16: return backward_partial_bytes<__half>(out_dim, batch) + overflow_rows * batch * 4;    // parts in fp32
     case DL_F32: return backward_partial_bytes<float>(out_dim, batch) + overflow_rows * batch * 4;
     case DL_F64: return backward_partial_bytes<double>(out_dim, batch) + overflow_rows * batch * 8;
     default: return -DL_ERR_DTYPE;

@@ -1,0 +1,66 @@
+"""Half activations: an input gradient is summed in fp32 and rounded to half ONCE, also where its parts come from several
+positions of the schedule."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+N = 1536
+
+
+def _corners(p):
+    """Corner sums in fp32, in the kernels' order of additions."""
+    at = lambda i: ((p[:, i[0]] + p[:, i[1]]) + (p[:, i[2]] + p[:, i[3]])) + ((p[:, i[4]] + p[:, i[5]]) + (p[:, i[6]] + p[:, i[7]]))  # noqa: E731
+    return (at((8, 9, 10, 11, 12, 13, 14, 15)), at((4, 5, 6, 7, 12, 13, 14, 15)), at((2, 3, 6, 7, 10, 11, 14, 15)),
+            at((1, 3, 5, 7, 9, 11, 13, 15)))
+
+
+def _fma32(x, y, z):
+    return (x.astype(np.float64) * y + z).astype(np.float32)          # the product of a half and a float is exact in fp64
+
+
+@pytest.fixture(scope="module")
+def wiring():
+    """Every input feeds two neurons: its gradient is a sum of two terms, the same in either order."""
+    rng = np.random.default_rng(5)
+    a = rng.permutation(N)
+    b = np.roll(a, 1)[np.argsort(rng.random(N))]
+    while (a == b).any():
+        b = rng.permutation(N)
+    return a, b
+
+
+def _case(wiring, batch, wdtype):
+    a, b = wiring
+    g = torch.Generator().manual_seed(batch)
+    x = torch.rand(N, batch, generator=g).half()
+    gy = torch.randn(N, batch, generator=g).half()
+    p = torch.softmax(torch.randn(N, 16, generator=g), -1).to(wdtype)
+    p00, p01, p10, p11 = (c[:, None] for c in _corners(p.float().numpy()))
+    av, bv, gv = x.numpy()[a].astype(np.float32), x.numpy()[b].astype(np.float32), gy.numpy().astype(np.float32)
+    d0, d1 = p01 - p00, p11 - p10
+    dd, da = d1 - d0, p10 - p00
+    acc = np.zeros((N, batch), np.float32)
+    acc[a] = gv * _fma32(bv, dd, da)
+    acc[b] += gv * _fma32(av, dd, d0)
+    return x, gy, p, acc
+
+
+def _same(got, want):
+    got = got.cpu().numpy()
+    assert got.dtype == np.float16 and got.shape == want.shape
+    wrong = (got != want).sum()
+    assert wrong == 0, (wrong, want.size)
+
+
+@pytest.mark.parametrize("batch", [64, 256, 512, 1024, 4096])
+def test_sums_over_positions_on_whole_vectors(monkeypatch, wiring, batch):
+    """(Scale 1: the product with another scale is rounded to fp32 first for some elements of a whole vector.)"""
+    from difflogic_amd import difflogic_cuda as ext
+    monkeypatch.setattr(ext, "BACKWARD_CHAIN_MAX_OVERFLOW", 1e9)
+    x, gy, p, acc = _case(wiring, batch, torch.float32)
+    a, b = (torch.as_tensor(t).cuda() for t in wiring)
+    sched = ext.schedule_for(a, b, N)
+    assert sched.backward_plan()[4] > 0
+    _same(ext.backward_chained(x.cuda(), p.cuda(), gy.cuda(), sched)[1], acc.astype(np.float16))
