@@ -24,7 +24,8 @@ template <typename T, int N, bool RAG = false> struct alignas(RAG ? sizeof(T) : 
 
 // Rows of `batch` elements are read and written as vectors 0 .. ceil(batch / VEC) - 1.  RAG: the last vector of a row is
 // moved back to end with the row, so it repeats `dup` elements of the vector before it.  Elementwise results are then
-// written twice with the same value; sums over the batch leave the repeated elements out (own_part).  What that buys
+// written twice with the same value (the conversion to half by round_fma, which does not depend on an element's place in
+// its vector); sums over the batch leave the repeated elements out (own_part).  What that buys
 // over one element per lane: half rows of 500 elements on six 64000-wide layers, forward + backward 2.11 -> 0.61 ms.
 template <int VEC> __device__ __forceinline__ int64_t vec_count(int64_t batch) {
     return (int64_t) ((uint64_t) (batch + VEC - 1) / VEC);
@@ -58,6 +59,23 @@ template <> __device__ __forceinline__ __half down<__half, float>(float v) { ret
 __device__ __forceinline__ float dl_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double dl_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
+// fma(a, b, c) as a T, and v * s as a T.  Left to itself the compiler folds the conversion to half into the multiply-add
+// for some elements of a vector (v_fma_mixlo_f16: one rounding) and not for others (two); ONCE says which it is: one
+// rounding for every element, as the kernels that take one element per lane have it.
+template <typename T, bool ONCE, typename C> __device__ __forceinline__ T round_fma(C a, C b, C c) {
+    if constexpr (ONCE && sizeof(T) == 2) {
+        uint32_t r;                                              // (the instruction writes the low half)
+        asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+        return __builtin_bit_cast(T, (uint16_t) r);
+    } else {
+        return down<T, C>(dl_fma(a, b, c));
+    }
+}
+template <typename T, bool ONCE, typename C> __device__ __forceinline__ T round_scaled(C v, C s) {
+    if constexpr (ONCE && sizeof(T) == 2) return round_fma<T, ONCE, C>(v, s, (C) -0.0);      // (keeps the sign of a zero)
+    else return down<T, C>(v * s);
+}
+
 // Gate weights (probabilities or logits) and their gradients sit next to activations of type T either in T as well
 // or, `w32`, in fp32 whatever T is: what a layer with fp32 weights needs for half / double activations (the
 // reference's --training-bit-count 16 / 64).  The pointers keep the type T* and are reinterpreted.
@@ -74,10 +92,10 @@ template <typename T> __device__ __forceinline__ void wstore(T *__restrict__ w, 
 }
 
 // y = lerp(lerp(P00, P01, b), lerp(P10, P11, b), a), three fused multiply-adds.
-template <typename C> __device__ __forceinline__ C mix(C av, C bv, C p00, C p10, C d0, C d1) {
+template <typename T, bool ONCE, typename C> __device__ __forceinline__ T mix(C av, C bv, C p00, C p10, C d0, C d1) {
     const C lo = dl_fma(bv, d0, p00);
     const C hi = dl_fma(bv, d1, p10);
-    return dl_fma(av, hi - lo, lo);
+    return round_fma<T, ONCE, C>(av, hi - lo, lo);
 }
 
 // The four corner values of neuron n's gate mixture.
@@ -292,7 +310,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_kernel(const T *__restrict__
                 P r;
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
-                    r.v[e] = down<T, C>(mix<C>(up<T>(va[j].v[e]), up<T>(vb[j].v[e]), p00[j], p10[j], d0[j], d1[j]));
+                    r.v[e] = mix<T, RAG, C>(up<T>(va[j].v[e]), up<T>(vb[j].v[e]), p00[j], p10[j], d0[j], d1[j]);
                 }
                 row_vec<P, VEC, RAG>(y, (n0 + j), batch, ncols, col) = r;
             }
@@ -480,7 +498,7 @@ __device__ __forceinline__ void backward_x_block(int64_t block, int64_t tile, in
         }
         P r;
 #pragma unroll
-        for (int q = 0; q < VEC; ++q) r.v[q] = down<T, C>(acc[q] * scale);
+        for (int q = 0; q < VEC; ++q) r.v[q] = round_scaled<T, RAG, C>(acc[q], scale);
         row_vec<P, VEC, RAG>(gx, c, batch, ncols, col) = r;
     }
 }
@@ -522,8 +540,9 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_both_kernel(
 // neuron[s] from (verts[s], verts[s + 1]); flip[s] tells which of the two is the neuron's `a`
 // input.  The shared row stays in registers, so a neuron costs one gathered row instead of two.
 // Arithmetic and summation order per element are those of the unchained kernels: the fp32 and
-// fp64 results are bit-identical (fp16 outputs can differ in the last bit, where the compiler
-// folds the final conversion into a fused multiply-add in one kernel and not in the other).
+// fp64 results are bit-identical, and so are half results on rows that end inside a vector (on rows of whole vectors
+// they can differ in the last bit, where the compiler folds the final conversion into a fused multiply-add in one
+// kernel and not in the other).
 // ------------------------------------------------------------------------------------------
 template <typename T, int VEC, int CHUNK, int GATES, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__restrict__ x,
@@ -566,7 +585,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__rest
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
                     const C u0 = up<T>(rows[j].v[e]), u1 = up<T>(rows[j + 1].v[e]);
-                    r.v[e] = down<T, C>(mix<C>(f ? u1 : u0, f ? u0 : u1, p00[i], p10[i], d0[i], d1[i]));
+                    r.v[e] = mix<T, RAG, C>(f ? u1 : u0, f ? u0 : u1, p00[i], p10[i], d0[i], d1[i]);
                 }
                 if (live && n[i] >= 0) row_vec<P, VEC, RAG>(y, (int64_t) n[i], batch, ncols, cl) = r;
             }
@@ -646,7 +665,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
                 if (j <= CHUNK) {
 #pragma unroll
                     for (int e = 0; e < VEC; ++e)
-                        rows[j].v[e] = down<T, C>(mix<C>(up<T>(va[i].v[e]), up<T>(vb[i].v[e]), lp00[j], lp10[j], ld0[j], ld1[j]));
+                        rows[j].v[e] = mix<T, RAG, C>(up<T>(va[i].v[e]), up<T>(vb[i].v[e]), lp00[j], lp10[j], ld0[j], ld1[j]);
                 }
             }
         }
@@ -657,7 +676,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const C u0 = up<T>(rows[j].v[e]), u1 = up<T>(rows[j + 1].v[e]);
-                r.v[e] = down<T, C>(mix<C>(f ? u1 : u0, f ? u0 : u1, p00[j], p10[j], d0[j], d1[j]));
+                r.v[e] = mix<T, RAG, C>(f ? u1 : u0, f ? u0 : u1, p00[j], p10[j], d0[j], d1[j]);
             }
             if (live && n[j] >= 0) row_vec<P, VEC, RAG>(y, (int64_t) n[j], batch, ncols, cl) = r;
         }
@@ -718,7 +737,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *_
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) {
                         const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]);
-                        r.v[e] = down<T, C>(mix<C>(f ? u1 : u0, f ? u0 : u1, p00[i], p10[i], d0[i], d1[i]));
+                        r.v[e] = mix<T, RAG, C>(f ? u1 : u0, f ? u0 : u1, p00[i], p10[i], d0[i], d1[i]);
                     }
                     if (n[i] >= 0 && col < ncols) row_vec<P, VEC, RAG>(y, (int64_t) n[i], batch, ncols, col) = r;
                 }
@@ -828,6 +847,12 @@ template <typename T> struct LowerLayer {
 template <typename T, int VEC, bool RAG>
 using OverflowPack = Pack<typename Acc<T>::type, VEC, RAG || sizeof(T) != sizeof(typename Acc<T>::type)>;
 
+// dy/da or dy/db of a neuron, k + u * dd.  SPLIT: in two roundings, as backward_x_kernel has it.
+template <bool SPLIT, typename C> __device__ __forceinline__ C slope(C u, C dd, C k) {
+    if constexpr (SPLIT) return k + u * dd;
+    else return dl_fma(u, dd, k);
+}
+
 template <typename T, int VEC, int CPL, int LOWER, bool RAG>
 __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const T *__restrict__ x, const int32_t *__restrict__ verts, const int32_t *__restrict__ neuron,
@@ -840,6 +865,9 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     typedef Pack<T, VEC, RAG> P;
     const int64_t ncols = vec_count<VEC>(batch);
     constexpr bool RECOMPUTE = LOWER == 2;
+    // a last-bit difference in fp32 turns a half result by 2^-11 now and then: with SPLIT, half rows of any length get the
+    // bits of backward_x_kernel whether or not their layer is walked along its schedule
+    constexpr bool SPLIT = RAG && sizeof(T) == 2;
     constexpr int LCPL = LOWER ? CPL : 1;                       // registers for lower rows only where they are used
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
@@ -879,7 +907,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
         for (int q = 0; q < CPL; ++q)
 #pragma unroll
             for (int e = 0; e < VEC; ++e)
-                out[q].v[e] = down<T, C>(mix<C>(up<T>(la[q].v[e]), up<T>(lb[q].v[e]), p00, p10, d0, d1));
+                out[q].v[e] = mix<T, RAG, C>(up<T>(la[q].v[e]), up<T>(lb[q].v[e]), p00, p10, d0, d1);
     };
     // la, lb: with LOWER, the two input rows of neuron `row` of the layer below
     auto store_row = [&](int32_t row, const C (&val)[CPL][VEC], const P *la, const P *lb) {
@@ -892,7 +920,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
                 const int dup = vec_dup<VEC, RAG>(col0 + lane + q * DL_WAVE, batch);
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
-                    const C g = own_part<RAG>(up<T>(down<T, C>(val[q][e] * scale)), e, dup);
+                    const C g = own_part<RAG>(up<T>(round_scaled<T, RAG, C>(val[q][e], scale)), e, dup);
                     const C av = up<T>(la[q].v[e]), bv = up<T>(lb[q].v[e]);
                     const C ga = g * av, gna = g - ga;
                     const C t11 = ga * bv, t01 = gna * bv;
@@ -923,7 +951,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
             const int64_t col = col0 + lane + q * DL_WAVE;
             P r;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) r.v[e] = down<T, C>(val[q][e] * scale);
+            for (int e = 0; e < VEC; ++e) r.v[e] = round_scaled<T, RAG, C>(val[q][e], scale);
             if (col < ncols) row_vec<P, VEC, RAG>(gx, row, batch, ncols, col) = r;
         }
     };
@@ -962,7 +990,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
 #pragma unroll
         for (int q = 0; q < CPL; ++q)
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) carry[q][e] = up<T>(g[q].v[e]) * dl_fma(up<T>(before[q].v[e]), dd, kv);
+            for (int e = 0; e < VEC; ++e) carry[q][e] = up<T>(g[q].v[e]) * slope<SPLIT, C>(up<T>(before[q].v[e]), dd, kv);
     }
     // The chunk's schedule entries are fetched once, one per lane (chunk <= 64), and handed out by
     // readlane, so the step loop waits for no scalar loads; the rows of step i + 1 are requested
@@ -1030,8 +1058,8 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
                 s10 += ga - t11;
                 s01 += t01;
                 s00 += gna - t01;
-                out[q][e] = carry[q][e] + gg * dl_fma(u1, dd, ku);
-                carry[q][e] = gg * dl_fma(u0, dd, kv);
+                out[q][e] = carry[q][e] + gg * slope<SPLIT, C>(u1, dd, ku);
+                carry[q][e] = gg * slope<SPLIT, C>(u0, dd, kv);
             }
         }
         wave_sum4(s00, s01, s10, s11, lane);
@@ -1109,7 +1137,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_fix_kernel(const typename A
         }
         P res;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) res.v[e] = down<T, C>(acc[e] * scale);
+        for (int e = 0; e < VEC; ++e) res.v[e] = round_scaled<T, RAG, C>(acc[e], scale);
         row_vec<P, VEC, RAG>(gx, v, batch, ncols, col) = res;
     }
 }
@@ -1394,7 +1422,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
                     // rounded to T like the stored activation would have been
-                    acc[e] += up<T>(down<T, C>(mix<C>(up<T>(va[j].v[e]), up<T>(vb[j].v[e]), p00[j], p10[j], d0[j], d1[j])));
+                    acc[e] += up<T>(mix<T, RAG, C>(up<T>(va[j].v[e]), up<T>(vb[j].v[e]), p00[j], p10[j], d0[j], d1[j]));
                 }
             }
         }
@@ -1463,7 +1491,7 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_backward_kernel(const T *_
         const int64_t cls = n / per_class;
         if (cls != cached_cls) {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) val.v[e] = down<T, C>(up<T>(g[(at + e) * k + cls]) * inv_tau);
+            for (int e = 0; e < VEC; ++e) val.v[e] = round_scaled<T, RAG, C>(up<T>(g[(at + e) * k + cls]), inv_tau);
             cached_cls = cls;
         }
         row_vec<P, VEC, RAG>(gx, n, batch, ncols, col) = val;

@@ -1,5 +1,6 @@
-"""Half activations: an input gradient is summed in fp32 and rounded to half ONCE, also where its parts come from several
-positions of the schedule."""
+"""Half activations: every output and input-gradient element is the fp32 (fp64 for the product under test) value of its
+formula rounded to half ONCE, whatever its place in a vector, on rows that end inside a 16-byte vector (whose last elements
+are written by two lanes) and on inputs whose gradient is summed from several positions of the schedule."""
 import numpy as np
 import pytest
 import torch
@@ -40,11 +41,15 @@ def _case(wiring, batch, wdtype):
     p00, p01, p10, p11 = (c[:, None] for c in _corners(p.float().numpy()))
     av, bv, gv = x.numpy()[a].astype(np.float32), x.numpy()[b].astype(np.float32), gy.numpy().astype(np.float32)
     d0, d1 = p01 - p00, p11 - p10
+    lo, hi = _fma32(bv, d0, p00), _fma32(bv, d1, p10)
+    y = (av.astype(np.float64) * (hi - lo) + lo).astype(np.float16)
     dd, da = d1 - d0, p10 - p00
-    acc = np.zeros((N, batch), np.float32)
-    acc[a] = gv * _fma32(bv, dd, da)
-    acc[b] += gv * _fma32(av, dd, d0)
-    return x, gy, p, acc
+    acc = []
+    for term in (lambda u, v, w: u * v + w, _fma32):     # in two roundings; fused (rows of whole vectors along the schedule)
+        acc.append(np.zeros((N, batch), np.float32))
+        acc[-1][a] = gv * term(bv, dd, da)
+        acc[-1][b] += gv * term(av, dd, d0)
+    return x, gy, p, y, *acc
 
 
 def _same(got, want):
@@ -54,12 +59,35 @@ def _same(got, want):
     assert wrong == 0, (wrong, want.size)
 
 
+@pytest.mark.parametrize("wdtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("batch", [9, 63, 255, 257, 500, 515, 1025, 2047, 2050])
+def test_rows_that_end_inside_a_vector(monkeypatch, wiring, batch, wdtype):
+    from difflogic_amd import difflogic_cuda as ext
+    from difflogic_amd.functional import build_reverse_index
+    monkeypatch.setattr(ext, "BACKWARD_CHAIN_MAX_OVERFLOW", 1e9)
+    x, gy, p, y, acc, _ = _case(wiring, batch, wdtype)
+    a, b = (torch.as_tensor(t).cuda() for t in wiring)
+    start, idx = (t.cuda() for t in build_reverse_index(a.cpu(), b.cpu(), N))
+    x, gy, p = x.cuda(), gy.cuda(), p.cuda()
+    sched = ext.schedule_for(a, b, N)
+    for schedule in (None, sched):
+        _same(ext.forward(x, a, b, p, schedule), y)
+    for scale in (1.0, 1.5):
+        want = (acc.astype(np.float64) * scale).astype(np.float16)
+        _same(ext.backward_x(x, a, b, p, gy, start, idx, scale), want)
+        _same(ext.backward_both(x, a, b, p, gy, start, idx, scale)[1], want)
+        _same(ext.backward_chained(x, p, gy, sched, scale, any_rows=True)[1], want)
+    g = torch.randn(batch, 4, generator=torch.Generator().manual_seed(1)).half()
+    want = (g.double().numpy().T * np.float64(np.float32(1 / 3.0))).astype(np.float16).repeat(8, 0)
+    _same(ext.group_sum_backward(g.cuda(), 32, 3.0), want)
+
+
 @pytest.mark.parametrize("batch", [64, 256, 512, 1024, 4096])
 def test_sums_over_positions_on_whole_vectors(monkeypatch, wiring, batch):
     """(Scale 1: the product with another scale is rounded to fp32 first for some elements of a whole vector.)"""
     from difflogic_amd import difflogic_cuda as ext
     monkeypatch.setattr(ext, "BACKWARD_CHAIN_MAX_OVERFLOW", 1e9)
-    x, gy, p, acc = _case(wiring, batch, torch.float32)
+    x, gy, p, _, _, acc = _case(wiring, batch, torch.float32)
     a, b = (torch.as_tensor(t).cuda() for t in wiring)
     sched = ext.schedule_for(a, b, N)
     assert sched.backward_plan()[4] > 0
