@@ -55,6 +55,10 @@ template <typename T> __device__ __forceinline__ typename Acc<T>::type up(T v) {
 template <> __device__ __forceinline__ float up<__half>(__half v) { return __half2float(v); }
 template <typename T, typename C> __device__ __forceinline__ T down(C v) { return (T) v; }
 template <> __device__ __forceinline__ __half down<__half, float>(float v) { return __float2half(v); }
+template <typename T> __device__ __forceinline__ T from_double(double v) {
+    if constexpr (sizeof(T) == 2) return __builtin_bit_cast(T, (_Float16) v);        // (not by way of float)
+    else return (T) v;
+}
 
 __device__ __forceinline__ float dl_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double dl_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
@@ -1443,8 +1447,8 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
 
 // One wave per 64 consecutive samples of one class; the four waves of a workgroup take
 // interleaved splits and are added in wave order, so the summation order is fixed.  The partial sums are added and scaled
-// in double and rounded once: a score of 64 is 8e-6 from its neighbours, which is what the gradients of a net with large
-// class sums see.
+// (by the reciprocal of tau) in double and rounded to T once: an fp32 score of 64 is 8e-6 from its neighbours, which is
+// what the gradients of a net with large class sums see.
 template <typename T>
 __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typename Acc<T>::type *__restrict__ partial,
                                                                     T *__restrict__ y, int64_t batch, int64_t k,
@@ -1467,7 +1471,7 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typena
     lds[wave][lane] = sum;
     __syncthreads();
     if (wave == 0 && r < batch)
-        y[r * k + c] = down<T, C>((C) (((lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane])) * inv_tau));
+        y[r * k + c] = from_double<T>(((lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane])) * inv_tau);
 }
 
 template <typename T, int VEC, bool RAG>

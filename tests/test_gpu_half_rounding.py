@@ -1,6 +1,6 @@
-"""Half activations: every output and input-gradient element is the fp32 (fp64 for the product under test) value of its
-formula rounded to half ONCE, whatever its place in a vector, on rows that end inside a 16-byte vector (whose last elements
-are written by two lanes) and on inputs whose gradient is summed from several positions of the schedule."""
+"""Half activations: every output, input-gradient element and class score is the fp32 (fp64 for the last product) value of
+its formula rounded to half ONCE, whatever its place in a vector, on rows that end inside a 16-byte vector (whose last
+elements are written by two lanes) and on inputs whose gradient is summed from several positions of the schedule."""
 import numpy as np
 import pytest
 import torch
@@ -92,3 +92,17 @@ def test_sums_over_positions_on_whole_vectors(monkeypatch, wiring, batch):
     sched = ext.schedule_for(a, b, N)
     assert sched.backward_plan()[4] > 0
     _same(ext.backward_chained(x.cuda(), p.cuda(), gy.cuda(), sched)[1], acc.astype(np.float16))
+
+
+@pytest.mark.parametrize("batch,per_class,tau", [(70001, 40, 1.7), (120000, 130, 0.9)])
+def test_class_sums(batch, per_class, tau):
+    """Values whose fp32 sums are exact (and have all 24 bits): a score is the sum times the reciprocal of tau in fp64,
+    rounded once."""
+    from difflogic_amd import difflogic_cuda as ext
+    k = 4
+    g = torch.Generator().manual_seed(batch)
+    x = torch.zeros(k, per_class, batch, dtype=torch.float64)
+    x[:, 0] = torch.randint(1024, 2048, (k, batch), generator=g).double()
+    x[:, per_class // 2] = torch.randint(0, 1024, (k, batch), generator=g).double() / 8192
+    want = (x.sum(1).numpy().T * (1.0 / tau)).astype(np.float16)
+    _same(ext.group_sum_forward(x.view(k * per_class, batch).half().cuda(), k, tau), want)
