@@ -1224,6 +1224,8 @@ template <typename T> Rows rows_kind(int64_t batch, const void *p0, const void *
     return batch >= V ? Rows::ragged : Rows::single;
 }
 
+#define DL_GRID_MAX (0xffffffffLL / DL_BLOCK)         // workgroups along x: HIP counts the threads in 32 bits
+
 unsigned col_tiles(int64_t ncols) {
     int64_t t = dl_ceil_div(ncols, DL_WAVE);
     return (unsigned) (t > 65535 ? 65535 : t);
@@ -1303,7 +1305,11 @@ int backward_both_t(const void *x, const int64_t *a, const int64_t *b, const voi
     const bool split = ncols >= 8 * DL_WAVE;                                         // as backward_w_t
     const int64_t row_blocks = dl_ceil_div(in_dim, 4), x_blocks = row_blocks * col_tiles(ncols);
     const int64_t blocks = x_blocks + (split ? dl_ceil_div(out_dim, NPW) : dl_ceil_div(out_dim, 4 * NPW));
-    if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
+    if (blocks > DL_GRID_MAX) {
+        // a launch holds less than 2^32 threads along x, where this one has the column tiles too: one launch each
+        const int st = backward_w_t<T>(x, a, b, gy, softmax_backward ? w : nullptr, gw, out_dim, batch, s, gdiv, w32);
+        return st != DL_OK ? st : backward_x_t<T>(x, a, b, w, gy, start, idx, gx, in_dim, batch, scale, s, gdiv, w32);
+    }
 #define DL_LAUNCH_BOTH(VV, WPN, RAG)                                                                                       \
     DL_LAUNCH((backward_both_kernel<T, VV, NPW, WPN, RAG>), dim3((unsigned) blocks), dim3(DL_BLOCK), 0, s, (const T *) x, a, \
               b, (const T *) w, (const T *) gy, softmax_backward ? (const T *) w : nullptr, start, idx, (T *) gw, (T *) gx, \

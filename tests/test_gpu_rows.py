@@ -162,3 +162,21 @@ def test_layers_walk_their_schedule_where_their_rows_are_long(ext, monkeypatch):
     (y0, w0, x0), (y1, w1, x1) = grads
     assert torch.equal(y0, y1) and torch.equal(w0, w1)
     assert within_budget(x0, x1, None, 1e-5)[0]
+
+
+def test_both_gradients_of_more_rows_than_one_launch_takes(ext):
+    """One workgroup per four input rows and the ones of grad_w after them are more than a launch takes along x."""
+    in_dim, out_dim = (1 << 26) - 4, 16
+    g = torch.Generator(device="cuda").manual_seed(0)
+    a, b = (torch.randint(0, in_dim, (out_dim,), device="cuda", generator=g) for _ in range(2))
+    a[0], b[1], a[2], b[3] = 0, in_dim - 1, in_dim - 1, 0
+    inputs, idx = torch.cat([a, b]).sort()
+    idx %= out_dim
+    start = torch.searchsorted(inputs, torch.arange(in_dim + 1, device="cuda"))
+    x = torch.rand(in_dim, 1, device="cuda", generator=g)
+    gy = torch.randn(out_dim, 1, device="cuda", generator=g)
+    p = torch.softmax(torch.randn(out_dim, 16, device="cuda", generator=g), -1)
+    gw, gx = ext.backward_both(x, a, b, p, gy, start, idx, 1.5, softmax_backward=True)
+    assert torch.equal(gw, ext.backward_logits(x, a, b, gy, p))
+    assert torch.equal(gx, ext.backward_x(x, a, b, p, gy, start, idx, 1.5))
+    assert torch.equal(gx.nonzero()[:, 0], inputs.unique())
