@@ -168,9 +168,9 @@ class LogicLayer(torch.nn.Module):
             return None
         a, b = self.indices
         schedule = difflogic_cuda.built_schedule(a, b, self.in_dim)
-        if schedule is not None and (not self.training or schedule._backward is not None):
+        if schedule is not None:
             return schedule
-        # building the schedule and its backward plan copies to and from the host
+        # building it copies to and from the host
         return None if torch.cuda.is_current_stream_capturing() else difflogic_cuda.schedule_for(a, b, self.in_dim)
 
     def _gate_ids(self):

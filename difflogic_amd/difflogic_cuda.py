@@ -361,9 +361,10 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
     if in_dim == 0 or out_dim == 0 or batch == 0:
         return None
     _check_schedule(schedule, in_dim, out_dim, dev)
-    dst, fix_vertex, fix_start, n_fix, rows = schedule.backward_plan()
-    if rows > in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
+    plan = schedule.backward_plan()
+    if plan is None or plan[4] > in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
         return None
+    dst, fix_vertex, fix_start, n_fix, rows = plan
     grad_w, grad_x = torch.empty_like(w), torch.empty_like(x)
     lib = _lib.load()
     ws_bytes = schedule.backward_bytes(rows, batch, code)
@@ -458,9 +459,10 @@ def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_
     if x is None and dtype == torch.float16:
         return None
     _check_schedule(schedule, in_dim, out_dim, dev)
-    dst, fix_vertex, fix_start, n_fix, rows = schedule.backward_plan()
-    if rows > in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
+    plan = schedule.backward_plan()
+    if plan is None or plan[4] > in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
         return None
+    dst, fix_vertex, fix_start, n_fix, rows = plan
     grad_w = torch.empty((out_dim, 16), dtype=dtype, device=dev)
     grad_w_lower = torch.empty((in_dim, 16), dtype=dtype, device=dev)
     fix_rows = torch.empty((n_fix, batch), dtype=dtype, device=dev) if n_fix else None
@@ -817,8 +819,11 @@ class EvalSchedule:
     def backward_plan(self):
         """(dst, fix_vertex, fix_start, n_fix, overflow_rows) for backward_chained, built on first
         use: where each schedule position's grad_x row goes and which inputs are summed from
-        several partial rows afterwards."""
+        several partial rows afterwards.  None where it would have to be built while a graph is being captured
+        (building it copies from the host)."""
         if self._backward is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
             import ctypes
             import numpy as np
             lib = _lib.load()
@@ -1302,8 +1307,9 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
     if want_x and want_w and schedule is not None:
         chained_code = code | _lib.DL_ROWS_ANY
         _check_schedule(schedule, in_dim, out_dim, dev)
-        dst, fix_vertex, fix_start, n_fix, rows = schedule.backward_plan()
-        if rows <= in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
+        plan = schedule.backward_plan()
+        if plan is not None and plan[4] <= in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
+            dst, fix_vertex, fix_start, n_fix, rows = plan
             grad_w = torch.empty((out_dim, 16), dtype=x.dtype, device=dev)
             grad_x = torch.empty_like(x)
             ws_bytes = lib.dl_logic_backward_chained_workspace_bytes(rows, out_dim, batch, chained_code)

@@ -140,3 +140,63 @@ def test_graphed_packed_inference_equals_eager_on_every_replay(F, widths, k, B):
     with torch.no_grad():
         eager = model(dl.PackBitsTensor(xs[1], bit_count=32))
     assert torch.equal(got, eager)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_captured_step_walks_the_schedules_of_the_warm_up(monkeypatch, fused):
+    """A layer whose input needs no gradient never builds the plan of the one-pass backward; its captured step runs along
+    the schedule all the same."""
+    import difflogic_amd as dl
+    from difflogic_amd.graphs import GraphedTrainStep
+    torch.manual_seed(0)
+    model = torch.nn.Sequential(dl.LogicLayer(4200, 20000), dl.LogicLayer(20000, 20000), dl.GroupSum(10, 100.0))
+    layers = [m for m in model if isinstance(m, dl.LogicLayer)]
+    model = (dl.fuse_for_training(model) if fused else model).train()
+    x, y = torch.rand(32, 4200, device="cuda"), torch.randint(0, 10, (32,), device="cuda")
+    asked, real = [], dl.LogicLayer._train_schedule
+
+    def spy(self, *args):
+        schedule = real(self, *args)
+        if torch.cuda.is_current_stream_capturing():
+            asked.append((layers.index(self), schedule is not None))
+        return schedule
+
+    monkeypatch.setattr(dl.LogicLayer, "_train_schedule", spy)
+    step = GraphedTrainStep(model, torch.nn.functional.cross_entropy, x, y)
+    assert {i for i, _ in asked} == {0, 1} and all(ok for _, ok in asked)
+    for _ in range(3):
+        loss = step.step().item()
+        grads = [p.grad.clone() for p in model.parameters()]
+        model.zero_grad(set_to_none=False)
+        eager = torch.nn.functional.cross_entropy(model(x), y)
+        eager.backward()
+        assert eager.item() == loss and all(torch.equal(p.grad, g) for p, g in zip(model.parameters(), grads))
+
+
+def test_capture_without_the_backward_plan():
+    """A schedule that only forward passes have used: its backward plan is not built under capture, the gradients come from
+    the other kernels."""
+    import difflogic_amd as dl
+    torch.manual_seed(0)
+    layer = dl.LogicLayer(4200, 20000).train()
+    x = torch.rand(32, 4200, device="cuda").requires_grad_()
+    with torch.no_grad():
+        layer(x)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        other = dl.LogicLayer(4200, 4200).train()(x)                   # (the autograd thread starts outside the capture)
+        torch.autograd.grad(other.sum(), x)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gx, gw = torch.autograd.grad(layer(x).square().sum(), (x, layer.weights))
+    schedule = dl.difflogic_cuda.built_schedule(*layer.indices, 4200)
+    assert schedule._backward is None
+    want_x, want_w = torch.autograd.grad(layer(x).square().sum(), (x, layer.weights))
+    assert schedule._backward is not None
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.allclose(gx, want_x, rtol=1e-5, atol=1e-5) and torch.equal(gw, want_w)
