@@ -1351,17 +1351,17 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_partial_kernel(const T *__
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = (C) 0;
     if (col < ncols) {
-        const T *xc = x + (cls * per_class) * batch;
+        const T *xc = x + (cls * per_class) * batch + at;
         int64_t r = r0 + wave;
         for (; r + 12 < r1; r += 16) {      // four independent row loads in flight per wave
             P v[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = row_vec<P, VEC, RAG>(xc, r + 4 * i, batch, ncols, col);
+            for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const P *>(xc + (r + 4 * i) * batch);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] += (up<T>(v[0].v[e]) + up<T>(v[1].v[e])) + (up<T>(v[2].v[e]) + up<T>(v[3].v[e]));
         }
         for (; r < r1; r += 4) {
-            const P v = row_vec<P, VEC, RAG>(xc, r, batch, ncols, col);
+            const P v = *reinterpret_cast<const P *>(xc + r * batch);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] += up<T>(v.v[e]);
         }
@@ -1454,7 +1454,9 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_group_sum_kernel(const T *__
 // One wave per 64 consecutive samples of one class; the four waves of a workgroup take
 // interleaved splits and are added in wave order, so the summation order is fixed.  The partial sums are added and scaled
 // (by the reciprocal of tau) in double and rounded to T once: an fp32 score of 64 is 8e-6 from its neighbours, which is
-// what the gradients of a net with large class sums see.
+// what the gradients of a net with large class sums see.  Bound by the latency of the partial sums, which come from the
+// other XCDs: eight loads in flight per wave, none of them behind a branch (a load under `s < splits` is one: the compiler
+// waits for each in turn).  GroupSum over 64000 rows at batch 100, 2 classes 36 -> 12 us, 10 classes 13 -> 8.
 template <typename T>
 __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typename Acc<T>::type *__restrict__ partial,
                                                                     T *__restrict__ y, int64_t batch, int64_t k,
@@ -1467,12 +1469,13 @@ __global__ __launch_bounds__(DL_BLOCK) void group_sum_finish_kernel(const typena
     const int64_t c = blockIdx.y;
     double sum = 0.0;
     if (r < batch)
-        for (int s = wave; s < splits; s += 64) {                // sixteen partial sums in flight, added in order
-            C v[16];
+        for (int s = wave; s < splits; s += 32) {
+            C v[8];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = s + 4 * i < splits ? partial[((int64_t) (s + 4 * i) * k + c) * batch + r] : (C) 0;
+            for (int i = 0; i < 8; ++i)                          // (past the end: the wave's own again, and not added)
+                v[i] = partial[((int64_t) (s + 4 * i < splits ? s + 4 * i : s) * k + c) * batch + r];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sum += (double) v[i];
+            for (int i = 0; i < 8; ++i) sum += s + 4 * i < splits ? (double) v[i] : 0.0;
         }
     lds[wave][lane] = sum;
     __syncthreads();
@@ -1590,9 +1593,10 @@ int forward_group_sum_t(const void *x, const int64_t *a, const int64_t *b, const
     return dl_launch_status();
 }
 
-// Number of row splits per class: enough workgroups to fill the chip, at least 32 rows each (64: layer and GroupSum on 8000
-// rows at batch 128 9.4 against 7.4 us).  Twice the workgroups: GroupSum over 128000 rows at batch 1024 97 -> 90 us, but
-// the finishing pass over the partial sums of 64000 rows at 512 5.3 -> 9.0.
+// Number of row splits per class: enough workgroups to fill the chip, at least 32 rows each (64 / 32: layer and GroupSum on
+// 8000 rows, 10 classes, batch 100 9.0 / 6.1 us; the GroupSum alone on 16000 rows at 500 7.3 / 8.5).  Twice the workgroups,
+// with a finishing pass that waited for its loads one by one: GroupSum over 128000 rows at batch 1024 97 -> 90 us, but the
+// finish over the partial sums of 64000 rows at 512 5.3 -> 9.0.
 int group_sum_splits(int64_t out_dim, int64_t batch, int64_t k) {
     const int64_t per_class = out_dim / k;
     const int64_t col_tiles = dl_ceil_div(batch, 4 * DL_WAVE);

@@ -180,3 +180,12 @@ def test_both_gradients_of_more_rows_than_one_launch_takes(ext):
     assert torch.equal(gw, ext.backward_logits(x, a, b, gy, p))
     assert torch.equal(gx, ext.backward_x(x, a, b, p, gy, start, idx, 1.5))
     assert torch.equal(gx.nonzero()[:, 0], inputs.unique())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("splits", [1, 3, 4, 5, 28, 29, 32, 33, 60, 61, 64, 65, 129, 1024])
+def test_partial_class_sums(ext, dtype, splits):
+    """The finishing pass of GroupSum around the four waves and the eight partial sums each takes at a time; sums that are
+    exact in every type."""
+    x = torch.randint(0, 8, (32 * splits, 65), generator=torch.Generator().manual_seed(splits)).double() / 8
+    assert torch.equal(ext.group_sum_forward(x.to(dtype).cuda(), 1, 1.0).cpu().double()[:, 0], x.sum(0).to(dtype).double())
