@@ -120,13 +120,13 @@ class LogicLayer(torch.nn.Module):
             w = torch.nn.functional.softmax(self.weights, dim=-1).to(x.dtype)
             return LogicLayerCudaFunction.apply(x, a, b, w, *tail, self._train_schedule(x)).transpose(0, 1)
         # eval mode: the discretised net on float inputs (no gradients)
+        schedule = _forward_walk(self._train_schedule(x), self.out_dim, x)
         if (same or mixed) and self.weights.is_cuda and self.weights.is_contiguous():
             with torch.no_grad():
-                return difflogic_cuda.forward(x, a, b, self.weights.detach(), self._train_schedule(x),
-                                              argmax=True).transpose(0, 1)
+                return difflogic_cuda.forward(x, a, b, self.weights.detach(), schedule, argmax=True).transpose(0, 1)
         w = torch.nn.functional.one_hot(self.weights.argmax(-1), 16).to(x.dtype)
         with torch.no_grad():
-            return difflogic_cuda.forward(x, a, b, w, self._train_schedule(x)).transpose(0, 1)
+            return difflogic_cuda.forward(x, a, b, w, schedule).transpose(0, 1)
 
     def forward_cuda_eval(self, x: PackBitsTensor):
         """Packed inference.  Updates ``x`` in place (as the reference rebinds ``x.t``) and
@@ -150,9 +150,9 @@ class LogicLayer(torch.nn.Module):
     # second gather of a row hits there; above it the chained kernels halve the gathered rows.
     _CHAIN_MIN_IN_DIM = 4096
     # Narrower layers are latency-bound: a wave walking 8 neurons in sequence only lengthens that, unless their rows are
-    # long.  Backward along the schedule / without, square fp32 layers: 16000 wide at batch 32 12.1 / 10.8 us, 100 14.0 /
-    # 13.1, 256 16.7 / 22.1; 30000 at 32 15.1 / 19.6; 8000 at 256 13.4 / 12.1, 512 16.7 / 22.2; 2000 at 2048 22.2 / 21.9.
-    # Forward at 16000: batch 100 6.0 / 6.0, 256 7.7 / 8.9.
+    # long.  Both gradients in one pass along the schedule / in one launch without, square fp32 layers: 16000 wide at batch 32
+    # 12.1 / 10.8 us, 100 14.0 / 13.1, 256 16.7 / 22.1; 30000 at 32 15.1 / 19.6; 8000 at 256 13.4 / 12.1, 512 16.7 / 22.2;
+    # 2000 at 2048 22.2 / 21.9.  (Which of their kernels take a schedule that is there: _forward_walk, _weights_walk.)
     _CHAIN_MIN_OUT_DIM = 20000
     _CHAIN_MIN_BYTES = 16_000_000           # ... of output rows: a quarter of the width is enough
 
@@ -225,6 +225,59 @@ class GroupSum(torch.nn.Module):
         return "k={}, tau={}".format(self.k, self.tau)
 
 
+# Layers of this many neurons walk their schedule in every kernel.  Narrower ones (LogicLayer._train_schedule) take the
+# one-pass backward along it and, kernel by kernel, what is measured to gain (fp32, whole vectors, with / without the
+# schedule): their own gathers are mostly served by the caches, and a wave walking its neurons in sequence is the longer
+# for it.
+_WALK_ALWAYS_OUT_DIM = 32768
+
+
+def _forward_pays(out_dim, x):
+    """Whether the forward kernels of a narrower layer gain on feature-major input like ``x``, as far as sizes tell.
+    20000 wide at batch 256 9.0 / 11.0 us, 6000 at 1024 12.4 / 15.6, but 668 11.3 / 9.2 and 24000 at 100 7.6 / 6.8; half
+    16000 at 1024 13.8 / 16.0, 20000 at 257 11.2 / 7.7; double 20000 at 256 16.7 / 21.3, 100 10.6 / 10.1."""
+    row = x.shape[1] * x.element_size()
+    if x.element_size() == 4:
+        return out_dim * row >= (16_000_000 if row <= 2048 else 24_000_000)
+    return out_dim * row >= 30_000_000 and row <= 8192
+
+
+def _forward_walk(schedule, out_dim, x):
+    """``schedule`` where the forward kernel of a layer of ``out_dim`` neurons takes it on ``x``, else None.  Half and double
+    only gain along trails that seldom break (16000 -> 24000, three uses of every input: 181 / 173 us at 2048 in double)."""
+    if schedule is None or out_dim >= _WALK_ALWAYS_OUT_DIM:
+        return schedule
+    return schedule if _forward_pays(out_dim, x) and (x.element_size() == 4 or 5 * schedule.steps <= 6 * out_dim) else None
+
+
+def _weights_walk(schedule, out_dim, x):
+    """The same for backward_w alone: 16000 wide at batch 512 14.1 / 16.9 us, 8000 at 1024 14.9 / 16.0, 512 11.3 / 9.6; double
+    16000 at 512 26.7 / 32.3, 257 22.5 / 21.0; half 20000 at 1024 22.1 / 20.5, 100 14.0 / 8.2."""
+    if schedule is None or out_dim >= _WALK_ALWAYS_OUT_DIM:
+        return schedule
+    row = x.shape[1] * x.element_size()
+    pays = out_dim * row >= 32_000_000 and (x.element_size() == 4 or (x.element_size() == 8 and 3584 <= row <= 4096))
+    return schedule if pays else None
+
+
+def _both_gradients(x, a, b, w, grad_y, start, idx, schedule, scale, softmax_backward):
+    """(grad of w or of its logits, grad_x) of a layer, x and grad_y not empty: in one pass along its schedule where it has one
+    and that applies, else without it.  (Widening layers have too many inputs at several positions: 24000 -> 30000 at
+    batch 100, two launches with backward_w along the schedule / without / one launch 30 / 26 / 22 us; 64000 -> 128000 at
+    1024, 559 / 580 / 571.)"""
+    if schedule is not None:
+        both = difflogic_cuda.backward_chained(x, w, grad_y, schedule, scale, softmax_backward=softmax_backward, any_rows=True)
+        if both is not None:
+            return both
+    out_dim = grad_y.shape[0]
+    if schedule is None or out_dim < _WALK_ALWAYS_OUT_DIM:
+        return difflogic_cuda.backward_both(x, a, b, w, grad_y, start, idx, scale, softmax_backward=softmax_backward)
+    grad_x = difflogic_cuda.backward_x(x, a, b, w, grad_y, start, idx, scale)
+    if softmax_backward:
+        return difflogic_cuda.backward_logits(x, a, b, grad_y, w, schedule), grad_x
+    return difflogic_cuda.backward_w(x, a, b, grad_y, schedule), grad_x
+
+
 class LogicLayerCudaFunction(torch.autograd.Function):
     """Feature-major forward/backward of one layer (difflogic/difflogic.py:205-221).  The
     optional trailing ``grad_factor`` is folded into backward_x instead of a separate
@@ -236,28 +289,22 @@ class LogicLayerCudaFunction(torch.autograd.Function):
         ctx.save_for_backward(x, a, b, w, given_x_indices_of_y_start, given_x_indices_of_y)
         ctx.grad_factor = grad_factor
         ctx.schedule = schedule
-        return difflogic_cuda.forward(x, a, b, w, schedule)
+        return difflogic_cuda.forward(x, a, b, w, _forward_walk(schedule, w.shape[0], x))
 
     @staticmethod
     def backward(ctx, grad_y):
         x, a, b, w, given_x_indices_of_y_start, given_x_indices_of_y = ctx.saved_tensors
         grad_y = grad_y.contiguous()
         grad_w = grad_x = None
-        if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is not None:
-            # one pass along the schedule yields both gradients
-            both = difflogic_cuda.backward_chained(x, w, grad_y, ctx.schedule, ctx.grad_factor, any_rows=True)
-            if both is not None:
-                return both[1], None, None, both[0], None, None, None, None
-        if (ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is None and x.numel() > 0
-                and grad_y.numel() > 0):
-            grad_w, grad_x = difflogic_cuda.backward_both(x, a, b, w, grad_y, given_x_indices_of_y_start,
-                                                          given_x_indices_of_y, ctx.grad_factor)
+        if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and x.numel() > 0 and grad_y.numel() > 0:
+            grad_w, grad_x = _both_gradients(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indices_of_y,
+                                             ctx.schedule, ctx.grad_factor, False)
             return grad_x, None, None, grad_w, None, None, None, None
         if ctx.needs_input_grad[0]:
             grad_x = difflogic_cuda.backward_x(x, a, b, w, grad_y, given_x_indices_of_y_start,
                                                given_x_indices_of_y, ctx.grad_factor)
         if ctx.needs_input_grad[3]:
-            grad_w = difflogic_cuda.backward_w(x, a, b, grad_y, ctx.schedule)
+            grad_w = difflogic_cuda.backward_w(x, a, b, grad_y, _weights_walk(ctx.schedule, w.shape[0], x))
         return grad_x, None, None, grad_w, None, None, None, None
 
 
@@ -268,7 +315,8 @@ class LogicLayerLogitsFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, a, b, logits, given_x_indices_of_y_start, given_x_indices_of_y, grad_factor=1.0,
                 schedule=None):
-        y, probs = difflogic_cuda.forward_logits(x, a, b, logits.detach().contiguous(), schedule)
+        y, probs = difflogic_cuda.forward_logits(x, a, b, logits.detach().contiguous(),
+                                                 _forward_walk(schedule, logits.shape[0], x))
         ctx.save_for_backward(x, a, b, probs, given_x_indices_of_y_start, given_x_indices_of_y)
         ctx.grad_factor = grad_factor
         ctx.schedule = schedule
@@ -279,21 +327,16 @@ class LogicLayerLogitsFunction(torch.autograd.Function):
         x, a, b, probs, given_x_indices_of_y_start, given_x_indices_of_y = ctx.saved_tensors
         grad_y = grad_y.contiguous()
         grad_logits = grad_x = None
-        if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is not None:
-            # one pass along the schedule yields both gradients
-            both = difflogic_cuda.backward_chained(x, probs, grad_y, ctx.schedule, ctx.grad_factor,
-                                                   softmax_backward=True, any_rows=True)
-            if both is not None:
-                return both[1], None, None, both[0], None, None, None, None
-        if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and ctx.schedule is None and grad_y.numel() > 0:
-            grad_logits, grad_x = difflogic_cuda.backward_both(x, a, b, probs, grad_y, given_x_indices_of_y_start,
-                                                               given_x_indices_of_y, ctx.grad_factor, softmax_backward=True)
+        if ctx.needs_input_grad[0] and ctx.needs_input_grad[3] and x.numel() > 0 and grad_y.numel() > 0:
+            grad_logits, grad_x = _both_gradients(x, a, b, probs, grad_y, given_x_indices_of_y_start, given_x_indices_of_y,
+                                                  ctx.schedule, ctx.grad_factor, True)
             return grad_x, None, None, grad_logits, None, None, None, None
         if ctx.needs_input_grad[0]:
             grad_x = difflogic_cuda.backward_x(x, a, b, probs, grad_y, given_x_indices_of_y_start,
                                                given_x_indices_of_y, ctx.grad_factor)
         if ctx.needs_input_grad[3]:
-            grad_logits = difflogic_cuda.backward_logits(x, a, b, grad_y, probs, ctx.schedule)
+            grad_logits = difflogic_cuda.backward_logits(x, a, b, grad_y, probs,
+                                                         _weights_walk(ctx.schedule, probs.shape[0], x))
         return grad_x, None, None, grad_logits, None, None, None, None
 
 
@@ -401,8 +444,8 @@ class LogicLayerPairFunction(torch.autograd.Function):
             y1 = None
             ctx.save_for_backward(x, a1, b1, probs1, a2, b2, probs2, start2, idx2)
         else:
-            y1, probs1 = difflogic_cuda.forward_logits(x, a1, b1, l1, schedule1)
-            y2, probs2 = difflogic_cuda.forward_logits(y1, a2, b2, l2, schedule2)
+            y1, probs1 = difflogic_cuda.forward_logits(x, a1, b1, l1, _forward_walk(schedule1, l1.shape[0], x))
+            y2, probs2 = difflogic_cuda.forward_logits(y1, a2, b2, l2, _forward_walk(schedule2, l2.shape[0], y1))
             ctx.save_for_backward(x, a1, b1, probs1, a2, b2, probs2, start2, idx2, y1)
         ctx.recompute = y1 is None
         ctx.grad_factor2, ctx.schedule1, ctx.schedule2 = grad_factor2, schedule1, schedule2
@@ -423,17 +466,15 @@ class LogicLayerPairFunction(torch.autograd.Function):
                 return None, None, None, g1, None, None, None, g2, None, None, None, None
         # the separate kernels, as two LogicLayers in a row would run them
         if y1 is None:
-            y1 = difflogic_cuda.forward(x, a1, b1, probs1, ctx.schedule1)
+            y1 = difflogic_cuda.forward(x, a1, b1, probs1, _forward_walk(ctx.schedule1, probs1.shape[0], x))
         if want1:
-            both = difflogic_cuda.backward_chained(y1, probs2, grad_y, ctx.schedule2, ctx.grad_factor2,
-                                                   softmax_backward=True, any_rows=True) if want2 else None
-            if both is not None:
-                g2, grad_y1 = both
+            if want2:
+                g2, grad_y1 = _both_gradients(y1, a2, b2, probs2, grad_y, start2, idx2, ctx.schedule2, ctx.grad_factor2, True)
             else:
                 grad_y1 = difflogic_cuda.backward_x(y1, a2, b2, probs2, grad_y, start2, idx2, ctx.grad_factor2)
-            g1 = difflogic_cuda.backward_logits(x, a1, b1, grad_y1, probs1, ctx.schedule1)
+            g1 = difflogic_cuda.backward_logits(x, a1, b1, grad_y1, probs1, _weights_walk(ctx.schedule1, probs1.shape[0], x))
         if want2 and g2 is None:
-            g2 = difflogic_cuda.backward_logits(y1, a2, b2, grad_y, probs2, ctx.schedule2)
+            g2 = difflogic_cuda.backward_logits(y1, a2, b2, grad_y, probs2, _weights_walk(ctx.schedule2, probs2.shape[0], y1))
         return None, None, None, g1, None, None, None, g2, None, None, None, None
 
 

@@ -189,3 +189,64 @@ def test_partial_class_sums(ext, dtype, splits):
     exact in every type."""
     x = torch.randint(0, 8, (32 * splits, 65), generator=torch.Generator().manual_seed(splits)).double() / 8
     assert torch.equal(ext.group_sum_forward(x.to(dtype).cuda(), 1, 1.0).cpu().double()[:, 0], x.sum(0).to(dtype).double())
+
+
+F16, F32, F64 = DTYPES
+
+
+@pytest.mark.parametrize("in_dim,out_dim,batch,dtype,forward,weights", [
+    (4200, 20000, 32, F32, False, False), (4200, 20000, 199, F32, False, False), (4200, 20000, 200, F32, True, False),
+    (4200, 8400, 714, F32, False, False), (4200, 8400, 715, F32, True, False), (4200, 8400, 952, F32, True, False),
+    (4200, 8400, 953, F32, True, True), (4200, 20000, 749, F16, False, False), (4200, 20000, 751, F16, True, False),
+    (4200, 8400, 447, F64, True, False), (4200, 8400, 477, F64, True, True), (4200, 6300, 600, F64, False, False),
+    (4200, 8400, 445, F64, False, False), (4200, 8400, 1025, F64, False, False), (4200, 33000, 4, F32, True, True),
+    (4200, 33000, 9, F16, True, True)])
+def test_kernels_of_narrower_layers_take_the_schedule_where_it_gains(ext, monkeypatch, in_dim, out_dim, batch, dtype, forward,
+                                                                     weights):
+    """Either side of the lines at which a layer below 32768 neurons walks its schedule, kernel by kernel; outputs and
+    gradients are those of the kernels without it."""
+    import difflogic_amd as dl
+    torch.manual_seed(batch)
+    layer = dl.LogicLayer(in_dim, out_dim).train()
+    x, gy = torch.rand(batch, in_dim, device="cuda").to(dtype), torch.randn(batch, out_dim, device="cuda").to(dtype)
+    walked, real_forward, real_weights = {}, ext.forward_logits, ext.backward_logits
+
+    def spy_forward(x, a, b, logits, schedule=None):
+        walked["forward"] = schedule is not None
+        return real_forward(x, a, b, logits, schedule)
+
+    def spy_weights(x, a, b, grad_y, probs, schedule=None):
+        walked["weights"] = schedule is not None
+        return real_weights(x, a, b, grad_y, probs, schedule)
+
+    monkeypatch.setattr(ext, "forward_logits", spy_forward)
+    monkeypatch.setattr(ext, "backward_logits", spy_weights)
+    y = layer(x)
+    y.backward(gy)
+    assert walked == {"forward": forward, "weights": weights}
+    xt, gt = x.t().contiguous(), gy.t().contiguous()
+    want, probs = real_forward(xt, *layer.indices, layer.weights.detach())
+    assert torch.equal(y.detach().t(), want) if dtype != F16 else within_budget(y.t(), want, None, RTOL[dtype])[0]
+    want = real_weights(xt, *layer.indices, gt, probs)
+    assert within_budget(layer.weights.grad, want, None, 1e-6)[0]
+
+
+@pytest.mark.parametrize("in_dim,out_dim,calls", [(8000, 20000, ["both"]), (20000, 40000, ["x", "weights"]), (20000, 20000, [])])
+def test_layers_that_widen(ext, monkeypatch, in_dim, out_dim, calls):
+    """Where the one-pass backward does not apply, narrower layers form both gradients in one launch."""
+    import difflogic_amd as dl
+    torch.manual_seed(1)
+    layer = dl.LogicLayer(in_dim, out_dim, grad_factor=1.5).train()
+    x = torch.rand(24, in_dim, device="cuda").requires_grad_()
+    gy = torch.randn(24, out_dim, device="cuda")
+    seen = []
+    for name, fn in (("x", "backward_x"), ("weights", "backward_logits"), ("both", "backward_both")):
+        real = getattr(ext, fn)
+        monkeypatch.setattr(ext, fn, lambda *a, real=real, name=name, **kw: seen.append(name) or real(*a, **kw))
+    layer(x).backward(gy)
+    assert seen == calls
+    monkeypatch.setattr(dl.LogicLayer, "_train_schedule", lambda self, x=None: None)
+    got = x.grad, layer.weights.grad
+    x.grad = layer.weights.grad = None
+    layer(x).backward(gy)
+    assert within_budget(got[0], x.grad, None, 1e-5)[0] and within_budget(got[1], layer.weights.grad, None, 1e-6)[0]
