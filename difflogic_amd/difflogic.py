@@ -121,6 +121,7 @@ class LogicLayer(torch.nn.Module):
             return LogicLayerCudaFunction.apply(x, a, b, w, *tail, self._train_schedule(x)).transpose(0, 1)
         # eval mode: the discretised net on float inputs (no gradients)
         schedule = _forward_walk(self._train_schedule(x), self.out_dim, x)
+        self._evaluated = True
         if (same or mixed) and self.weights.is_cuda and self.weights.is_contiguous():
             with torch.no_grad():
                 return difflogic_cuda.forward(x, a, b, self.weights.detach(), schedule, argmax=True).transpose(0, 1)
@@ -155,6 +156,7 @@ class LogicLayer(torch.nn.Module):
     # 2000 at 2048 22.2 / 21.9.  (Which of their kernels take a schedule that is there: _forward_walk, _weights_walk.)
     _CHAIN_MIN_OUT_DIM = 20000
     _CHAIN_MIN_BYTES = 16_000_000           # ... of output rows: a quarter of the width is enough
+    _evaluated = False                      # whether forward has run in eval mode on float inputs
 
     def _train_schedule(self, x=None):
         """Evaluation schedule of this layer's wiring for the chained forward / backward kernels (cached per
@@ -170,6 +172,10 @@ class LogicLayer(torch.nn.Module):
         schedule = difflogic_cuda.built_schedule(a, b, self.in_dim)
         if schedule is not None:
             return schedule
+        if not self.training and self.out_dim < _WALK_ALWAYS_OUT_DIM and not (
+                self._evaluated and x is not None and _forward_pays(self.out_dim, x)):
+            # building it takes milliseconds, which evaluating a narrower net once does not earn back
+            return None
         # building it copies to and from the host
         return None if torch.cuda.is_current_stream_capturing() else difflogic_cuda.schedule_for(a, b, self.in_dim)
 

@@ -140,7 +140,8 @@ def test_layers_walk_their_schedule_where_their_rows_are_long(ext, monkeypatch):
     import difflogic_amd as dl
     torch.manual_seed(2)
     layer = dl.LogicLayer(5000, 6000, grad_factor=1.5)
-    long, short = torch.rand(668, 5000, device="cuda"), torch.rand(600, 5000, device="cuda")
+    # (the forward kernel of 6000 neurons gains from 24 MB of rows on, batch 1000; up to then, 8.9 -> 11.5 us at 668, it loses)
+    long, short = torch.rand(1024, 5000, device="cuda"), torch.rand(600, 5000, device="cuda")
     graph, fresh = torch.cuda.CUDAGraph(), dl.LogicLayer(5000, 6000).eval()
     layer(short), torch.cuda.synchronize()
     with torch.cuda.graph(graph), torch.no_grad():
@@ -150,7 +151,7 @@ def test_layers_walk_their_schedule_where_their_rows_are_long(ext, monkeypatch):
     with torch.no_grad():
         assert torch.equal(out, fresh(long)) and ext.built_schedule(*fresh.indices, 5000) is not None
     assert layer._train_schedule(short.t()) is None and layer._train_schedule(long.t()) is not None
-    gy = torch.randn(668, 6000, device="cuda")
+    gy = torch.randn(1024, 6000, device="cuda")
     grads = []
     for least in (layer._CHAIN_MIN_BYTES, 1 << 60):
         monkeypatch.setattr(dl.LogicLayer, "_CHAIN_MIN_BYTES", least)
@@ -250,3 +251,23 @@ def test_layers_that_widen(ext, monkeypatch, in_dim, out_dim, calls):
     x.grad = layer.weights.grad = None
     layer(x).backward(gy)
     assert within_budget(got[0], x.grad, None, 1e-5)[0] and within_budget(got[1], layer.weights.grad, None, 1e-6)[0]
+
+
+def test_first_evaluation_builds_no_schedule(ext):
+    """A narrower layer evaluated once takes the kernels without a schedule; from the second evaluation on it has one, where
+    that gains.  Wider layers and training as ever."""
+    import difflogic_amd as dl
+    x, short = torch.rand(1024, 4200, device="cuda"), torch.rand(100, 4200, device="cuda")
+    built = lambda layer: ext.built_schedule(*layer.indices, 4200) is not None  # noqa: E731
+    layer = dl.LogicLayer(4200, 8400).eval()
+    first = layer(x)
+    assert not built(layer)
+    assert torch.equal(layer(x), first) and built(layer)
+    layer = dl.LogicLayer(4200, 20000).eval()
+    layer(short), layer(short)
+    assert not built(layer)
+    layer.train()(short)
+    assert built(layer)
+    layer = dl.LogicLayer(4200, 33000).eval()
+    layer(short)
+    assert built(layer)
