@@ -77,7 +77,9 @@ class GraphedPackedInference:
 
         def run():
             with torch.no_grad():
-                return model(PackBitsTensor(self.x, bit_count=bit_count))
+                packed = PackBitsTensor(self.x, bit_count=bit_count)
+                packed._replayed = True
+                return model(packed)
 
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())

@@ -39,10 +39,16 @@ _LAUNCH_SECONDS = 3e-6       # per kernel on the stream; decides between plans f
 # layer at once costs 4 us and the traffic of its rows.  784 -> 6 x 64000, graph replay, deferred / at once: batch 100
 # 188 / 48 us, 1000 190 / 76, 4000 196 / 135, 8000 200 / 202; 4 x 256000: batch 2000 249 / 166, 3000 252 / 265 (the bytes of
 # a layer's rows decide).  Narrower layers are bound by latency instead: 6 x 16000 at 12000 188 / 118, 4 x 32000 162 / 131
-# there; nets that fit in LDS run in one workgroup per 128 samples, 6 x 8000 at 100 74 / 35, 4000 75 / 62, 6000 75 / 75, 12000 77 / 101.
+# there; nets that fit in LDS run in one workgroup per 128 samples, 6 x 8000 at 100 74 / 35, 4000 75 / 58, 6000 76 / 68, 12000
+# 77 / 101.  The gates of the net change the deferred side: of nets that fit in LDS, 6 x 8000 with two-input gates only at 4000
+# 61 / 59, 5000 61 / 68, 6 x 6000 60 / 64, 6 x 4000 at 6000 67 / 60, half pass-through gates 6 x 8000 at 5000 61 / 63 (so
+# there a replayed graph has a line of its own; called eagerly, bound by the host, 144 / 91 at 6000); of wider nets both gain at
+# every limit (6 x 64000 at 7900, two-input 271 / 218, pass-through 213 / 185; 4 x 256000 at 2000 289 / 172, 261 / 170).
 _DIRECT_BYTES = 64 << 20         # rows of a layer's output
 _DIRECT_ROW_BYTES = 1536         # ... and one row of them
 _DIRECT_ROW_BYTES_LDS = 768      # one row, for layers that the LDS kernel takes
+_REPLAYED_ROW_BYTES_LDS = 512    # ... in a replayed graph, where a layer's output has more than
+_REPLAYED_BYTES_LDS = 3_300_000  # ... this many
 _DIRECT_MIN_OUT = 1000           # smaller layers, and the tapering end of a net below 4096, stay with the LDS kernel
 
 
@@ -56,10 +62,15 @@ _STORED_BYTES = 160 << 20        # rows of the last layer
 _STORED_ROW_BYTES = 5120         # ... and one row of them
 
 
-def _direct(in_dim, out_dim, row_bytes, lds_width):
-    """Whether a layer on rows of ``row_bytes`` is evaluated at once (above)."""
-    return (out_dim >= min(max(in_dim, _DIRECT_MIN_OUT), 4096) and 0 < out_dim * row_bytes <= _DIRECT_BYTES
-            and row_bytes <= (_DIRECT_ROW_BYTES_LDS if max(in_dim, out_dim) <= lds_width else _DIRECT_ROW_BYTES))
+def _direct(in_dim, out_dim, row_bytes, lds_width, replayed):
+    """Whether a layer on rows of ``row_bytes`` is evaluated at once (above); ``replayed``: as part of a replayed graph."""
+    if out_dim < min(max(in_dim, _DIRECT_MIN_OUT), 4096) or not 0 < out_dim * row_bytes <= _DIRECT_BYTES:
+        return False
+    if max(in_dim, out_dim) > lds_width:
+        return row_bytes <= _DIRECT_ROW_BYTES
+    if replayed and out_dim * row_bytes > _REPLAYED_BYTES_LDS:
+        return row_bytes <= _REPLAYED_ROW_BYTES_LDS
+    return row_bytes <= _DIRECT_ROW_BYTES_LDS
 
 
 def _chained(depth):
@@ -201,6 +212,8 @@ class PackBitsTensor:
     as int64 words: the same bytes as words of any of the four widths, so every batch size and word
     width runs the same vector kernels.  ``.t`` is a view of those rows where their length allows
     it and a copy cut to ``ceil(B / bit_count)`` words otherwise."""
+
+    _replayed = False                 # set by GraphedPackedInference, on the inputs of its warm-up calls and of the captured one
 
     def __init__(self, t: torch.BoolTensor, bit_count=32, device="cuda"):
         assert len(t.shape) == 2, t.shape
@@ -379,7 +392,7 @@ class PackBitsTensor:
     def takes_weights(self, out_dim):
         """Whether a layer of ``out_dim`` neurons applied next is best evaluated at once, from its weights (apply_weights)."""
         return not self._pending and _direct(self._in_features(), out_dim, self._row_bytes(self._batch),
-                                             difflogic_cuda.net_lds_max_width())
+                                             difflogic_cuda.net_lds_max_width(), self._replayed)
 
     def apply_weights(self, a, b, weights):
         """Applies the gate layer with wiring ``a``, ``b`` and the argmax gates of ``weights`` [out, 16], now."""

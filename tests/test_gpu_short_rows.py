@@ -128,3 +128,25 @@ def test_words_written_between_layers_at_once():
         assert np.array_equal(p.group_sum(10).cpu().numpy(), po.groupbitsum(top, p.pad_len, 10))
         assert np.array_equal(p.t.cpu().numpy(), top)
         assert tuple(model(dl.PackBitsTensor(torch.zeros(0, F, dtype=torch.bool, device="cuda"))).shape) == (0, 10)
+
+
+@pytest.mark.parametrize("width,B,at_once", [(6500, 4096, True), (6500, 4097, False), (4290, 6144, True), (4300, 6144, False)])
+def test_replayed_net_that_fits_in_lds(monkeypatch, width, B, at_once):
+    """Either side of the lines that hold for a replayed graph, in its warm-up calls too; every replay gives the oracle's
+    counts.  Called eagerly all of them are evaluated at once."""
+    import difflogic_amd as dl
+    from difflogic_amd.graphs import GraphedPackedInference
+    rng = np.random.default_rng(B + width)
+    layers = random_layers(rng, 50, [width, width])
+    x, other = (rng.random((B, 50)) < 0.4 for _ in range(2))
+    model = build_model(50, layers, 10).eval()
+    calls, real = [], dl.PackBitsTensor.apply_weights
+    monkeypatch.setattr(dl.PackBitsTensor, "apply_weights", lambda self, *a: calls.append(1) or real(self, *a))
+    graph = GraphedPackedInference(model, torch.as_tensor(x).cuda())
+    assert len(calls) == (6 if at_once else 0)                         # two warm-up calls and the captured one, two layers each
+    for batch in (x, other, x):
+        assert np.array_equal(graph(torch.as_tensor(batch).cuda()).cpu().numpy(), interp.net_eval(batch, layers, 10))
+    calls.clear()
+    with torch.no_grad():
+        model(dl.PackBitsTensor(torch.as_tensor(x).cuda()))
+    assert len(calls) == 2

@@ -168,3 +168,17 @@ def test_wiring_cache_lives_and_dies_with_its_tensors():
     # a new tensor that happens to reuse a freed address is never served a dead tensor's entry
     a = torch.arange(6)
     assert cache.get((a, b), (7,), build) is not v2
+
+
+def test_layers_evaluated_at_once():
+    """Sizes either side of the lines between layers evaluated when they are applied and deferred ones; in a replayed graph a
+    net that fits in LDS is deferred where its gates may make that the faster way."""
+    from difflogic_amd.packbitstensor import _direct
+    eager, replayed = (lambda *a, c=c: _direct(*a, 10240, c) for c in (False, True))  # noqa: E731
+    for in_dim, out_dim, row, eagerly, in_graph in (
+            (8000, 8000, 512, True, True), (8000, 8000, 528, True, False), (6000, 6000, 640, True, False),
+            (8000, 8000, 768, True, False), (8000, 8000, 784, False, False), (4000, 4000, 768, True, True),
+            (4296, 4296, 768, True, True), (4297, 4297, 768, True, False), (64000, 64000, 1040, True, True),
+            (64000, 64000, 1056, False, False), (10250, 10250, 1536, True, True), (10250, 10250, 1552, False, False),
+            (784, 999, 16, False, False), (784, 1000, 16, True, True), (8000, 4000, 16, False, False), (784, 8000, 0, False, False)):
+        assert (eager(in_dim, out_dim, row), replayed(in_dim, out_dim, row)) == (eagerly, in_graph), (in_dim, out_dim, row)
