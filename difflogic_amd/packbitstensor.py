@@ -276,6 +276,14 @@ class PackBitsTensor:
         self._src = None
         return self._rows
 
+    def _held_row_bytes(self):
+        """Length of a row as `_words` returns it, without packing or copying anything."""
+        if self._rows is not None:
+            return self._rows.shape[1] * 8
+        if self._public is not None:
+            return 16 * -(-self._public.shape[1] * self._public.element_size() // 16)
+        return self._row_bytes(self._batch)
+
     def _pad(self, rows):
         """Padding bits at the end of a padded row."""
         return rows.shape[1] * 64 - self._batch
@@ -323,6 +331,12 @@ class PackBitsTensor:
             _LIVE_SHARES[key] = share
         return share
 
+    @staticmethod
+    def _run_group(rows, group, out_live=None):
+        if _chained(len(group)):
+            return difflogic_cuda.eval_chained(rows, group, out_live=out_live)
+        return difflogic_cuda.eval_fused(rows, group)
+
     def _run_groups(self, groups, live=None):
         """Evaluates the first sum(groups) pending layers group by group.  ``live`` (difflogic_cuda.live_inputs of
         the pending layers): rows that the layers still pending afterwards do not look at need not be written; the
@@ -333,10 +347,7 @@ class PackBitsTensor:
         for depth in groups:
             group = self._pending[pos:pos + depth]
             pos += depth
-            if _chained(depth):
-                rows = difflogic_cuda.eval_chained(rows, group, out_live=live[pos] if live and pos < len(live) else None)
-            else:
-                rows = difflogic_cuda.eval_fused(rows, group)
+            rows = self._run_group(rows, group, live[pos] if live and pos < len(live) else None)
         if pos:
             self._rows, self._public = rows, None
         self._pending = self._pending[pos:]
@@ -424,7 +435,7 @@ class PackBitsTensor:
                                                   folded=self._folded)
                 if out is not None:
                     return out
-            row_bytes = self._words().shape[1] * 8
+            row_bytes = self._held_row_bytes()
             if row_bytes <= _STORED_ROW_BYTES and self.features * row_bytes <= _STORED_BYTES:
                 self._run_groups(plan_groups(self._dims(), False, self._words64(), share))
                 rows = self._words()

@@ -150,3 +150,34 @@ def test_replayed_net_that_fits_in_lds(monkeypatch, width, B, at_once):
     with torch.no_grad():
         model(dl.PackBitsTensor(torch.as_tensor(x).cuda()))
     assert len(calls) == 2
+
+
+@pytest.mark.parametrize("widths", [[12000], [6000, 12000], [6000, 6000, 6000, 12000]])
+def test_counting_stored_rows(monkeypatch, widths):
+    """Counting deferred layers from stored rows: words that are no whole vectors are copied into padded rows once, not to
+    learn their length, and the object can be counted and read again."""
+    import difflogic_amd as dl
+    from difflogic_amd import packbitstensor as pbt
+    monkeypatch.setattr(pbt, "_DIRECT_BYTES", 0)
+    monkeypatch.setattr(pbt, "lds_tail", lambda *a, **kw: 0)
+    rng = np.random.default_rng(9)
+    F, k, batch = 50, 10, 4064
+    layers = random_layers(rng, F, widths)
+    logic = [m for m in build_model(F, layers, k).eval() if isinstance(m, dl.LogicLayer)]
+    words = rng.integers(-2**31, 2**31, (F, batch // 32), dtype=np.int32)            # 508 bytes: no whole 16-byte vectors
+    x = np.unpackbits(words.view(np.uint8), axis=1, bitorder="little").T[:batch].astype(bool)
+    want = interp.net_eval(x, layers, k)
+    with torch.no_grad():
+        p = dl.PackBitsTensor(torch.zeros(batch, F, dtype=torch.bool, device="cuda"), bit_count=32)
+        p.t = _dev(words)
+        for m in logic:
+            p = m(p)
+        copies, real = [], pbt.PackBitsTensor._adopt
+        monkeypatch.setattr(pbt.PackBitsTensor, "_adopt", lambda self, v: copies.append(v.shape) or real(self, v))
+        assert np.array_equal(p.group_sum(k).cpu().numpy(), want) and len(copies) == 1
+        assert np.array_equal(p.group_sum(k).cpu().numpy(), want)
+        want = words
+        for a, b, op in layers:
+            want = po.eval_layer(want, a, b, op)
+        assert np.array_equal(p.t.cpu().numpy(), want)
+        assert np.array_equal(p.group_sum(k).cpu().numpy(), po.groupbitsum(want, p.pad_len, k))
