@@ -437,8 +437,12 @@ class PackBitsTensor:
                     return out
             row_bytes = self._held_row_bytes()
             if row_bytes <= _STORED_ROW_BYTES and self.features * row_bytes <= _STORED_BYTES:
-                self._run_groups(plan_groups(self._dims(), False, self._words64(), share))
-                rows = self._words()
+                groups = plan_groups(self._dims(), False, self._words64(), share)
+                if len(groups) > 1:
+                    self._run_groups(groups[:-1])
+                # the last group stays pending and its rows are not kept: the object's state does not change by counting
+                self._fold_pending()
+                rows = self._run_group(self._words(), self._pending)
                 return difflogic_cuda.groupbitsum(rows, self._pad(rows), k)
             self._fold_pending()
             groups = plan_groups(self._dims(), True, self._words64(), share)

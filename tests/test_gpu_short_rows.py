@@ -154,8 +154,8 @@ def test_replayed_net_that_fits_in_lds(monkeypatch, width, B, at_once):
 
 @pytest.mark.parametrize("widths", [[12000], [6000, 12000], [6000, 6000, 6000, 12000]])
 def test_counting_stored_rows(monkeypatch, widths):
-    """Counting deferred layers from stored rows: words that are no whole vectors are copied into padded rows once, not to
-    learn their length, and the object can be counted and read again."""
+    """Counting deferred layers from stored rows: the last layer's rows are given back, the object can be counted and read
+    again, and words that are no whole vectors are copied into padded rows once, not to learn their length."""
     import difflogic_amd as dl
     from difflogic_amd import packbitstensor as pbt
     monkeypatch.setattr(pbt, "_DIRECT_BYTES", 0)
@@ -174,7 +174,10 @@ def test_counting_stored_rows(monkeypatch, widths):
             p = m(p)
         copies, real = [], pbt.PackBitsTensor._adopt
         monkeypatch.setattr(pbt.PackBitsTensor, "_adopt", lambda self, v: copies.append(v.shape) or real(self, v))
+        p._live_share(), torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
         assert np.array_equal(p.group_sum(k).cpu().numpy(), want) and len(copies) == 1
+        assert torch.cuda.memory_allocated() - before < 12000 * 512              # at most the rows of an earlier layer
         assert np.array_equal(p.group_sum(k).cpu().numpy(), want)
         want = words
         for a, b, op in layers:
