@@ -1626,10 +1626,10 @@ int chain_chunk(int64_t steps) {
 
 template <typename T, int GATES>
 int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps,
-                    const void *w, void *y, void *probs, int64_t batch, hipStream_t s, bool w32 = false) {
+                    const void *w, void *y, void *probs, int64_t batch, bool any_rows, hipStream_t s, bool w32 = false) {
     constexpr int V = Vec16<T>::n;
     const Rows kind = rows_kind<T>(batch, x, y);
-    if (kind == Rows::single) return DL_ERR_TOO_LARGE;
+    if (kind != Rows::whole && !(any_rows && kind == Rows::ragged)) return DL_ERR_TOO_LARGE;
     const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
     const T *xp = (const T *) x, *wp = (const T *) w;
     const dim3 block(DL_BLOCK);
@@ -1697,11 +1697,11 @@ int forward_chain_lower_t(const void *lx, const int64_t *la, const int64_t *lb, 
 
 template <typename T>
 int backward_w_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps,
-                       const void *gy, const void *probs, void *gw, int64_t batch, hipStream_t s, int64_t gdiv = 0,
-                       bool w32 = false) {
+                       const void *gy, const void *probs, void *gw, int64_t batch, bool any_rows, hipStream_t s,
+                       int64_t gdiv = 0, bool w32 = false) {
     constexpr int V = Vec16<T>::n;
     const Rows kind = rows_kind<T>(batch, x, gy);
-    if (kind == Rows::single) return DL_ERR_TOO_LARGE;
+    if (kind != Rows::whole && !(any_rows && kind == Rows::ragged)) return DL_ERR_TOO_LARGE;
     const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
     const int64_t blocks = dl_ceil_div(nchunks, 4);
     if (blocks > 0x7fffffffLL || ncols > 4 * DL_WAVE) return DL_ERR_TOO_LARGE;   // a lane holds at most 4 vectors of a row
@@ -1933,7 +1933,7 @@ extern "C" int dl_logic_backward_chained_lower(const void *x, const int32_t *ver
 extern "C" int dl_logic_forward_chained(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip,
                                         int64_t steps, const void *w, void *y, void *probs, int64_t in_dim,
                                         int64_t out_dim, int64_t batch, int dtype, void *stream) {
-    const bool argmax = gates_argmax(dtype), w32 = weights_fp32(dtype);
+    const bool any = takes_any_rows(dtype), argmax = gates_argmax(dtype), w32 = weights_fp32(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim < 0 || out_dim < 0 || batch <= 0 || steps < out_dim || steps % DL_TRAIN_CHUNK != 0)
         return DL_ERR_INVALID_ARGUMENT;
@@ -1943,22 +1943,22 @@ extern "C" int dl_logic_forward_chained(const void *x, const int32_t *verts, con
     hipStream_t s = (hipStream_t) stream;
     if (probs) {
         switch (dtype) {
-        case DL_F16: return forward_chain_t<__half, true>(x, verts, neuron, flip, steps, w, y, probs, batch, s, w32);
-        case DL_F32: return forward_chain_t<float, true>(x, verts, neuron, flip, steps, w, y, probs, batch, s);
-        default: return forward_chain_t<double, true>(x, verts, neuron, flip, steps, w, y, probs, batch, s, w32);
+        case DL_F16: return forward_chain_t<__half, true>(x, verts, neuron, flip, steps, w, y, probs, batch, any, s, w32);
+        case DL_F32: return forward_chain_t<float, true>(x, verts, neuron, flip, steps, w, y, probs, batch, any, s);
+        default: return forward_chain_t<double, true>(x, verts, neuron, flip, steps, w, y, probs, batch, any, s, w32);
         }
     }
     if (argmax) {
         switch (dtype) {
-        case DL_F16: return forward_chain_t<__half, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s, w32);
-        case DL_F32: return forward_chain_t<float, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s);
-        default: return forward_chain_t<double, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s, w32);
+        case DL_F16: return forward_chain_t<__half, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
+        case DL_F32: return forward_chain_t<float, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s);
+        default: return forward_chain_t<double, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
         }
     }
     switch (dtype) {
-    case DL_F16: return forward_chain_t<__half, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s, w32);
-    case DL_F32: return forward_chain_t<float, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s);
-    default: return forward_chain_t<double, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, s, w32);
+    case DL_F16: return forward_chain_t<__half, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
+    case DL_F32: return forward_chain_t<float, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s);
+    default: return forward_chain_t<double, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
     }
 }
 
@@ -1997,7 +1997,7 @@ extern "C" int dl_logic_backward_w_chained(const void *x, const int32_t *verts, 
                                            const uint8_t *flip, int64_t steps, const void *grad_y, const void *probs,
                                            void *grad_w, int64_t in_dim, int64_t out_dim, int64_t batch, int dtype,
                                            void *stream) {
-    const bool w32 = weights_fp32(dtype);
+    const bool any = takes_any_rows(dtype), w32 = weights_fp32(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim < 0 || out_dim < 0 || batch <= 0 || steps < out_dim || steps % DL_TRAIN_CHUNK != 0)
         return DL_ERR_INVALID_ARGUMENT;
@@ -2005,9 +2005,9 @@ extern "C" int dl_logic_backward_w_chained(const void *x, const int32_t *verts, 
     if (!x || !verts || !neuron || !flip || !grad_y || !grad_w || in_dim == 0) return DL_ERR_INVALID_ARGUMENT;
     hipStream_t s = (hipStream_t) stream;
     switch (dtype) {
-    case DL_F16: return backward_w_chain_t<__half>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, s, 0, w32);
-    case DL_F32: return backward_w_chain_t<float>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, s);
-    default: return backward_w_chain_t<double>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, s, 0, w32);
+    case DL_F16: return backward_w_chain_t<__half>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, any, s, 0, w32);
+    case DL_F32: return backward_w_chain_t<float>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, any, s);
+    default: return backward_w_chain_t<double>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, any, s, 0, w32);
     }
 }
 

@@ -156,8 +156,8 @@ def forward(x, a, b, w, schedule=None, argmax=False):
         if schedule is not None and out_dim > 0 and batch > 0:
             _check_schedule(schedule, in_dim, out_dim, dev)
             st = lib.dl_logic_forward_chained(_p(x), _p(schedule.verts), _p(schedule.neuron), _p(schedule.flip),
-                                              schedule.steps, _p(w), _p(y), None, in_dim, out_dim, batch, code,
-                                              _stream(dev))
+                                              schedule.steps, _p(w), _p(y), None, in_dim, out_dim, batch,
+                                              code | _lib.DL_ROWS_ANY, _stream(dev))
         if st == _lib.DL_ERR_TOO_LARGE:
             st = lib.dl_logic_forward(_p(x), _p(a), _p(b), _p(w), _p(y), in_dim, out_dim, batch, code, _stream(dev))
     if st:
@@ -187,7 +187,7 @@ def backward_w(x, a, b, grad_y, schedule=None):
             _check_schedule(schedule, in_dim, out_dim, dev)
             st = lib.dl_logic_backward_w_chained(_p(x), _p(schedule.verts), _p(schedule.neuron), _p(schedule.flip),
                                                  schedule.steps, _p(grad_y), None, _p(grad_w), in_dim, out_dim, batch,
-                                                 code, _stream(dev))
+                                                 code | _lib.DL_ROWS_ANY, _stream(dev))
         if st == _lib.DL_ERR_TOO_LARGE:
             st = lib.dl_logic_backward_w(_p(x), _p(a), _p(b), _p(grad_y), _p(grad_w), in_dim, out_dim, batch, code,
                                          _stream(dev))
@@ -289,7 +289,7 @@ def forward_logits(x, a, b, logits, schedule=None):
         _check_schedule(schedule, in_dim, out_dim, x.device)
         st = _launch(index, lib.dl_logic_forward_chained, x.data_ptr(), schedule.verts.data_ptr(), schedule.neuron.data_ptr(),
                      schedule.flip.data_ptr(), schedule.steps, logits.data_ptr(), y.data_ptr(), probs.data_ptr(), in_dim,
-                     out_dim, batch, code)
+                     out_dim, batch, code | _lib.DL_ROWS_ANY)
     if st == _lib.DL_ERR_TOO_LARGE:
         st = _launch(index, lib.dl_logic_forward_logits, x.data_ptr(), a.data_ptr(), b.data_ptr(), logits.data_ptr(),
                      y.data_ptr(), probs.data_ptr(), in_dim, out_dim, batch, code)
@@ -330,7 +330,7 @@ def backward_logits(x, a, b, grad_y, probs, schedule=None):
         _check_schedule(schedule, in_dim, out_dim, x.device)
         st = _launch(index, lib.dl_logic_backward_w_chained, x.data_ptr(), schedule.verts.data_ptr(),
                      schedule.neuron.data_ptr(), schedule.flip.data_ptr(), schedule.steps, grad_y.data_ptr(),
-                     probs.data_ptr(), grad_logits.data_ptr(), in_dim, out_dim, batch, code)
+                     probs.data_ptr(), grad_logits.data_ptr(), in_dim, out_dim, batch, code | _lib.DL_ROWS_ANY)
     if st == _lib.DL_ERR_TOO_LARGE:
         st = _launch(index, lib.dl_logic_backward_logits, x.data_ptr(), a.data_ptr(), b.data_ptr(), grad_y.data_ptr(),
                      probs.data_ptr(), grad_logits.data_ptr(), in_dim, out_dim, batch, code)

@@ -53,9 +53,9 @@ typedef enum dl_status {
 typedef enum dl_dtype { DL_F16 = 0, DL_F32 = 1, DL_F64 = 2, DL_F16_W32 = 3, DL_F64_W32 = 4 } dl_dtype;
 
 /* Or'ed into `dtype`: rows that are not whole 16-byte vectors, or whose base address is not 16-byte
- * aligned, are taken as well, as long as a row holds at least 16 bytes (dl_logic_backward_chained,
- * its _lower and _grouped forms and its workspace size, dl_logic_forward_chained_lower; without it
- * these return DL_ERR_TOO_LARGE for such rows).  The workspace stays 16-byte aligned. */
+ * aligned, are taken as well, as long as a row holds at least 16 bytes (dl_logic_forward_chained and
+ * its _lower form, dl_logic_backward_w_chained, dl_logic_backward_chained, its _lower and _grouped
+ * forms and its workspace size; without it these return DL_ERR_TOO_LARGE for such rows).  The workspace stays 16-byte aligned. */
 #define DL_ROWS_ANY 0x100
 
 /* Or'ed into `dtype` of dl_logic_forward and dl_logic_forward_chained (probs NULL): `w` holds weights of which
@@ -103,15 +103,15 @@ int dl_logic_backward_logits(const void *x, const int64_t *a, const int64_t *b, 
 /* forward / backward_w walked along an evaluation schedule of the layer's wiring (built with
  * dl_eval_schedule_build, declared below): consecutive neurons share an input row, which stays in
  * registers, so a neuron costs one gathered row instead of two.  Results are bit-identical to
- * dl_logic_forward(_logits) / dl_logic_backward_w(_logits) in fp32 and fp64 (fp16 outputs can
- * differ in the last bit).  No counterpart in the reference.
+ * dl_logic_forward(_logits) / dl_logic_backward_w(_logits) in fp32 and fp64 (fp16 outputs on rows of
+ * whole vectors can differ in the last bit).  No counterpart in the reference.
  *   verts [steps+1], neuron [steps], flip [steps]: DEVICE copies of the schedule.
  *   probs: forward  - NULL: `w` holds probabilities; else `w` holds logits and probs receives
  *                     softmax(w) (as dl_logic_forward_logits);
  *          backward - NULL: plain grad_w; else the softmax backward is chained
  *                     (as dl_logic_backward_logits).
- * Return DL_ERR_TOO_LARGE where the chained kernels do not apply (rows shorter than 16 bytes;
- * backward_w: rows longer than 256 vectors of 16 bytes);
+ * Return DL_ERR_TOO_LARGE where the chained kernels do not apply (batch not a multiple of 16
+ * bytes of elements, unaligned buffers: see DL_ROWS_ANY; backward_w: rows longer than 256 vectors of 16 bytes);
  * the caller then uses the unchained entry points. */
 int dl_logic_forward_chained(const void *x, const int32_t *verts, const int32_t *neuron,
                              const uint8_t *flip, int64_t steps, const void *w, void *y, void *probs,

@@ -82,3 +82,17 @@ def test_library_shares_torchs_hip_runtime_whatever_the_import_order():
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT, timeout=300)
     assert out.returncode == 0, out.stderr
     assert out.stdout.split()[0] == "1", out.stdout
+
+
+def test_rows_that_are_no_whole_vectors_are_refused_without_the_flag():
+    """The chained entry points answer DL_ERR_TOO_LARGE before any launch (with DL_ROWS_ANY: for rows under 16 bytes)."""
+    from difflogic_amd import _lib
+    lib = _lib.load()
+    null, p, odd = ctypes.c_void_p(0), ctypes.c_void_p(4096), ctypes.c_void_p(4100)       # never dereferenced
+    forward = lambda x, batch, code, y=p: lib.dl_logic_forward_chained(x, p, p, p, 32, p, y, null, 4, 32, batch, code, null)  # noqa: E731
+    weights = lambda x, batch, code, g=p: lib.dl_logic_backward_w_chained(x, p, p, p, 32, g, null, p, 4, 32, batch, code, null)  # noqa: E731
+    for call in (forward, weights):
+        for code, vector in ((_lib.DL_F16, 8), (_lib.DL_F32, 4), (_lib.DL_F64, 2), (_lib.DL_F16_W32, 8), (_lib.DL_F64_W32, 2)):
+            assert call(p, vector + 1, code) == _lib.DL_ERR_TOO_LARGE
+            assert call(odd, vector, code) == _lib.DL_ERR_TOO_LARGE and call(p, vector, code, odd) == _lib.DL_ERR_TOO_LARGE
+            assert call(p, vector - 1, code | _lib.DL_ROWS_ANY) == _lib.DL_ERR_TOO_LARGE
