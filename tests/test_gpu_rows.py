@@ -271,3 +271,26 @@ def test_first_evaluation_builds_no_schedule(ext):
     layer = dl.LogicLayer(4200, 33000).eval()
     layer(short)
     assert built(layer)
+
+
+@pytest.mark.parametrize("dtype,batch", [c for c in CASES if c[0] != F16])
+def test_elements_that_two_lanes_write(ext, monkeypatch, dtype, batch):
+    """Outputs and input gradients on rows that end inside a vector are, bit for bit, those of the same call on the rows
+    padded to whole vectors (half: tests of its rounding)."""
+    from difflogic_amd.functional import build_reverse_index
+    monkeypatch.setattr(ext, "BACKWARD_CHAIN_MAX_OVERFLOW", 1e9)
+    in_dim, out_dim = 60, 88
+    g = torch.Generator().manual_seed(batch)
+    a, b = (torch.randint(0, in_dim, (out_dim,), generator=g) for _ in range(2))
+    start, idx = (t.cuda() for t in build_reverse_index(a, b, in_dim))
+    a, b = a.cuda(), b.cuda()
+    sched = ext.schedule_for(a, b, in_dim)
+    whole = -(-batch // 8) * 8
+    x = torch.rand(in_dim, whole, generator=g).to(dtype).cuda()
+    gy = torch.randn(out_dim, whole, generator=g).to(dtype).cuda()
+    p = torch.softmax(torch.randn(out_dim, 16, generator=g), -1).to(dtype).cuda()
+    xr, gr = x[:, :batch].contiguous(), gy[:, :batch].contiguous()
+    for call in (lambda x, gy: ext.forward(x, a, b, p), lambda x, gy: ext.forward(x, a, b, p, sched),
+                 lambda x, gy: ext.backward_x(x, a, b, p, gy, start, idx, 1.5),
+                 lambda x, gy: ext.backward_chained(x, p, gy, sched, 1.5, any_rows=True)[1]):
+        assert torch.equal(call(xr, gr), call(x, gy)[:, :batch])
