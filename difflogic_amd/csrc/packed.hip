@@ -2226,10 +2226,17 @@ static int pack_batch_major_rows(const uint8_t *x, void *out, int64_t batch, int
     const int64_t gx = dl_ceil_div(cols, 16);
     if (gx > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     const bool vectors = features % 16 == 0 && dl_aligned(x, 16);
-    // Up to 192 words per row (batch 12288) the tile kernels have too few workgroups (784 features: 17 us against 4 at batch
-    // 1000, 17 against 5 at 10000, 17 against 9 at 16000, 17 against 16 at 32000; 9216 features: 50 against 36 at 10000, 51
-    // against 55 at 16000; 785 features, byte loads: 45 against 20 at 10000, 39 against 36 at 16000).
-    if (out_row_bytes % 8 == 0 && cols <= 192) {
+    // Up to 192 words per row (batch 12288) the tile kernels have too few workgroups, unless there are many features: the
+    // ballot kernel reads a sample's row in pieces of 64 bytes, 2 TB/s at most, byte loads 0.35.  Tile / ballot kernel: 784
+    // features 17 / 4 us at batch 1000, 17 / 5 at 10000, (17 / 9 at 16000); 9216 at 10000 50 / 36, 12288 50 / 43; 12288 at
+    // 10000 47 / 46; 20000 at 4000 49 / 43, 5000 51 / 53; 100000 at 1000 52 / 53, 4000 111 / 212.  Four bytes at a time in
+    // the tile kernel: 4004 at 9990 114 / 106, 10004 at 3998 106 / 106, 5997 119 / 156.  Single bytes there: 785 at 10000
+    // 45 / 20, 9217 at 2000 83 / 64, 3000 84 / 91; where its workgroups come out even, one round: 2001 at 8000 39 / 46,
+    // 3001 at 3998 39 / 34.
+    const int64_t ballot_bytes = vectors ? (features <= 12288 ? 115000000 : 95000000)
+                                 : features % 4 == 0 && dl_aligned(x, 4) ? 40000000
+                                 : gx % 4 == 0 && gx * dl_ceil_div(features, 64) <= 256 ? 13500000 : 23000000;
+    if (out_row_bytes % 8 == 0 && cols <= 192 && batch * features <= ballot_bytes) {
         const dim3 grid((unsigned) dl_ceil_div(features, 64), (unsigned) cols);
         if (dl_ceil_div(features, 64) > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
         if (vectors) DL_LAUNCH(packbits_ballot_kernel<true>, grid, dim3(DL_BLOCK), 0, s, x, (uint64_t *) out, batch, features, cols);

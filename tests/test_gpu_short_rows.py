@@ -73,6 +73,20 @@ def test_pack_into_rows(ext, F, B):
     assert np.array_equal(bits[:, :B], (raw.numpy() != 0).T) and not bits[:, B:].any()
 
 
+# either side of the bytes up to which the kernel for few words takes the batch: 16-byte, 4-byte and single loads in the other
+@pytest.mark.parametrize("F,B", [(12288, 9358), (12288, 9359), (12304, 7721), (12304, 7722), (10004, 3998), (10004, 3999),
+                                 (2001, 6746), (2001, 7990), (9217, 2495), (9217, 2496)])
+def test_pack_many_features_into_rows(ext, F, B):
+    x = torch.rand(B, F, device="cuda", generator=torch.Generator(device="cuda").manual_seed(F + B)) < 0.3
+    words = -(-B // 64)
+    got = ext.tensor_packbits_batch_major_rows(x, 16 * -(-B // 128))
+    bit = torch.ones(64, dtype=torch.int64, device="cuda") << torch.arange(64, device="cuda")
+    for w in range(words):
+        piece = x[64 * w:64 * w + 64].long()
+        assert torch.equal(got[:, w], (piece * bit[:piece.shape[0], None]).sum(0)), w
+    assert not got[:, words:].any()
+
+
 @pytest.mark.parametrize("widths,B,bits", [
     ([1000, 1200, 2000], 1, 8), ([4096, 2100, 4096], 100, 16), ([6000, 6000], 6144, 32), ([6000, 6000], 6145, 64),
     ([10250, 11000], 12288, 64), ([10250, 11000], 12289, 64), ([10250, 10900], 40960, 32), ([10250, 10900], 40961, 64), ([1000, 999, 1900, 1000], 300, 64), ([2000, 4000], 1000, 64)])
