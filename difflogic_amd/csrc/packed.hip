@@ -1781,8 +1781,10 @@ void launch_groupbitsum(const void *bits, int32_t *out, int64_t row_bytes, int64
     const int64_t ncols = row_bytes / 16;
     // groupbitsum_kernel has one workgroup per class and kilobyte of the row: up to about 200 of them leave most of the
     // chip idle (64000 rows, 10 classes, 1264-byte rows: 201 us against 25; 16 KB rows = 160 workgroups: 213 against 200;
-    // 100 classes of 600 rows, 1600-byte rows = 200: 41 against 37; 4 KB rows = 400: 61 against 64).
-    if (vectors && k * dl_ceil_div(ncols, DL_WAVE) <= 200 && per_class <= 255 * 1024) {
+    // 100 classes of 600 rows, 1600-byte rows = 200: 41 against 37; 4 KB rows = 400: 61 against 64).  Classes of a few rows
+    // leave the 1024 threads idle instead: 100 classes of 100 rows, 2 KB rows = 200: 26 against 30; 40 classes of 100, 4 KB =
+    // 160: 22 against 24; 60 classes of 50, 2 KB = 120: 21 against 19.
+    if (vectors && k * dl_ceil_div(ncols, DL_WAVE) <= (per_class <= 200 ? 128 : 200) && per_class <= 255 * 1024) {
         const int nc = (int) ncols, pc = (int) per_class, kk = (int) k;
         // Columns per workgroup: wide enough for whole lines, narrow enough for about a hundred workgroups (64000 rows, 10
         // classes, with 1 / 2 / 4 / 8 columns: 7.4 / 7.4 / 8.9 / 12 us on 128-byte rows, 18 / 11 / 12 / 14 on 512,

@@ -46,7 +46,8 @@ def test_layer_from_its_weights(ext, vectors, out_dim, dtype):
 @pytest.mark.parametrize("per_class,k,words,pad", [
     (1, 1, 2, 0), (1023, 1, 2, 5), (8193, 1, 2, 63), (261120, 1, 2, 0), (261121, 1, 2, 1), (300, 7, 6, 3), (130560, 2, 102, 9),
     (130561, 2, 102, 0), (129, 10, 22, 0), (65280, 3, 234, 0), (65281, 3, 234, 63), (500, 9, 80, 1), (33, 16, 126, 0),
-    (1025, 17, 130, 7), (127, 20, 1152, 0), (40, 200, 18, 0), (40, 201, 18, 0), (5, 3, 1, 0), (77, 1, 2050, 64)])
+    (1025, 17, 130, 7), (127, 20, 1152, 0), (40, 200, 18, 0), (40, 201, 18, 0),
+    (200, 64, 130, 0), (200, 43, 300, 5), (200, 129, 16, 1), (201, 129, 16, 0), (5, 3, 1, 0), (77, 1, 2050, 64)])
 def test_bit_count_of_short_rows(ext, per_class, k, words, pad):
     g = torch.Generator(device="cuda").manual_seed(per_class + k)
     x = torch.randint(-2**62, 2**62, (per_class * k, words), device="cuda", generator=g)
