@@ -1224,6 +1224,11 @@ template <typename T> Rows rows_kind(int64_t batch, const void *p0, const void *
     return batch >= V ? Rows::ragged : Rows::single;
 }
 
+// Rows up to which both gradients share a launch.  On longer ones launches do not count and the two kernels get in each
+// other's way (fp32 1000 -> 1000, two launches / one: batch 4096 25.2 / 23.9 us, 8192 41.5 / 41.3, 16384 75.5 / 76.6, 65536
+// 303 / 349; 2000 -> 2000 at 16384 146 / 152, half at 65536 309 / 329).
+#define DL_BOTH_MAX_ROW_BYTES 32768
+
 #define DL_GRID_MAX (0xffffffffLL / DL_BLOCK)         // workgroups along x: HIP counts the threads in 32 bits
 
 unsigned col_tiles(int64_t ncols) {
@@ -1305,7 +1310,7 @@ int backward_both_t(const void *x, const int64_t *a, const int64_t *b, const voi
     const bool split = ncols >= 8 * DL_WAVE;                                         // as backward_w_t
     const int64_t row_blocks = dl_ceil_div(in_dim, 4), x_blocks = row_blocks * col_tiles(ncols);
     const int64_t blocks = x_blocks + (split ? dl_ceil_div(out_dim, NPW) : dl_ceil_div(out_dim, 4 * NPW));
-    if (blocks > DL_GRID_MAX) {
+    if (blocks > DL_GRID_MAX || batch * (int64_t) sizeof(T) > DL_BOTH_MAX_ROW_BYTES) {
         // a launch holds less than 2^32 threads along x, where this one has the column tiles too: one launch each
         const int st = backward_w_t<T>(x, a, b, gy, softmax_backward ? w : nullptr, gw, out_dim, batch, s, gdiv, w32);
         return st != DL_OK ? st : backward_x_t<T>(x, a, b, w, gy, start, idx, gx, in_dim, batch, scale, s, gdiv, w32);

@@ -134,8 +134,8 @@ int dl_logic_backward_x(const void *x, const int64_t *a, const int64_t *b, const
                         int64_t in_dim, int64_t out_dim, int64_t batch, double scale, int dtype,
                         void *stream);
 
-/* dl_logic_backward_w (softmax_backward: dl_logic_backward_logits with probs = w) and dl_logic_backward_x in one launch; the
- * same results.  k > 0: grad_y is the [k, batch] gradient of the class sums above the layer, as
+/* dl_logic_backward_w (softmax_backward: dl_logic_backward_logits with probs = w) and dl_logic_backward_x in one launch (two
+ * on rows above 32 KB, and where one does not hold their workgroups); the same results.  k > 0: grad_y is the [k, batch] gradient of the class sums above the layer, as
  * dl_logic_backward_x_grouped takes it; k = 0: grad_y is [out_dim, batch].  in_dim, out_dim, batch >= 1. */
 int dl_logic_backward_both(const void *x, const int64_t *a, const int64_t *b, const void *w, const void *grad_y,
                            int softmax_backward, const int64_t *start, const int64_t *idx, void *grad_w, void *grad_x,

@@ -109,7 +109,7 @@ def test_two_layers_at_once_on_rows_of_any_length(ext, monkeypatch, dtype, batch
 
 @pytest.mark.parametrize("dtype,wdtype", [(d, d) for d in DTYPES] + [(torch.float16, torch.float32), (torch.float64, torch.float32)])
 @pytest.mark.parametrize("in_dim,out_dim,batch", [(1, 1, 1), (30, 44, 3), (5, 9, 17), (33, 50, 128), (30, 44, 515), (64, 40, 2048),
-                                                  (20, 24, 4100)])
+                                                  (20, 24, 4100), (12, 16, 8196), (12, 16, 16392)])
 def test_both_gradients_in_one_launch(ext, dtype, wdtype, in_dim, out_dim, batch):
     """backward_both is backward_x and backward_w / backward_logits, bit for bit; rows of every kind, one and several
     column tiles, the batch split over the workgroup's waves, a layer under a GroupSum."""
