@@ -160,8 +160,8 @@ class LogicLayer(torch.nn.Module):
 
     def _train_schedule(self, x=None):
         """Evaluation schedule of this layer's wiring for the chained forward / backward kernels (cached per
-        wiring), or None where chaining does not pay on feature-major input like ``x`` (None: of any batch) or the schedule
-        would have to be built while a graph is being captured."""
+        wiring), or None where chaining does not pay on feature-major input like ``x`` (None: of any batch), or where the
+        schedule would have to be built while a graph is being captured or for the first evaluation of a narrower layer."""
         if self.in_dim < self._CHAIN_MIN_IN_DIM:
             return None
         if self.out_dim < self._CHAIN_MIN_OUT_DIM and (
