@@ -121,7 +121,8 @@ class LogicLayer(torch.nn.Module):
             return LogicLayerCudaFunction.apply(x, a, b, w, *tail, self._train_schedule(x)).transpose(0, 1)
         # eval mode: the discretised net on float inputs (no gradients)
         schedule = _forward_walk(self._train_schedule(x), self.out_dim, x)
-        self._evaluated = True
+        if not self._evaluated:
+            self._evaluated = True
         if (same or mixed) and self.weights.is_cuda and self.weights.is_contiguous():
             with torch.no_grad():
                 return difflogic_cuda.forward(x, a, b, self.weights.detach(), schedule, argmax=True).transpose(0, 1)
