@@ -68,17 +68,19 @@ class GraphedPackedInference:
     """
 
     def __init__(self, model, example_x, bit_count=64, warmup=2):
-        from .packbitstensor import PackBitsTensor
+        from .difflogic import LogicLayer
+        from .packbitstensor import PackBitsTensor, replayed_rows
         assert not model.training, "packed inference runs the discretised net: call model.eval() first"
         assert example_x.dtype == torch.bool and example_x.dim() == 2 and example_x.is_cuda, (
             example_x.dtype, tuple(example_x.shape), example_x.device)
         self.model, self.bit_count = model, bit_count
         self.x = example_x.detach().clone()
+        rows = replayed_rows([(m.in_dim, m.out_dim) for m in model.modules() if isinstance(m, LogicLayer)])
 
         def run():
             with torch.no_grad():
                 packed = PackBitsTensor(self.x, bit_count=bit_count)
-                packed._replayed = True
+                packed._replayed = rows
                 return model(packed)
 
         side = torch.cuda.Stream()

@@ -49,6 +49,11 @@ _DIRECT_ROW_BYTES = 1536         # ... and one row of them
 _DIRECT_ROW_BYTES_LDS = 768      # one row, for layers that the LDS kernel takes
 _REPLAYED_ROW_BYTES_LDS = 512    # ... in a replayed graph, where a layer's output has more than
 _REPLAYED_BYTES_LDS = 3_300_000  # ... this many
+# A net that narrows ends in the LDS kernel whatever comes before; with its first layers at once that kernel reads packed rows
+# instead of the bools.  Replayed, deferred as a whole / first layers at once, two-input gates: 8000-4000-2000-1000 at batch 64
+# 44 / 40 us, 1000 45 / 49, 4000 45 / 59; 2000-1000 at 1000 34 / 30, 4000 35 / 34; 3 x 8000-4000 at 1000 47 / 44, 4000 47 / 59.
+_NARROWING_ROW_BYTES = 32        # ... so one row of them in such a net, where less than half of the layers come before,
+_NARROWING_LATE_ROW_BYTES = 128  # ... or at least half
 _DIRECT_MIN_OUT = 1000           # smaller layers, and the tapering end of a net below 4096, stay with the LDS kernel
 
 
@@ -62,15 +67,30 @@ _STORED_BYTES = 160 << 20        # rows of the last layer
 _STORED_ROW_BYTES = 5120         # ... and one row of them
 
 
+def _narrows(in_dim, out_dim):
+    """Whether a layer is left to the LDS kernel for its width."""
+    return out_dim < min(max(in_dim, _DIRECT_MIN_OUT), 4096)
+
+
+def replayed_rows(dims):
+    """What `_direct` is told of a replayed net whose layers have ``dims`` = [(in_dim, out_dim), ...]: the longest row on which
+    those that fit in LDS are evaluated at once."""
+    first = next((i for i, d in enumerate(dims) if _narrows(*d)), None)
+    if first is None:
+        return _DIRECT_ROW_BYTES_LDS
+    return _NARROWING_LATE_ROW_BYTES if 2 * first >= len(dims) else _NARROWING_ROW_BYTES
+
+
 def _direct(in_dim, out_dim, row_bytes, lds_width, replayed):
-    """Whether a layer on rows of ``row_bytes`` is evaluated at once (above); ``replayed``: as part of a replayed graph."""
-    if out_dim < min(max(in_dim, _DIRECT_MIN_OUT), 4096) or not 0 < out_dim * row_bytes <= _DIRECT_BYTES:
+    """Whether a layer on rows of ``row_bytes`` is evaluated at once (above); ``replayed``: None, or as part of a replayed graph
+    what replayed_rows says of its net."""
+    if _narrows(in_dim, out_dim) or not 0 < out_dim * row_bytes <= _DIRECT_BYTES:
         return False
     if max(in_dim, out_dim) > lds_width:
         return row_bytes <= _DIRECT_ROW_BYTES
-    if replayed and out_dim * row_bytes > _REPLAYED_BYTES_LDS:
-        return row_bytes <= _REPLAYED_ROW_BYTES_LDS
-    return row_bytes <= _DIRECT_ROW_BYTES_LDS
+    if replayed is None:
+        return row_bytes <= _DIRECT_ROW_BYTES_LDS
+    return row_bytes <= (replayed if out_dim * row_bytes <= _REPLAYED_BYTES_LDS else min(replayed, _REPLAYED_ROW_BYTES_LDS))
 
 
 def _chained(depth):
@@ -213,7 +233,7 @@ class PackBitsTensor:
     width runs the same vector kernels.  ``.t`` is a view of those rows where their length allows
     it and a copy cut to ``ceil(B / bit_count)`` words otherwise."""
 
-    _replayed = False                 # set by GraphedPackedInference, on the inputs of its warm-up calls and of the captured one
+    _replayed = None                  # set by GraphedPackedInference, on the inputs of its warm-up calls and of the captured one
 
     def __init__(self, t: torch.BoolTensor, bit_count=32, device="cuda"):
         assert len(t.shape) == 2, t.shape

@@ -199,3 +199,21 @@ def test_counting_stored_rows(monkeypatch, widths):
             want = po.eval_layer(want, a, b, op)
         assert np.array_equal(p.t.cpu().numpy(), want)
         assert np.array_equal(p.group_sum(k).cpu().numpy(), po.groupbitsum(want, p.pad_len, k))
+
+
+@pytest.mark.parametrize("widths,B,at_once", [([4000, 2000, 1000], 256, 1), ([4000, 2000, 1000], 257, 0), ([2000, 1000], 1024, 1),
+                                              ([2000, 1000], 1025, 0), ([12000, 6000, 3000], 2000, 2)])
+def test_replayed_net_that_narrows(monkeypatch, widths, B, at_once):
+    """Layers before the narrow end are evaluated at once on short rows only, in the warm-up calls and the captured one."""
+    import difflogic_amd as dl
+    from difflogic_amd.graphs import GraphedPackedInference
+    rng = np.random.default_rng(B)
+    layers = random_layers(rng, 50, widths)
+    x = rng.random((B, 50)) < 0.4
+    model = build_model(50, layers, 10).eval()
+    calls, real = [], dl.PackBitsTensor.apply_weights
+    monkeypatch.setattr(dl.PackBitsTensor, "apply_weights", lambda self, *a: calls.append(1) or real(self, *a))
+    graph = GraphedPackedInference(model, torch.as_tensor(x).cuda())
+    assert len(calls) == 3 * at_once
+    for _ in range(3):
+        assert np.array_equal(graph(torch.as_tensor(x).cuda()).cpu().numpy(), interp.net_eval(x, layers, 10))

@@ -173,8 +173,8 @@ def test_wiring_cache_lives_and_dies_with_its_tensors():
 def test_layers_evaluated_at_once():
     """Sizes either side of the lines between layers evaluated when they are applied and deferred ones; in a replayed graph a
     net that fits in LDS is deferred where its gates may make that the faster way."""
-    from difflogic_amd.packbitstensor import _direct
-    eager, replayed = (lambda *a, c=c: _direct(*a, 10240, c) for c in (False, True))  # noqa: E731
+    from difflogic_amd.packbitstensor import _direct, replayed_rows
+    eager, replayed = (lambda *a, c=c: _direct(*a, 10240, c) for c in (None, replayed_rows([(784, 8000)])))  # noqa: E731
     for in_dim, out_dim, row, eagerly, in_graph in (
             (8000, 8000, 512, True, True), (8000, 8000, 528, True, False), (6000, 6000, 640, True, False),
             (8000, 8000, 768, True, False), (8000, 8000, 784, False, False), (4000, 4000, 768, True, True),
@@ -182,3 +182,9 @@ def test_layers_evaluated_at_once():
             (64000, 64000, 1056, False, False), (10250, 10250, 1536, True, True), (10250, 10250, 1552, False, False),
             (784, 999, 16, False, False), (784, 1000, 16, True, True), (8000, 4000, 16, False, False), (784, 8000, 0, False, False)):
         assert (eager(in_dim, out_dim, row), replayed(in_dim, out_dim, row)) == (eagerly, in_graph), (in_dim, out_dim, row)
+    # nets that narrow, replayed: the layers before the narrow end only on short rows, the shorter the less of them there are
+    early, late = ([(784, 8000), (8000, 4000), (4000, 2000)], [(784, 2000), (2000, 1000)])
+    assert replayed_rows(early) == 32 and replayed_rows(late) == 128 and replayed_rows([]) == 768
+    assert _direct(784, 8000, 32, 10240, 32) and not _direct(784, 8000, 48, 10240, 32) and _direct(784, 8000, 768, 10240, None)
+    assert _direct(784, 2000, 128, 10240, 128) and not _direct(784, 2000, 144, 10240, 128)
+    assert _direct(784, 64000, 1008, 10240, 32)                        # wider than the LDS kernel: as ever
