@@ -51,6 +51,40 @@ __device__ __forceinline__ P &row_vec(T *base, int64_t row, int64_t batch, int64
     return const_cast<P &>(row_vec<P, VEC, RAG>(const_cast<const T *>(base), row, batch, ncols, col));
 }
 
+// A vector read past the caches (NT: the row will not be read again soon, so it takes no place in the Infinity Cache).
+template <bool NT, typename P> __device__ __forceinline__ P load_vec(const P &at) {
+    if constexpr (!NT) {
+        return at;
+    } else {
+        constexpr size_t A = alignof(P) < 4 ? 2 : 4;
+        typedef std::conditional_t<A == 2, uint16_t, uint32_t> E;
+        typedef E V __attribute__((ext_vector_type(sizeof(P) / A), aligned(alignof(P))));
+        return __builtin_bit_cast(P, __builtin_nontemporal_load(reinterpret_cast<const V *>(&at)));
+    }
+}
+
+// Vector `col` of row `row` of a matrix of short rows, zeros where the row has no such vector, by every lane and without a
+// branch: behind one the compiler cannot count the loads in flight, and waits for all of them.  Whole rows are read through a
+// buffer resource that ends with the row: nothing is fetched, and zeros come back, where `valid` (wave-uniform) is false.
+// RAG: lanes past the row read its last vector; `row` must be there, and `valid` is the caller's to apply.
+template <typename P, int VEC, bool RAG, bool NT, typename T>
+__device__ __forceinline__ P row_part(const T *base, int64_t row, bool valid, int64_t batch, int64_t ncols, int64_t col) {
+    if constexpr (RAG) {
+        P v = load_vec<NT>(row_vec<P, VEC, RAG>(base, row, batch, ncols, col));
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v.v[e] = col < ncols ? v.v[e] : (T) 0;
+        return v;
+    } else {
+        static_assert(sizeof(P) == 16 || sizeof(P) == 8, "one buffer load per vector");
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T *>(base + row * batch), 0, valid ? (int) (batch * (int64_t) sizeof(T)) : 0, 0x00027000);
+        const int at = (int) col * (int) sizeof(P);
+        constexpr int policy = NT ? 2 : 0;
+        if constexpr (sizeof(P) == 16) return __builtin_bit_cast(P, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, policy));
+        else return __builtin_bit_cast(P, __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, policy));
+    }
+}
+
 template <typename T> __device__ __forceinline__ typename Acc<T>::type up(T v) { return (typename Acc<T>::type) v; }
 template <> __device__ __forceinline__ float up<__half>(__half v) { return __half2float(v); }
 template <typename T, typename C> __device__ __forceinline__ T down(C v) { return (T) v; }
@@ -88,11 +122,18 @@ template <typename T> __device__ __forceinline__ typename Acc<T>::type wload(con
     if constexpr (sizeof(T) == sizeof(float)) return w[at];
     else return w32 ? (C) reinterpret_cast<const float *>(w)[at] : up<T>(w[at]);
 }
-template <typename T> __device__ __forceinline__ void wstore(T *__restrict__ w, int64_t at, typename Acc<T>::type v, bool w32) {
+template <bool NT, typename E> __device__ __forceinline__ void store_elem(E *at, E v) {
+    typedef std::conditional_t<sizeof(E) == 2, uint16_t, std::conditional_t<sizeof(E) == 4, uint32_t, uint64_t>> U;
+    if constexpr (NT) __builtin_nontemporal_store(__builtin_bit_cast(U, v), reinterpret_cast<U *>(at));
+    else *at = v;
+}
+// (NT: past the Infinity Cache, as load_vec)
+template <typename T, bool NT = false>
+__device__ __forceinline__ void wstore(T *__restrict__ w, int64_t at, typename Acc<T>::type v, bool w32) {
     typedef typename Acc<T>::type C;
-    if constexpr (sizeof(T) == sizeof(float)) w[at] = v;
-    else if (w32) reinterpret_cast<float *>(w)[at] = (float) v;
-    else w[at] = down<T, C>(v);
+    if constexpr (sizeof(T) == sizeof(float)) store_elem<NT, T>(w + at, v);
+    else if (w32) store_elem<NT>(reinterpret_cast<float *>(w) + at, (float) v);
+    else store_elem<NT>(w + at, down<T, C>(v));
 }
 
 // y = lerp(lerp(P00, P01, b), lerp(P10, P11, b), a), three fused multiply-adds.
@@ -160,14 +201,19 @@ __device__ __forceinline__ float swap_add32(float v) {
     return __builtin_bit_cast(float, (unsigned) r[0]) + __builtin_bit_cast(float, (unsigned) r[1]);
 }
 
-__device__ __forceinline__ void wave_sum4(float &s0, float &s1, float &s2, float &s3, int lane) {
+// (in every lane the total of value lane & 3)
+__device__ __forceinline__ float wave_sum4_lane(float s0, float s1, float s2, float s3, int lane) {
     const bool odd = lane & 1, high = lane & 2;
     const float x = (odd ? s1 : s0) + dpp_f32<0xB1>(odd ? s0 : s1);          // quad_perm [1,0,3,2]: lane ^ 1
     const float y = (odd ? s3 : s2) + dpp_f32<0xB1>(odd ? s2 : s3);
     float z = (high ? y : x) + dpp_f32<0x4E>(high ? x : y);                  // quad_perm [2,3,0,1]: lane ^ 2
     z += dpp_f32<0x124>(z);                                                  // row_ror:4
     z += dpp_f32<0x128>(z);                                                  // row_ror:8
-    z = swap_add32(swap_add16(z));
+    return swap_add32(swap_add16(z));
+}
+
+__device__ __forceinline__ void wave_sum4(float &s0, float &s1, float &s2, float &s3, int lane) {
+    const float z = wave_sum4_lane(s0, s1, s2, s3, lane);
     s0 = lane_value(z, 0);
     s1 = lane_value(z, 1);
     s2 = lane_value(z, 2);
@@ -186,6 +232,15 @@ __device__ __forceinline__ void wave_sum4(double &s0, double &s1, double &s2, do
     s2 = wave_sum(s2);
     s3 = wave_sum(s3);
 }
+
+__device__ __forceinline__ double wave_sum4_lane(double s0, double s1, double s2, double s3, int lane) {
+    wave_sum4(s0, s1, s2, s3, lane);
+    return (lane & 2) ? ((lane & 1) ? s3 : s2) : ((lane & 1) ? s1 : s0);
+}
+
+// The value of lane I of the lane's 16-lane row (wave_sum4_lane: one of four sums; the quads of a row add in different orders).
+template <int I> __device__ __forceinline__ float row_value(float v) { return dpp_f32<0x150 + I>(v); }         // row_newbcast
+template <int I> __device__ __forceinline__ double row_value(double v) { return __shfl(v, (dl_lane() & ~15) | I, DL_WAVE); }
 
 // Sum over each aligned group of 16 lanes, result in every lane of the group.
 __device__ __forceinline__ float row16_sum(float v) {
@@ -237,7 +292,7 @@ constexpr int GATES_LOGITS = 1, GATES_ARGMAX = 2;
 // softmax (and stores it to `probs` if asked); otherwise `w` holds the probabilities.  The corner
 // sums are masked row sums whose association order is that of corners_of(), so the results are
 // bit-identical to it.  Returns, per neuron, the wave-uniform P00, P10, P01 - P00, P11 - P10.
-template <typename T, int GATES>
+template <typename T, int GATES, bool NT = false>
 __device__ __forceinline__ void corners4(const T *__restrict__ w, const int32_t (&n)[4], int lane, bool store_probs,
                                          T *__restrict__ probs, typename Acc<T>::type (&p00)[4],
                                          typename Acc<T>::type (&p10)[4], typename Acc<T>::type (&d0)[4],
@@ -251,7 +306,7 @@ __device__ __forceinline__ void corners4(const T *__restrict__ w, const int32_t 
     if (GATES == GATES_LOGITS) {
         const C e = dl_exp(p - row16_max(p));
         p = e / row16_sum(e);
-        if (store_probs && valid) wstore<T>(probs, at, p, w32);
+        if (store_probs && valid) wstore<T, NT>(probs, at, p, w32);
     } else if (GATES == GATES_ARGMAX) {
         // as argmax: the first of the largest, a NaN above every number (row16_max passes NaNs over)
         const uint32_t nans = (uint32_t) (__ballot(p != p) >> (16 * row)) & 0xffffu;
@@ -343,6 +398,25 @@ __device__ __forceinline__ void store_grad_w(int lane, bool neuron_valid, int64_
         r = p * (r - dot);
     }
     if (valid) wstore<T>(gw, n * 16 + lane, r, w32);
+}
+
+// The same for four neurons at once: the 16-lane row r of the wave holds neuron r's sums as wave_sum4_lane leaves them and, in
+// `p`, its probabilities (read only with `softmax`).  Same values, same order of additions.
+template <typename T, bool NT>
+__device__ __forceinline__ void store_grad_w4(int lane, bool valid, int64_t n, typename Acc<T>::type sums,
+                                              typename Acc<T>::type p, bool softmax, T *__restrict__ gw, bool w32) {
+    typedef typename Acc<T>::type C;
+    const C s00 = row_value<0>(sums), s01 = row_value<1>(sums), s10 = row_value<2>(sums), s11 = row_value<3>(sums);
+    C r = (C) 0;
+    if (lane & 8) r += s00;
+    if (lane & 4) r += s01;
+    if (lane & 2) r += s10;
+    if (lane & 1) r += s11;
+    if (softmax) {
+        const C dot = row16_sum(p * r);
+        r = p * (r - dot);
+    }
+    if (valid) wstore<T, NT>(gw, n * 16 + (lane & 15), r, w32);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -548,7 +622,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_both_kernel(
 // they can differ in the last bit, where the compiler folds the final conversion into a fused multiply-add in one
 // kernel and not in the other).
 // ------------------------------------------------------------------------------------------
-template <typename T, int VEC, int CHUNK, int GATES, bool RAG>
+template <typename T, int VEC, int CHUNK, int GATES, bool RAG, bool NT>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__restrict__ x,
                                                                  const int32_t *__restrict__ verts,
                                                                  const int32_t *__restrict__ neuron,
@@ -573,14 +647,15 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_kernel(const T *__rest
         // every row of the chunk is requested before the first one is used
         P rows[CHUNK + 1];
 #pragma unroll
-        for (int j = 0; j <= CHUNK; ++j) rows[j] = row_vec<P, VEC, RAG>(x, (int64_t) verts[s0 + j], batch, ncols, cl);
+        for (int j = 0; j <= CHUNK; ++j)
+            rows[j] = load_vec<NT>(row_vec<P, VEC, RAG>(x, (int64_t) verts[s0 + j], batch, ncols, cl));
 #pragma unroll
         for (int j0 = 0; j0 < CHUNK; j0 += 4) {
             int32_t n[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) n[i] = neuron[s0 + j0 + i];
             C p00[4], p10[4], d0[4], d1[4];
-            corners4<T, GATES>(w, n, lane, ct == 0, probs, p00, p10, d0, d1, w32);
+            corners4<T, GATES, NT>(w, n, lane, ct == 0, probs, p00, p10, d0, d1, w32);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int j = j0 + i;
@@ -691,7 +766,7 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_lower_kernel(
 // CPL * 64 consecutive vectors of the row (blockIdx.y picks the segment; lane l holds its vectors
 // l, l + 64, ...), so every gathered row is one contiguous request of up to 4 KB, and the next
 // step's row is requested before this step's arithmetic.
-template <typename T, int VEC, int CPL, int GATES, bool RAG>
+template <typename T, int VEC, int CPL, int GATES, bool RAG, bool NT>
 __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *__restrict__ x,
                                                                       const int32_t *__restrict__ verts,
                                                                       const int32_t *__restrict__ neuron,
@@ -708,55 +783,60 @@ __global__ __launch_bounds__(DL_BLOCK) void forward_chain_rows_kernel(const T *_
     if (s0 >= steps) return;
     const int64_t s1 = s0 + chunk < steps ? s0 + chunk : steps;
     const int64_t col0 = (int64_t) blockIdx.y * (CPL * DL_WAVE);
-    P zero;
+    auto load_row = [&](int64_t row, bool valid, P *out) {
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) zero.v[e] = down<T, C>((C) 0);
-    auto load_row = [&](int64_t row, P *out) {
-#pragma unroll
-        for (int q = 0; q < CPL; ++q) {
-            const int64_t col = col0 + lane + q * DL_WAVE;
-            out[q] = col < ncols ? row_vec<P, VEC, RAG>(x, row, batch, ncols, col) : zero;
-        }
+        for (int q = 0; q < CPL; ++q)
+            out[q] = row_part<P, VEC, RAG, NT>(x, row, valid, batch, ncols, col0 + lane + q * DL_WAVE);
     };
-    P prev[CPL], cur[CPL], next[CPL];
-    load_row(verts[s0], prev);
-    load_row(verts[s0 + 1], cur);
+    // the chunk's schedule entries, one per lane (chunk <= 64), handed out by readlane: no scalar loads in the step loop
+    const int cnt = (int) (s1 - s0);
+    const bool has = lane < cnt;
+    const int32_t sch_n = has ? neuron[s0 + lane] : -1;
+    const int32_t sch_v = has ? verts[s0 + 1 + lane] : 0;
+    const int32_t sch_f = has ? (int32_t) flip[s0 + lane] : 0;
+    constexpr int AHEAD = 3, SLOTS = AHEAD + 1;     // rows requested before their step; step i is in slot i % SLOTS
+    P prev[CPL], cur[SLOTS][CPL];
+    auto fetch = [&](int i, P *out) {
+        const bool there = i < cnt;
+        load_row(__builtin_amdgcn_readlane(sch_v, there ? i : cnt - 1), there, out);
+    };
+    load_row(verts[s0], true, prev);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) fetch(i, cur[i]);
 #pragma unroll 1
-    for (int64_t g = s0; g < s1; g += 4) {           // four steps per trip: their corners are computed together
+    for (int i0 = 0; i0 < cnt; i0 += 4) {            // four steps per trip: their corners are computed together
         int32_t n[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) n[i] = g + i < s1 ? neuron[g + i] : -1;
+        for (int j = 0; j < 4; ++j) n[j] = __builtin_amdgcn_readlane(sch_n, (i0 + j) & 63);
         C p00[4], p10[4], d0[4], d1[4];
-        corners4<T, GATES>(w, n, lane, col0 == 0, probs, p00, p10, d0, d1, w32);
+        corners4<T, GATES, NT>(w, n, lane, col0 == 0, probs, p00, p10, d0, d1, w32);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t s = g + i;
-            if (s < s1) {                            // wave-uniform
-                if (s + 1 < s1) load_row(verts[s + 2], next);
-                const bool f = flip[s] != 0;
+        for (int j = 0; j < 4; ++j) {
+            const int i = i0 + j;
+            if (i < cnt) {                           // wave-uniform
+                const int now = j % SLOTS;
+                fetch(i + AHEAD, cur[(j + AHEAD) % SLOTS]);
+                const bool f = __builtin_amdgcn_readlane(sch_f, i) != 0;
 #pragma unroll
                 for (int q = 0; q < CPL; ++q) {
                     const int64_t col = col0 + lane + q * DL_WAVE;
                     P r;
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) {
-                        const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]);
-                        r.v[e] = mix<T, RAG, C>(f ? u1 : u0, f ? u0 : u1, p00[i], p10[i], d0[i], d1[i]);
+                        const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[now][q].v[e]);
+                        r.v[e] = mix<T, RAG, C>(f ? u1 : u0, f ? u0 : u1, p00[j], p10[j], d0[j], d1[j]);
                     }
-                    if (n[i] >= 0 && col < ncols) row_vec<P, VEC, RAG>(y, (int64_t) n[i], batch, ncols, col) = r;
+                    if (n[j] >= 0 && col < ncols) row_vec<P, VEC, RAG>(y, (int64_t) n[j], batch, ncols, col) = r;
                 }
 #pragma unroll
-                for (int q = 0; q < CPL; ++q) {
-                    prev[q] = cur[q];
-                    cur[q] = next[q];
-                }
+                for (int q = 0; q < CPL; ++q) prev[q] = cur[now][q];
             }
         }
     }
 }
 
 // One wave owns CHUNK steps and the whole batch: lane l holds vectors l, l + 64, ... (CPL of them).
-template <typename T, int VEC, int CPL, int CHUNK, bool RAG>
+template <typename T, int VEC, int CPL, int CHUNK, bool RAG, bool NT>
 __global__ __launch_bounds__(DL_BLOCK) void backward_w_chain_kernel(const T *__restrict__ x,
                                                                     const int32_t *__restrict__ verts,
                                                                     const int32_t *__restrict__ neuron,
@@ -772,46 +852,53 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_w_chain_kernel(const T *__r
     const int64_t c = (int64_t) blockIdx.x * 4 + wave;
     if (c >= nchunks) return;
     const int64_t s0 = c * CHUNK;
-    P zero;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) zero.v[e] = down<T, C>((C) 0);
-
     auto load_row = [&](const T *base, int64_t row, P *dst) {
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
             const int64_t col = lane + q * DL_WAVE;
-            dst[q] = col < ncols ? row_vec<P, VEC, RAG>(base, row, batch, ncols, col) : zero;
+            dst[q] = row_part<P, VEC, RAG, NT>(base, row, true, batch, ncols, col);
         }
     };
+    static_assert(CHUNK % 4 == 0, "neurons are finished four at a time");
+    const int quarter = lane >> 4;                   // which of four neurons this lane finishes
     P prev[CPL];
     load_row(x, verts[s0], prev);
 #pragma unroll 1
-    for (int j = 0; j < CHUNK; ++j) {
-        const int32_t n = neuron[s0 + j];
-        const bool f = flip[s0 + j] != 0;
-        P cur[CPL], g[CPL];
-        load_row(x, verts[s0 + j + 1], cur);
-        load_row(gy, grad_row(n >= 0 ? n : 0, gdiv), g);
-        C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
+    for (int j0 = 0; j0 < CHUNK; j0 += 4) {
+        int32_t n[4];
 #pragma unroll
-        for (int q = 0; q < CPL; ++q) {
-            const int dup = vec_dup<VEC, RAG>(lane + q * DL_WAVE, batch);
+        for (int i = 0; i < 4; ++i) n[i] = neuron[s0 + j0 + i];
+        const int32_t mine = quarter == 0 ? n[0] : quarter == 1 ? n[1] : quarter == 2 ? n[2] : n[3];
+        const C p = probs != nullptr && mine >= 0 ? wload<T>(probs, (int64_t) mine * 16 + (lane & 15), w32) : (C) 0;
+        C sums = (C) 0;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]), gg = own_part<RAG>(up<T>(g[q].v[e]), e, dup);
-                const C av = f ? u1 : u0, bv = f ? u0 : u1;
-                const C ga = gg * av, gna = gg - ga;
-                const C t11 = ga * bv, t01 = gna * bv;
-                s11 += t11;
-                s10 += ga - t11;
-                s01 += t01;
-                s00 += gna - t01;
+        for (int i = 0; i < 4; ++i) {
+            const bool f = flip[s0 + j0 + i] != 0;
+            P cur[CPL], g[CPL];
+            load_row(x, verts[s0 + j0 + i + 1], cur);
+            load_row(gy, grad_row(n[i] >= 0 ? n[i] : 0, gdiv), g);
+            C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
+#pragma unroll
+            for (int q = 0; q < CPL; ++q) {
+                const int dup = vec_dup<VEC, RAG>(lane + q * DL_WAVE, batch);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]), gg = own_part<RAG>(up<T>(g[q].v[e]), e, dup);
+                    const C av = f ? u1 : u0, bv = f ? u0 : u1;
+                    const C ga = gg * av, gna = gg - ga;
+                    const C t11 = ga * bv, t01 = gna * bv;
+                    s11 += t11;
+                    s10 += ga - t11;
+                    s01 += t01;
+                    s00 += gna - t01;
+                }
             }
-        }
-        wave_sum4(s00, s01, s10, s11, lane);
-        store_grad_w<T>(lane, n >= 0, n >= 0 ? n : 0, s00, s01, s10, s11, probs, gw, w32);
+            const C z = wave_sum4_lane(s00, s01, s10, s11, lane);
+            sums = quarter == i ? z : sums;
 #pragma unroll
-        for (int q = 0; q < CPL; ++q) prev[q] = cur[q];
+            for (int q = 0; q < CPL; ++q) prev[q] = cur[q];
+        }
+        store_grad_w4<T, NT>(lane, mine >= 0, mine, sums, p, probs != nullptr, gw, w32);
     }
 }
 
@@ -857,7 +944,7 @@ template <bool SPLIT, typename C> __device__ __forceinline__ C slope(C u, C dd, 
     else return dl_fma(u, dd, k);
 }
 
-template <typename T, int VEC, int CPL, int LOWER, bool RAG>
+template <typename T, int VEC, int CPL, int LOWER, bool RAG, bool NT>
 __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const T *__restrict__ x, const int32_t *__restrict__ verts, const int32_t *__restrict__ neuron,
     const uint8_t *__restrict__ flip, const int32_t *__restrict__ dst, const T *__restrict__ w,
@@ -873,6 +960,9 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     // bits of backward_x_kernel whether or not their layer is walked along its schedule
     constexpr bool SPLIT = RAG && sizeof(T) == 2;
     constexpr int LCPL = LOWER ? CPL : 1;                       // registers for lower rows only where they are used
+    // steps whose rows are requested before they are walked: three on short fp32 rows (64000 -> 64000, one / three: batch 100
+    // 27.6 / 25.8 us, 128 28.6 / 26.2); half rows, whose steps hold more registers, lose by it (500: 45.8 / 47.4)
+    constexpr int AHEAD = CPL == 1 && LOWER == 0 && sizeof(T) == 4 ? 3 : 1, SLOTS = AHEAD + 1;
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
     const int64_t s0 = ((int64_t) blockIdx.x * 4 + wave) * chunk;
@@ -880,64 +970,73 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const int64_t s1 = s0 + chunk < steps ? s0 + chunk : steps;
     const int64_t col0 = (int64_t) blockIdx.y * (CPL * DL_WAVE);   // this wave's segment of the rows
     const int gate = lane & 15;
-    P zero;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) zero.v[e] = down<T, C>((C) 0);
-
-    auto load_row = [&](const T *base, int64_t row, bool valid, P *out) {
+    auto load_row_as = [&](auto once, const T *base, int64_t row, bool valid, P *out) {
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
             const int64_t col = col0 + lane + q * DL_WAVE;
-            out[q] = (valid && col < ncols) ? row_vec<P, VEC, RAG>(base, row, batch, ncols, col) : zero;
+            out[q] = row_part<P, VEC, RAG, decltype(once)::value>(base, row, valid, batch, ncols, col);
         }
+    };
+    auto load_row = [&](const T *base, int64_t row, bool valid, P *out) {          // of x or grad_y
+        load_row_as(std::bool_constant<NT>(), base, row, valid, out);
     };
     // the two input rows of neuron v of the layer below (v wave-uniform)
     auto lower_rows = [&](int64_t v, bool valid, P *la, P *lb) {
         if constexpr (LOWER != 0) {
             const int64_t r = valid ? v : 0;
-            load_row(low.x, low.a[r], valid, la);
-            load_row(low.x, low.b[r], valid, lb);
+            load_row_as(std::false_type(), low.x, low.a[r], valid, la);
+            load_row_as(std::false_type(), low.x, low.b[r], valid, lb);
         }
     };
-    // row v of x as the lower layer's forward kernel stored it: lane `gate` of every 16-lane row holds the
-    // neuron's probability of that gate; corner sums and their order as corners4()
-    auto lower_forward = [&](const P *la, const P *lb, C lp, P *out) {
-        const C zc = (C) 0;
-        const C q00 = row16_sum((gate & 8) ? lp : zc), q01 = row16_sum((gate & 4) ? lp : zc);
-        const C q10 = row16_sum((gate & 2) ? lp : zc), q11 = row16_sum((gate & 1) ? lp : zc);
-        const C p00 = lane_value(q00, 0), p10 = lane_value(q10, 0);
-        const C d0 = lane_value(q01 - q00, 0), d1 = lane_value(q11 - q10, 0);
+    // Corner sums of the probabilities in the lanes' 16-lane rows, in the association order of corners_of().
+    const C zc = (C) 0;
+    const int quarter = lane >> 4;                   // which of four steps this lane's row serves
+    auto corner_rows = [&](C p, C &q00, C &q10, C &d0, C &d1) {
+        q00 = row16_sum((gate & 8) ? p : zc);
+        q10 = row16_sum((gate & 2) ? p : zc);
+        d0 = row16_sum((gate & 4) ? p : zc) - q00;
+        d1 = row16_sum((gate & 1) ? p : zc) - q10;
+    };
+    auto pick = [&](const int32_t (&v)[4]) { return quarter == 0 ? v[0] : quarter == 1 ? v[1] : quarter == 2 ? v[2] : v[3]; };
+    // row v of x as the lower layer's forward kernel stored it, from its two input rows and corner coefficients
+    auto lower_forward = [&](const P *la, const P *lb, C p00, C p10, C d0, C d1, P *out) {
 #pragma unroll
         for (int q = 0; q < CPL; ++q)
 #pragma unroll
             for (int e = 0; e < VEC; ++e)
                 out[q].v[e] = mix<T, RAG, C>(up<T>(la[q].v[e]), up<T>(lb[q].v[e]), p00, p10, d0, d1);
     };
-    // la, lb: with LOWER, the two input rows of neuron `row` of the layer below
-    auto store_row = [&](int32_t row, const C (&val)[CPL][VEC], const P *la, const P *lb) {
-        if (row < 0) return;
-        if (LOWER != 0 && row < in_dim) {
-            // as backward_w_kernel on the row this would have stored: same values, same order of additions
-            C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
+    // ... of a single vertex
+    auto lower_row = [&](int64_t v, P *la, P *lb, P *out) {
+        lower_rows(v, true, la, lb);
+        C q00, q10, d0, d1;
+        corner_rows(up<T>(low.w[v * 16 + gate]), q00, q10, d0, d1);
+        lower_forward(la, lb, lane_value(q00, 0), lane_value(q10, 0), lane_value(d0, 0), lane_value(d1, 0), out);
+    };
+    // (LOWER) corner sums of the layer below for a finished vertex, whose lower rows are la, lb: as backward_w_kernel on the
+    // row that would have been stored, same values, same order of additions
+    auto lower_sums = [&](const C (&val)[CPL][VEC], const P *la, const P *lb) {
+        C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
 #pragma unroll
-            for (int q = 0; q < CPL; ++q) {
-                const int dup = vec_dup<VEC, RAG>(col0 + lane + q * DL_WAVE, batch);
+        for (int q = 0; q < CPL; ++q) {
+            const int dup = vec_dup<VEC, RAG>(col0 + lane + q * DL_WAVE, batch);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    const C g = own_part<RAG>(up<T>(round_scaled<T, RAG, C>(val[q][e], scale)), e, dup);
-                    const C av = up<T>(la[q].v[e]), bv = up<T>(lb[q].v[e]);
-                    const C ga = g * av, gna = g - ga;
-                    const C t11 = ga * bv, t01 = gna * bv;
-                    s11 += t11;
-                    s10 += ga - t11;
-                    s01 += t01;
-                    s00 += gna - t01;
-                }
+            for (int e = 0; e < VEC; ++e) {
+                const C g = own_part<RAG>(up<T>(round_scaled<T, RAG, C>(val[q][e], scale)), e, dup);
+                const C av = up<T>(la[q].v[e]), bv = up<T>(lb[q].v[e]);
+                const C ga = g * av, gna = g - ga;
+                const C t11 = ga * bv, t01 = gna * bv;
+                s11 += t11;
+                s10 += ga - t11;
+                s01 += t01;
+                s00 += gna - t01;
             }
-            wave_sum4(s00, s01, s10, s11, lane);
-            store_grad_w<T>(lane, true, row, s00, s01, s10, s11, low.probs, low.gw);
-            return;
         }
+        return wave_sum4_lane(s00, s01, s10, s11, lane);
+    };
+    // a finished position's row to where dst says; with LOWER only parts of sums are stored
+    auto store_row = [&](int32_t row, const C (&val)[CPL][VEC]) {
+        if (row < 0 || (LOWER != 0 && row < in_dim)) return;
         if (row >= in_dim) {                                     // a part of a sum: in C, scaled here only if that is T
             typedef OverflowPack<T, VEC, RAG> O;
 #pragma unroll
@@ -964,13 +1063,8 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     // which also serve that vertex's backward_w at step 0
     P prev[CPL], pla[LCPL], plb[LCPL];
     C carry[CPL][VEC];
-    if constexpr (RECOMPUTE) {
-        const int64_t v0 = verts[s0];
-        lower_rows(v0, true, pla, plb);
-        lower_forward(pla, plb, up<T>(low.w[v0 * 16 + gate]), prev);
-    } else {
-        load_row(x, verts[s0], true, prev);
-    }
+    if constexpr (RECOMPUTE) lower_row(verts[s0], pla, plb, prev);
+    else load_row(x, verts[s0], true, prev);
 #pragma unroll
     for (int q = 0; q < CPL; ++q)
 #pragma unroll
@@ -980,10 +1074,8 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
         const bool f = flip[s0 - 1] != 0;
         P before[CPL], g[CPL];
         if constexpr (RECOMPUTE) {
-            const int64_t vb = verts[s0 - 1];
             P ba[LCPL], bb[LCPL];
-            lower_rows(vb, true, ba, bb);
-            lower_forward(ba, bb, up<T>(low.w[vb * 16 + gate]), before);
+            lower_row(verts[s0 - 1], ba, bb, before);
         } else {
             load_row(x, verts[s0 - 1], true, before);
         }
@@ -1005,107 +1097,144 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const int32_t sch_v = has ? verts[s0 + 1 + lane] : 0;
     const int32_t sch_d = has ? dst[s0 + lane] : -1;
     const int32_t sch_f = has ? (int32_t) flip[s0 + lane] : 0;
-    // Rows of step i: the new input row (RECOMPUTE: the two lower rows and the lower probabilities it is
-    // recomputed from), the neuron's grad_y row (zero for a step without a neuron) and, in every 16-lane
-    // row, the neuron's 16 gate probabilities.  LOWER == 1: la, lb are the lower rows of the vertex that
-    // step i finishes (dst[i]); RECOMPUTE: of the vertex that step i brings in.
-    auto fetch = [&](int i, P *row, P *grad, C &prob, P *la, P *lb, C &lprob) {
+    // Rows of step i: the new input row (RECOMPUTE: the two lower rows it is recomputed from) and the neuron's grad_y
+    // row (zero for a step without a neuron).  LOWER == 1: la, lb are the lower rows of the vertex that step i
+    // finishes (dst[i]); RECOMPUTE: of the vertex that step i brings in.
+    auto fetch = [&](int i, P *row, P *grad, P *la, P *lb) {
+        const bool there = i < cnt;
+        if (!there) i = cnt - 1;
         const int32_t n = __builtin_amdgcn_readlane(sch_n, i);
-        const bool valid = n >= 0;
-        const int64_t nn = valid ? n : 0;
         const int32_t v = __builtin_amdgcn_readlane(sch_v, i);
         if constexpr (RECOMPUTE) {
-            lower_rows(v, true, la, lb);
-            lprob = up<T>(low.w[(int64_t) v * 16 + gate]);
+            lower_rows(v, there, la, lb);
         } else {
-            load_row(x, v, true, row);
+            load_row(x, v, there, row);
             if constexpr (LOWER == 1) {
                 const int32_t d = __builtin_amdgcn_readlane(sch_d, i);
-                lower_rows(d, d >= 0 && d < in_dim, la, lb);
+                lower_rows(d, there && d >= 0 && d < in_dim, la, lb);
             }
         }
-        load_row(gy, grad_row(nn, gdiv), valid, grad);
-        prob = wload<T>(w, nn * 16 + gate, w32);
+        load_row(gy, grad_row(n >= 0 ? n : 0, gdiv), there && n >= 0, grad);
     };
-    P cur[CPL], g[CPL], la[LCPL], lb[LCPL];
-    C pw, lpw = (C) 0;
-    fetch(0, cur, g, pw, la, lb, lpw);
-#pragma unroll 1
-    for (int i = 0; i < cnt; ++i) {
-        P ncur[CPL], ng[CPL], nla[LCPL], nlb[LCPL];
-        C npw = (C) 0, nlpw = (C) 0;
-        if (i + 1 < cnt) fetch(i + 1, ncur, ng, npw, nla, nlb, nlpw);
-        if constexpr (RECOMPUTE) lower_forward(la, lb, lpw, cur);
-        const int32_t n = __builtin_amdgcn_readlane(sch_n, i);
-        const bool valid = n >= 0;
-        const int64_t nn = valid ? n : 0;
-        const bool f = __builtin_amdgcn_readlane(sch_f, i) != 0;
-        // corner sums of the probabilities, in the association order of corners_of()
-        const C zc = (C) 0;
-        const C p00 = lane_value(row16_sum((gate & 8) ? pw : zc), 0), p01 = lane_value(row16_sum((gate & 4) ? pw : zc), 0);
-        const C p10 = lane_value(row16_sum((gate & 2) ? pw : zc), 0), p11 = lane_value(row16_sum((gate & 1) ? pw : zc), 0);
-        const C d0 = p01 - p00, dd = (p11 - p10) - d0, da = p10 - p00;
-        const C ku = f ? d0 : da, kv = f ? da : d0;
-        C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
-        C out[CPL][VEC];
+    // What is needed once per neuron is done for four steps at a time, a 16-lane row each: of the group that starts at
+    // step i the neurons' probabilities, (RECOMPUTE) those of the vertices the steps bring in, and (LOWER) those of the
+    // vertices they finish.
+    auto entries = [&](int32_t sch, int i, int32_t (&v)[4]) {
 #pragma unroll
-        for (int q = 0; q < CPL; ++q) {
-            const int dup = vec_dup<VEC, RAG>(col0 + lane + q * DL_WAVE, batch);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[q].v[e]), gg = up<T>(g[q].v[e]);
-                const C av = f ? u1 : u0, bv = f ? u0 : u1;
-                const C gs = own_part<RAG>(gg, e, dup);
-                const C ga = gs * av, gna = gs - ga;
-                const C t11 = ga * bv, t01 = gna * bv;
-                s11 += t11;
-                s10 += ga - t11;
-                s01 += t01;
-                s00 += gna - t01;
-                out[q][e] = carry[q][e] + gg * slope<SPLIT, C>(u1, dd, ku);
-                carry[q][e] = gg * slope<SPLIT, C>(u0, dd, kv);
-            }
-        }
-        wave_sum4(s00, s01, s10, s11, lane);
-        if (partial == nullptr) {
-            // as store_grad_w, with the probabilities already at hand
-            C r = (C) 0;
-            if (lane & 8) r += s00;
-            if (lane & 4) r += s01;
-            if (lane & 2) r += s10;
-            if (lane & 1) r += s11;
-            if (probs != nullptr) {
-                const C pr = (valid && lane < 16) ? pw : zc;
-                const C dot = row16_sum(pr * r);
-                r = pr * (r - dot);
-            }
-            if (valid && lane < 16) wstore<T>(gw, nn * 16 + lane, r, w32);
-        } else if (valid && lane < 4) {              // several segments: backward_w_finish_kernel adds them
-            const C mine = lane == 0 ? s00 : lane == 1 ? s01 : lane == 2 ? s10 : s11;
-            partial[((int64_t) blockIdx.y * out_dim + nn) * 4 + lane] = mine;
-        }
-        // the vertex at position s0 + i is finished: RECOMPUTE keeps its lower rows from the step that brought it in
-        store_row(__builtin_amdgcn_readlane(sch_d, i), out, RECOMPUTE ? pla : la, RECOMPUTE ? plb : lb);
-#pragma unroll
-        for (int q = 0; q < CPL; ++q) {
-            prev[q] = cur[q];
-            cur[q] = ncur[q];
-            g[q] = ng[q];
+        for (int j = 0; j < 4; ++j) v[j] = __builtin_amdgcn_readlane(sch, (i + j) & 63);
+    };
+    auto fetch_probs = [&](int i, C &p, C &lp, C &dp) {
+        int32_t v[4];
+        entries(sch_n, i, v);
+        const int32_t n = pick(v);
+        p = wload<T>(w, (int64_t) (n >= 0 ? n : 0) * 16 + gate, w32);
+        if constexpr (RECOMPUTE) {
+            entries(sch_v, i, v);
+            lp = up<T>(low.w[(int64_t) pick(v) * 16 + gate]);
         }
         if constexpr (LOWER != 0) {
+            entries(sch_d, i, v);
+            const int32_t d = pick(v);
+            if (low.probs != nullptr) dp = up<T>(low.probs[(int64_t) (d >= 0 && d < in_dim ? d : 0) * 16 + gate]);
+        }
+    };
+    P cur[SLOTS][CPL], g[SLOTS][CPL], la[SLOTS][LCPL], lb[SLOTS][LCPL];       // step i is in slot i % SLOTS
+    C pw, lpw = zc, dpw = zc;
 #pragma unroll
-            for (int q = 0; q < LCPL; ++q) {
-                if constexpr (RECOMPUTE) pla[q] = la[q], plb[q] = lb[q];
-                la[q] = nla[q], lb[q] = nlb[q];
+    for (int i = 0; i < AHEAD; ++i) fetch(i, cur[i], g[i], la[i], lb[i]);
+    fetch_probs(0, pw, lpw, dpw);
+#pragma unroll 1
+    for (int i0 = 0; i0 < cnt; i0 += 4) {
+        int32_t n[4], d[4], fl[4];
+        entries(sch_n, i0, n);
+        entries(sch_d, i0, d);
+        entries(sch_f, i0, fl);
+        C npw = zc, nlpw = zc, ndpw = zc;
+        if (i0 + 4 < cnt) fetch_probs(i0 + 4, npw, nlpw, ndpw);
+        C c00, c10, cd0, cd1, l00 = zc, l10 = zc, ld0 = zc, ld1 = zc;
+        corner_rows(pw, c00, c10, cd0, cd1);
+        const C cdd = cd1 - cd0, cda = c10 - c00;
+        const bool frow = pick(fl) != 0;
+        const C cku = frow ? cd0 : cda, ckv = frow ? cda : cd0;
+        if constexpr (RECOMPUTE) corner_rows(lpw, l00, l10, ld0, ld1);
+        C sums = zc, lsums = zc;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = i0 + j;
+            if (i < cnt) {                               // (wave-uniform)
+                const int now = j % SLOTS, ahead = (j + AHEAD) % SLOTS;
+                fetch(i + AHEAD, cur[ahead], g[ahead], la[ahead], lb[ahead]);
+                if constexpr (RECOMPUTE)
+                    lower_forward(la[now], lb[now], lane_value(l00, 16 * j), lane_value(l10, 16 * j), lane_value(ld0, 16 * j),
+                                  lane_value(ld1, 16 * j), cur[now]);
+                if (RAG && n[j] < 0)
+#pragma unroll
+                    for (int q = 0; q < CPL; ++q) g[now][q] = P{};
+                const bool f = fl[j] != 0;
+                const C dd = lane_value(cdd, 16 * j), ku = lane_value(cku, 16 * j), kv = lane_value(ckv, 16 * j);
+                C s00 = zc, s01 = zc, s10 = zc, s11 = zc;
+                C out[CPL][VEC];
+#pragma unroll
+                for (int q = 0; q < CPL; ++q) {
+                    const int dup = vec_dup<VEC, RAG>(col0 + lane + q * DL_WAVE, batch);
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        const C u0 = up<T>(prev[q].v[e]), u1 = up<T>(cur[now][q].v[e]), gg = up<T>(g[now][q].v[e]);
+                        const C av = f ? u1 : u0, bv = f ? u0 : u1;
+                        const C gs = own_part<RAG>(gg, e, dup);
+                        const C ga = gs * av, gna = gs - ga;
+                        const C t11 = ga * bv, t01 = gna * bv;
+                        s11 += t11;
+                        s10 += ga - t11;
+                        s01 += t01;
+                        s00 += gna - t01;
+                        out[q][e] = carry[q][e] + gg * slope<SPLIT, C>(u1, dd, ku);
+                        carry[q][e] = gg * slope<SPLIT, C>(u0, dd, kv);
+                    }
+                }
+                const C z = wave_sum4_lane(s00, s01, s10, s11, lane);
+                sums = quarter == j ? z : sums;
+                // the vertex at position s0 + i is finished: RECOMPUTE keeps its lower rows from the step that brought it in
+                if constexpr (LOWER != 0) {
+                    if (d[j] >= 0 && d[j] < in_dim) {
+                        const C lz = lower_sums(out, RECOMPUTE ? pla : la[now], RECOMPUTE ? plb : lb[now]);
+                        lsums = quarter == j ? lz : lsums;
+                    }
+                }
+                store_row(d[j], out);
+#pragma unroll
+                for (int q = 0; q < CPL; ++q) prev[q] = cur[now][q];
+                if constexpr (RECOMPUTE) {
+#pragma unroll
+                    for (int q = 0; q < LCPL; ++q) pla[q] = la[now][q], plb[q] = lb[now][q];
+                }
             }
+        }
+        const int32_t mine = pick(n);                    // (-1 past the end: the lanes beyond hold no entry)
+        if (partial == nullptr) {
+            store_grad_w4<T, NT>(lane, mine >= 0, mine, sums, pw, probs != nullptr, gw, w32);
+        } else if (mine >= 0 && gate < 4) {              // several segments: backward_w_finish_kernel adds them
+            store_elem<NT>(partial + ((int64_t) blockIdx.y * out_dim + mine) * 4 + gate, sums);
+        }
+        if constexpr (LOWER != 0) {
+            const int32_t done = pick(d);
+            store_grad_w4<T, NT>(lane, done >= 0 && done < in_dim, done, lsums, dpw, low.probs != nullptr, low.gw, false);
         }
         pw = npw;
         lpw = nlpw;
+        dpw = ndpw;
     }
-    if (s1 == steps) {                                // the schedule's last position
+    if (s1 == steps) {                                   // the schedule's last position
         const int32_t last = dst[steps];
-        if constexpr (LOWER == 1) lower_rows(last, last >= 0 && last < in_dim, la, lb);
-        store_row(last, carry, RECOMPUTE ? pla : la, RECOMPUTE ? plb : lb);
+        if constexpr (LOWER != 0) {
+            if (last >= 0 && last < in_dim) {
+                if constexpr (LOWER == 1) lower_rows(last, true, pla, plb);
+                const C lz = lower_sums(carry, pla, plb);
+                const C p = low.probs != nullptr ? up<T>(low.probs[(int64_t) last * 16 + gate]) : zc;
+                store_grad_w4<T, NT>(lane, quarter == 0, last, lz, p, low.probs != nullptr, low.gw, false);
+            }
+        }
+        store_row(last, carry);
     }
 }
 
@@ -1619,23 +1748,48 @@ int group_sum_splits(int64_t out_dim, int64_t batch, int64_t k) {
 // Longest row (in 16-byte vectors) the whole-row kernels take: 16 segments of 256.
 #define DL_ROWS_MAX_VECTORS (16 * 4 * DL_WAVE)
 
+// Rows past the Infinity Cache (NT).  A walk reads every row of x (and of grad_y) once, and what it writes is what the next
+// kernel reads.  Read the ordinary way, rows that nobody wants again push the new ones out of the 256 MB; written the ordinary
+// way, 64 bytes of probabilities or weight gradients a neuron cost as much as half a kilobyte of rows (half a cache line each).
+// Six square fp32 layers in a row, us a layer, ordinary / past the cache, by the bytes of x:
+//   forward of training    31 MB 15.1 / 18.0, 51 MB 26.1 / 25.4, 66 MB 30.9 / 28.4, 131 MB 57 / 51, 262 MB 112 / 95, 524 MB 231 / 206,
+//                          1 GB 452 / 452
+//   discretised forward    66 MB 22.5 / 25.4, 131 MB 49.2 / 49.7, 179 MB 75 / 72, 262 MB 105 / 94, 524 MB 219 / 203, 1 GB 441 / 445
+//   one-pass backward      66 MB 41.8 / 41.6, 98 MB 64 / 58, 131 MB 90 / 73, 262 MB 173 / 137, 524 MB 347 / 330, 1 GB 685 / 696
+//   backward_w alone       131 MB 44 / 50, 179 MB 66 / 70, 262 MB 98 / 95, 524 MB 203 / 190, 1 GB 502 / 503
+// Smaller matrices stay in the caches from one kernel to the next; rows that are read several times (a layer much wider
+// than its input, the classes' gradient rows) are read the ordinary way.
+struct PastCache { int64_t from, to; };
+constexpr PastCache DL_PAST_FORWARD = {50000000, INT64_MAX}, DL_PAST_ARGMAX = {140000000, 700000000},
+                    DL_PAST_BACKWARD = {80000000, 700000000}, DL_PAST_WEIGHTS = {240000000, INT64_MAX};
+
+bool past_cache(PastCache limits, int64_t steps, int64_t in_dim, int64_t row_bytes) {
+    const int64_t bytes = in_dim * row_bytes;
+    return 4 * steps <= 5 * in_dim && bytes >= limits.from && bytes <= limits.to;
+}
+
 int row_segments(int64_t ncols) { return (int) dl_ceil_div(ncols, 4 * DL_WAVE); }
 
 // Steps per wave of the kernels in which a wave owns whole rows: long chunks re-read fewer rows at
-// their seams, short ones give more waves to hide latency with; keep about three waves per SIMD.
-int chain_chunk(int64_t steps) {
+// their seams, short ones give more waves to hide latency with; keep about three waves per SIMD (`waves`).
+constexpr int64_t DL_CHAIN_WAVES = 3000;
+// ... and two in the one-pass backward of rows longer than 2 KB (64000 -> 64000, 32 / 16 steps: batch 1024 137 / 142 us, 512 80 / 74)
+constexpr int64_t DL_CHAIN_WAVES_LONG = 2000;
+int chain_chunk(int64_t steps, int64_t waves = DL_CHAIN_WAVES) {
     for (int chunk = 32; chunk > 8; chunk /= 2)
-        if (steps / chunk >= 3000) return chunk;
+        if (steps / chunk >= waves) return chunk;
     return 8;
 }
 
 template <typename T, int GATES>
 int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps,
-                    const void *w, void *y, void *probs, int64_t batch, bool any_rows, hipStream_t s, bool w32 = false) {
+                    const void *w, void *y, void *probs, int64_t in_dim, int64_t batch, bool any_rows, hipStream_t s,
+                    bool w32 = false) {
     constexpr int V = Vec16<T>::n;
     const Rows kind = rows_kind<T>(batch, x, y);
     if (kind != Rows::whole && !(any_rows && kind == Rows::ragged)) return DL_ERR_TOO_LARGE;
     const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
+    const bool past = past_cache(probs ? DL_PAST_FORWARD : DL_PAST_ARGMAX, steps, in_dim, batch * (int64_t) sizeof(T));
     const T *xp = (const T *) x, *wp = (const T *) w;
     const dim3 block(DL_BLOCK);
     if (ncols > DL_FWD_ROWS_MIN && ncols <= DL_ROWS_MAX_VECTORS) {
@@ -1645,9 +1799,14 @@ int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, 
         const int64_t blocks = dl_ceil_div(dl_ceil_div(steps, chunk), 4);
         if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
         const dim3 grid((unsigned) blocks, (unsigned) segments);
+#define DL_LAUNCH_ROWS_AS(CPL, RAG, NT)                                                                                 \
+    DL_LAUNCH((forward_chain_rows_kernel<T, V, CPL, GATES, RAG, NT>), grid, block, 0, s, xp, verts, neuron, flip, wp,   \
+              (T *) y, (T *) probs, steps, chunk, batch, w32)
 #define DL_LAUNCH_ROWS(CPL, RAG)                                                                                        \
-    DL_LAUNCH((forward_chain_rows_kernel<T, V, CPL, GATES, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, (T *) y, \
-              (T *) probs, steps, chunk, batch, w32)
+    do {                                                                                                                \
+        if (past) DL_LAUNCH_ROWS_AS(CPL, RAG, true);                                                                    \
+        else DL_LAUNCH_ROWS_AS(CPL, RAG, false);                                                                        \
+    } while (0)
         if (ncols <= 2 * DL_WAVE) {
             if (kind == Rows::whole) DL_LAUNCH_ROWS(2, false);
             else DL_LAUNCH_ROWS(2, true);
@@ -1656,6 +1815,7 @@ int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, 
             else DL_LAUNCH_ROWS(4, true);
         }
 #undef DL_LAUNCH_ROWS
+#undef DL_LAUNCH_ROWS_AS
         return dl_launch_status();
     }
     const int64_t blocks = dl_ceil_div(nchunks, 4);
@@ -1664,9 +1824,14 @@ int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, 
     // short rows: 8-byte vectors put a row on all 64 lanes instead of half of them
     const bool half = V >= 2 && ncols <= DL_WAVE / 2;
     const dim3 grid((unsigned) blocks, half ? 1 : col_tiles(ncols));
+#define DL_LAUNCH_CHAIN_AS(VV, RAG, NT)                                                                                \
+    DL_LAUNCH((forward_chain_kernel<T, VV, DL_TRAIN_CHUNK, GATES, RAG, NT>), grid, block, 0, s, xp, verts, neuron, flip, \
+              wp, (T *) y, (T *) probs, nchunks, batch, w32)
 #define DL_LAUNCH_CHAIN(VV, RAG)                                                                                       \
-    DL_LAUNCH((forward_chain_kernel<T, VV, DL_TRAIN_CHUNK, GATES, RAG>), grid, block, 0, s, xp, verts, neuron, flip, wp, \
-              (T *) y, (T *) probs, nchunks, batch, w32)
+    do {                                                                                                               \
+        if (past) DL_LAUNCH_CHAIN_AS(VV, RAG, true);                                                                   \
+        else DL_LAUNCH_CHAIN_AS(VV, RAG, false);                                                                       \
+    } while (0)
     if (half) {
         if (kind == Rows::whole) DL_LAUNCH_CHAIN(H, false);
         else DL_LAUNCH_CHAIN(H, true);
@@ -1675,6 +1840,7 @@ int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, 
         else DL_LAUNCH_CHAIN(V, true);
     }
 #undef DL_LAUNCH_CHAIN
+#undef DL_LAUNCH_CHAIN_AS
     return dl_launch_status();
 }
 
@@ -1702,7 +1868,7 @@ int forward_chain_lower_t(const void *lx, const int64_t *la, const int64_t *lb, 
 
 template <typename T>
 int backward_w_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps,
-                       const void *gy, const void *probs, void *gw, int64_t batch, bool any_rows, hipStream_t s,
+                       const void *gy, const void *probs, void *gw, int64_t in_dim, int64_t batch, bool any_rows, hipStream_t s,
                        int64_t gdiv = 0, bool w32 = false) {
     constexpr int V = Vec16<T>::n;
     const Rows kind = rows_kind<T>(batch, x, gy);
@@ -1710,21 +1876,22 @@ int backward_w_chain_t(const void *x, const int32_t *verts, const int32_t *neuro
     const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
     const int64_t blocks = dl_ceil_div(nchunks, 4);
     if (blocks > 0x7fffffffLL || ncols > 4 * DL_WAVE) return DL_ERR_TOO_LARGE;   // a lane holds at most 4 vectors of a row
+    const bool past = gdiv == 0 && past_cache(DL_PAST_WEIGHTS, steps, in_dim, batch * (int64_t) sizeof(T));
+#define DL_LAUNCH_W_CHAIN_AS(CPL, RAG, NT)                                                                             \
+    DL_LAUNCH((backward_w_chain_kernel<T, V, CPL, DL_TRAIN_CHUNK, RAG, NT>), dim3((unsigned) blocks), dim3(DL_BLOCK),  \
+              0, s, (const T *) x, verts, neuron, flip, (const T *) gy, (const T *) probs, (T *) gw, nchunks, batch, gdiv, w32)
 #define DL_LAUNCH_W_CHAIN(CPL)                                                                                         \
     do {                                                                                                               \
-        if (kind == Rows::whole)                                                                                       \
-            DL_LAUNCH((backward_w_chain_kernel<T, V, CPL, DL_TRAIN_CHUNK, false>), dim3((unsigned) blocks), dim3(DL_BLOCK), \
-                      0, s, (const T *) x, verts, neuron, flip, (const T *) gy, (const T *) probs, (T *) gw, nchunks,  \
-                      batch, gdiv, w32);                                                                               \
-        else                                                                                                           \
-            DL_LAUNCH((backward_w_chain_kernel<T, V, CPL, DL_TRAIN_CHUNK, true>), dim3((unsigned) blocks), dim3(DL_BLOCK), \
-                      0, s, (const T *) x, verts, neuron, flip, (const T *) gy, (const T *) probs, (T *) gw, nchunks,  \
-                      batch, gdiv, w32);                                                                               \
+        if (kind == Rows::whole && past) DL_LAUNCH_W_CHAIN_AS(CPL, false, true);                                       \
+        else if (kind == Rows::whole) DL_LAUNCH_W_CHAIN_AS(CPL, false, false);                                         \
+        else if (past) DL_LAUNCH_W_CHAIN_AS(CPL, true, true);                                                          \
+        else DL_LAUNCH_W_CHAIN_AS(CPL, true, false);                                                                   \
     } while (0)
     if (ncols <= DL_WAVE) DL_LAUNCH_W_CHAIN(1);
     else if (ncols <= 2 * DL_WAVE) DL_LAUNCH_W_CHAIN(2);
     else DL_LAUNCH_W_CHAIN(4);
 #undef DL_LAUNCH_W_CHAIN
+#undef DL_LAUNCH_W_CHAIN_AS
     return dl_launch_status();
 }
 
@@ -1758,27 +1925,29 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
     if ((partial_bytes > 0 || overflow_rows > 0) && workspace == nullptr) return DL_ERR_INVALID_ARGUMENT;
     C *partial = partial_bytes > 0 ? (C *) workspace : nullptr;
     C *overflow = (C *) ((char *) workspace + partial_bytes);
-    const int chunk = chain_chunk(steps * segments);
+    const int chunk = chain_chunk(steps * segments, ncols > 2 * DL_WAVE ? DL_CHAIN_WAVES_LONG : DL_CHAIN_WAVES);
     const int64_t blocks = dl_ceil_div(dl_ceil_div(steps, chunk), 4), fix_blocks = dl_ceil_div(n_fix, 4);
     if (blocks > 0x7fffffffLL || fix_blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     const dim3 grid((unsigned) blocks, (unsigned) segments), block(DL_BLOCK);
     const T *xp = (const T *) x, *wp = (const T *) w, *gp = (const T *) gy, *pp = softmax_backward ? wp : nullptr;
     constexpr int H = V >= 2 ? V / 2 : 1;
-#define DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, LOWER, RAG)                                                                 \
-    DL_LAUNCH((backward_chain_kernel<T, VV, CPL, LOWER, RAG>), grid, block, 0, s, xp, verts, neuron, flip, dst, wp, gp, pp, \
-              (T *) gw, partial, (T *) gx, overflow, steps, chunk, in_dim, out_dim, batch, (C) scale, gdiv,             \
+    const bool past = gdiv == 0 && past_cache(DL_PAST_BACKWARD, steps, in_dim, batch * (int64_t) sizeof(T));
+#define DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, LOWER, RAG, NT)                                                             \
+    DL_LAUNCH((backward_chain_kernel<T, VV, CPL, LOWER, RAG, NT>), grid, block, 0, s, xp, verts, neuron, flip, dst, wp, gp, \
+              pp, (T *) gw, partial, (T *) gx, overflow, steps, chunk, in_dim, out_dim, batch, (C) scale, gdiv,         \
               LOWER ? *lower : none, LOWER ? false : w32)
+#define DL_LAUNCH_BACKWARD_CHAIN_RAG(VV, CPL, RAG, NT)                                                                   \
+    do {                                                                                                                 \
+        if (lower && !x) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, RAG, NT);                                               \
+        else if (lower) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 1, RAG, NT);                                                \
+        else DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 0, RAG, NT);                                                           \
+    } while (0)
 #define DL_LAUNCH_BACKWARD_CHAIN(VV, CPL)                                                                                \
     do {                                                                                                                 \
-        if (kind == Rows::whole) {                                                                                       \
-            if (lower && !x) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, false);                                             \
-            else if (lower) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 1, false);                                              \
-            else DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 0, false);                                                         \
-        } else {                                                                                                         \
-            if (lower && !x) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, true);                                              \
-            else if (lower) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 1, true);                                               \
-            else DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 0, true);                                                          \
-        }                                                                                                                \
+        if (kind == Rows::whole && past) DL_LAUNCH_BACKWARD_CHAIN_RAG(VV, CPL, false, true);                             \
+        else if (kind == Rows::whole) DL_LAUNCH_BACKWARD_CHAIN_RAG(VV, CPL, false, false);                               \
+        else if (past) DL_LAUNCH_BACKWARD_CHAIN_RAG(VV, CPL, true, true);                                                \
+        else DL_LAUNCH_BACKWARD_CHAIN_RAG(VV, CPL, true, false);                                                         \
     } while (0)
     if (V >= 2 && ncols <= DL_WAVE / 2)
         DL_LAUNCH_BACKWARD_CHAIN(H, 1);              // short rows: 8-byte vectors use all 64 lanes
@@ -1789,6 +1958,7 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
     else
         DL_LAUNCH_BACKWARD_CHAIN(V, 4);
 #undef DL_LAUNCH_BACKWARD_CHAIN_AS
+#undef DL_LAUNCH_BACKWARD_CHAIN_RAG
 #undef DL_LAUNCH_BACKWARD_CHAIN
     int st = dl_launch_status();
     if (st != DL_OK) return st;
@@ -1948,22 +2118,22 @@ extern "C" int dl_logic_forward_chained(const void *x, const int32_t *verts, con
     hipStream_t s = (hipStream_t) stream;
     if (probs) {
         switch (dtype) {
-        case DL_F16: return forward_chain_t<__half, true>(x, verts, neuron, flip, steps, w, y, probs, batch, any, s, w32);
-        case DL_F32: return forward_chain_t<float, true>(x, verts, neuron, flip, steps, w, y, probs, batch, any, s);
-        default: return forward_chain_t<double, true>(x, verts, neuron, flip, steps, w, y, probs, batch, any, s, w32);
+        case DL_F16: return forward_chain_t<__half, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, batch, any, s, w32);
+        case DL_F32: return forward_chain_t<float, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, batch, any, s);
+        default: return forward_chain_t<double, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, batch, any, s, w32);
         }
     }
     if (argmax) {
         switch (dtype) {
-        case DL_F16: return forward_chain_t<__half, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
-        case DL_F32: return forward_chain_t<float, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s);
-        default: return forward_chain_t<double, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
+        case DL_F16: return forward_chain_t<__half, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
+        case DL_F32: return forward_chain_t<float, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s);
+        default: return forward_chain_t<double, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
         }
     }
     switch (dtype) {
-    case DL_F16: return forward_chain_t<__half, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
-    case DL_F32: return forward_chain_t<float, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s);
-    default: return forward_chain_t<double, false>(x, verts, neuron, flip, steps, w, y, nullptr, batch, any, s, w32);
+    case DL_F16: return forward_chain_t<__half, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
+    case DL_F32: return forward_chain_t<float, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s);
+    default: return forward_chain_t<double, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
     }
 }
 
@@ -2010,9 +2180,9 @@ extern "C" int dl_logic_backward_w_chained(const void *x, const int32_t *verts, 
     if (!x || !verts || !neuron || !flip || !grad_y || !grad_w || in_dim == 0) return DL_ERR_INVALID_ARGUMENT;
     hipStream_t s = (hipStream_t) stream;
     switch (dtype) {
-    case DL_F16: return backward_w_chain_t<__half>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, any, s, 0, w32);
-    case DL_F32: return backward_w_chain_t<float>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, any, s);
-    default: return backward_w_chain_t<double>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, batch, any, s, 0, w32);
+    case DL_F16: return backward_w_chain_t<__half>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, in_dim, batch, any, s, 0, w32);
+    case DL_F32: return backward_w_chain_t<float>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, in_dim, batch, any, s);
+    default: return backward_w_chain_t<double>(x, verts, neuron, flip, steps, grad_y, probs, grad_w, in_dim, batch, any, s, 0, w32);
     }
 }
 
