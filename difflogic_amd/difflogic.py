@@ -2,10 +2,13 @@
 the gfx950 kernels through ``difflogic_cuda``."""
 import torch
 
-from . import difflogic_cuda
+from . import _host, difflogic_cuda
 from .functional import (GradFactor, bin_op_s, build_reverse_index, get_random_connections,
                          get_unique_connections)
 from .packbitstensor import PackBitsTensor
+
+
+_PLAIN = (torch.nn.Parameter, torch.Tensor)
 
 
 class LogicLayer(torch.nn.Module):
@@ -103,6 +106,13 @@ class LogicLayer(torch.nn.Module):
 
     def forward_cuda(self, x):
         if self.training:
+            if (type(x) is torch.Tensor and type(self.weights) in _PLAIN and torch._C._get_tracing_state() is None
+                    and (self.in_dim < self._CHAIN_MIN_IN_DIM or self._train_schedule(x.transpose(0, 1)) is None)):
+                # a layer without a schedule: one native call (784 -> 4 x 8000 at batch 100 as written: NNN us a step)
+                y = _host.train_layer(x, self.weights, *self.indices, self.given_x_indices_of_y_start,
+                                      self.given_x_indices_of_y, float(self.grad_factor))
+                if y is not None:
+                    return y
             assert x.device.type == "cuda", x.device
         assert x.ndim == 2, x.ndim
         x = x.transpose(0, 1).contiguous()                  # feature-major [in, B]
@@ -138,11 +148,12 @@ class LogicLayer(torch.nn.Module):
         assert isinstance(x, PackBitsTensor)
         assert x.features == self.in_dim, (x.features, self.in_dim)
         a, b = self.indices
-        key = (self.weights.data_ptr(), self.weights._version, self.out_dim)
         w = self.weights.detach()
-        if w.is_cuda and w.is_contiguous() and w.dtype in (torch.float16, torch.float32, torch.float64):
-            if x.takes_weights(self.out_dim):
-                return x.apply_weights(a, b, w)
+        plain = w.is_cuda and w.is_contiguous() and w.dtype in (torch.float16, torch.float32, torch.float64)
+        if plain and x.takes_weights(self.out_dim):
+            return x.apply_weights(a, b, w)
+        key = (self.weights.data_ptr(), self.weights._version, self.out_dim)
+        if plain:
             # the argmax gates with the constants among x's rows folded in, in one kernel (x tracks which rows those are)
             ids, state = difflogic_cuda.gate_ids_folded(w, a, b, x.row_state(a.device))
             return x.defer_layer(a, b, ids, key=key, state=state)
@@ -221,6 +232,11 @@ class GroupSum(torch.nn.Module):
         if isinstance(x, PackBitsTensor):
             return x.group_sum(self.k)
         assert x.shape[-1] % self.k == 0, (x.shape, self.k)
+        if (type(x) is torch.Tensor and self.k <= self._HIP_MAX_K and x.shape[-1] <= self._HIP_MAX_OUT_DIM
+                and torch._C._get_tracing_state() is None):
+            y = _host.group_sum(x, int(self.k), float(self.tau))            # the case below in one native call
+            if y is not None:
+                return y
         if (x.is_cuda and x.dim() == 2 and x.dtype in (torch.float16, torch.float32, torch.float64)
                 and x.numel() > 0 and x.stride(0) == 1 and x.stride(1) == x.shape[0]
                 and self.k <= self._HIP_MAX_K and x.shape[1] <= self._HIP_MAX_OUT_DIM):

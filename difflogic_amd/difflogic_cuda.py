@@ -15,7 +15,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 
 _FLOAT_CODES = {torch.float16: _lib.DL_F16, torch.float32: _lib.DL_F32, torch.float64: _lib.DL_F64}
 _WORD_BITS = {torch.int8: 8, torch.uint8: 8, torch.int16: 16, torch.int32: 32, torch.int64: 64}
@@ -531,6 +531,9 @@ def gate_ids(weights):
 def eval_weights(x, a, b, weights):
     """``eval(x, a, b, gate_ids(weights))`` in one kernel, on rows ``x`` int64 [in, W] of whole 16-byte vectors (W even).
     Not part of the reference's extension; PackBitsTensor uses it for short rows."""
+    y = _host.eval_weights(x, a, b, weights)
+    if y is not None:
+        return y
     index = x.get_device()
     ready = _ready(index, (x, a, b, weights))
     if not ready:
@@ -559,6 +562,9 @@ def gate_ids_folded(weights, a, b, state=None):
     ``a``, ``b`` whose input rows are constant where ``state`` says so (uint8 [in]: 0 varies, 1 all zeros, 2 all
     ones; None: all vary).  ``ids`` uint8 [out] are the argmax gates with those constants folded in, ``state_out``
     uint8 [out] the constants among the layer's outputs.  Not part of the reference's extension."""
+    both = _host.gate_ids_folded(weights, a, b, state)
+    if both is not None:
+        return both
     index = weights.get_device()
     ready = _ready(index, (weights, a, b) if state is None else (weights, a, b, state))
     if not ready:
@@ -658,6 +664,9 @@ def tensor_packbits_batch_major_rows(x, row_bytes):
     B bits); sample s is bit s % 64 of word s / 64, bits past the batch are zero.  The bytes are
     those of int{8,16,32} words as well.  Not part of the reference's extension; PackBitsTensor
     uses it."""
+    out = _host.pack_rows(x, row_bytes)
+    if out is not None:
+        return out
     _check_input(x, "x")
     if x.dtype != torch.bool or x.dim() != 2:
         raise RuntimeError(f"expected x to be a 2-D bool tensor, got {x.dtype} with {x.dim()} dims")
@@ -674,6 +683,10 @@ def tensor_packbits_batch_major_rows(x, row_bytes):
 
 def groupbitsum(b, pad_len, k):
     """int words [out,W] -> int32 [W*bits - pad_len, k]   (difflogic.cpp:75-83)."""
+    if b.dtype is torch.int64:
+        out = _host.count_rows(b, int(pad_len), int(k))
+        if out is not None:
+            return out
     _check_input(b, "b")
     bits = _WORD_BITS.get(b.dtype)
     if bits is None or b.dim() != 2:
