@@ -39,20 +39,67 @@ bool index_of(const Tensor &t, c10::DeviceIndex device, int64_t numel) {
     return t.scalar_type() == at::kLong && t.dim() == 1 && t.size(0) == numel && plain(t, device);
 }
 
-// LogicLayerLogitsFunction without a schedule: feature-major x [in, B] and gate logits -> y [out, B].
+// A layer's walk along its evaluation schedule: difflogic_cuda.EvalSchedule and the plan of its one-pass backward
+// ([verts, neuron, flip, dst, fix_vertex, fix_start]; none: the layer has no schedule), and which of the kernels take it.
+struct Walk {
+    std::vector<Tensor> tables;
+    int64_t steps = 0, n_fix = 0, rows = 0;
+    bool forward = false, weights = false;
+
+    const int32_t *i32(int i) const { return tables[i].const_data_ptr<int32_t>(); }
+    const uint8_t *flip() const { return tables[2].const_data_ptr<uint8_t>(); }
+};
+
+bool fits(const Walk &w, c10::DeviceIndex device) {
+    if (w.tables.empty()) return true;
+    if (w.tables.size() != 6 || w.steps < 0 || w.n_fix < 0 || w.rows < 0) return false;
+    const int64_t sizes[6] = {w.steps + 1, w.steps, w.steps, w.steps + 1, w.n_fix, w.n_fix + 1};
+    for (int i = 0; i < 6; ++i)
+        if (w.tables[i].scalar_type() != (i == 2 ? at::kByte : at::kInt) || w.tables[i].numel() != sizes[i] || !plain(w.tables[i], device))
+            return false;
+    return true;
+}
+
+Tensor forward_into(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &logits, const Tensor &probs, int code,
+                    const Walk &walk) {
+    const int64_t out_dim = logits.size(0);
+    Tensor y = at::empty({out_dim, x.size(1)}, x.options());
+    int st = DL_ERR_TOO_LARGE;
+    if (!walk.tables.empty() && walk.forward)
+        st = dl_logic_forward_chained(x.const_data_ptr(), walk.i32(0), walk.i32(1), walk.flip(), walk.steps, logits.const_data_ptr(),
+                                      y.mutable_data_ptr(), probs.mutable_data_ptr(), x.size(0), out_dim, x.size(1),
+                                      code | DL_ROWS_ANY, stream_of(x));
+    if (st == DL_ERR_TOO_LARGE)
+        st = dl_logic_forward_logits(x.const_data_ptr(), a.const_data_ptr<int64_t>(), b.const_data_ptr<int64_t>(),
+                                     logits.const_data_ptr(), y.mutable_data_ptr(), probs.mutable_data_ptr(), x.size(0), out_dim,
+                                     x.size(1), code, stream_of(x));
+    check(st, "logic_layer_cuda_forward_logits");
+    return y;
+}
+
+void backward_both_into(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &probs, const Tensor &gy,
+                        const Tensor &start, const Tensor &idx, const Tensor &gw, const Tensor &gx, int64_t gdiv_classes,
+                        double scale, bool softmax, int code) {
+    check(dl_logic_backward_both(x.const_data_ptr(), a.const_data_ptr<int64_t>(), b.const_data_ptr<int64_t>(),
+                                 probs.const_data_ptr(), gy.const_data_ptr(), softmax ? 1 : 0, start.const_data_ptr<int64_t>(),
+                                 idx.const_data_ptr<int64_t>(), gw.mutable_data_ptr(), gx.mutable_data_ptr(), x.size(0),
+                                 probs.size(0), x.size(1), gdiv_classes, scale, code, stream_of(x)),
+          "logic_layer_cuda_backward_both");
+}
+
+// LogicLayerLogitsFunction: feature-major x [in, B] and gate logits -> y [out, B].
 struct LayerFunction : torch::autograd::Function<LayerFunction> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &logits, const Tensor &a, const Tensor &b,
-                          const Tensor &start, const Tensor &idx, double scale, int64_t code) {
-        const int64_t out_dim = logits.size(0);
-        Tensor w = logits.detach();
-        Tensor y = at::empty({out_dim, x.size(1)}, x.options()), probs = at::empty_like(w);
-        check(dl_logic_forward_logits(x.const_data_ptr(), a.const_data_ptr<int64_t>(), b.const_data_ptr<int64_t>(),
-                                      w.const_data_ptr(), y.mutable_data_ptr(), probs.mutable_data_ptr(), x.size(0), out_dim,
-                                      x.size(1), (int) code, stream_of(x)),
-              "logic_layer_cuda_forward_logits");
+                          const Tensor &start, const Tensor &idx, double scale, int64_t code, const Walk *walk) {
+        const Tensor w = logits.detach(), probs = at::empty_like(w);
+        Tensor y = forward_into(x, a, b, w, probs, (int) code, *walk);
         ctx->save_for_backward({x, a, b, probs, start, idx});
         ctx->saved_data["scale"] = scale;
         ctx->saved_data["code"] = code;
+        if (!walk->tables.empty()) {
+            ctx->saved_data["tables"] = walk->tables;
+            ctx->saved_data["sizes"] = std::vector<int64_t>{walk->steps, walk->n_fix, walk->rows, walk->weights};
+        }
         return y;
     }
 
@@ -61,6 +108,13 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
         const Tensor &x = saved[0], &a = saved[1], &b = saved[2], &probs = saved[3], &start = saved[4], &idx = saved[5];
         const double scale = ctx->saved_data["scale"].toDouble();
         const int code = (int) ctx->saved_data["code"].toInt();
+        Walk walk;
+        const auto tables = ctx->saved_data.find("tables");
+        if (tables != ctx->saved_data.end()) {
+            walk.tables = tables->second.toTensorVector();
+            const std::vector<int64_t> sizes = ctx->saved_data["sizes"].toIntVector();
+            walk.steps = sizes[0], walk.n_fix = sizes[1], walk.rows = sizes[2], walk.weights = sizes[3] != 0;
+        }
         const c10::DeviceGuard guard(x.device());
         const Tensor gy = grads[0].contiguous();
         TORCH_CHECK(gy.scalar_type() == x.scalar_type() && gy.dim() == 2 && gy.size(0) == probs.size(0) && gy.size(1) == x.size(1)
@@ -69,37 +123,123 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
         const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1);
         const int64_t in_dim = x.size(0), out_dim = probs.size(0), batch = x.size(1);
         const int64_t *ap = a.const_data_ptr<int64_t>(), *bp = b.const_data_ptr<int64_t>();
-        const int64_t *sp = start.const_data_ptr<int64_t>(), *ip = idx.const_data_ptr<int64_t>();
         Tensor gx = want_x ? at::empty_like(x) : Tensor(), gw = want_w ? at::empty_like(probs) : Tensor();
-        if (want_x && want_w)
-            check(dl_logic_backward_both(x.const_data_ptr(), ap, bp, probs.const_data_ptr(), gy.const_data_ptr(), 1, sp, ip,
-                                         gw.mutable_data_ptr(), gx.mutable_data_ptr(), in_dim, out_dim, batch, 0, scale, code,
-                                         stream_of(x)),
-                  "logic_layer_cuda_backward_both");
-        else if (want_x)
-            check(dl_logic_backward_x(x.const_data_ptr(), ap, bp, probs.const_data_ptr(), gy.const_data_ptr(), sp, ip,
-                                      gx.mutable_data_ptr(), in_dim, out_dim, batch, scale, code, stream_of(x)),
+        int st = DL_ERR_TOO_LARGE;
+        if (want_x && want_w) {
+            if (!walk.tables.empty()) {
+                const int64_t bytes = dl_logic_backward_chained_workspace_bytes(walk.rows, out_dim, batch, code | DL_ROWS_ANY);
+                check(bytes < 0 ? (int) -bytes : DL_OK, "logic_layer_cuda_backward_chained");
+                const Tensor ws = bytes ? at::empty({bytes}, x.options().dtype(at::kByte)) : Tensor();
+                st = dl_logic_backward_chained(x.const_data_ptr(), walk.i32(0), walk.i32(1), walk.flip(), walk.i32(3), walk.steps,
+                                               probs.const_data_ptr(), gy.const_data_ptr(), 1,
+                                               walk.n_fix ? walk.i32(4) : nullptr, walk.n_fix ? walk.i32(5) : nullptr, walk.n_fix,
+                                               walk.rows, gw.mutable_data_ptr(), gx.mutable_data_ptr(),
+                                               bytes ? ws.mutable_data_ptr() : nullptr, in_dim, out_dim, batch, scale,
+                                               code | DL_ROWS_ANY, stream_of(x));
+                if (st != DL_ERR_TOO_LARGE) check(st, "logic_layer_cuda_backward_chained");
+            }
+            if (st == DL_ERR_TOO_LARGE)
+                backward_both_into(x, a, b, probs, gy, start, idx, gw, gx, 0, scale, true, code);
+        } else if (want_x) {
+            check(dl_logic_backward_x(x.const_data_ptr(), ap, bp, probs.const_data_ptr(), gy.const_data_ptr(),
+                                      start.const_data_ptr<int64_t>(), idx.const_data_ptr<int64_t>(), gx.mutable_data_ptr(),
+                                      in_dim, out_dim, batch, scale, code, stream_of(x)),
                   "logic_layer_cuda_backward_x");
-        else if (want_w)
-            check(dl_logic_backward_logits(x.const_data_ptr(), ap, bp, gy.const_data_ptr(), probs.const_data_ptr(),
-                                           gw.mutable_data_ptr(), in_dim, out_dim, batch, code, stream_of(x)),
-                  "logic_layer_cuda_backward_w");
-        return {gx, gw, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        } else if (want_w) {
+            if (!walk.tables.empty() && walk.weights)
+                st = dl_logic_backward_w_chained(x.const_data_ptr(), walk.i32(0), walk.i32(1), walk.flip(), walk.steps,
+                                                 gy.const_data_ptr(), probs.const_data_ptr(), gw.mutable_data_ptr(), in_dim,
+                                                 out_dim, batch, code | DL_ROWS_ANY, stream_of(x));
+            if (st == DL_ERR_TOO_LARGE)
+                st = dl_logic_backward_logits(x.const_data_ptr(), ap, bp, gy.const_data_ptr(), probs.const_data_ptr(),
+                                              gw.mutable_data_ptr(), in_dim, out_dim, batch, code, stream_of(x));
+            check(st, "logic_layer_cuda_backward_w");
+        }
+        return {gx, gw, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
-// A training layer on x [B, in] as LogicLayer.forward_cuda runs one that has no schedule: y [B, out], a view of [out, B].
-c10::optional<Tensor> train_layer(const Tensor &x, const Tensor &weights, const Tensor &a, const Tensor &b, const Tensor &start,
-                                  const Tensor &idx, double scale) {
-    if (!x.is_cuda() || x.dim() != 2 || weights.dim() != 2 || weights.size(1) != 16) return c10::nullopt;
+// Feature-major x and the layer's tensors as the kernels take them; the dtype code, or -1.
+int layer_args(const Tensor &x, const Tensor &w, const Tensor &a, const Tensor &b) {
+    if (!x.is_cuda() || x.dim() != 2 || w.dim() != 2 || w.size(1) != 16 || x.numel() == 0 || w.size(0) == 0) return -1;
     const c10::DeviceIndex device = x.get_device();
-    const int code = layer_code(x.scalar_type(), weights.scalar_type());
-    const int64_t out_dim = weights.size(0), in_dim = x.size(1);
-    if (code < 0 || x.size(0) == 0 || in_dim == 0 || out_dim == 0 || !plain(weights, device) || !index_of(a, device, out_dim)
-        || !index_of(b, device, out_dim) || !index_of(start, device, in_dim + 1) || !index_of(idx, device, 2 * out_dim))
+    if (!plain(w, device) || !index_of(a, device, w.size(0)) || !index_of(b, device, w.size(0))) return -1;
+    return layer_code(x.scalar_type(), w.scalar_type());
+}
+
+bool reverse_args(const Tensor &start, const Tensor &idx, c10::DeviceIndex device, int64_t in_dim, int64_t out_dim) {
+    return index_of(start, device, in_dim + 1) && index_of(idx, device, 2 * out_dim);
+}
+
+// A training layer on x [B, in] as LogicLayer.forward_cuda runs it: y [B, out], a view of [out, B].
+c10::optional<Tensor> train_layer(const Tensor &x, const Tensor &weights, const Tensor &a, const Tensor &b, const Tensor &start,
+                                  const Tensor &idx, double scale, std::vector<Tensor> tables, int64_t steps, int64_t n_fix,
+                                  int64_t rows, bool walk_forward, bool walk_weights) {
+    const int code = layer_args(x, weights, a, b);
+    const Walk walk{std::move(tables), steps, n_fix, rows, walk_forward, walk_weights};
+    if (code < 0 || !reverse_args(start, idx, x.get_device(), x.size(1), weights.size(0)) || !fits(walk, x.get_device()))
         return c10::nullopt;
     const c10::DeviceGuard guard(x.device());
-    return LayerFunction::apply(x.transpose(0, 1).contiguous(), weights, a, b, start, idx, scale, (int64_t) code).transpose(0, 1);
+    return LayerFunction::apply(x.transpose(0, 1).contiguous(), weights, a, b, start, idx, scale, (int64_t) code, &walk)
+        .transpose(0, 1);
+}
+
+// difflogic_cuda.forward_logits without a schedule.
+c10::optional<std::tuple<Tensor, Tensor>> forward_logits(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &logits) {
+    const int code = layer_args(x, logits, a, b);
+    if (code < 0 || !x.is_contiguous()) return c10::nullopt;
+    const c10::DeviceGuard guard(x.device());
+    Tensor probs = at::empty_like(logits);
+    Tensor y = forward_into(x, a, b, logits, probs, code, Walk());
+    return std::make_tuple(y, probs);
+}
+
+// difflogic_cuda.backward_both; classes > 0: gy is the [classes, B] gradient of a GroupSum behind the layer.
+c10::optional<std::tuple<Tensor, Tensor>> backward_both(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &w,
+                                                        const Tensor &gy, const Tensor &start, const Tensor &idx, double scale,
+                                                        bool softmax, int64_t classes) {
+    const int code = layer_args(x, w, a, b);
+    if (code < 0 || !x.is_contiguous() || !reverse_args(start, idx, x.get_device(), x.size(0), w.size(0))
+        || !plain(gy, x.get_device()) || gy.dim() != 2 || gy.scalar_type() != x.scalar_type() || gy.size(1) != x.size(1)
+        || gy.size(0) != (classes ? classes : w.size(0)) || classes < 0
+        || (classes && (w.size(0) % classes || !softmax || w.scalar_type() != x.scalar_type())))
+        return c10::nullopt;
+    const c10::DeviceGuard guard(x.device());
+    Tensor gw = at::empty_like(w), gx = at::empty_like(x);
+    backward_both_into(x, a, b, w, gy, start, idx, gw, gx, classes, scale, softmax, code);
+    return std::make_tuple(gw, gx);
+}
+
+// difflogic_cuda.backward_logits without a schedule.
+c10::optional<Tensor> backward_logits(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &gy, const Tensor &probs) {
+    const int code = layer_args(x, probs, a, b);
+    if (code < 0 || !x.is_contiguous() || !plain(gy, x.get_device()) || gy.dim() != 2 || gy.scalar_type() != x.scalar_type()
+        || gy.size(0) != probs.size(0) || gy.size(1) != x.size(1))
+        return c10::nullopt;
+    const c10::DeviceGuard guard(x.device());
+    Tensor gw = at::empty_like(probs);
+    check(dl_logic_backward_logits(x.const_data_ptr(), a.const_data_ptr<int64_t>(), b.const_data_ptr<int64_t>(),
+                                   gy.const_data_ptr(), probs.const_data_ptr(), gw.mutable_data_ptr(), x.size(0), probs.size(0),
+                                   x.size(1), code, stream_of(x)),
+          "logic_layer_cuda_backward_logits");
+    return gw;
+}
+
+// difflogic_cuda.forward_group_sum: (scores [B, k], probs).
+c10::optional<std::tuple<Tensor, Tensor>> forward_group_sum(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &logits,
+                                                            int64_t k, double tau) {
+    const int code = layer_args(x, logits, a, b);
+    if (code < 0 || x.scalar_type() != logits.scalar_type() || !x.is_contiguous() || k <= 0 || logits.size(0) % k)
+        return c10::nullopt;
+    const c10::DeviceGuard guard(x.device());
+    Tensor y = at::empty({x.size(1), k}, x.options()), probs = at::empty_like(logits);
+    const int64_t bytes = dl_group_sum_workspace_bytes(logits.size(0), x.size(1), k, code);
+    const Tensor ws = at::empty({std::max<int64_t>(1, bytes)}, x.options().dtype(at::kByte));
+    check(dl_logic_forward_group_sum(x.const_data_ptr(), a.const_data_ptr<int64_t>(), b.const_data_ptr<int64_t>(),
+                                     logits.const_data_ptr(), probs.mutable_data_ptr(), y.mutable_data_ptr(),
+                                     ws.mutable_data_ptr(), x.size(0), logits.size(0), x.size(1), k, tau, code, stream_of(x)),
+          "logic_layer_cuda_forward_group_sum");
+    return std::make_tuple(y, probs);
 }
 
 // GroupSumCudaFunction: feature-major x [out, B] -> scores [B, k].
@@ -211,6 +351,10 @@ c10::optional<Tensor> count_rows(const Tensor &b, int64_t pad, int64_t k) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     typedef py::call_guard<py::gil_scoped_release> unlocked;
     m.def("train_layer", &train_layer, unlocked());
+    m.def("forward_logits", &forward_logits, unlocked());
+    m.def("backward_both", &backward_both, unlocked());
+    m.def("backward_logits", &backward_logits, unlocked());
+    m.def("forward_group_sum", &forward_group_sum, unlocked());
     m.def("group_sum", &group_sum, unlocked());
     m.def("eval_weights", &eval_weights, unlocked());
     m.def("gate_ids_folded", &gate_ids_folded, unlocked());

@@ -9,6 +9,7 @@ from .packbitstensor import PackBitsTensor
 
 
 _PLAIN = (torch.nn.Parameter, torch.Tensor)
+_NO_WALK = ([], 0, 0, 0, False, False)
 
 
 class LogicLayer(torch.nn.Module):
@@ -106,13 +107,13 @@ class LogicLayer(torch.nn.Module):
 
     def forward_cuda(self, x):
         if self.training:
-            if (type(x) is torch.Tensor and type(self.weights) in _PLAIN and torch._C._get_tracing_state() is None
-                    and (self.in_dim < self._CHAIN_MIN_IN_DIM or self._train_schedule(x.transpose(0, 1)) is None)):
-                # a layer without a schedule: one native call (784 -> 4 x 8000 at batch 100 as written: NNN us a step)
-                y = _host.train_layer(x, self.weights, *self.indices, self.given_x_indices_of_y_start,
-                                      self.given_x_indices_of_y, float(self.grad_factor))
-                if y is not None:
-                    return y
+            if type(x) is torch.Tensor and type(self.weights) in _PLAIN and torch._C._get_tracing_state() is None:
+                walk = self._native_walk(x)
+                if walk is not None:
+                    y = _host.train_layer(x, self.weights, *self.indices, self.given_x_indices_of_y_start,
+                                          self.given_x_indices_of_y, float(self.grad_factor), *walk)
+                    if y is not None:
+                        return y
             assert x.device.type == "cuda", x.device
         assert x.ndim == 2, x.ndim
         x = x.transpose(0, 1).contiguous()                  # feature-major [in, B]
@@ -169,6 +170,24 @@ class LogicLayer(torch.nn.Module):
     _CHAIN_MIN_OUT_DIM = 20000
     _CHAIN_MIN_BYTES = 16_000_000           # ... of output rows: a quarter of the width is enough
     _evaluated = False                      # whether forward has run in eval mode on float inputs
+
+    def _native_walk(self, x):
+        """What _host.train_layer is told of the layer's schedule for x [B, in], or None where the call stays in Python: the
+        layer walks a schedule and does not form both gradients in one pass along it."""
+        if self.in_dim < self._CHAIN_MIN_IN_DIM or x.ndim != 2 or x.shape[1] != self.in_dim:
+            return _NO_WALK
+        xt = x.transpose(0, 1)
+        schedule = self._train_schedule(xt)
+        if schedule is None:
+            return _NO_WALK
+        if not (x.requires_grad and self.weights.requires_grad and torch.is_grad_enabled()
+                and x.is_cuda and schedule.verts.device == x.device):
+            return None
+        plan = schedule.backward_plan()
+        if plan is None or plan[4] > self.in_dim * difflogic_cuda.BACKWARD_CHAIN_MAX_OVERFLOW:
+            return None
+        return ([schedule.verts, schedule.neuron, schedule.flip, *plan[:3]], schedule.steps, *plan[3:],
+                _forward_walk(schedule, self.out_dim, xt) is not None, _weights_walk(schedule, self.out_dim, xt) is not None)
 
     def _train_schedule(self, x=None):
         """Evaluation schedule of this layer's wiring for the chained forward / backward kernels (cached per

@@ -230,6 +230,9 @@ def backward_both(x, a, b, w, grad_y, given_x_indices_of_y_start, given_x_indice
     returned) and backward_x in one launch: (grad_w [out,16] of w's dtype, grad_x [in,B]), the values of the two.  Not
     part of the reference's extension."""
     start, idx = given_x_indices_of_y_start, given_x_indices_of_y
+    both = _host.backward_both(x, a, b, w, grad_y, start, idx, float(scale), bool(softmax_backward), 0)
+    if both is not None:
+        return both
     index = x.get_device()
     ready = _ready(index, (x, a, b, w, grad_y, start, idx))
     for t, n in () if ready else ((x, "x"), (a, "a"), (b, "b"), (w, "w"), (grad_y, "grad_y"),
@@ -267,6 +270,10 @@ def forward_logits(x, a, b, logits, schedule=None):
     and so is what backward_logits / backward_chained return for them).
     ``schedule`` (an EvalSchedule of (a, b)) selects the chained kernel: same result, one
     gathered input row per neuron instead of two."""
+    if schedule is None:
+        both = _host.forward_logits(x, a, b, logits)
+        if both is not None:
+            return both
     index = x.get_device()
     ready = _ready(index, (x, a, b, logits))
     if not ready:
@@ -308,6 +315,10 @@ def backward_logits(x, a, b, grad_y, probs, schedule=None):
     """Gradient with respect to the gate logits: backward_w chained with the softmax backward,
     ``p * (g - (p * g).sum(-1, keepdim=True))`` with ``g = backward_w(x, a, b, grad_y)``.
     ``schedule`` selects the chained kernel (bit-identical result)."""
+    if schedule is None:
+        grad_logits = _host.backward_logits(x, a, b, grad_y, probs)
+        if grad_logits is not None:
+            return grad_logits
     index = x.get_device()
     ready = _ready(index, (x, a, b, grad_y, probs))
     for t, n in () if ready else ((x, "x"), (a, "a"), (b, "b"), (grad_y, "grad_y"), (probs, "probs")):
@@ -1277,6 +1288,9 @@ def forward_group_sum(x, a, b, logits, k, tau):
     """``group_sum_forward(forward_logits(x, a, b, logits)[0], k, tau)`` without the layer's output
     ever being written: returns (sums [B, k], probs [out, 16]).  Not part of the reference's
     extension."""
+    both = _host.forward_group_sum(x, a, b, logits, int(k), float(tau))
+    if both is not None:
+        return both
     for t, n in ((x, "x"), (a, "a"), (b, "b"), (logits, "logits")):
         _check_input(t, n)
     code = _float_code(x, "logic_layer_cuda_forward")
@@ -1306,6 +1320,10 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
     """Gradients of forward_group_sum: ``grad_cls`` [k, B] is the gradient of the sums, transposed
     and already divided by tau; every neuron of class c sees row c as its grad_y (the broadcast
     matrix is never built).  Returns (grad_logits or None, grad_x or None)."""
+    if want_x and want_w and schedule is None and grad_cls.dim() == 2:
+        both = _host.backward_both(x, a, b, probs, grad_cls, start, idx, float(scale), True, grad_cls.shape[0])
+        if both is not None:
+            return both
     for t, n in ((x, "x"), (a, "a"), (b, "b"), (probs, "probs"), (grad_cls, "grad_cls")):
         _check_input(t, n)
     code = _float_code(x, "logic_layer_cuda_backward")
