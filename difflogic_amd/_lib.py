@@ -19,6 +19,7 @@ DL_ERR_CAPTURING = 8
 DL_F16, DL_F32, DL_F64, DL_F16_W32, DL_F64_W32 = 0, 1, 2, 3, 4
 DL_ROWS_ANY = 0x100
 DL_GATES_OF_ARGMAX = 0x200
+DL_FIX_POSITIONS = 0x400
 
 DL_STATIC_SCRATCH_BYTES = 64 << 20      # include/difflogic_hip.h
 

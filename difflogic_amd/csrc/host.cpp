@@ -53,7 +53,7 @@ struct Walk {
 bool fits(const Walk &w, c10::DeviceIndex device) {
     if (w.tables.empty()) return true;
     if (w.tables.size() != 6 || w.steps < 0 || w.n_fix < 0 || w.rows < 0) return false;
-    const int64_t sizes[6] = {w.steps + 1, w.steps, w.steps, w.steps + 1, w.n_fix, w.n_fix + 1};
+    const int64_t sizes[6] = {w.steps + 1, w.steps, w.steps, w.steps + 1, w.n_fix, w.n_fix + 1 + w.rows};
     for (int i = 0; i < 6; ++i)
         if (w.tables[i].scalar_type() != (i == 2 ? at::kByte : at::kInt) || w.tables[i].numel() != sizes[i] || !plain(w.tables[i], device))
             return false;
@@ -135,7 +135,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
                                                walk.n_fix ? walk.i32(4) : nullptr, walk.n_fix ? walk.i32(5) : nullptr, walk.n_fix,
                                                walk.rows, gw.mutable_data_ptr(), gx.mutable_data_ptr(),
                                                bytes ? ws.mutable_data_ptr() : nullptr, in_dim, out_dim, batch, scale,
-                                               code | DL_ROWS_ANY, stream_of(x));
+                                               code | DL_ROWS_ANY | DL_FIX_POSITIONS, stream_of(x));
                 if (st != DL_ERR_TOO_LARGE) check(st, "logic_layer_cuda_backward_chained");
             }
             if (st == DL_ERR_TOO_LARGE)

@@ -934,6 +934,15 @@ template <typename T> struct LowerLayer {
     T *gw;                      // [in_dim, 16]
 };
 
+// Vertices of several positions (or none) that further workgroups of the launch finish, a wave each, forming their parts
+// anew: `vertex` [count] with positions[start[i]] .. positions[start[i + 1] - 1].  positions == nullptr: the walks store the
+// parts to overflow rows and backward_fix_kernel adds them.
+struct FixHere {
+    const int32_t *vertex, *start, *positions;
+    int count;
+    uint32_t first_block;
+};
+
 // A vector of an overflow row.  (Eight floats for half rows: two 16-byte accesses, no 32-byte alignment asked for.)
 template <typename T, int VEC, bool RAG>
 using OverflowPack = Pack<typename Acc<T>::type, VEC, RAG || sizeof(T) != sizeof(typename Acc<T>::type)>;
@@ -951,7 +960,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     const T *__restrict__ gy, const T *__restrict__ probs, T *__restrict__ gw,
     typename Acc<T>::type *__restrict__ partial, T *__restrict__ gx, typename Acc<T>::type *__restrict__ overflow,
     int64_t steps, int chunk, int64_t in_dim, int64_t out_dim, int64_t batch, typename Acc<T>::type scale, int64_t gdiv, LowerLayer<T> low,
-    bool w32) {
+    FixHere fix, bool w32) {
     typedef typename Acc<T>::type C;
     typedef Pack<T, VEC, RAG> P;
     const int64_t ncols = vec_count<VEC>(batch);
@@ -965,8 +974,9 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     constexpr int AHEAD = CPL == 1 && LOWER == 0 && sizeof(T) == 4 ? 3 : 1, SLOTS = AHEAD + 1;
     const int wave = dl_wave_in_block();
     const int lane = dl_lane();
-    const int64_t s0 = ((int64_t) blockIdx.x * 4 + wave) * chunk;
-    if (s0 >= steps) return;
+    const bool fixes = blockIdx.x >= fix.first_block;            // (uniform) a workgroup that finishes vertices of several positions
+    const int64_t s0 = ((int64_t) (fixes ? 0 : blockIdx.x) * 4 + wave) * chunk;
+    if (!fixes && s0 >= steps) return;
     const int64_t s1 = s0 + chunk < steps ? s0 + chunk : steps;
     const int64_t col0 = (int64_t) blockIdx.y * (CPL * DL_WAVE);   // this wave's segment of the rows
     const int gate = lane & 15;
@@ -1015,7 +1025,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     };
     // (LOWER) corner sums of the layer below for a finished vertex, whose lower rows are la, lb: as backward_w_kernel on the
     // row that would have been stored, same values, same order of additions
-    auto lower_sums = [&](const C (&val)[CPL][VEC], const P *la, const P *lb) {
+    auto lower_sums = [&](const C (&val)[CPL][VEC], const P *la, const P *lb, C scale) {
         C s00 = (C) 0, s01 = (C) 0, s10 = (C) 0, s11 = (C) 0;
 #pragma unroll
         for (int q = 0; q < CPL; ++q) {
@@ -1038,6 +1048,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     auto store_row = [&](int32_t row, const C (&val)[CPL][VEC]) {
         if (row < 0 || (LOWER != 0 && row < in_dim)) return;
         if (row >= in_dim) {                                     // a part of a sum: in C, scaled here only if that is T
+            if (fix.positions != nullptr) return;                // ... or formed where the sum is taken
             typedef OverflowPack<T, VEC, RAG> O;
 #pragma unroll
             for (int q = 0; q < CPL; ++q) {
@@ -1059,6 +1070,76 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
         }
     };
 
+    // The share of neuron n = neuron[s], between positions s and s + 1, of the vertex at `own`, from the row of the other.
+    auto share_of = [&](int64_t s, bool own_first, C (&share)[CPL][VEC]) {
+        const int32_t n = neuron[s];
+        const bool f = flip[s] != 0;
+        P other[CPL], g[CPL];
+        const int64_t v = verts[own_first ? s + 1 : s];
+        if constexpr (RECOMPUTE) {
+            P oa[LCPL], ob[LCPL];
+            lower_row(v, oa, ob, other);
+        } else {
+            load_row(x, v, true, other);
+        }
+        load_row(gy, grad_row(n, gdiv), true, g);
+        const Corners<C> k = corners<T>(w, n, w32);
+        const C d0 = k.p01 - k.p00, dd = (k.p11 - k.p10) - d0, da = k.p10 - k.p00;
+        const C kk = f == own_first ? d0 : da;
+#pragma unroll
+        for (int q = 0; q < CPL; ++q)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) share[q][e] = up<T>(g[q].v[e]) * slope<SPLIT, C>(up<T>(other[q].v[e]), dd, kk);
+    };
+    if (fixes) {
+        // a wave per vertex: the parts of its positions as the walks form them, added in the order of the overflow rows
+        const int i = (int) (blockIdx.x - fix.first_block) * 4 + wave;
+        if (i >= fix.count) return;
+        const int64_t v = fix.vertex[i];
+        C acc[CPL][VEC];
+#pragma unroll
+        for (int q = 0; q < CPL; ++q)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) acc[q][e] = (C) 0;
+        const int32_t r1 = fix.start[i + 1];
+#pragma unroll 1
+        for (int32_t r = fix.start[i]; r < r1; ++r) {
+            const int64_t p = fix.positions[r];
+            C part[CPL][VEC], next[CPL][VEC];
+#pragma unroll
+            for (int q = 0; q < CPL; ++q)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) part[q][e] = next[q][e] = (C) 0;
+            if (p > 0 && neuron[p - 1] >= 0) share_of(p - 1, false, part);
+            if (p < steps && neuron[p] >= 0) share_of(p, true, next);
+#pragma unroll
+            for (int q = 0; q < CPL; ++q)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    const C both = part[q][e] + next[q][e];
+                    acc[q][e] += sizeof(T) == sizeof(C) ? both * scale : both;
+                }
+        }
+        const C rest = sizeof(T) == sizeof(C) ? (C) 1 : scale;
+        if constexpr (LOWER != 0) {
+            P fa[LCPL], fb[LCPL];
+            lower_rows(v, true, fa, fb);
+            const C lz = lower_sums(acc, fa, fb, rest);
+            const C p = low.probs != nullptr ? up<T>(low.probs[v * 16 + gate]) : zc;
+            store_grad_w4<T, NT>(lane, quarter == 0, v, lz, p, low.probs != nullptr, low.gw, false);
+        } else {
+#pragma unroll
+            for (int q = 0; q < CPL; ++q) {
+                const int64_t col = col0 + lane + q * DL_WAVE;
+                P r;
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) r.v[e] = round_scaled<T, RAG, C>(acc[q][e], rest);
+                if (col < ncols) row_vec<P, VEC, RAG>(gx, v, batch, ncols, col) = r;
+            }
+        }
+        return;
+    }
+
     // prev: row of the vertex at the chunk's first position; pla, plb: (RECOMPUTE) the lower rows it came from,
     // which also serve that vertex's backward_w at step 0
     P prev[CPL], pla[LCPL], plb[LCPL];
@@ -1069,25 +1150,8 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
     for (int q = 0; q < CPL; ++q)
 #pragma unroll
         for (int e = 0; e < VEC; ++e) carry[q][e] = (C) 0;
-    if (s0 > 0 && neuron[s0 - 1] >= 0) {             // share of the neuron that ends at this chunk's first vertex
-        const int32_t n = neuron[s0 - 1];
-        const bool f = flip[s0 - 1] != 0;
-        P before[CPL], g[CPL];
-        if constexpr (RECOMPUTE) {
-            P ba[LCPL], bb[LCPL];
-            lower_row(verts[s0 - 1], ba, bb, before);
-        } else {
-            load_row(x, verts[s0 - 1], true, before);
-        }
-        load_row(gy, grad_row(n, gdiv), true, g);
-        const Corners<C> k = corners<T>(w, n, w32);
-        const C d0 = k.p01 - k.p00, dd = (k.p11 - k.p10) - d0, da = k.p10 - k.p00;
-        const C kv = f ? da : d0;
-#pragma unroll
-        for (int q = 0; q < CPL; ++q)
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) carry[q][e] = up<T>(g[q].v[e]) * slope<SPLIT, C>(up<T>(before[q].v[e]), dd, kv);
-    }
+    // the share of the neuron that ends at this chunk's first vertex
+    if (s0 > 0 && neuron[s0 - 1] >= 0) share_of(s0 - 1, false, carry);
     // The chunk's schedule entries are fetched once, one per lane (chunk <= 64), and handed out by
     // readlane, so the step loop waits for no scalar loads; the rows of step i + 1 are requested
     // before the arithmetic of step i.
@@ -1197,7 +1261,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
                 // the vertex at position s0 + i is finished: RECOMPUTE keeps its lower rows from the step that brought it in
                 if constexpr (LOWER != 0) {
                     if (d[j] >= 0 && d[j] < in_dim) {
-                        const C lz = lower_sums(out, RECOMPUTE ? pla : la[now], RECOMPUTE ? plb : lb[now]);
+                        const C lz = lower_sums(out, RECOMPUTE ? pla : la[now], RECOMPUTE ? plb : lb[now], scale);
                         lsums = quarter == j ? lz : lsums;
                     }
                 }
@@ -1229,7 +1293,7 @@ __global__ __launch_bounds__(DL_BLOCK) void backward_chain_kernel(
         if constexpr (LOWER != 0) {
             if (last >= 0 && last < in_dim) {
                 if constexpr (LOWER == 1) lower_rows(last, true, pla, plb);
-                const C lz = lower_sums(carry, pla, plb);
+                const C lz = lower_sums(carry, pla, plb, scale);
                 const C p = low.probs != nullptr ? up<T>(low.probs[(int64_t) last * 16 + gate]) : zc;
                 store_grad_w4<T, NT>(lane, quarter == 0, last, lz, p, low.probs != nullptr, low.gw, false);
             }
@@ -1757,14 +1821,16 @@ int group_sum_splits(int64_t out_dim, int64_t batch, int64_t k) {
 //   discretised forward    66 MB 22.5 / 25.4, 131 MB 49.2 / 49.7, 179 MB 75 / 72, 262 MB 105 / 94, 524 MB 219 / 203, 1 GB 441 / 445
 //   one-pass backward      66 MB 41.8 / 41.6, 98 MB 64 / 58, 131 MB 90 / 73, 262 MB 173 / 137, 524 MB 347 / 330, 1 GB 685 / 696
 //   backward_w alone       131 MB 44 / 50, 179 MB 66 / 70, 262 MB 98 / 95, 524 MB 203 / 190, 1 GB 502 / 503
+// (The discretised forward goes by the bytes of x and y: a layer that narrows, 80000 -> 40000 at batch 512, 164 MB and 82 MB,
+// is still better off with both in the cache, three layers 112 / 117 us.)
 // Smaller matrices stay in the caches from one kernel to the next; rows that are read several times (a layer much wider
 // than its input, the classes' gradient rows) are read the ordinary way.
 struct PastCache { int64_t from, to; };
-constexpr PastCache DL_PAST_FORWARD = {50000000, INT64_MAX}, DL_PAST_ARGMAX = {140000000, 700000000},
+constexpr PastCache DL_PAST_FORWARD = {50000000, INT64_MAX}, DL_PAST_ARGMAX = {280000000, 1400000000},
                     DL_PAST_BACKWARD = {80000000, 700000000}, DL_PAST_WEIGHTS = {240000000, INT64_MAX};
 
-bool past_cache(PastCache limits, int64_t steps, int64_t in_dim, int64_t row_bytes) {
-    const int64_t bytes = in_dim * row_bytes;
+bool past_cache(PastCache limits, int64_t steps, int64_t in_dim, int64_t row_bytes, int64_t rows_written = 0) {
+    const int64_t bytes = (in_dim + rows_written) * row_bytes;
     return 4 * steps <= 5 * in_dim && bytes >= limits.from && bytes <= limits.to;
 }
 
@@ -1783,13 +1849,15 @@ int chain_chunk(int64_t steps, int64_t waves = DL_CHAIN_WAVES) {
 
 template <typename T, int GATES>
 int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, int64_t steps,
-                    const void *w, void *y, void *probs, int64_t in_dim, int64_t batch, bool any_rows, hipStream_t s,
+                    const void *w, void *y, void *probs, int64_t in_dim, int64_t out_dim, int64_t batch, bool any_rows, hipStream_t s,
                     bool w32 = false) {
     constexpr int V = Vec16<T>::n;
     const Rows kind = rows_kind<T>(batch, x, y);
     if (kind != Rows::whole && !(any_rows && kind == Rows::ragged)) return DL_ERR_TOO_LARGE;
     const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
-    const bool past = past_cache(probs ? DL_PAST_FORWARD : DL_PAST_ARGMAX, steps, in_dim, batch * (int64_t) sizeof(T));
+    const int64_t row_bytes = batch * (int64_t) sizeof(T);
+    const bool past = probs ? past_cache(DL_PAST_FORWARD, steps, in_dim, row_bytes)
+                            : past_cache(DL_PAST_ARGMAX, steps, in_dim, row_bytes, out_dim);
     const T *xp = (const T *) x, *wp = (const T *) w;
     const dim3 block(DL_BLOCK);
     if (ncols > DL_FWD_ROWS_MIN && ncols <= DL_ROWS_MAX_VECTORS) {
@@ -1895,6 +1963,11 @@ int backward_w_chain_t(const void *x, const int32_t *verts, const int32_t *neuro
     return dl_launch_status();
 }
 
+// Vertices (and overflow rows) up to which the one-pass backward finishes them in its own launch.  Each costs four row reads
+// instead of a written and a read row; the launch that goes takes 4 to 5 us a layer (784 -> 4 x 64000, a captured step at
+// batch 100: fp32 fused 187 -> 167 us with the pair's second launch gone too, half 226 -> 213).
+constexpr int64_t DL_FIX_HERE = 64;
+
 template <typename T> int64_t backward_partial_bytes(int64_t out_dim, int64_t batch) {
     constexpr int V = Vec16<T>::n;
     const int segments = row_segments(dl_ceil_div(batch, V));
@@ -1905,7 +1978,7 @@ template <typename T>
 int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, const uint8_t *flip, const int32_t *dst,
                      int64_t steps, const void *w, const void *gy, bool softmax_backward, const int32_t *fix_vertex,
                      const int32_t *fix_start, int64_t n_fix, int64_t overflow_rows, void *gw, void *gx, void *workspace,
-                     int64_t in_dim, int64_t out_dim, int64_t batch, double scale, bool any_rows, hipStream_t s,
+                     int64_t in_dim, int64_t out_dim, int64_t batch, double scale, bool any_rows, bool fix_positions, hipStream_t s,
                      int64_t gdiv = 0, const LowerLayer<T> *lower = nullptr, bool w32 = false) {
     typedef typename Acc<T>::type C;
     constexpr int V = Vec16<T>::n;
@@ -1928,14 +2001,17 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
     const int chunk = chain_chunk(steps * segments, ncols > 2 * DL_WAVE ? DL_CHAIN_WAVES_LONG : DL_CHAIN_WAVES);
     const int64_t blocks = dl_ceil_div(dl_ceil_div(steps, chunk), 4), fix_blocks = dl_ceil_div(n_fix, 4);
     if (blocks > 0x7fffffffLL || fix_blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-    const dim3 grid((unsigned) blocks, (unsigned) segments), block(DL_BLOCK);
+    // a few vertices are finished by further workgroups of the same launch; many are cheaper through overflow rows
+    const bool here = fix_positions && n_fix > 0 && n_fix <= DL_FIX_HERE && overflow_rows <= DL_FIX_HERE && blocks + fix_blocks <= 0x7fffffffLL;
+    const FixHere fix = {fix_vertex, fix_start, here ? fix_start + n_fix + 1 : nullptr, here ? (int) n_fix : 0, (uint32_t) blocks};
+    const dim3 grid((unsigned) (blocks + (here ? fix_blocks : 0)), (unsigned) segments), block(DL_BLOCK);
     const T *xp = (const T *) x, *wp = (const T *) w, *gp = (const T *) gy, *pp = softmax_backward ? wp : nullptr;
     constexpr int H = V >= 2 ? V / 2 : 1;
     const bool past = gdiv == 0 && past_cache(DL_PAST_BACKWARD, steps, in_dim, batch * (int64_t) sizeof(T));
 #define DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, LOWER, RAG, NT)                                                             \
     DL_LAUNCH((backward_chain_kernel<T, VV, CPL, LOWER, RAG, NT>), grid, block, 0, s, xp, verts, neuron, flip, dst, wp, gp, \
               pp, (T *) gw, partial, (T *) gx, overflow, steps, chunk, in_dim, out_dim, batch, (C) scale, gdiv,         \
-              LOWER ? *lower : none, LOWER ? false : w32)
+              LOWER ? *lower : none, fix, LOWER ? false : w32)
 #define DL_LAUNCH_BACKWARD_CHAIN_RAG(VV, CPL, RAG, NT)                                                                   \
     do {                                                                                                                 \
         if (lower && !x) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, RAG, NT);                                               \
@@ -1970,7 +2046,7 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
         st = dl_launch_status();
         if (st != DL_OK) return st;
     }
-    if (n_fix == 0) return DL_OK;
+    if (n_fix == 0 || here) return DL_OK;
     const dim3 fix_grid((unsigned) fix_blocks, col_tiles(ncols));
     const C fix_scale = sizeof(T) == sizeof(C) ? (C) 1 : (C) scale;
     if (kind == Rows::whole)
@@ -2011,6 +2087,13 @@ bool gates_argmax(int &dtype) {
     return argmax;
 }
 
+// DL_FIX_POSITIONS in a dtype code: taken out of it, and returned
+bool takes_fix_positions(int &dtype) {
+    const bool there = (dtype & DL_FIX_POSITIONS) != 0;
+    dtype &= ~DL_FIX_POSITIONS;
+    return there;
+}
+
 // DL_ROWS_ANY in a dtype code: taken out of it, and returned
 bool takes_any_rows(int &dtype) {
     const bool any = (dtype & DL_ROWS_ANY) != 0;
@@ -2024,6 +2107,7 @@ extern "C" int64_t dl_logic_backward_chained_workspace_bytes(int64_t overflow_ro
                                                              int dtype) {
     if (overflow_rows < 0 || out_dim < 0 || batch < 0) return -DL_ERR_INVALID_ARGUMENT;
     takes_any_rows(dtype);
+    takes_fix_positions(dtype);
     weights_fp32(dtype);
     switch (dtype) {
     case DL_F16: return backward_partial_bytes<__half>(out_dim, batch) + overflow_rows * batch * 4;    // parts in fp32
@@ -2039,7 +2123,7 @@ extern "C" int dl_logic_backward_chained(const void *x, const int32_t *verts, co
                                          int64_t n_fix, int64_t overflow_rows, void *grad_w, void *grad_x,
                                          void *workspace, int64_t in_dim, int64_t out_dim, int64_t batch, double scale,
                                          int dtype, void *stream) {
-    const bool any = takes_any_rows(dtype), w32 = weights_fp32(dtype);
+    const bool any = takes_any_rows(dtype), fp = takes_fix_positions(dtype), w32 = weights_fp32(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim <= 0 || out_dim <= 0 || batch <= 0 || steps < out_dim || n_fix < 0 || n_fix > in_dim || overflow_rows < 0)
         return DL_ERR_INVALID_ARGUMENT;
@@ -2050,14 +2134,14 @@ extern "C" int dl_logic_backward_chained(const void *x, const int32_t *verts, co
     switch (dtype) {
     case DL_F16:
         return backward_chain_t<__half>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, 0, nullptr,
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, fp, s, 0, nullptr,
                                         w32);
     case DL_F32:
         return backward_chain_t<float>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s);
+                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, fp, s);
     default:
         return backward_chain_t<double>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, 0, nullptr,
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, fp, s, 0, nullptr,
                                         w32);
     }
 }
@@ -2071,6 +2155,7 @@ extern "C" int dl_logic_backward_chained_lower(const void *x, const int32_t *ver
                                                int softmax_backward_lower, void *grad_w_lower, int64_t in_dim,
                                                int64_t out_dim, int64_t batch, double scale, int dtype, void *stream) {
     const bool any = takes_any_rows(dtype);
+    const bool fp = takes_fix_positions(dtype);
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (in_dim <= 0 || out_dim <= 0 || batch <= 0 || steps < out_dim || n_fix < 0 || n_fix > in_dim || overflow_rows < 0)
         return DL_ERR_INVALID_ARGUMENT;
@@ -2088,19 +2173,19 @@ extern "C" int dl_logic_backward_chained_lower(const void *x, const int32_t *ver
         const LowerLayer<__half> low = {(const __half *) x_lower, a_lower, b_lower, (const __half *) w_lower,
                                         softmax_backward_lower ? (const __half *) w_lower : nullptr, (__half *) grad_w_lower};
         return backward_chain_t<__half>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, s, 0, &low);
+                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, fp, s, 0, &low);
     }
     case DL_F32: {
         const LowerLayer<float> low = {(const float *) x_lower, a_lower, b_lower, (const float *) w_lower,
                                        softmax_backward_lower ? (const float *) w_lower : nullptr, (float *) grad_w_lower};
         return backward_chain_t<float>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                       overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, s, 0, &low);
+                                       overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, fp, s, 0, &low);
     }
     default: {
         const LowerLayer<double> low = {(const double *) x_lower, a_lower, b_lower, (const double *) w_lower,
                                         softmax_backward_lower ? (const double *) w_lower : nullptr, (double *) grad_w_lower};
         return backward_chain_t<double>(x, verts, neuron, flip, dst, steps, w, grad_y, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, s, 0, &low);
+                                        overflow_rows, grad_w, fix_rows, workspace, in_dim, out_dim, batch, scale, any, fp, s, 0, &low);
     }
     }
 }
@@ -2118,22 +2203,22 @@ extern "C" int dl_logic_forward_chained(const void *x, const int32_t *verts, con
     hipStream_t s = (hipStream_t) stream;
     if (probs) {
         switch (dtype) {
-        case DL_F16: return forward_chain_t<__half, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, batch, any, s, w32);
-        case DL_F32: return forward_chain_t<float, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, batch, any, s);
-        default: return forward_chain_t<double, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, batch, any, s, w32);
+        case DL_F16: return forward_chain_t<__half, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, out_dim, batch, any, s, w32);
+        case DL_F32: return forward_chain_t<float, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, out_dim, batch, any, s);
+        default: return forward_chain_t<double, true>(x, verts, neuron, flip, steps, w, y, probs, in_dim, out_dim, batch, any, s, w32);
         }
     }
     if (argmax) {
         switch (dtype) {
-        case DL_F16: return forward_chain_t<__half, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
-        case DL_F32: return forward_chain_t<float, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s);
-        default: return forward_chain_t<double, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
+        case DL_F16: return forward_chain_t<__half, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, out_dim, batch, any, s, w32);
+        case DL_F32: return forward_chain_t<float, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, out_dim, batch, any, s);
+        default: return forward_chain_t<double, GATES_ARGMAX>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, out_dim, batch, any, s, w32);
         }
     }
     switch (dtype) {
-    case DL_F16: return forward_chain_t<__half, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
-    case DL_F32: return forward_chain_t<float, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s);
-    default: return forward_chain_t<double, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, batch, any, s, w32);
+    case DL_F16: return forward_chain_t<__half, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, out_dim, batch, any, s, w32);
+    case DL_F32: return forward_chain_t<float, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, out_dim, batch, any, s);
+    default: return forward_chain_t<double, false>(x, verts, neuron, flip, steps, w, y, nullptr, in_dim, out_dim, batch, any, s, w32);
     }
 }
 
@@ -2403,6 +2488,7 @@ extern "C" int dl_logic_backward_chained_grouped(const void *x, const int32_t *v
                                                  int64_t out_dim, int64_t batch, int64_t k, double scale, int dtype,
                                                  void *stream) {
     const bool any = takes_any_rows(dtype);
+    const bool fp = takes_fix_positions(dtype);
     const int st = grouped_args(in_dim, out_dim, batch, k, dtype);
     if (st != DL_OK) return st;
     if (steps < out_dim || n_fix < 0 || n_fix > in_dim || overflow_rows < 0) return DL_ERR_INVALID_ARGUMENT;
@@ -2414,13 +2500,13 @@ extern "C" int dl_logic_backward_chained_grouped(const void *x, const int32_t *v
     switch (dtype) {
     case DL_F16:
         return backward_chain_t<__half>(x, verts, neuron, flip, dst, steps, w, grad_cls, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, per_class);
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, fp, s, per_class);
     case DL_F32:
         return backward_chain_t<float>(x, verts, neuron, flip, dst, steps, w, grad_cls, sb, fix_vertex, fix_start, n_fix,
-                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, per_class);
+                                       overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, fp, s, per_class);
     default:
         return backward_chain_t<double>(x, verts, neuron, flip, dst, steps, w, grad_cls, sb, fix_vertex, fix_start, n_fix,
-                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, s, per_class);
+                                        overflow_rows, grad_w, grad_x, workspace, in_dim, out_dim, batch, scale, any, fp, s, per_class);
     }
 }
 

@@ -365,7 +365,7 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
             or w.shape != (grad_y.shape[0], 16)):
         raise RuntimeError(f"expected x [in,B], w [out,16], grad_y [out,B] of one dtype, got {tuple(x.shape)}, "
                            f"{tuple(w.shape)}, {tuple(grad_y.shape)}")
-    code = _layer_code(x, w, "logic_layer_cuda_backward") | (_lib.DL_ROWS_ANY if any_rows else 0)
+    code = _layer_code(x, w, "logic_layer_cuda_backward") | _lib.DL_FIX_POSITIONS | (_lib.DL_ROWS_ANY if any_rows else 0)
     dev = x.device if ready else _same_device(x, w, grad_y)
     in_dim, batch = x.shape
     out_dim = grad_y.shape[0]
@@ -448,7 +448,7 @@ def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_
     for t, n in ((w, "w"), (grad_y, "grad_y"), (x_lower, "x_lower"), (a_lower, "a_lower"), (b_lower, "b_lower"),
                  (w_lower, "w_lower")):
         _check_input(t, n)
-    code = _float_code(grad_y, "logic_layer_cuda_backward") | (_lib.DL_ROWS_ANY if any_rows else 0)
+    code = _float_code(grad_y, "logic_layer_cuda_backward") | _lib.DL_FIX_POSITIONS | (_lib.DL_ROWS_ANY if any_rows else 0)
     dtype = grad_y.dtype
     out_dim, batch = grad_y.shape if grad_y.dim() == 2 else (0, 0)
     in_dim = w_lower.shape[0]
@@ -843,7 +843,7 @@ class EvalSchedule:
     def backward_plan(self):
         """(dst, fix_vertex, fix_start, n_fix, overflow_rows) for backward_chained, built on first
         use: where each schedule position's grad_x row goes and which inputs are summed from
-        several partial rows afterwards.  None where it would have to be built while a graph is being captured
+        several partial rows afterwards (fix_start is followed by the overflow rows' positions).  None where it would have to be built while a graph is being captured
         (building it copies from the host)."""
         if self._backward is None:
             if torch.cuda.is_current_stream_capturing():
@@ -863,8 +863,11 @@ class EvalSchedule:
                 _raise(-rows, "backward_schedule_build")
             n = int(n_fix.value)
             dev = self.verts.device
+            overflow = np.flatnonzero(dst >= self.in_dim)
+            positions = np.empty(int(rows), dtype=np.int32)
+            positions[dst[overflow] - self.in_dim] = overflow                # DL_FIX_POSITIONS
             self._backward = (torch.from_numpy(dst).to(dev), torch.from_numpy(fix_vertex[:n].copy()).to(dev),
-                              torch.from_numpy(fix_start[:n + 1].copy()).to(dev), n, int(rows))
+                              torch.from_numpy(np.concatenate((fix_start[:n + 1], positions))).to(dev), n, int(rows))
         return self._backward
 
 
@@ -1336,7 +1339,7 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
     dev = _same_device(x, a, b, probs, grad_cls)
     lib = _lib.load()
     if want_x and want_w and schedule is not None:
-        chained_code = code | _lib.DL_ROWS_ANY
+        chained_code = code | _lib.DL_ROWS_ANY | _lib.DL_FIX_POSITIONS
         _check_schedule(schedule, in_dim, out_dim, dev)
         plan = schedule.backward_plan()
         if plan is not None and plan[4] <= in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
