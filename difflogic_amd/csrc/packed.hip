@@ -1952,33 +1952,6 @@ extern "C" int dl_tensor_packbits(const uint8_t *t, void *out, int64_t features,
     return dl_launch_status();
 }
 
-// Gate ids of a layer for packed inference: argmax over each neuron's 16 weights, as
-// weights.argmax(-1).to(uint8): the first maximal value wins, a NaN counts as maximal.
-template <typename T, typename C> __device__ __forceinline__ uint32_t argmax16(const T *__restrict__ w) {
-    C best = (C) w[0];
-    uint32_t at = 0;
-    if (best == best) {                                   // not NaN: look on
-#pragma unroll
-        for (int i = 1; i < 16; ++i) {
-            const C v = (C) w[i];
-            if (v != v) {                                 // the first NaN
-                at = i;
-                break;
-            }
-            if (v > best) best = v, at = i;
-        }
-    }
-    return at;
-}
-
-template <typename T, typename C>
-__global__ __launch_bounds__(DL_BLOCK) void gate_ids_kernel(const T *__restrict__ w, uint8_t *__restrict__ ids,
-                                                            int64_t out_dim) {
-    const int64_t n = (int64_t) blockIdx.x * DL_BLOCK + threadIdx.x;
-    if (n >= out_dim) return;
-    ids[n] = (uint8_t) argmax16<T, C>(w + n * 16);
-}
-
 // ------------------------------------------------------------------------------------------
 // One layer straight from its weights, for short rows: argmax gate and gate evaluation in one launch, no records, no
 // schedule, no liveness.  A wave owns 16 neurons: four lanes take the argmax of a neuron's 16 weights (one coalesced
@@ -1995,8 +1968,30 @@ template <typename C> __device__ __forceinline__ void argmax_take(C &v, uint32_t
     const bool tie = (nan && onan) || v == ov;
     if (tie ? oat < at : (onan || (!nan && ov > v))) v = ov, at = oat;
 }
-__device__ __forceinline__ float lane_xor(float v, int m) { return __shfl_xor(v, m, DL_WAVE); }
-__device__ __forceinline__ double lane_xor(double v, int m) { return __shfl_xor(v, m, DL_WAVE); }
+// the value of lane ^ 1 (M = 1) or lane ^ 2 (M = 2), by quad permutation
+template <int M> __device__ __forceinline__ uint32_t quad_xor(uint32_t v) {
+    constexpr int CTRL = M == 1 ? 0xB1 : 0x4E;
+    return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, CTRL, 0xf, 0xf, true);
+}
+template <int M> __device__ __forceinline__ float quad_xor(float v) {
+    return __builtin_bit_cast(float, quad_xor<M>(__builtin_bit_cast(uint32_t, v)));
+}
+template <int M> __device__ __forceinline__ double quad_xor(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(double, ((uint64_t) quad_xor<M>((uint32_t) (u >> 32)) << 32) | quad_xor<M>((uint32_t) u));
+}
+
+// Gate id of a neuron as weights.argmax(-1) has it (the first maximal value wins, a NaN counts as maximal), from four lanes
+// that hold four consecutive weights each; in all four.
+template <typename T, typename C> __device__ __forceinline__ uint32_t argmax_quad(const Weights4<T> &part, int lane) {
+    C best = (C) part.v[0];
+    uint32_t at = 4 * (lane & 3);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) argmax_take<C>(best, at, (C) part.v[i], 4 * (lane & 3) + i);
+    argmax_take<C>(best, at, quad_xor<1>(best), quad_xor<1>(at));
+    argmax_take<C>(best, at, quad_xor<2>(best), quad_xor<2>(at));
+    return at;
+}
 
 template <typename T, typename C, int P>
 __global__ __launch_bounds__(DL_BLOCK) void eval_weights_kernel(const dl_u32x4 *__restrict__ x, const int64_t *__restrict__ a,
@@ -2011,12 +2006,7 @@ __global__ __launch_bounds__(DL_BLOCK) void eval_weights_kernel(const dl_u32x4 *
     // lanes 0 .. 15 hold the neurons' `a`, lanes 16 .. 31 their `b`
     const int64_t ni = n0 + (lane & 15) < out_dim ? n0 + (lane & 15) : out_dim - 1;
     const int32_t idx = (int32_t) ((lane & 16) ? b[ni] : a[ni]);
-    C best = (C) part.v[0];
-    uint32_t at = 4 * (lane & 3);
-#pragma unroll
-    for (int i = 1; i < 4; ++i) argmax_take<C>(best, at, (C) part.v[i], 4 * (lane & 3) + i);
-#pragma unroll
-    for (int m = 1; m < 4; m <<= 1) argmax_take<C>(best, at, lane_xor(best, m), (uint32_t) __shfl_xor((int) at, m, DL_WAVE));
+    const uint32_t at = argmax_quad<T, C>(part, lane);
 
     constexpr int PER = DL_WAVE / P;                                     // neurons side by side
     constexpr int PASSES = 16 / PER > 0 ? 16 / PER : 1;
@@ -2073,20 +2063,30 @@ __device__ __forceinline__ uint32_t fold_gate(uint32_t op, uint32_t sa, uint32_t
     return op;
 }
 
-// gate_ids_kernel and fold_gate_constants_kernel in one: the argmax gate with the constants among the layer's input
-// rows folded in, and which of the layer's own outputs are constant
-template <typename T, typename C>
-__global__ __launch_bounds__(DL_BLOCK) void gate_ids_folded_kernel(const T *__restrict__ w, const int64_t *__restrict__ a,
-                                                                   const int64_t *__restrict__ b,
-                                                                   const uint8_t *__restrict__ state_in,
-                                                                   uint8_t *__restrict__ ids, uint8_t *__restrict__ state_out,
-                                                                   int64_t out_dim) {
-    const int64_t n = (int64_t) blockIdx.x * DL_BLOCK + threadIdx.x;
-    if (n >= out_dim) return;
-    const uint32_t sa = state_in ? state_in[a[n]] : 0u, sb = state_in ? state_in[b[n]] : 0u;
-    const uint32_t op = fold_gate(argmax16<T, C>(w + n * 16), sa, sb);
-    ids[n] = (uint8_t) op;
-    state_out[n] = op == 0u ? 1 : op == 15u ? 2 : 0;
+// Gate ids of a layer for packed inference.  Four lanes take a neuron's 16 weights, so a wave reads a contiguous kilobyte (fp32)
+// at once; one lane per neuron read 64 bytes of 64 lines four times.  With `a`: the constants among the layer's input rows
+// are folded in (state_in: 1 all zeros, 2 all ones, 0 varies; null: all vary), and state_out says which of the layer's own
+// outputs are constant.  Bound by latency: 64000 neurons (5 MB) N.N us, launch included, N.N before; 128000 N.N, N.N before.
+template <typename T, typename C, bool FOLD>
+__global__ __launch_bounds__(DL_BLOCK) void gate_ids_kernel(const T *__restrict__ w, const int64_t *__restrict__ a,
+                                                            const int64_t *__restrict__ b, const uint8_t *__restrict__ state_in,
+                                                            uint8_t *__restrict__ ids, uint8_t *__restrict__ state_out,
+                                                            int64_t out_dim) {
+    const int lane = dl_lane();
+    const int64_t n = ((int64_t) blockIdx.x * DL_BLOCK + threadIdx.x) >> 2;
+    const int64_t nw = n < out_dim ? n : out_dim - 1;                      // (whole quads: the permutations need their lanes)
+    const Weights4<T> part = *reinterpret_cast<const Weights4<T> *>(w + nw * 16 + 4 * (lane & 3));
+    uint32_t state = 0;                                                    // of `a` in the even lanes, of `b` in the odd ones
+    if (FOLD && state_in != nullptr) state = state_in[(lane & 1) ? b[nw] : a[nw]];
+    uint32_t op = argmax_quad<T, C>(part, lane);
+    const uint32_t other = quad_xor<1>(state);
+    if ((lane & 3) == 0 && n < out_dim) {
+        if (FOLD) {
+            op = fold_gate(op, state, other);
+            state_out[n] = op == 0u ? 1 : op == 15u ? 2 : 0;
+        }
+        ids[n] = (uint8_t) op;
+    }
 }
 
 template <typename T, typename C>
@@ -2124,19 +2124,30 @@ extern "C" int dl_logic_eval_weights(const void *x, const int64_t *a, const int6
     return dl_launch_status();
 }
 
+template <bool FOLD>
+static int launch_gate_ids(const void *w, int dtype, const int64_t *a, const int64_t *b, const uint8_t *state_in, uint8_t *ids,
+                           uint8_t *state_out, int64_t out_dim, hipStream_t s) {
+    constexpr int64_t MOST = 1LL << 29;              // neurons of a launch, whose threads HIP counts in 32 bits
+    for (int64_t n = 0; n < out_dim; n += MOST) {
+        const int64_t count = out_dim - n < MOST ? out_dim - n : MOST;
+        const dim3 grid((unsigned) dl_ceil_div(count, DL_BLOCK / 4)), block(DL_BLOCK);
+#define DL_LAUNCH_GATE_IDS(T, C)                                                                                          \
+    DL_LAUNCH((gate_ids_kernel<T, C, FOLD>), grid, block, 0, s, (const T *) w + n * 16, FOLD ? a + n : a, FOLD ? b + n : b, \
+              state_in, ids + n, FOLD ? state_out + n : state_out, count)
+        if (dtype == DL_F16) DL_LAUNCH_GATE_IDS(__half, float);
+        else if (dtype == DL_F32) DL_LAUNCH_GATE_IDS(float, float);
+        else DL_LAUNCH_GATE_IDS(double, double);
+#undef DL_LAUNCH_GATE_IDS
+    }
+    return dl_launch_status();
+}
+
 extern "C" int dl_gate_ids(const void *w, uint8_t *ids, int64_t out_dim, int dtype, void *stream) {
     if (dtype != DL_F16 && dtype != DL_F32 && dtype != DL_F64) return DL_ERR_DTYPE;
     if (out_dim < 0) return DL_ERR_INVALID_ARGUMENT;
     if (out_dim == 0) return DL_OK;
     if (!w || !ids) return DL_ERR_INVALID_ARGUMENT;
-    const int64_t blocks = dl_ceil_div(out_dim, DL_BLOCK);
-    if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-    hipStream_t s = (hipStream_t) stream;
-    const dim3 grid((unsigned) blocks), block(DL_BLOCK);
-    if (dtype == DL_F16) DL_LAUNCH((gate_ids_kernel<__half, float>), grid, block, 0, s, (const __half *) w, ids, out_dim);
-    else if (dtype == DL_F32) DL_LAUNCH((gate_ids_kernel<float, float>), grid, block, 0, s, (const float *) w, ids, out_dim);
-    else DL_LAUNCH((gate_ids_kernel<double, double>), grid, block, 0, s, (const double *) w, ids, out_dim);
-    return dl_launch_status();
+    return launch_gate_ids<false>(w, dtype, nullptr, nullptr, nullptr, ids, nullptr, out_dim, (hipStream_t) stream);
 }
 
 extern "C" int dl_gate_ids_folded(const void *w, int dtype, const int64_t *a, const int64_t *b, const uint8_t *state_in,
@@ -2145,20 +2156,7 @@ extern "C" int dl_gate_ids_folded(const void *w, int dtype, const int64_t *a, co
     if (out_dim < 0) return DL_ERR_INVALID_ARGUMENT;
     if (out_dim == 0) return DL_OK;
     if (!w || !a || !b || !ids || !state_out) return DL_ERR_INVALID_ARGUMENT;
-    const int64_t blocks = dl_ceil_div(out_dim, DL_BLOCK);
-    if (blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
-    hipStream_t s = (hipStream_t) stream;
-    const dim3 grid((unsigned) blocks), block(DL_BLOCK);
-    if (dtype == DL_F16)
-        DL_LAUNCH((gate_ids_folded_kernel<__half, float>), grid, block, 0, s, (const __half *) w, a, b, state_in, ids, state_out,
-                  out_dim);
-    else if (dtype == DL_F32)
-        DL_LAUNCH((gate_ids_folded_kernel<float, float>), grid, block, 0, s, (const float *) w, a, b, state_in, ids, state_out,
-                  out_dim);
-    else
-        DL_LAUNCH((gate_ids_folded_kernel<double, double>), grid, block, 0, s, (const double *) w, a, b, state_in, ids,
-                  state_out, out_dim);
-    return dl_launch_status();
+    return launch_gate_ids<true>(w, dtype, a, b, state_in, ids, state_out, out_dim, (hipStream_t) stream);
 }
 
 // Constants folded into the gates above them.  A neuron whose gate is constant (ids 0 and 15), or becomes so
