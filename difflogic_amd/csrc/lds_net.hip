@@ -128,8 +128,8 @@ __global__ __launch_bounds__(DL_BLOCK) void compose_net_kernel(NetWiring t, uint
 // ------------------------------------------------------------------------------------------
 struct ThinTables {
     uint8_t *folded[DL_NET_MAX_DEPTH];          // gate ids of layer l with the constants below folded in
-    uint8_t *live[DL_NET_MAX_DEPTH];            // hidden layer l: neuron n is looked at (the last layer: null)
-    int32_t *rank[DL_NET_MAX_DEPTH];            // rank of neuron n among the neurons left (of its class, in the last layer)
+    uint32_t *left;                             // [depth + 1][DL_NET_MASK_WORDS]: bit n = neuron n of layer l is left; then
+                                                // the constant ones of the last layer
     int32_t *thin;
     int32_t k;
 };
@@ -137,11 +137,11 @@ struct ThinTables {
 __device__ __forceinline__ bool net_gate_uses_a(uint32_t op) { return (((op >> 3) ^ (op >> 1)) & 1u) || (((op >> 2) ^ op) & 1u); }
 __device__ __forceinline__ bool net_gate_uses_b(uint32_t op) { return (((op >> 3) ^ (op >> 2)) & 1u) || (((op >> 1) ^ op) & 1u); }
 
-#define DL_NET_RANK_ITEMS (DL_NET_MAX_WIDTH / DL_NET_THREADS)        // consecutive neurons per thread
+#define DL_NET_RANK_ITEMS (DL_NET_MAX_WIDTH / DL_NET_THREADS)        // neurons per thread
+#define DL_NET_MASK_WORDS (DL_NET_MAX_WIDTH / 32)
 
-// Gate ids of layer l with the constants of the layer below folded in (launched layer by layer, upwards); clears
-// the layer's marks.  Gate ids are (f(0,0) f(0,1) f(1,0) f(1,1)), most significant bit first.
-__global__ __launch_bounds__(DL_BLOCK) void net_thin_fold_kernel(NetWiring t, ThinTables thin, int l, int depth) {
+// Gate ids of layer l with the constants of the layer below folded in (launched layer by layer, upwards).  Gate ids are (f(0,0) f(0,1) f(1,0) f(1,1)), most significant bit first.
+__global__ __launch_bounds__(DL_BLOCK) void net_thin_fold_kernel(NetWiring t, ThinTables thin, int l) {
     const int n = (int) (blockIdx.x * DL_BLOCK + threadIdx.x);
     if (n >= t.width[l]) return;
     uint32_t op = t.w[l][n] & 15u;
@@ -157,116 +157,138 @@ __global__ __launch_bounds__(DL_BLOCK) void net_thin_fold_kernel(NetWiring t, Th
         }
     }
     thin.folded[l][n] = (uint8_t) op;
-    if (l + 1 < depth) thin.live[l][n] = 0;
 }
 
-// Where the caller's gate ids are folded already: only the marks of the hidden layers are cleared (in one launch;
-// `marks` is the first layer's, the others follow it, `total` bytes in all).
-__global__ __launch_bounds__(DL_BLOCK) void net_thin_clear_kernel(uint8_t *__restrict__ marks, int64_t total) {
-    const int64_t i = (int64_t) blockIdx.x * DL_BLOCK + threadIdx.x;
-    if (i < total) marks[i] = 0;
+// A barrier for what is in LDS alone: global loads and stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Marks the neurons of layer l - 1 that a neuron of layer l which is itself looked at (the last layer: every neuron)
-// looks at (launched layer by layer, downwards).  A constant neuron marks nothing and, its readers having been
-// folded, is marked by nobody.
-__global__ __launch_bounds__(DL_BLOCK) void net_thin_mark_kernel(NetWiring t, ThinTables thin, int l, int depth) {
-    const int n = (int) (blockIdx.x * DL_BLOCK + threadIdx.x);
-    if (n >= t.width[l] || (l + 1 < depth && !thin.live[l][n])) return;
-    const uint32_t op = thin.folded[l][n];
-    if (net_gate_uses_a(op)) thin.live[l - 1][t.a[l][n]] = 1;
-    if (net_gate_uses_b(op)) thin.live[l - 1][t.b[l][n]] = 1;
-}
+// Which neurons are left, for the whole net in one launch of one workgroup that walks the layers downwards: a neuron that is
+// left marks the ones that its gate looks at (a constant neuron marks nothing and, its readers having been folded, is
+// marked by nobody).  The marks of two layers take turns in LDS, one barrier a layer; the next layer's wiring is requested
+// before this one marks.  Bound by what one CU gets through: 24 us for six layers of 8000, where a launch per layer, one that
+// cleared the marks and one for the ranks took 35 (784 -> 6 x 8000 at batch 12000: 132 -> 87 us a call, replayed 71 -> 66).
+// With ranks and records in it as well the workgroup took 43.  Neuron n of a layer belongs to thread n % 1024, so a ballot is a word of the masks.
+__global__ __launch_bounds__(DL_NET_THREADS) void net_thin_mark_kernel(NetWiring t, ThinTables thin, int depth) {
+    constexpr int ITEMS = DL_NET_RANK_ITEMS, WAVES = DL_NET_THREADS / DL_WAVE;
+    static_assert(DL_NET_MAX_WIDTH + DL_NET_THREADS <= 1 << DL_NET_ID_BITS, "neurons and the threads' idle marks");
+    __shared__ uint8_t marks[2][1 << DL_NET_ID_BITS];
+    const int tid = (int) threadIdx.x, lane = dl_lane(), wave = dl_wave_in_block();
+    for (int i = tid; i < (int) sizeof(marks) / 4; i += DL_NET_THREADS) reinterpret_cast<uint32_t *>(marks)[i] = 0;
 
-// blockIdx.x = layer: exclusive prefix sums of "this neuron is left" over the layer's neurons.  One scan carries two
-// counts: the neurons left in the low half of the word and, in the last layer, the constant-one neurons in the high
-// half (neither exceeds DL_NET_MAX_WIDTH < 2^16, and both only grow along the layer, so differences of two scan
-// values are the differences of the halves).
-__global__ __launch_bounds__(DL_NET_THREADS) void net_thin_rank_kernel(NetWiring t, ThinTables thin, int depth) {
-    static_assert(DL_NET_MAX_WIDTH < (1 << 16), "two counts per word");
-    __shared__ int32_t wave_total[DL_NET_THREADS / DL_WAVE];
-    __shared__ int32_t class_at[DL_NET_MAX_WIDTH + 1];       // last layer: the scan at each class's first neuron, then the total
-    const int l = blockIdx.x, tid = (int) threadIdx.x, lane = dl_lane(), wave = dl_wave_in_block();
-    const int width = t.width[l];
-    const bool last = l == depth - 1;
-    const uint8_t *flag_src = last ? thin.folded[l] : thin.live[l];
-    int32_t local[DL_NET_RANK_ITEMS], sum = 0;
+    struct Raw { uint32_t a[ITEMS], b[ITEMS], w[ITEMS]; };
+    auto load = [&](int l, Raw &r) {                         // (neuron numbers are below 2^14: the low halves)
+        const int width = t.width[l];
 #pragma unroll
-    for (int i = 0; i < DL_NET_RANK_ITEMS; ++i) {
-        const int n = tid * DL_NET_RANK_ITEMS + i;
-        int32_t f = 0;
-        if (n < width) {
-            const uint32_t v = flag_src[n];
-            f = last ? (int32_t) (v != 0u && v != 15u) | ((int32_t) (v == 15u) << 16) : (int32_t) (v != 0u);
+        for (int i = 0; i < ITEMS; ++i) {
+            const int n = i * DL_NET_THREADS + tid, at = n < width ? n : 0;
+            r.a[i] = reinterpret_cast<const uint32_t *>(t.a[l])[2 * at];
+            r.b[i] = reinterpret_cast<const uint32_t *>(t.b[l])[2 * at];
+            r.w[i] = thin.folded[l][at];
         }
-        local[i] = sum;
-        sum += f;
-    }
-    int32_t incl = sum;                                      // inclusive scan of the threads' sums within the wave
+    };
+    auto store_mask = [&](int row, int i, bool flag) {
+        const uint64_t m = __ballot(flag);
+        if (lane < 2) thin.left[row * DL_NET_MASK_WORDS + (i * WAVES + wave) * 2 + lane] = (uint32_t) (m >> (32 * lane));
+    };
+    Raw cur;
+    load(depth - 1, cur);
+    uint32_t left = 0;                                       // bit i: the thread's i-th neuron is left
 #pragma unroll
-    for (int off = 1; off < DL_WAVE; off <<= 1) {
-        const int32_t up = __shfl_up(incl, off, DL_WAVE);
-        if (lane >= off) incl += up;
+    for (int i = 0; i < ITEMS; ++i) {
+        const bool there = i * DL_NET_THREADS + tid < t.width[depth - 1];
+        const bool varies = there && cur.w[i] != 0u && cur.w[i] != 15u;
+        if (varies) left |= 1u << i;
+        store_mask(depth - 1, i, varies);
+        store_mask(depth, i, there && cur.w[i] == 15u);
     }
-    if (lane == DL_WAVE - 1) wave_total[wave] = incl;
-    __syncthreads();
-    int32_t before = 0, total = 0;
-    for (int w = 0; w < DL_NET_THREADS / DL_WAVE; ++w) {
-        if (w < wave) before += wave_total[w];
-        total += wave_total[w];
-    }
-    const int32_t mine = before + incl - sum;                // the scan before this thread's first neuron
-    int32_t *rank = thin.rank[l];
-    if (!last) {
+    lds_barrier();
+#pragma unroll 1
+    for (int l = depth - 1; l > 0; --l) {
+        Raw next;
+        load(l - 1, next);
+        uint8_t *const mark = marks[l & 1];
+        constexpr uint32_t ID = (1u << DL_NET_ID_BITS) - 1;
 #pragma unroll
-        for (int i = 0; i < DL_NET_RANK_ITEMS; ++i) {
-            const int n = tid * DL_NET_RANK_ITEMS + i;
-            if (n < width) rank[n] = mine + local[i];
+        for (int i = 0; i < ITEMS; ++i) {
+            // (what marks nothing writes past the widest layer: no branches)
+            const bool is = (left >> i) & 1u;
+            mark[is && net_gate_uses_a(cur.w[i]) ? cur.a[i] & ID : (uint32_t) (DL_NET_MAX_WIDTH + tid)] = 1;
+            mark[is && net_gate_uses_b(cur.w[i]) ? cur.b[i] & ID : (uint32_t) (DL_NET_MAX_WIDTH + tid)] = 1;
         }
-        if (tid == 0) thin.thin[l] = total;
-        return;
-    }
-    // the last layer: ranks within each class, the classes' numbers of neurons left and of constant ones
-    const int per_class = width / thin.k;
+        lds_barrier();
+        left = 0;
 #pragma unroll
-    for (int i = 0; i < DL_NET_RANK_ITEMS; ++i) {
-        const int n = tid * DL_NET_RANK_ITEMS + i;
-        if (n < width && n % per_class == 0) class_at[n / per_class] = mine + local[i];
-    }
-    if (tid == 0) class_at[thin.k] = total;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < DL_NET_RANK_ITEMS; ++i) {
-        const int n = tid * DL_NET_RANK_ITEMS + i;
-        if (n < width) rank[n] = ((mine + local[i]) & 0xffff) - (class_at[n / per_class] & 0xffff);
-    }
-    for (int c = tid; c < thin.k; c += DL_NET_THREADS) {
-        const int32_t d = class_at[c + 1] - class_at[c];
-        thin.thin[depth - 1 + c] = d & 0xffff;
-        thin.thin[depth - 1 + thin.k + c] = d >> 16;
+        for (int i = 0; i < ITEMS; ++i) {
+            const int n = i * DL_NET_THREADS + tid;
+            const bool live = n < t.width[l - 1] && mark[n] != 0;
+            if (live) left |= 1u << i;
+            store_mask(l - 1, i, live);
+            mark[n] = 0;                                     // for the layer after next, a barrier away
+        }
+        cur = next;
     }
 }
 
-// records of the neurons left (layer blockIdx.y): a | b << 14 | gate << 28 at the neuron's rank, the inputs' rows being
-// the ranks of the layer below (an input that the gate does not look at: row 0)
+// Records of the neurons left (layer blockIdx.y): a | b << 14 | gate << 28 at the neuron's rank among those left (of its
+// class, in the last layer), the inputs' rows being the ranks of the layer below (an input that the gate does not look at:
+// row 0); and the numbers of neurons left.  A rank is the count of the mask's words below, scanned by a wave per mask, and
+// of the bits below in the neuron's own word.
 __global__ __launch_bounds__(DL_BLOCK) void compose_net_thin_kernel(NetWiring t, ThinTables thin, int depth,
                                                                     uint32_t *__restrict__ rec) {
-    const int l = blockIdx.y;
+    __shared__ uint32_t mask[3][DL_NET_MASK_WORDS], before[3][DL_NET_MASK_WORDS + 1];     // own layer, layer below, constant ones
+    const int l = blockIdx.y, width = t.width[l], lane = dl_lane(), wave = dl_wave_in_block();
+    const bool last = l == depth - 1;
     const int n = (int) (blockIdx.x * DL_BLOCK + threadIdx.x);
-    if (n >= t.width[l]) return;
-    const uint32_t gate = thin.folded[l][n];
-    int64_t at;
-    if (l < depth - 1) {
-        if (!thin.live[l][n]) return;
-        at = thin.rank[l][n];
-    } else {
-        if (gate == 0u || gate == 15u) return;
-        const int per_class = t.width[l] / thin.k;
-        at = (int64_t) (n / per_class) * per_class + thin.rank[l][n];
+    if ((int) (blockIdx.x * DL_BLOCK) >= width) return;
+    const int at = n < width ? n : 0;
+    const uint32_t gate = thin.folded[l][at], a = (uint32_t) t.a[l][at], b = (uint32_t) t.b[l][at];
+    const int row = wave == 0 ? l : wave == 1 ? (l > 0 ? l - 1 : -1) : wave == 2 && last ? depth : -1;
+    if (row >= 0) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (int w0 = 0; w0 < DL_NET_MASK_WORDS; w0 += DL_WAVE) {
+            const uint32_t m = thin.left[row * DL_NET_MASK_WORDS + w0 + lane];
+            uint32_t v = (uint32_t) __popc(m);
+            const uint32_t own = v;
+#pragma unroll
+            for (int off = 1; off < DL_WAVE; off <<= 1) {
+                const uint32_t up = __shfl_up(v, off, DL_WAVE);
+                if (lane >= off) v += up;
+            }
+            mask[wave][w0 + lane] = m;
+            before[wave][w0 + lane] = sum + v - own;
+            sum += (uint32_t) __builtin_amdgcn_readlane((int) v, DL_WAVE - 1);
+        }
+        if (lane == 0) before[wave][DL_NET_MASK_WORDS] = sum;
     }
-    auto row = [&](int64_t v) -> uint32_t { return (uint32_t) (l == 0 ? v + t.in_base : thin.rank[l - 1][v]); };
-    const uint32_t ra = net_gate_uses_a(gate) ? row(t.a[l][n]) : 0u, rb = net_gate_uses_b(gate) ? row(t.b[l][n]) : 0u;
-    rec[t.offset[l] + at] = ra | (rb << DL_NET_ID_BITS) | (gate << (2 * DL_NET_ID_BITS));
+    __syncthreads();
+    auto rank = [&](int which, uint32_t v) -> uint32_t {     // (v: up to DL_NET_MAX_WIDTH)
+        const uint32_t word = v >> 5;
+        return before[which][word] + (word < DL_NET_MASK_WORDS ? (uint32_t) __popc(mask[which][word] & ((1u << (v & 31u)) - 1u)) : 0u);
+    };
+    const int per_class = last ? width / thin.k : 1;
+    if (blockIdx.x == 0) {
+        if (!last && threadIdx.x == 0) thin.thin[l] = (int32_t) before[0][DL_NET_MASK_WORDS];
+        if (last)
+            for (int c = (int) threadIdx.x; c < thin.k; c += DL_BLOCK) {
+                const uint32_t c0 = (uint32_t) (c * per_class), c1 = c0 + (uint32_t) per_class;
+                thin.thin[depth - 1 + c] = (int32_t) (rank(0, c1) - rank(0, c0));
+                thin.thin[depth - 1 + thin.k + c] = (int32_t) (rank(2, c1) - rank(2, c0));
+            }
+    }
+    if (n >= width || !((mask[0][n >> 5] >> (n & 31)) & 1u)) return;
+    uint32_t place = rank(0, (uint32_t) n);
+    if (last) {
+        const uint32_t c0 = (uint32_t) (n / per_class) * (uint32_t) per_class;
+        place += c0 - rank(0, c0);
+    }
+    auto input = [&](uint32_t v) { return l == 0 ? v + (uint32_t) t.in_base : rank(1, v); };
+    const uint32_t ra = net_gate_uses_a(gate) ? input(a) : 0u, rb = net_gate_uses_b(gate) ? input(b) : 0u;
+    rec[t.offset[l] + place] = ra | (rb << DL_NET_ID_BITS) | (gate << (2 * DL_NET_ID_BITS));
 }
 
 // COLS 64-bit words as 2 * COLS dwords
@@ -743,8 +765,8 @@ extern "C" int64_t dl_logic_net_lds_workspace_bytes(int depth, const int64_t *di
     if (depth < 1 || depth > DL_NET_MAX_DEPTH || !dims) return 0;
     // per layer: the records (9 per chunk of a schedule of at most width + width / 4 + 32 steps, chunks
     // rounded up to whole waves) and width row ids
-    // (thinned: a record, a rank, a folded gate id and a mark per neuron = 10 bytes, and three numbers per layer /
-    // class: fits the same bound with the last term, k <= dims[depth])
+    // (thinned: a record and a folded gate id per neuron = 5 bytes, a mask of 1280 bytes per layer and one more, and three
+    // numbers per layer / class: fits the same bound with the last term, k <= dims[depth])
     int64_t bytes = 0;
     for (int l = 1; l <= depth; ++l) {
         const int64_t w = dims[l] > 0 ? dims[l] : 0;
@@ -850,39 +872,23 @@ static int net_lds_run(const void *x, bool bool_input, int64_t batch, int depth,
     const int32_t *thin = nullptr;
     int st;
     if (thinned) {
-        // ranks follow the records, then the numbers of neurons left, the folded gate ids and the marks
+        // the numbers of neurons left follow the records, then the masks of those left and the folded gate ids
         ThinTables th;
-        int32_t *rank = (int32_t *) workspace + offset;
-        for (int l = 0; l < DL_NET_MAX_DEPTH; ++l) th.folded[l] = th.live[l] = nullptr, th.rank[l] = nullptr;
-        for (int l = 0; l < depth; ++l) {
-            th.rank[l] = rank;
-            rank += dims[l + 1];
-        }
-        th.thin = rank;
+        for (int l = 0; l < DL_NET_MAX_DEPTH; ++l) th.folded[l] = nullptr;
+        th.thin = (int32_t *) workspace + offset;
         th.k = (int32_t) k;
-        uint8_t *bytes = (uint8_t *) (rank + depth + 2 * k);
-        uint8_t *marks = bytes;                                  // the hidden layers' marks, one after the other
-        int64_t nmarks = 0;
-        for (int l = 0; l + 1 < depth; ++l) th.live[l] = bytes, bytes += dims[l + 1], nmarks += dims[l + 1];
+        th.left = (uint32_t *) (th.thin + depth + 2 * k);
+        uint8_t *bytes = (uint8_t *) (th.left + (depth + 1) * DL_NET_MASK_WORDS);
         for (int l = 0; l < depth; ++l) {
             // (folded already: the caller's gate ids are read where the folded ones would be; nothing writes them)
             if (folded) th.folded[l] = const_cast<uint8_t *>(w[l]);
             else th.folded[l] = bytes, bytes += dims[l + 1];
         }
         if ((char *) bytes - (char *) workspace > dl_logic_net_lds_workspace_bytes(depth, dims)) return DL_ERR_INVALID_ARGUMENT;
-        if (folded) {
-            if (nmarks > 0) DL_LAUNCH(net_thin_clear_kernel, dim3((unsigned) dl_ceil_div(nmarks, DL_BLOCK)), dim3(DL_BLOCK), 0, s, marks, nmarks);
-        } else {
+        if (!folded)
             for (int l = 0; l < depth; ++l)
-                DL_LAUNCH(net_thin_fold_kernel, dim3((unsigned) dl_ceil_div(dims[l + 1], DL_BLOCK)), dim3(DL_BLOCK), 0, s, wiring, th,
-                          l, depth);
-        }
-        for (int l = depth - 1; l >= 1; --l)
-            DL_LAUNCH(net_thin_mark_kernel, dim3((unsigned) dl_ceil_div(dims[l + 1], DL_BLOCK)), dim3(DL_BLOCK), 0, s, wiring, th, l,
-                      depth);
-        DL_LAUNCH(net_thin_rank_kernel, dim3((unsigned) depth), dim3(DL_NET_THREADS), 0, s, wiring, th, depth);
-        st = dl_launch_status();
-        if (st != DL_OK) return st;
+                DL_LAUNCH(net_thin_fold_kernel, dim3((unsigned) dl_ceil_div(dims[l + 1], DL_BLOCK)), dim3(DL_BLOCK), 0, s, wiring, th, l);
+        DL_LAUNCH(net_thin_mark_kernel, dim3(1), dim3(DL_NET_THREADS), 0, s, wiring, th, depth);
         DL_LAUNCH(compose_net_thin_kernel, dim3((unsigned) dl_ceil_div(entries, DL_BLOCK), (unsigned) depth), dim3(DL_BLOCK), 0, s,
                   wiring, th, depth, rec);
         thin = th.thin;
