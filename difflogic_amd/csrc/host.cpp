@@ -184,6 +184,33 @@ c10::optional<Tensor> train_layer(const Tensor &x, const Tensor &weights, const 
         .transpose(0, 1);
 }
 
+// A layer in eval mode on float x [B, in] (LogicLayer.forward_cuda): all of each neuron's argmax gate, no gradients.
+// `tables`: verts, neuron and flip of the schedule that the kernel walks, or none.
+c10::optional<Tensor> eval_layer(const Tensor &x, const Tensor &weights, const Tensor &a, const Tensor &b,
+                                 const std::vector<Tensor> &tables, int64_t steps, int64_t in_dim) {
+    const int code = layer_args(x, weights, a, b);
+    if (code < 0 || x.size(1) != in_dim || (!tables.empty() && tables.size() != 3)) return c10::nullopt;
+    for (size_t i = 0; i < tables.size(); ++i)
+        if (tables[i].scalar_type() != (i == 2 ? at::kByte : at::kInt) || tables[i].numel() != steps + (i == 0)
+            || !plain(tables[i], x.get_device()))
+            return c10::nullopt;
+    const at::NoGradGuard no_grad;
+    const c10::DeviceGuard guard(x.device());
+    const Tensor xt = x.transpose(0, 1).contiguous();
+    const int64_t out_dim = weights.size(0), batch = xt.size(1);
+    Tensor y = at::empty({out_dim, batch}, xt.options());
+    int st = DL_ERR_TOO_LARGE;
+    if (!tables.empty())
+        st = dl_logic_forward_chained(xt.const_data_ptr(), tables[0].const_data_ptr<int32_t>(), tables[1].const_data_ptr<int32_t>(),
+                                      tables[2].const_data_ptr<uint8_t>(), steps, weights.const_data_ptr(), y.mutable_data_ptr(),
+                                      nullptr, in_dim, out_dim, batch, code | DL_GATES_OF_ARGMAX | DL_ROWS_ANY, stream_of(xt));
+    if (st == DL_ERR_TOO_LARGE)
+        st = dl_logic_forward(xt.const_data_ptr(), a.const_data_ptr<int64_t>(), b.const_data_ptr<int64_t>(), weights.const_data_ptr(),
+                              y.mutable_data_ptr(), in_dim, out_dim, batch, code | DL_GATES_OF_ARGMAX, stream_of(xt));
+    check(st, "logic_layer_cuda_forward");
+    return y.transpose(0, 1);
+}
+
 // difflogic_cuda.forward_logits without a schedule.
 c10::optional<std::tuple<Tensor, Tensor>> forward_logits(const Tensor &x, const Tensor &a, const Tensor &b, const Tensor &logits) {
     const int code = layer_args(x, logits, a, b);
@@ -351,6 +378,7 @@ c10::optional<Tensor> count_rows(const Tensor &b, int64_t pad, int64_t k) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     typedef py::call_guard<py::gil_scoped_release> unlocked;
     m.def("train_layer", &train_layer, unlocked());
+    m.def("eval_layer", &eval_layer, unlocked());
     m.def("forward_logits", &forward_logits, unlocked());
     m.def("backward_both", &backward_both, unlocked());
     m.def("backward_logits", &backward_logits, unlocked());

@@ -116,6 +116,17 @@ class LogicLayer(torch.nn.Module):
                         return y
             assert x.device.type == "cuda", x.device
         assert x.ndim == 2, x.ndim
+        if (not self.training and type(x) is torch.Tensor and type(self.weights) in _PLAIN and x.is_cuda
+                and x.shape[1] == self.in_dim and torch._C._get_tracing_state() is None):
+            # the discretised net on float inputs in one native call
+            xt = x.transpose(0, 1)
+            schedule = None if self.in_dim < self._CHAIN_MIN_IN_DIM else _forward_walk(self._train_schedule(xt), self.out_dim, xt)
+            tables = [] if schedule is None else [schedule.verts, schedule.neuron, schedule.flip]
+            y = _host.eval_layer(x, self.weights, *self.indices, tables, 0 if schedule is None else schedule.steps, self.in_dim)
+            if y is not None:
+                if not self._evaluated:
+                    self._evaluated = True
+                return y
         x = x.transpose(0, 1).contiguous()                  # feature-major [in, B]
         assert x.shape[0] == self.in_dim, (x.shape, self.in_dim)
         a, b = self.indices
