@@ -39,6 +39,20 @@ bool index_of(const Tensor &t, c10::DeviceIndex device, int64_t numel) {
     return t.scalar_type() == at::kLong && t.dim() == 1 && t.size(0) == numel && plain(t, device);
 }
 
+// Saved tensors may have been through a caller's hooks: [x, a, b, probabilities, start, idx] for each layer, as they were saved.
+void check_saved(const variable_list &saved) {
+    for (size_t i = 0; i + 5 < saved.size(); i += 6) {
+        const Tensor &x = saved[i], &probs = saved[i + 3];
+        TORCH_CHECK(x.is_cuda() && x.dim() == 2 && probs.dim() == 2 && probs.size(1) == 16, "saved tensors changed");
+        const c10::DeviceIndex device = x.get_device();
+        const int64_t in_dim = x.size(0), out_dim = probs.size(0);
+        TORCH_CHECK(plain(x, device) && plain(probs, device) && index_of(saved[i + 1], device, out_dim)
+                        && index_of(saved[i + 2], device, out_dim) && index_of(saved[i + 4], device, in_dim + 1)
+                        && index_of(saved[i + 5], device, 2 * out_dim),
+                    "saved tensors have to come back as they were: contiguous and on their device");
+    }
+}
+
 // A layer's walk along its evaluation schedule: difflogic_cuda.EvalSchedule and the plan of its one-pass backward
 // ([verts, neuron, flip, dst, fix_vertex, fix_start]; none: the layer has no schedule), and which of the kernels take it.
 struct Walk {
@@ -105,6 +119,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
 
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
+        check_saved(saved);
         const Tensor &x = saved[0], &a = saved[1], &b = saved[2], &probs = saved[3], &start = saved[4], &idx = saved[5];
         const double scale = ctx->saved_data["scale"].toDouble();
         const int code = (int) ctx->saved_data["code"].toInt();
@@ -299,6 +314,142 @@ struct GroupSumFunction : torch::autograd::Function<GroupSumFunction> {
     }
 };
 
+// LogicNetFunction's work for layers without schedules: all of a net's layers and its GroupSum, each way.  fused: the last layer and
+// the GroupSum in one kernel each way (LogicLayerGroupSumFunction).
+struct Net {
+    std::vector<Tensor> a, b, start, idx;
+    std::vector<double> scale;
+    std::vector<int64_t> code;
+    int64_t k = 0;
+    double tau = 1.0;
+    bool fused = false;
+};
+
+// Forward: (scores [B, k], what the backward pass needs: six tensors a layer).
+std::tuple<Tensor, variable_list> net_forward_of(const Tensor &x, const variable_list &weights, const Net *net) {
+    const size_t layers = net->a.size();
+    variable_list saved;
+    saved.reserve(6 * layers);
+    Tensor cur = x;
+    for (size_t l = 0; l < layers; ++l) {
+        const Tensor w = weights[l].detach(), probs = at::empty_like(w);
+        saved.insert(saved.end(), {cur, net->a[l], net->b[l], probs, net->start[l], net->idx[l]});
+        if (l + 1 < layers || !net->fused) {
+            cur = forward_into(cur, net->a[l], net->b[l], w, probs, (int) net->code[l], Walk());
+            continue;
+        }
+        const int code = (int) net->code[l];
+        const int64_t out_dim = w.size(0), batch = cur.size(1);
+        Tensor y = at::empty({batch, net->k}, cur.options());
+        const int64_t bytes = dl_group_sum_workspace_bytes(out_dim, batch, net->k, code);
+        const Tensor ws = at::empty({std::max<int64_t>(1, bytes)}, cur.options().dtype(at::kByte));
+        check(dl_logic_forward_group_sum(cur.const_data_ptr(), net->a[l].const_data_ptr<int64_t>(),
+                                         net->b[l].const_data_ptr<int64_t>(), w.const_data_ptr(), probs.mutable_data_ptr(),
+                                         y.mutable_data_ptr(), ws.mutable_data_ptr(), cur.size(0), out_dim, batch, net->k,
+                                         net->tau, code, stream_of(cur)),
+              "logic_layer_cuda_forward_group_sum");
+        cur = y;
+    }
+    if (!net->fused) {
+        const int code = layer_code(cur.scalar_type(), cur.scalar_type());
+        const int64_t out_dim = cur.size(0), batch = cur.size(1);
+        Tensor y = at::empty({batch, net->k}, cur.options());
+        const int64_t bytes = dl_group_sum_workspace_bytes(out_dim, batch, net->k, code);
+        const Tensor ws = at::empty({std::max<int64_t>(1, bytes)}, cur.options().dtype(at::kByte));
+        check(dl_group_sum_forward(cur.const_data_ptr(), y.mutable_data_ptr(), ws.mutable_data_ptr(), out_dim, batch, net->k,
+                                   net->tau, code, stream_of(cur)),
+              "group_sum_forward");
+        cur = y;
+    }
+    return {cur, saved};
+}
+
+// Backward, from the gradient of the scores: the gradients of x and the weights as `wanted`.  (A node's own checks have been
+// made: saved is what net_forward returned.)
+std::vector<c10::optional<Tensor>> net_backward(const variable_list &saved, Tensor g, const std::vector<bool> &wanted,
+                                                const std::vector<double> &scale, const std::vector<int64_t> &codes, int64_t k,
+                                                double tau, bool fused) {
+    const int64_t layers = (int64_t) saved.size() / 6;
+    TORCH_CHECK(layers > 0 && (int64_t) wanted.size() == layers + 1 && (int64_t) scale.size() == layers && (int64_t) codes.size() == layers,
+                "net_backward: lists of one length expected");
+    check_saved(saved);
+    const c10::DeviceGuard guard(saved[0].device());
+    const Tensor &top = saved[6 * (layers - 1)];             // the last layer's input
+    TORCH_CHECK(g.dim() == 2 && g.size(0) == top.size(1) && g.size(1) == k && g.scalar_type() == top.scalar_type()
+                    && g.device() == top.device(),
+                "expected the gradient of the scores [B,k] in their dtype and on their device");
+    if (fused) {
+        g = (g / tau).t().contiguous();                      // [k, B]: a few KB
+    } else {
+        g = g.contiguous();
+        const int64_t out_dim = saved[6 * (layers - 1) + 3].size(0);
+        Tensor gx = at::empty({out_dim, g.size(0)}, g.options());
+        check(dl_group_sum_backward(g.const_data_ptr(), gx.mutable_data_ptr(), out_dim, g.size(0), k, tau,
+                                    layer_code(g.scalar_type(), g.scalar_type()), stream_of(g)),
+              "group_sum_backward");
+        g = gx;
+    }
+    std::vector<c10::optional<Tensor>> out((size_t) layers + 1);       // of x, of the weights
+    for (int64_t l = layers - 1; l >= 0; --l) {
+        const Tensor *s = &saved[(size_t) (6 * l)];
+        const Tensor &x = s[0], &a = s[1], &b = s[2], &probs = s[3], &start = s[4], &idx = s[5];
+        bool want_x = wanted[0];
+        for (int64_t below = 0; below < l; ++below) want_x = want_x || wanted[(size_t) (1 + below)];
+        const bool want_w = wanted[(size_t) (1 + l)];
+        const int64_t in_dim = x.size(0), out_dim = probs.size(0), batch = x.size(1);
+        const int code = (int) codes[(size_t) l];
+        const int64_t classes = fused && l == layers - 1 ? k : 0;
+        const int64_t *ap = a.const_data_ptr<int64_t>(), *bp = b.const_data_ptr<int64_t>();
+        const int64_t *sp = start.const_data_ptr<int64_t>(), *ip = idx.const_data_ptr<int64_t>();
+        Tensor gx = want_x ? at::empty_like(x) : Tensor(), gw = want_w ? at::empty_like(probs) : Tensor();
+        if (want_x && want_w)
+            backward_both_into(x, a, b, probs, g, start, idx, gw, gx, classes, scale[(size_t) l], true, code);
+        else if (want_x)
+            check(classes ? dl_logic_backward_x_grouped(x.const_data_ptr(), ap, bp, probs.const_data_ptr(), g.const_data_ptr(), sp,
+                                                        ip, gx.mutable_data_ptr(), in_dim, out_dim, batch, classes,
+                                                        scale[(size_t) l], code, stream_of(x))
+                          : dl_logic_backward_x(x.const_data_ptr(), ap, bp, probs.const_data_ptr(), g.const_data_ptr(), sp, ip,
+                                                gx.mutable_data_ptr(), in_dim, out_dim, batch, scale[(size_t) l], code,
+                                                stream_of(x)),
+                  "logic_layer_cuda_backward_x");
+        else if (want_w)
+            check(classes ? dl_logic_backward_logits_grouped(x.const_data_ptr(), ap, bp, g.const_data_ptr(),
+                                                             probs.const_data_ptr(), gw.mutable_data_ptr(), in_dim, out_dim,
+                                                             batch, classes, code, stream_of(x))
+                          : dl_logic_backward_logits(x.const_data_ptr(), ap, bp, g.const_data_ptr(), probs.const_data_ptr(),
+                                                     gw.mutable_data_ptr(), in_dim, out_dim, batch, code, stream_of(x)),
+                  "logic_layer_cuda_backward_w");
+        if (want_w) out[(size_t) (1 + l)] = gw;
+        if (!want_x) break;                                  // nothing below wants a gradient
+        g = gx;
+        if (l == 0 && wanted[0]) out[0] = gx;
+    }
+    return out;
+}
+
+// A net on feature-major x [in, B] (LogicNetFunction): scores, saved tensors and the layers' dtype codes.
+c10::optional<std::tuple<Tensor, variable_list, std::vector<int64_t>>> net_forward(const Tensor &x, const variable_list &weights, std::vector<Tensor> a, std::vector<Tensor> b,
+                                std::vector<Tensor> start, std::vector<Tensor> idx, std::vector<double> scale, int64_t k, double tau,
+                                bool fused) {
+    const size_t layers = weights.size();
+    if (layers == 0 || a.size() != layers || b.size() != layers || start.size() != layers || idx.size() != layers
+        || scale.size() != layers || k <= 0 || !x.is_contiguous())
+        return c10::nullopt;
+    Net net{std::move(a), std::move(b), std::move(start), std::move(idx), std::move(scale), {}, k, tau, fused};
+    int64_t in_dim = x.dim() == 2 ? x.size(0) : 0;
+    for (size_t l = 0; l < layers; ++l) {
+        const int code = layer_args(x, weights[l], net.a[l], net.b[l]);
+        if (code < 0 || !reverse_args(net.start[l], net.idx[l], x.get_device(), in_dim, weights[l].size(0))) return c10::nullopt;
+        net.code.push_back(code);
+        in_dim = weights[l].size(0);
+    }
+    if (in_dim % k || (fused && weights.back().scalar_type() != x.scalar_type())) return c10::nullopt;
+    const c10::DeviceGuard guard(x.device());
+    const at::NoGradGuard no_grad;
+    auto [y, saved] = net_forward_of(x, weights, &net);
+    return std::make_tuple(y, saved, net.code);
+}
+
 // GroupSum on the transposed view [B, out] that a layer returns.
 c10::optional<Tensor> group_sum(const Tensor &x, int64_t k, double tau) {
     if (!x.is_cuda() || x.dim() != 2 || x.numel() == 0 || x.stride(0) != 1 || x.stride(1) != x.size(0) || k <= 0
@@ -378,6 +529,8 @@ c10::optional<Tensor> count_rows(const Tensor &b, int64_t pad, int64_t k) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     typedef py::call_guard<py::gil_scoped_release> unlocked;
     m.def("train_layer", &train_layer, unlocked());
+    m.def("net_forward", &net_forward, unlocked());
+    m.def("net_backward", &net_backward, unlocked());
     m.def("eval_layer", &eval_layer, unlocked());
     m.def("forward_logits", &forward_logits, unlocked());
     m.def("backward_both", &backward_both, unlocked());
