@@ -711,7 +711,7 @@ class LogicNetFunction(torch.autograd.Function):
     @staticmethod
     def _native(x, stages, weights):
         """(_host.net_forward's results, (scale, k, tau, fused)) where no stage walks a schedule, else None: the same kernels, less
-        host work per layer (784 -> 8 x 2140 at batch 33, double: NNN us a step)."""
+        host work per layer (48 -> 4 x 11162 at batch 165: 513 -> 241 us a step)."""
         layers, k, tau, fused = [], 0, 1.0, False
         for fn, args, _ in stages:
             if fn is GroupSumCudaFunction:
