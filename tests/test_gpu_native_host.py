@@ -1,0 +1,148 @@
+"""The calls that are made in C++ (difflogic_amd._host) against the Python functions they stand in for: the same kernels, so the
+same bits, for every form of argument they take, and the same refusals for the others."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+F16, F32, F64 = torch.float16, torch.float32, torch.float64
+
+
+@pytest.fixture(scope="module")
+def dl():
+    import difflogic_amd
+    return difflogic_amd
+
+
+def _python_only(monkeypatch, dl):
+    for name in ("train_layer", "group_sum", "eval_layer", "net_forward", "eval_weights", "gate_ids_folded", "pack_rows", "count_rows",
+                 "forward_logits", "backward_both", "backward_logits", "forward_group_sum"):
+        monkeypatch.setattr(dl._host, name, lambda *a: None)
+
+
+def _views(x):
+    """x [B, in] as it is, as the transposed view a layer returns, and as columns of a wider matrix."""
+    wide = torch.zeros(x.shape[0], 2 * x.shape[1], dtype=x.dtype, device=x.device)
+    wide[:, ::2] = x
+    return x, x.t().contiguous().t(), wide[:, ::2]
+
+
+@pytest.mark.parametrize("dtype,wdtype", [(F32, F32), (F16, F32), (F64, F32), (F16, F16), (F64, F64)])
+@pytest.mark.parametrize("in_dim,out_dim,batch", [(20, 30, 1), (64, 50, 3), (300, 200, 100), (4200, 20000, 33)])
+def test_layer_and_group_sum(dl, monkeypatch, dtype, wdtype, in_dim, out_dim, batch):
+    torch.manual_seed(batch)
+    layer, total = dl.LogicLayer(in_dim, out_dim, grad_factor=1.5).train(), dl.GroupSum(10, 7.0)
+    layer.weights = torch.nn.Parameter(layer.weights.detach().to(wdtype))
+    x0 = torch.rand(batch, in_dim, device="cuda").to(dtype)
+    gy, gs = torch.randn(batch, out_dim, device="cuda").to(dtype), torch.randn(batch, 10, device="cuda").to(dtype)
+
+    def run():
+        out = []
+        for view in range(3):
+            for want_x, want_w in ((True, True), (True, False), (False, True), (False, False)):
+                layer.weights.requires_grad_(want_w)
+                layer.weights.grad = None
+                x = x0.detach().clone().requires_grad_(want_x)
+                y = layer(_views(x)[view])
+                assert y.requires_grad == (want_x or want_w) and y.stride() == (1, batch)
+                out.append(y.detach())
+                if y.requires_grad:
+                    torch.autograd.backward((y, total(y)), (gy, gs[:1].expand(batch, 10)), retain_graph=True)
+                    out += [t.grad.clone() for t in (x, layer.weights) if t.grad is not None]
+                    wanted = [t for t in (x, layer.weights) if t.requires_grad]
+                    out += [t for one in wanted for t in torch.autograd.grad(y, one, gy, retain_graph=True)]
+        with torch.no_grad():
+            out.append(layer(x0))
+        layer.eval()
+        out += [layer(v).detach() for v in _views(x0.clone().requires_grad_())] + [total(layer(x0))]
+        layer.train()
+        layer.weights.requires_grad_(True)
+        return out
+
+    native = run()
+    assert not native[-1].requires_grad
+    _python_only(monkeypatch, dl)
+    for u, v in zip(native, run(), strict=True):
+        assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v)
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, F64])
+@pytest.mark.parametrize("want_x,frozen", [(False, ()), (True, (1,)), (True, (0, 1, 2)), (False, (0,)), (False, (2,))])
+def test_fused_net(dl, monkeypatch, dtype, want_x, frozen):
+    torch.manual_seed(3)
+    net = torch.nn.Sequential(dl.LogicLayer(60, 90, grad_factor=2.0), dl.LogicLayer(90, 120), dl.LogicLayer(120, 80), dl.GroupSum(4, 3.0))
+    for i in frozen:
+        net[i].weights.requires_grad_(False)
+    fused = dl.fuse_for_training(net).train()
+    x0, g = torch.rand(37, 60, device="cuda").to(dtype), torch.randn(37, 4, device="cuda").to(dtype)
+
+    def run():
+        fused.zero_grad(set_to_none=True)
+        x = x0.clone().requires_grad_(want_x)
+        y = fused(x)
+        y.backward(g, retain_graph=True)
+        first = [p.grad.clone() for p in fused.parameters() if p.grad is not None]
+        y.backward(g)                                                 # a retained graph is walked again: gradients add up
+        return [y.detach()] + ([x.grad] if want_x else []) + first + [p.grad for p in fused.parameters() if p.grad is not None]
+
+    native = run()
+    _python_only(monkeypatch, dl)
+    for u, v in zip(native, run(), strict=True):
+        assert torch.equal(u, v)
+
+
+def test_hooks_streams_and_freed_graphs(dl):
+    torch.manual_seed(4)
+    layer = dl.LogicLayer(300, 200).train()
+    x = torch.rand(50, 300, device="cuda", requires_grad=True)
+    layer(x).sum().backward()
+    want = x.grad.clone(), layer.weights.grad.clone()
+    x.grad = layer.weights.grad = None
+    with torch.autograd.graph.save_on_cpu():
+        y = layer(x)
+    y.sum().backward()
+    assert torch.equal(x.grad, want[0]) and torch.equal(layer.weights.grad, want[1])
+    with pytest.raises(RuntimeError):
+        y.sum().backward()                                            # the graph is freed
+    y = layer(x)
+    with torch.no_grad():
+        x.add_(0)                                                     # (x itself is not what was saved: a transposed copy is)
+    y.sum().backward()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    x.grad = layer.weights.grad = None
+    with torch.cuda.stream(side):
+        layer(x).sum().backward()
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(x.grad, want[0]) and torch.equal(layer.weights.grad, want[1])
+
+
+def test_what_is_refused_stays_refused(dl):
+    layer = dl.LogicLayer(30, 40).train()
+    good = torch.rand(5, 30, device="cuda")
+    for bad, error in ((torch.rand(5, 31, device="cuda"), AssertionError), (torch.rand(5, 30), AssertionError),
+                       (torch.rand(30, device="cuda"), AssertionError), (good.int(), (RuntimeError, TypeError))):
+        with pytest.raises(error):
+            layer(bad).sum().backward()
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(layer)(good[None])
+    with pytest.raises(RuntimeError):
+        torch.func.jvp(layer, (good,), (good,))
+    with pytest.raises(AssertionError):
+        dl.GroupSum(7)(layer(good))
+    assert layer(torch.rand(0, 30, device="cuda")).shape == (0, 40)
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert torch.equal(layer(good.as_subclass(Sub)).as_subclass(torch.Tensor), layer(good))
+
+
+@pytest.mark.parametrize("batch,bits", [(1, 8), (100, 32), (129, 64), (5000, 16)])
+def test_packed_layers(dl, monkeypatch, batch, bits):
+    torch.manual_seed(batch)
+    net = torch.nn.Sequential(dl.LogicLayer(100, 1200), dl.LogicLayer(1200, 1000), dl.GroupSum(10)).eval()
+    x = torch.rand(batch, 100, device="cuda") < 0.3
+    native = net(dl.PackBitsTensor(x, bit_count=bits))
+    _python_only(monkeypatch, dl)
+    assert torch.equal(native, net(dl.PackBitsTensor(x, bit_count=bits)))
