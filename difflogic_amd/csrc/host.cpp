@@ -39,13 +39,19 @@ bool index_of(const Tensor &t, c10::DeviceIndex device, int64_t numel) {
     return t.scalar_type() == at::kLong && t.dim() == 1 && t.size(0) == numel && plain(t, device);
 }
 
-// Saved tensors may have been through a caller's hooks: [x, a, b, probabilities, start, idx] for each layer, as they were saved.
-void check_saved(const variable_list &saved) {
+// Saved tensors may have been through a caller's hooks: [x, a, b, probabilities, start, idx] for each layer, as they were saved
+// (code(layer): the layer's dtype code then; the layers are a chain on one device).
+template <typename Code>
+void check_saved(const variable_list &saved, const Code &code) {
     for (size_t i = 0; i + 5 < saved.size(); i += 6) {
         const Tensor &x = saved[i], &probs = saved[i + 3];
-        TORCH_CHECK(x.is_cuda() && x.dim() == 2 && probs.dim() == 2 && probs.size(1) == 16, "saved tensors changed");
-        const c10::DeviceIndex device = x.get_device();
+        TORCH_CHECK(x.is_cuda() && x.dim() == 2 && probs.dim() == 2 && probs.size(1) == 16
+                        && layer_code(x.scalar_type(), probs.scalar_type()) == code(i / 6),
+                    "saved tensors have to come back as they were: in their shape and dtype");
+        const c10::DeviceIndex device = saved[0].get_device();
         const int64_t in_dim = x.size(0), out_dim = probs.size(0);
+        TORCH_CHECK(i == 0 || (in_dim == saved[i - 3].size(0) && x.size(1) == saved[0].size(1)),
+                    "saved tensors have to come back as they were: in their shape and dtype");
         TORCH_CHECK(plain(x, device) && plain(probs, device) && index_of(saved[i + 1], device, out_dim)
                         && index_of(saved[i + 2], device, out_dim) && index_of(saved[i + 4], device, in_dim + 1)
                         && index_of(saved[i + 5], device, 2 * out_dim),
@@ -119,10 +125,10 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
 
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
-        check_saved(saved);
+        const int code = (int) ctx->saved_data["code"].toInt();
+        check_saved(saved, [&](size_t) { return code; });
         const Tensor &x = saved[0], &a = saved[1], &b = saved[2], &probs = saved[3], &start = saved[4], &idx = saved[5];
         const double scale = ctx->saved_data["scale"].toDouble();
-        const int code = (int) ctx->saved_data["code"].toInt();
         Walk walk;
         const auto tables = ctx->saved_data.find("tables");
         if (tables != ctx->saved_data.end()) {
@@ -372,7 +378,7 @@ std::vector<c10::optional<Tensor>> net_backward(const variable_list &saved, Tens
     const int64_t layers = (int64_t) saved.size() / 6;
     TORCH_CHECK(layers > 0 && (int64_t) wanted.size() == layers + 1 && (int64_t) scale.size() == layers && (int64_t) codes.size() == layers,
                 "net_backward: lists of one length expected");
-    check_saved(saved);
+    check_saved(saved, [&](size_t layer) { return codes[layer]; });
     const c10::DeviceGuard guard(saved[0].device());
     const Tensor &top = saved[6 * (layers - 1)];             // the last layer's input
     TORCH_CHECK(g.dim() == 2 && g.size(0) == top.size(1) && g.size(1) == k && g.scalar_type() == top.scalar_type()

@@ -117,6 +117,20 @@ def test_hooks_streams_and_freed_graphs(dl):
     assert torch.equal(x.grad, want[0]) and torch.equal(layer.weights.grad, want[1])
 
 
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("change", ["dtype", "rows", "device"])
+def test_saved_tensors_that_hooks_changed_are_refused(dl, fused, change):
+    net = torch.nn.Sequential(dl.LogicLayer(30, 40), dl.LogicLayer(40, 50), dl.GroupSum(10)).train()
+    net = dl.fuse_for_training(net) if fused else net
+    x = torch.rand(5, 30, device="cuda", requires_grad=True)
+    changes = {"dtype": lambda t: t.half(), "rows": lambda t: t[1:].contiguous(), "device": lambda t: t.cpu()}
+    probabilities = lambda t: t.dim() == 2 and t.shape[1] == 16
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: changes[change](t) if probabilities(t) else t):
+        y = net(x)
+    with pytest.raises(RuntimeError):
+        y.sum().backward()
+
+
 def test_what_is_refused_stays_refused(dl):
     layer = dl.LogicLayer(30, 40).train()
     good = torch.rand(5, 30, device="cuda")
