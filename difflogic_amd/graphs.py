@@ -32,8 +32,12 @@ class GraphedTrainStep:
     def __init__(self, model, loss_fn, example_x, example_y, optimizer=None, warmup=3):
         self.model, self.loss_fn, self.optimizer = model, loss_fn, optimizer
         # a model that starts with a logic layer reads its input feature-major: the static buffer is kept that way, so that the
-        # copy into it is the transposition as well (784 -> 4 x 8000 at batch 128, with the gradient below: 91.6 -> 87.2 us a step)
-        self.x = (example_x.detach().t().contiguous().t() if _reads_feature_major(model, example_x) else example_x.detach().clone())
+        # copy into it is the transposition as well (784 -> 4 x 8000 at batch 128, with the gradient below: 91.6 -> 87.2 us a step);
+        # a buffer of its own in either layout, also where the example is feature-major already
+        if _reads_feature_major(model, example_x):
+            self.x = example_x.detach().t().clone(memory_format=torch.contiguous_format).t()
+        else:
+            self.x = example_x.detach().clone()
         self.y = example_y.detach().clone()
         self._one = None                       # the loss's own gradient
         side = torch.cuda.Stream()

@@ -41,6 +41,27 @@ def test_graphed_step_equals_eager_on_every_replay():
             assert pg.grad is not None and torch.equal(pg.grad, pe.grad), rep
 
 
+@pytest.mark.parametrize("batch,features,feature_major", [(1, 60, False), (7, 1, False), (7, 60, True), (7, 60, False)])
+def test_the_static_input_is_a_buffer_of_its_own(batch, features, feature_major):
+    """Also where the example's transposed view is contiguous: one sample, one feature, a feature-major example."""
+    import difflogic_amd as dl
+    from difflogic_amd.graphs import GraphedTrainStep
+    torch.manual_seed(2)
+    model = torch.nn.Sequential(torch.nn.Flatten(), dl.LogicLayer(features, 40), dl.GroupSum(10, 10.0)).train()
+    loss_fn = torch.nn.CrossEntropyLoss()
+    example = torch.rand(features, batch, device="cuda").t() if feature_major else torch.rand(batch, features, device="cuda")
+    y = torch.zeros(batch, dtype=torch.long, device="cuda")
+    kept, other = example.clone(), torch.rand(batch, features, device="cuda")
+    graphed = GraphedTrainStep(model, loss_fn, example, y)
+    assert graphed.x.data_ptr() != example.data_ptr()
+    for x in (other, kept, other):
+        loss = graphed.step(x).clone()
+        assert torch.equal(example, kept)
+        assert torch.equal(loss, loss_fn(model(x), y).detach())
+    example.fill_(0.5)                                # what the caller writes there later is not what is replayed
+    assert torch.equal(graphed.step(), loss)
+
+
 def test_graphed_step_with_optimizer_tracks_eager_training():
     import copy
 
