@@ -12,6 +12,13 @@ _PLAIN = (torch.nn.Parameter, torch.Tensor)
 _NO_WALK = ([], 0, 0, 0, False, False)
 
 
+def _in_one_call(x):
+    """Whether a native call may take ``x``: a CUDA tensor, not a subclass, of a call that nobody traces (the compiler cannot
+    look into a native function; torch.jit would record nothing of it)."""
+    return (type(x) is torch.Tensor and x.is_cuda and not torch.compiler.is_compiling()
+            and torch._C._get_tracing_state() is None)
+
+
 class LogicLayer(torch.nn.Module):
     """A layer of ``out_dim`` two-input logic gates, each a learnable mixture of the 16 gates
     over two fixed inputs (difflogic/difflogic.py:11-169).
@@ -107,7 +114,7 @@ class LogicLayer(torch.nn.Module):
 
     def forward_cuda(self, x):
         if self.training:
-            if type(x) is torch.Tensor and type(self.weights) in _PLAIN and torch._C._get_tracing_state() is None:
+            if _in_one_call(x) and type(self.weights) in _PLAIN:
                 walk = self._native_walk(x)
                 if walk is not None:
                     y = _host.train_layer(x, self.weights, *self.indices, self.given_x_indices_of_y_start,
@@ -116,8 +123,7 @@ class LogicLayer(torch.nn.Module):
                         return y
             assert x.device.type == "cuda", x.device
         assert x.ndim == 2, x.ndim
-        if (not self.training and type(x) is torch.Tensor and type(self.weights) in _PLAIN and x.is_cuda
-                and x.shape[1] == self.in_dim and torch._C._get_tracing_state() is None):
+        if not self.training and _in_one_call(x) and type(self.weights) in _PLAIN and x.shape[1] == self.in_dim:
             # the discretised net on float inputs in one native call
             xt = x.transpose(0, 1)
             schedule = None if self.in_dim < self._CHAIN_MIN_IN_DIM else _forward_walk(self._train_schedule(xt), self.out_dim, xt)
@@ -262,8 +268,7 @@ class GroupSum(torch.nn.Module):
         if isinstance(x, PackBitsTensor):
             return x.group_sum(self.k)
         assert x.shape[-1] % self.k == 0, (x.shape, self.k)
-        if (type(x) is torch.Tensor and self.k <= self._HIP_MAX_K and x.shape[-1] <= self._HIP_MAX_OUT_DIM
-                and torch._C._get_tracing_state() is None):
+        if _in_one_call(x) and self.k <= self._HIP_MAX_K and x.shape[-1] <= self._HIP_MAX_OUT_DIM:
             y = _host.group_sum(x, int(self.k), float(self.tau))            # the case below in one native call
             if y is not None:
                 return y

@@ -160,3 +160,15 @@ def test_packed_layers(dl, monkeypatch, batch, bits):
     native = net(dl.PackBitsTensor(x, bit_count=bits))
     _python_only(monkeypatch, dl)
     assert torch.equal(native, net(dl.PackBitsTensor(x, bit_count=bits)))
+
+
+@pytest.mark.parametrize("train", [True, False])
+def test_compiled_modules(dl, train):
+    """The compiler sees what it saw without the native calls: GroupSum on row-major scores is one graph, a net of the kernels
+    runs with breaks around them."""
+    torch.manual_seed(6)
+    torch._dynamo.reset()
+    total, x = dl.GroupSum(5, 3.0), torch.rand(7, 30, device="cuda")
+    assert torch.equal(torch.compile(total, fullgraph=True, backend="eager")(x), total(x))
+    net = torch.nn.Sequential(dl.LogicLayer(30, 40), dl.LogicLayer(40, 50), total).train(train)
+    assert torch.equal(torch.compile(net, backend="eager")(x), net(x))

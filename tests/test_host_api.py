@@ -188,3 +188,18 @@ def test_layers_evaluated_at_once():
     assert _direct(784, 8000, 32, 10240, 32) and not _direct(784, 8000, 48, 10240, 32) and _direct(784, 8000, 768, 10240, None)
     assert _direct(784, 2000, 128, 10240, 128) and not _direct(784, 2000, 144, 10240, 128)
     assert _direct(784, 64000, 1008, 10240, 32)                        # wider than the LDS kernel: as ever
+
+
+@pytest.mark.parametrize("train", [True, False])
+def test_python_implementation_compiles_whole(train):
+    """torch.compile makes one graph of the python implementation and of GroupSum: nothing native is in its way."""
+    torch.manual_seed(5)
+    net = torch.nn.Sequential(dl.LogicLayer(20, 40, device="cpu"), dl.LogicLayer(40, 30, device="cpu"), dl.GroupSum(5, 3.0))
+    x = torch.rand(7, 20)
+    for module, inputs in ((net.train(train), x), (dl.GroupSum(5, 3.0), torch.rand(7, 30)), (dl.GroupSum(5, 3.0), torch.rand(30, 7).t())):
+        torch._dynamo.reset()
+        got = torch.compile(module, fullgraph=True, backend="eager")(inputs)
+        assert torch.equal(got, module(inputs))
+    if train:
+        torch.compile(net, fullgraph=True, backend="eager")(x).sum().backward()
+        assert all(p.grad is not None for p in net.parameters())
