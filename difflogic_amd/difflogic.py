@@ -268,14 +268,15 @@ class GroupSum(torch.nn.Module):
         if isinstance(x, PackBitsTensor):
             return x.group_sum(self.k)
         assert x.shape[-1] % self.k == 0, (x.shape, self.k)
-        if _in_one_call(x) and self.k <= self._HIP_MAX_K and x.shape[-1] <= self._HIP_MAX_OUT_DIM:
-            y = _host.group_sum(x, int(self.k), float(self.tau))            # the case below in one native call
-            if y is not None:
-                return y
+        # (k and tau are converted where the kernels take the call alone: the formula below broadcasts a tau per class)
         if (x.is_cuda and x.dim() == 2 and x.dtype in (torch.float16, torch.float32, torch.float64)
                 and x.numel() > 0 and x.stride(0) == 1 and x.stride(1) == x.shape[0]
                 and self.k <= self._HIP_MAX_K and x.shape[1] <= self._HIP_MAX_OUT_DIM):
             # the transposed view a 'cuda' LogicLayer returns: sum on the feature-major storage
+            if _in_one_call(x):
+                y = _host.group_sum(x, int(self.k), float(self.tau))
+                if y is not None:
+                    return y
             return GroupSumCudaFunction.apply(x.transpose(0, 1), self.k, float(self.tau))
         return x.reshape(*x.shape[:-1], self.k, x.shape[-1] // self.k).sum(-1) / self.tau
 

@@ -172,3 +172,17 @@ def test_compiled_modules(dl, train):
     assert torch.equal(torch.compile(total, fullgraph=True, backend="eager")(x), total(x))
     net = torch.nn.Sequential(dl.LogicLayer(30, 40), dl.LogicLayer(40, 50), total).train(train)
     assert torch.equal(torch.compile(net, backend="eager")(x), net(x))
+
+
+def test_group_sum_converts_tau_where_the_kernels_take_the_call(dl):
+    """A tau per class broadcasts over scores that go to the torch formula, and the device is not waited for there."""
+    x = torch.rand(7, 30, device="cuda")
+    tau = torch.arange(1.0, 6.0, device="cuda")
+    want = x.reshape(7, 5, 6).sum(-1)
+    assert torch.equal(dl.GroupSum(5, tau)(x), want / tau)
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        got = dl.GroupSum(5, tau[1])(x)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    assert torch.equal(got, want / tau[1])

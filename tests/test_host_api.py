@@ -203,3 +203,10 @@ def test_python_implementation_compiles_whole(train):
     if train:
         torch.compile(net, fullgraph=True, backend="eager")(x).sum().backward()
         assert all(p.grad is not None for p in net.parameters())
+
+
+def test_group_sum_with_a_tau_per_class():
+    x, tau = torch.rand(4, 20), torch.arange(1.0, 6.0)
+    want = x.reshape(4, 5, 4).sum(-1) / tau
+    assert torch.equal(dl.GroupSum(5, tau)(x), want)
+    assert torch.equal(dl.GroupSum(5, tau)(x.t().contiguous().t()), want)
