@@ -10,11 +10,17 @@ import torch
 
 
 def _reads_feature_major(model, x):
-    """Whether ``model`` is a Sequential whose first module that does anything to 2-D input is a 'cuda' logic layer."""
-    from .difflogic import FusedLogicLayerGroupSum, FusedLogicLayerPair, LogicLayer
-    if x.dim() != 2 or not isinstance(model, torch.nn.Sequential):
+    """Whether ``model`` is a Sequential whose first module that does anything to 2-D input is a 'cuda' logic layer, and nothing
+    else sees its input: a subclass's own forward, or a hook, may want the strides of the example."""
+    from .difflogic import FusedLogicLayerGroupSum, FusedLogicLayerPair, FusedSequential, LogicLayer
+    if x.dim() != 2 or type(model) not in (torch.nn.Sequential, FusedSequential):
         return False
     first = next((m for m in model if type(m) is not torch.nn.Flatten), None)
+    for m in (model, *model):
+        if m._forward_pre_hooks or m._forward_hooks:
+            return False
+        if m is first:
+            break
     if type(first) in (FusedLogicLayerGroupSum, FusedLogicLayerPair):
         first = first.layer if type(first) is FusedLogicLayerGroupSum else first.layer1
     return type(first) is LogicLayer and first.implementation == "cuda"
@@ -26,7 +32,7 @@ class GraphedTrainStep:
     ``step(x, y)`` copies the batch into the static input buffers, replays the graph and returns
     the static loss tensor (valid until the next replay).  Parameter gradients are the
     ``.grad`` tensors of the parameters, rewritten by every replay.  Shapes and dtypes are fixed
-    at construction.  With ``optimizer`` given it must be constructed with ``capturable=True``.
+    at construction; the static input ``x`` may be laid out feature-major (written with ``copy_``, not through a flat view).  With ``optimizer`` given it must be constructed with ``capturable=True``.
     """
 
     def __init__(self, model, loss_fn, example_x, example_y, optimizer=None, warmup=3):

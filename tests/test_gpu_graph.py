@@ -62,6 +62,35 @@ def test_the_static_input_is_a_buffer_of_its_own(batch, features, feature_major)
     assert torch.equal(graphed.step(), loss)
 
 
+@pytest.mark.parametrize("who", ["subclass", "pre-hook of the model", "pre-hook of the layer", "hook of Flatten"])
+def test_other_readers_of_the_static_input_see_its_strides(who):
+    """A Sequential subclass with a forward of its own, and hooks, get the input laid out as the example is."""
+    import difflogic_amd as dl
+    from difflogic_amd.graphs import GraphedTrainStep
+
+    class Halves(torch.nn.Sequential):
+        def forward(self, x):
+            return super().forward(x.view(-1, 30))        # (of a transposed view this would raise)
+
+    torch.manual_seed(3)
+    features = 30 if who == "subclass" else 60
+    mods = [torch.nn.Flatten(), dl.LogicLayer(features, 40), dl.GroupSum(10, 10.0)]
+    model = (Halves if who == "subclass" else torch.nn.Sequential)(*mods).train()
+    seen = []
+    if who == "pre-hook of the model":
+        model.register_forward_pre_hook(lambda m, a: seen.append(a[0].view(-1)))
+    elif who == "pre-hook of the layer":
+        mods[1].register_forward_pre_hook(lambda m, a: seen.append(a[0].view(-1)))
+    elif who == "hook of Flatten":
+        mods[0].register_forward_hook(lambda m, a, y: seen.append(y.view(-1)))
+    loss_fn = torch.nn.CrossEntropyLoss()
+    x, other = torch.rand(8, 60, device="cuda"), torch.rand(8, 60, device="cuda")
+    y = torch.zeros(16 if who == "subclass" else 8, dtype=torch.long, device="cuda")
+    graphed = GraphedTrainStep(model, loss_fn, x, y)
+    for inp in (other, x, other):
+        assert torch.equal(graphed.step(inp), loss_fn(model(inp), y).detach())
+
+
 def test_graphed_step_with_optimizer_tracks_eager_training():
     import copy
 
