@@ -45,14 +45,19 @@ class GraphedTrainStep:
         else:
             self.x = example_x.detach().clone()
         self.y = example_y.detach().clone()
-        self._one = None                       # the loss's own gradient
+        self._one, loss = None, None           # the loss's own gradient (made by backward() it would be a launch in every replay)
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
             for _ in range(warmup):
-                self._eager()
+                loss = self._eager()
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
+        if loss is not None and loss.dim() == 0:
+            # on this stream, whose later work waits for the replays: memory of the warm-up's stream could be handed out
+            # again beside the last of them
+            self._one = torch.ones_like(loss, requires_grad=False)
+        loss = None
         self.graph = torch.cuda.CUDAGraph()
         self._zero_grad()
         with torch.cuda.graph(self.graph):
@@ -68,9 +73,7 @@ class GraphedTrainStep:
         if zero:
             self._zero_grad()
         loss = self.loss_fn(self.model(self.x), self.y)
-        if self._one is None and loss.dim() == 0:
-            self._one = torch.ones_like(loss, requires_grad=False)
-        loss.backward(self._one)               # (made by backward() it would be a launch in every replay)
+        loss.backward(self._one)
         if self.optimizer is not None:
             self.optimizer.step()
         return loss

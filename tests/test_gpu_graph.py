@@ -91,6 +91,29 @@ def test_other_readers_of_the_static_input_see_its_strides(who):
         assert torch.equal(graphed.step(inp), loss_fn(model(inp), y).detach())
 
 
+def test_what_replays_read_is_no_memory_of_the_warm_up_stream():
+    """Buffers kept beside the graph come from the stream that the graph is made and replayed on, so that freeing them waits for
+    the replays; without warm-up steps the gradient of the loss is part of the graph."""
+    import difflogic_amd as dl
+    from difflogic_amd.graphs import GraphedTrainStep
+    torch.manual_seed(4)
+    model = torch.nn.Sequential(dl.LogicLayer(60, 40), dl.GroupSum(10, 10.0)).train()
+    loss_fn = torch.nn.CrossEntropyLoss()
+    x, y = torch.rand(8, 60, device="cuda"), torch.zeros(8, dtype=torch.long, device="cuda")
+    for warmup in (2, 0):
+        graphed = GraphedTrainStep(model, loss_fn, x, y, warmup=warmup)
+        kept = [t for t in vars(graphed).values() if torch.is_tensor(t) and t is not graphed.loss]
+        here = torch.cuda.current_stream().cuda_stream
+        for t in kept:
+            segment, = [s for s in torch.cuda.memory_snapshot() if s["address"] <= t.data_ptr() < s["address"] + s["total_size"]]
+            assert segment["stream"] == here
+        want = loss_fn(model(x), y)
+        grads = torch.autograd.grad(want, list(model.parameters()))
+        for _ in range(3):
+            assert torch.equal(graphed.step(x), want.detach())
+            assert all(torch.equal(p.grad, g) for p, g in zip(model.parameters(), grads))
+
+
 def test_graphed_step_with_optimizer_tracks_eager_training():
     import copy
 
