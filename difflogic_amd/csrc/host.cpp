@@ -60,11 +60,12 @@ void check_saved(const variable_list &saved, const Code &code) {
 }
 
 // A layer's walk along its evaluation schedule: difflogic_cuda.EvalSchedule and the plan of its one-pass backward
-// ([verts, neuron, flip, dst, fix_vertex, fix_start]; none: the layer has no schedule), and which of the kernels take it.
+// ([verts, neuron, flip, dst, fix_vertex, fix_start]; none: the layer has no schedule), whether the inputs at several
+// positions are finished in the launch (DL_FIX_POSITIONS), and which of the kernels take the schedule.
 struct Walk {
     std::vector<Tensor> tables;
     int64_t steps = 0, n_fix = 0, rows = 0;
-    bool forward = false, weights = false;
+    bool here = false, forward = false, weights = false;
 
     const int32_t *i32(int i) const { return tables[i].const_data_ptr<int32_t>(); }
     const uint8_t *flip() const { return tables[2].const_data_ptr<uint8_t>(); }
@@ -118,7 +119,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
         ctx->saved_data["code"] = code;
         if (!walk->tables.empty()) {
             ctx->saved_data["tables"] = walk->tables;
-            ctx->saved_data["sizes"] = std::vector<int64_t>{walk->steps, walk->n_fix, walk->rows, walk->weights};
+            ctx->saved_data["sizes"] = std::vector<int64_t>{walk->steps, walk->n_fix, walk->rows, walk->here, walk->weights};
         }
         return y;
     }
@@ -134,7 +135,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
         if (tables != ctx->saved_data.end()) {
             walk.tables = tables->second.toTensorVector();
             const std::vector<int64_t> sizes = ctx->saved_data["sizes"].toIntVector();
-            walk.steps = sizes[0], walk.n_fix = sizes[1], walk.rows = sizes[2], walk.weights = sizes[3] != 0;
+            walk.steps = sizes[0], walk.n_fix = sizes[1], walk.rows = sizes[2], walk.here = sizes[3] != 0, walk.weights = sizes[4] != 0;
         }
         const c10::DeviceGuard guard(x.device());
         const Tensor gy = grads[0].contiguous();
@@ -156,7 +157,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
                                                walk.n_fix ? walk.i32(4) : nullptr, walk.n_fix ? walk.i32(5) : nullptr, walk.n_fix,
                                                walk.rows, gw.mutable_data_ptr(), gx.mutable_data_ptr(),
                                                bytes ? ws.mutable_data_ptr() : nullptr, in_dim, out_dim, batch, scale,
-                                               code | DL_ROWS_ANY | DL_FIX_POSITIONS, stream_of(x));
+                                               code | DL_ROWS_ANY | (walk.here ? DL_FIX_POSITIONS : 0), stream_of(x));
                 if (st != DL_ERR_TOO_LARGE) check(st, "logic_layer_cuda_backward_chained");
             }
             if (st == DL_ERR_TOO_LARGE)
@@ -195,9 +196,9 @@ bool reverse_args(const Tensor &start, const Tensor &idx, c10::DeviceIndex devic
 // A training layer on x [B, in] as LogicLayer.forward_cuda runs it: y [B, out], a view of [out, B].
 c10::optional<Tensor> train_layer(const Tensor &x, const Tensor &weights, const Tensor &a, const Tensor &b, const Tensor &start,
                                   const Tensor &idx, double scale, std::vector<Tensor> tables, int64_t steps, int64_t n_fix,
-                                  int64_t rows, bool walk_forward, bool walk_weights) {
+                                  int64_t rows, bool here, bool walk_forward, bool walk_weights) {
     const int code = layer_args(x, weights, a, b);
-    const Walk walk{std::move(tables), steps, n_fix, rows, walk_forward, walk_weights};
+    const Walk walk{std::move(tables), steps, n_fix, rows, here, walk_forward, walk_weights};
     if (code < 0 || !reverse_args(start, idx, x.get_device(), x.size(1), weights.size(0)) || !fits(walk, x.get_device()))
         return c10::nullopt;
     const c10::DeviceGuard guard(x.device());

@@ -1985,7 +1985,8 @@ int backward_w_chain_t(const void *x, const int32_t *verts, const int32_t *neuro
 
 // Vertices (and overflow rows) up to which the one-pass backward finishes them in its own launch.  Each costs four row reads
 // instead of a written and a read row; the launch that goes takes 4 to 5 us a layer (784 -> 4 x 64000, a captured step at
-// batch 100: fp32 fused 187 -> 167 us with the pair's second launch gone too, half 226 -> 213).
+// batch 100: fp32 fused 187 -> 167 us with the pair's second launch gone too, half 226 -> 213).  (A vertex of many positions is
+// one wave's serial work: the caller says DL_FIX_POSITIONS where there is none.)
 constexpr int64_t DL_FIX_HERE = 64;
 
 template <typename T> int64_t backward_partial_bytes(int64_t out_dim, int64_t batch) {

@@ -9,7 +9,7 @@ from .packbitstensor import PackBitsTensor
 
 
 _PLAIN = (torch.nn.Parameter, torch.Tensor)
-_NO_WALK = ([], 0, 0, 0, False, False)
+_NO_WALK = ([], 0, 0, 0, False, False, False)
 
 
 def _in_one_call(x):

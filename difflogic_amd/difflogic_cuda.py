@@ -365,7 +365,7 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
             or w.shape != (grad_y.shape[0], 16)):
         raise RuntimeError(f"expected x [in,B], w [out,16], grad_y [out,B] of one dtype, got {tuple(x.shape)}, "
                            f"{tuple(w.shape)}, {tuple(grad_y.shape)}")
-    code = _layer_code(x, w, "logic_layer_cuda_backward") | _lib.DL_FIX_POSITIONS | (_lib.DL_ROWS_ANY if any_rows else 0)
+    code = _layer_code(x, w, "logic_layer_cuda_backward") | (_lib.DL_ROWS_ANY if any_rows else 0)
     dev = x.device if ready else _same_device(x, w, grad_y)
     in_dim, batch = x.shape
     out_dim = grad_y.shape[0]
@@ -375,7 +375,7 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
     plan = schedule.backward_plan()
     if plan is None or plan[4] > in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
         return None
-    dst, fix_vertex, fix_start, n_fix, rows = plan
+    dst, fix_vertex, fix_start, n_fix, rows, _ = plan
     grad_w, grad_x = torch.empty_like(w), torch.empty_like(x)
     lib = _lib.load()
     ws_bytes = schedule.backward_bytes(rows, batch, code)
@@ -385,7 +385,7 @@ def backward_chained(x, w, grad_y, schedule, scale=1.0, softmax_backward=False, 
         schedule.flip.data_ptr(), dst.data_ptr(), schedule.steps, w.data_ptr(), grad_y.data_ptr(),
         1 if softmax_backward else 0, fix_vertex.data_ptr() if n_fix else None, fix_start.data_ptr() if n_fix else None,
         n_fix, rows, grad_w.data_ptr(), grad_x.data_ptr(), workspace.data_ptr() if ws_bytes else None, in_dim, out_dim,
-        batch, float(scale), code)
+        batch, float(scale), code | _fix_code(plan))
     if st == _lib.DL_ERR_TOO_LARGE:
         return None
     if st:
@@ -448,7 +448,7 @@ def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_
     for t, n in ((w, "w"), (grad_y, "grad_y"), (x_lower, "x_lower"), (a_lower, "a_lower"), (b_lower, "b_lower"),
                  (w_lower, "w_lower")):
         _check_input(t, n)
-    code = _float_code(grad_y, "logic_layer_cuda_backward") | _lib.DL_FIX_POSITIONS | (_lib.DL_ROWS_ANY if any_rows else 0)
+    code = _float_code(grad_y, "logic_layer_cuda_backward") | (_lib.DL_ROWS_ANY if any_rows else 0)
     dtype = grad_y.dtype
     out_dim, batch = grad_y.shape if grad_y.dim() == 2 else (0, 0)
     in_dim = w_lower.shape[0]
@@ -473,7 +473,7 @@ def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_
     plan = schedule.backward_plan()
     if plan is None or plan[4] > in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
         return None
-    dst, fix_vertex, fix_start, n_fix, rows = plan
+    dst, fix_vertex, fix_start, n_fix, rows, _ = plan
     grad_w = torch.empty((out_dim, 16), dtype=dtype, device=dev)
     grad_w_lower = torch.empty((in_dim, 16), dtype=dtype, device=dev)
     fix_rows = torch.empty((n_fix, batch), dtype=dtype, device=dev) if n_fix else None
@@ -488,7 +488,8 @@ def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_
             schedule.steps, _p(w), _p(grad_y), 1 if softmax_backward else 0, _p(fix_vertex) if n_fix else None,
             _p(fix_start) if n_fix else None, n_fix, rows, _p(grad_w), _p(fix_rows) if n_fix else None,
             _p(workspace) if ws_bytes else None, _p(x_lower), _p(a_lower), _p(b_lower), _p(w_lower),
-            1 if softmax_backward_lower else 0, _p(grad_w_lower), in_dim, out_dim, batch, float(scale), code, _stream(dev))
+            1 if softmax_backward_lower else 0, _p(grad_w_lower), in_dim, out_dim, batch, float(scale), code | _fix_code(plan),
+            _stream(dev))
     if st == _lib.DL_ERR_TOO_LARGE:
         return None
     if st:
@@ -499,6 +500,16 @@ def backward_chained_lower(x, w, grad_y, schedule, x_lower, a_lower, b_lower, w_
 # backward_chained gives way to the separate kernels when the partial rows it would park in the
 # overflow buffer exceed this fraction of the input rows (wirings with many high-degree inputs).
 BACKWARD_CHAIN_MAX_OVERFLOW = 0.25
+
+# Inputs at several schedule positions are finished in the launch of backward_chained itself (DL_FIX_POSITIONS) where none is
+# at more positions than this: one wave forms them one after the other.  64000 -> 64000, one input read by 8 / 16 / 32 / 64 /
+# 110 neurons (5 / 10 / 18 / 34 / 56 positions), overflow rows and a second launch / in the launch: fp32 batch 100 25.7 / 22.4,
+# 26.0 / 23.5, 29.2 / 33.6, 32.8 / 52.7, 37.8 / 82.1 us, half 500 47.5 / 43.4, 48.4 / 50.0, 49.9 / 77.4, 54.5 / 129, 61.1 / 204.
+FIX_HERE_MAX_POSITIONS = 8
+
+
+def _fix_code(plan):
+    return _lib.DL_FIX_POSITIONS if plan[5] else 0
 
 
 def eval(x, a, b, w):  # noqa: A001  (the reference's name)
@@ -841,10 +852,11 @@ class EvalSchedule:
         return nbytes
 
     def backward_plan(self):
-        """(dst, fix_vertex, fix_start, n_fix, overflow_rows) for backward_chained, built on first
+        """(dst, fix_vertex, fix_start, n_fix, overflow_rows, here) for backward_chained, built on first
         use: where each schedule position's grad_x row goes and which inputs are summed from
-        several partial rows afterwards (fix_start is followed by the overflow rows' positions).  None where it would have to be built while a graph is being captured
-        (building it copies from the host)."""
+        several partial rows afterwards (fix_start is followed by the overflow rows' positions;
+        ``here``: whether a call says so, FIX_HERE_MAX_POSITIONS).  None where it would have to be built
+        while a graph is being captured (building it copies from the host)."""
         if self._backward is None:
             if torch.cuda.is_current_stream_capturing():
                 return None
@@ -866,8 +878,9 @@ class EvalSchedule:
             overflow = np.flatnonzero(dst >= self.in_dim)
             positions = np.empty(int(rows), dtype=np.int32)
             positions[dst[overflow] - self.in_dim] = overflow                # DL_FIX_POSITIONS
+            here = n > 0 and int(np.diff(fix_start[:n + 1]).max()) <= FIX_HERE_MAX_POSITIONS
             self._backward = (torch.from_numpy(dst).to(dev), torch.from_numpy(fix_vertex[:n].copy()).to(dev),
-                              torch.from_numpy(np.concatenate((fix_start[:n + 1], positions))).to(dev), n, int(rows))
+                              torch.from_numpy(np.concatenate((fix_start[:n + 1], positions))).to(dev), n, int(rows), here)
         return self._backward
 
 
@@ -1339,11 +1352,11 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
     dev = _same_device(x, a, b, probs, grad_cls)
     lib = _lib.load()
     if want_x and want_w and schedule is not None:
-        chained_code = code | _lib.DL_ROWS_ANY | _lib.DL_FIX_POSITIONS
+        chained_code = code | _lib.DL_ROWS_ANY
         _check_schedule(schedule, in_dim, out_dim, dev)
         plan = schedule.backward_plan()
         if plan is not None and plan[4] <= in_dim * BACKWARD_CHAIN_MAX_OVERFLOW:
-            dst, fix_vertex, fix_start, n_fix, rows = plan
+            dst, fix_vertex, fix_start, n_fix, rows, _ = plan
             grad_w = torch.empty((out_dim, 16), dtype=x.dtype, device=dev)
             grad_x = torch.empty_like(x)
             ws_bytes = lib.dl_logic_backward_chained_workspace_bytes(rows, out_dim, batch, chained_code)
@@ -1355,7 +1368,7 @@ def backward_group_sum(x, a, b, probs, grad_cls, start, idx, schedule, scale, wa
                     _p(x), _p(schedule.verts), _p(schedule.neuron), _p(schedule.flip), _p(dst), schedule.steps, _p(probs),
                     _p(grad_cls), 1, _p(fix_vertex) if n_fix else None, _p(fix_start) if n_fix else None, n_fix, rows,
                     _p(grad_w), _p(grad_x), _p(workspace) if ws_bytes else None, in_dim, out_dim, batch, k, float(scale),
-                    chained_code, _stream(dev))
+                    chained_code | _fix_code(plan), _stream(dev))
             if st == _lib.DL_OK:
                 return grad_w, grad_x
             if st != _lib.DL_ERR_TOO_LARGE:

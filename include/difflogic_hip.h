@@ -60,7 +60,8 @@ typedef enum dl_dtype { DL_F16 = 0, DL_F32 = 1, DL_F64 = 2, DL_F16_W32 = 3, DL_F
 
 /* Or'ed into `dtype` of dl_logic_backward_chained and its _lower and _grouped forms: `fix_start` is followed by the schedule
  * positions of the overflow rows, int32 [overflow_rows] (row r: the position p with dst[p] = in_dim + r).  The kernels may then
- * finish fix_vertex in the launch itself, without overflow rows; the workspace is asked for and passed as without it. */
+ * finish fix_vertex in the launch itself, without overflow rows; the workspace is asked for and passed as without it.  Worth it
+ * where no vertex has more than some eight positions: a wave takes a vertex's positions one after the other. */
 #define DL_FIX_POSITIONS 0x400
 
 /* Or'ed into `dtype` of dl_logic_forward and dl_logic_forward_chained (probs NULL): `w` holds weights of which

@@ -6,8 +6,9 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
-from difflogic_amd import _lib
+from difflogic_amd import _lib, difflogic_cuda
 from oracle import connections as oc
 
 
@@ -224,3 +225,16 @@ def test_launch_plan_follows_the_traffic_model():
     assert pbt.lds_cost(c2, 16384, True, 0.95) == pbt.lds_cost(c2, 16384, True)
     assert pbt.lds_tail(c2, 16384, 0.5, from_bool=True) == 6
     assert pbt.plan_groups([784], True) == []
+
+
+@pytest.mark.parametrize("reads,here", [(2, True), (14, True), (40, False), (200, False)])
+def test_inputs_at_many_positions_are_not_left_to_one_wave(monkeypatch, reads, here):
+    """The plan of the one-pass backward asks for inputs to be finished in its launch where none is at many positions: one wave
+    adds a vertex's positions one after the other."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)          # (asks for a device)
+    rng = np.random.default_rng(reads)
+    a, b = (torch.as_tensor(rng.permutation(5000)) for _ in range(2))
+    a[rng.permutation(5000)[:reads]] = 7
+    plan = difflogic_cuda.EvalSchedule(a, b, 5000).backward_plan()
+    start = plan[2][:plan[3] + 1].numpy()
+    assert (np.diff(start).max() <= difflogic_cuda.FIX_HERE_MAX_POSITIONS) == plan[5] == here
