@@ -145,23 +145,26 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
         const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1);
         const int64_t in_dim = x.size(0), out_dim = probs.size(0), batch = x.size(1);
         const int64_t *ap = a.const_data_ptr<int64_t>(), *bp = b.const_data_ptr<int64_t>();
-        Tensor gx = want_x ? at::empty_like(x) : Tensor(), gw = want_w ? at::empty_like(probs) : Tensor();
+        // Along a schedule the one pass forms both gradients faster than the other kernels form grad_x alone (a task that asks for
+        // x only, both wanting gradients: 128000 -> 128000 at batch 1024 349 / 470 us, 64000 at 512 94 / 104).
+        const bool one_pass = want_x && !walk.tables.empty(), both = want_x && want_w;
+        Tensor gx = want_x ? at::empty_like(x) : Tensor(), gw = want_w || one_pass ? at::empty_like(probs) : Tensor();
         int st = DL_ERR_TOO_LARGE;
-        if (want_x && want_w) {
-            if (!walk.tables.empty()) {
-                const int64_t bytes = dl_logic_backward_chained_workspace_bytes(walk.rows, out_dim, batch, code | DL_ROWS_ANY);
-                check(bytes < 0 ? (int) -bytes : DL_OK, "logic_layer_cuda_backward_chained");
-                const Tensor ws = bytes ? at::empty({bytes}, x.options().dtype(at::kByte)) : Tensor();
-                st = dl_logic_backward_chained(x.const_data_ptr(), walk.i32(0), walk.i32(1), walk.flip(), walk.i32(3), walk.steps,
-                                               probs.const_data_ptr(), gy.const_data_ptr(), 1,
-                                               walk.n_fix ? walk.i32(4) : nullptr, walk.n_fix ? walk.i32(5) : nullptr, walk.n_fix,
-                                               walk.rows, gw.mutable_data_ptr(), gx.mutable_data_ptr(),
-                                               bytes ? ws.mutable_data_ptr() : nullptr, in_dim, out_dim, batch, scale,
-                                               code | DL_ROWS_ANY | (walk.here ? DL_FIX_POSITIONS : 0), stream_of(x));
-                if (st != DL_ERR_TOO_LARGE) check(st, "logic_layer_cuda_backward_chained");
-            }
-            if (st == DL_ERR_TOO_LARGE)
-                backward_both_into(x, a, b, probs, gy, start, idx, gw, gx, 0, scale, true, code);
+        if (one_pass) {
+            const int64_t bytes = dl_logic_backward_chained_workspace_bytes(walk.rows, out_dim, batch, code | DL_ROWS_ANY);
+            check(bytes < 0 ? (int) -bytes : DL_OK, "logic_layer_cuda_backward_chained");
+            const Tensor ws = bytes ? at::empty({bytes}, x.options().dtype(at::kByte)) : Tensor();
+            st = dl_logic_backward_chained(x.const_data_ptr(), walk.i32(0), walk.i32(1), walk.flip(), walk.i32(3), walk.steps,
+                                           probs.const_data_ptr(), gy.const_data_ptr(), 1,
+                                           walk.n_fix ? walk.i32(4) : nullptr, walk.n_fix ? walk.i32(5) : nullptr, walk.n_fix,
+                                           walk.rows, gw.mutable_data_ptr(), gx.mutable_data_ptr(),
+                                           bytes ? ws.mutable_data_ptr() : nullptr, in_dim, out_dim, batch, scale,
+                                           code | DL_ROWS_ANY | (walk.here ? DL_FIX_POSITIONS : 0), stream_of(x));
+            if (st != DL_ERR_TOO_LARGE) check(st, "logic_layer_cuda_backward_chained");
+        }
+        if (st == DL_OK) {                                   // formed above
+        } else if (both) {
+            backward_both_into(x, a, b, probs, gy, start, idx, gw, gx, 0, scale, true, code);
         } else if (want_x) {
             check(dl_logic_backward_x(x.const_data_ptr(), ap, bp, probs.const_data_ptr(), gy.const_data_ptr(),
                                       start.const_data_ptr<int64_t>(), idx.const_data_ptr<int64_t>(), gx.mutable_data_ptr(),
@@ -177,7 +180,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
                                               gw.mutable_data_ptr(), in_dim, out_dim, batch, code, stream_of(x));
             check(st, "logic_layer_cuda_backward_w");
         }
-        return {gx, gw, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        return {gx, want_w ? gw : Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 

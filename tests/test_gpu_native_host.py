@@ -20,6 +20,25 @@ def _python_only(monkeypatch, dl):
         monkeypatch.setattr(dl._host, name, lambda *a: None)
 
 
+def _answered(monkeypatch, dl):
+    """Counts the native calls that answered: {name: times}, train_layer along a schedule as "train_layer walked"."""
+    counts = {}
+
+    def counted(name, fn):
+        def call(*args):
+            out = fn(*args)
+            if out is not None:
+                key = name + (" walked" if name == "train_layer" and args[7] else "")
+                counts[key] = counts.get(key, 0) + 1
+            return out
+        return call
+
+    for name in ("train_layer", "group_sum", "eval_layer", "net_forward", "net_backward", "eval_weights", "gate_ids_folded", "pack_rows",
+                 "count_rows", "forward_logits", "backward_both", "backward_logits", "forward_group_sum"):
+        monkeypatch.setattr(dl._host, name, counted(name, getattr(dl._host, name)))
+    return counts
+
+
 def _views(x):
     """x [B, in] as it is, as the transposed view a layer returns, and as columns of a wider matrix."""
     wide = torch.zeros(x.shape[0], 2 * x.shape[1], dtype=x.dtype, device=x.device)
@@ -28,7 +47,10 @@ def _views(x):
 
 
 @pytest.mark.parametrize("dtype,wdtype", [(F32, F32), (F16, F32), (F64, F32), (F16, F16), (F64, F64)])
-@pytest.mark.parametrize("in_dim,out_dim,batch", [(20, 30, 1), (64, 50, 3), (300, 200, 100), (4200, 20000, 33)])
+@pytest.mark.parametrize("in_dim,out_dim,batch", [(20, 30, 1), (64, 50, 3), (300, 200, 100),
+                                                  (4200, 20000, 33),       # a schedule, but too many inputs at several positions
+                                                  (20000, 20000, 33),      # one-pass backward along the schedule
+                                                  (33000, 33000, 30)])     # every kernel along it
 def test_layer_and_group_sum(dl, monkeypatch, dtype, wdtype, in_dim, out_dim, batch):
     torch.manual_seed(batch)
     layer, total = dl.LogicLayer(in_dim, out_dim, grad_factor=1.5).train(), dl.GroupSum(10, 7.0)
@@ -37,7 +59,7 @@ def test_layer_and_group_sum(dl, monkeypatch, dtype, wdtype, in_dim, out_dim, ba
     gy, gs = torch.randn(batch, out_dim, device="cuda").to(dtype), torch.randn(batch, 10, device="cuda").to(dtype)
 
     def run():
-        out = []
+        out, alone = [], []                               # alone: gradients of the weights in a task that asks for nothing else
         for view in range(3):
             for want_x, want_w in ((True, True), (True, False), (False, True), (False, False)):
                 layer.weights.requires_grad_(want_w)
@@ -49,21 +71,39 @@ def test_layer_and_group_sum(dl, monkeypatch, dtype, wdtype, in_dim, out_dim, ba
                 if y.requires_grad:
                     torch.autograd.backward((y, total(y)), (gy, gs[:1].expand(batch, 10)), retain_graph=True)
                     out += [t.grad.clone() for t in (x, layer.weights) if t.grad is not None]
-                    wanted = [t for t in (x, layer.weights) if t.requires_grad]
-                    out += [t for one in wanted for t in torch.autograd.grad(y, one, gy, retain_graph=True)]
+                    if want_x:
+                        out += torch.autograd.grad(y, x, gy, retain_graph=True)
+                    if want_w:
+                        alone += torch.autograd.grad(y, layer.weights, gy, retain_graph=True)
         with torch.no_grad():
             out.append(layer(x0))
         layer.eval()
         out += [layer(v).detach() for v in _views(x0.clone().requires_grad_())] + [total(layer(x0))]
         layer.train()
         layer.weights.requires_grad_(True)
-        return out
+        return out, alone
 
-    native = run()
+    counts = _answered(monkeypatch, dl)
+    native, alone = run()
     assert not native[-1].requires_grad
+    assert counts["eval_layer"] == 4 and counts["group_sum"] > 0
+    if in_dim < 4096:
+        assert counts["train_layer"] == 13 and "train_layer walked" not in counts         # the four wants of three views, no_grad
+    elif in_dim < out_dim:
+        assert "train_layer" not in counts and "train_layer walked" not in counts and counts["backward_both"] > 0
+    else:
+        assert "train_layer" not in counts and counts["train_layer walked"] == 3          # where both gradients are wanted
     _python_only(monkeypatch, dl)
-    for u, v in zip(native, run(), strict=True):
+    want, want_alone = run()
+    for u, v in zip(native, want, strict=True):
         assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v)
+    for u, v in zip(alone, want_alone, strict=True):
+        # (Python forms both gradients in one pass along a schedule, which adds the terms of short rows in another order: each
+        # of the 16 sums has `batch` terms of at most |gy|, and the softmax multiplies by at most 1)
+        eps = 2.0 ** -53 if dtype == F64 and wdtype == F64 else 2.0 ** -24
+        bound = 4 * (batch + 2) * eps * gy.double().abs().sum(0)[:, None] + (2.0 ** -10 if wdtype == F16 else 0) * v.double().abs()
+        assert u.dtype == v.dtype and u.shape == v.shape
+        assert torch.equal(u, v) if in_dim < 20000 else bool(((u.double() - v.double()).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("dtype", [F32, F16, F64])
@@ -85,7 +125,9 @@ def test_fused_net(dl, monkeypatch, dtype, want_x, frozen):
         y.backward(g)                                                 # a retained graph is walked again: gradients add up
         return [y.detach()] + ([x.grad] if want_x else []) + first + [p.grad for p in fused.parameters() if p.grad is not None]
 
+    counts = _answered(monkeypatch, dl)
     native = run()
+    assert counts["net_forward"] == 1 and counts["net_backward"] == 2
     _python_only(monkeypatch, dl)
     for u, v in zip(native, run(), strict=True):
         assert torch.equal(u, v)
@@ -153,11 +195,19 @@ def test_what_is_refused_stays_refused(dl):
 
 
 @pytest.mark.parametrize("batch,bits", [(1, 8), (100, 32), (129, 64), (5000, 16)])
-def test_packed_layers(dl, monkeypatch, batch, bits):
+@pytest.mark.parametrize("top", [1000, 1200])
+def test_packed_layers(dl, monkeypatch, batch, bits, top):
     torch.manual_seed(batch)
-    net = torch.nn.Sequential(dl.LogicLayer(100, 1200), dl.LogicLayer(1200, 1000), dl.GroupSum(10)).eval()
+    net = torch.nn.Sequential(dl.LogicLayer(100, 1200), dl.LogicLayer(1200, top), dl.GroupSum(10)).eval()
     x = torch.rand(batch, 100, device="cuda") < 0.3
+    counts = _answered(monkeypatch, dl)
     native = net(dl.PackBitsTensor(x, bit_count=bits))
+    if top < 1200:                                    # a layer that narrows is deferred
+        assert counts == {"pack_rows": 1, "eval_weights": 1, "gate_ids_folded": 1}
+    elif batch <= 129:
+        assert counts == {"pack_rows": 1, "eval_weights": 2, "count_rows": 1}
+    else:
+        assert counts["eval_weights"] + counts.get("gate_ids_folded", 0) == 2
     _python_only(monkeypatch, dl)
     assert torch.equal(native, net(dl.PackBitsTensor(x, bit_count=bits)))
 
