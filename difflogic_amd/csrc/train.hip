@@ -1857,13 +1857,26 @@ bool past_cache(PastCache limits, int64_t steps, int64_t in_dim, int64_t row_byt
 int row_segments(int64_t ncols) { return (int) dl_ceil_div(ncols, 4 * DL_WAVE); }
 
 // Steps per wave of the kernels in which a wave owns whole rows: long chunks re-read fewer rows at
-// their seams, short ones give more waves to hide latency with; keep about three waves per SIMD (`waves`).
-constexpr int64_t DL_CHAIN_WAVES = 3000;
-// ... and two in the one-pass backward of rows longer than 2 KB (64000 -> 64000, 32 / 16 steps: batch 1024 137 / 142 us, 512 80 / 74)
-constexpr int64_t DL_CHAIN_WAVES_LONG = 2000;
-int chain_chunk(int64_t steps, int64_t waves = DL_CHAIN_WAVES) {
+// their seams, short ones give more waves to hide latency with; keep about three waves per SIMD.
+int chain_chunk(int64_t steps) {
     for (int chunk = 32; chunk > 8; chunk /= 2)
-        if (steps / chunk >= waves) return chunk;
+        if (steps / chunk >= 3000) return chunk;
+    return 8;
+}
+
+// ... of the one-pass backward of rows longer than 2 KB, whose 1024 SIMDs hold three waves each: a chunk is also long enough where
+// its waves are there at once and spread evenly, at most two to a SIMD (1536 < waves <= 2048: chunks of half the length would
+// need a second go) or mostly three (from 2560).  Square layers, us with chunks of 32 / 16, by the waves that 32 gives: fp32 at
+// batch 1024 1500 (48000 wide) 111 / 103, 1531 112 / 105, 1562 113 / 120, 1750 120 / 129, 2000 138 / 142, 2250 181 / 171, 2500
+// 193 / 190, 2562 197 / 202, 2750 211 / 222, 3000 233 / 242; at 600 1500 74 / 65, 1625 76 / 81, 2000 84 / 89, 2250 109 / 101, 2500
+// 115 / 108, 2750 120 / 125; half at 1200 1750 101 / 102, 2000 103 / 105, 2500 149 / 130, 2625 149 / 148; at 2048 2562 211 / 209, 2625
+// 214 / 222; double at 512 1750 121 / 131, 2500 196 / 191, 2625 202 / 215.  Chunks of 16 / 8, by the waves of 16: fp32 at 1024 1500
+// (24000 wide) 58 / 55, 1750 62 / 68, 2062 84 / 80, 2500 93 / 91, 2562 93 / 94, 2750 97 / 103; half at 1200 2062 77 / 68, 2625 80 / 81.
+int chain_chunk_long(int64_t steps) {
+    for (int chunk = 32; chunk > 8; chunk /= 2) {
+        const int64_t waves = steps / chunk;
+        if (waves >= 2560 || (waves > 1536 && waves <= 2048)) return chunk;
+    }
     return 8;
 }
 
@@ -2019,7 +2032,7 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
     if ((partial_bytes > 0 || overflow_rows > 0) && workspace == nullptr) return DL_ERR_INVALID_ARGUMENT;
     C *partial = partial_bytes > 0 ? (C *) workspace : nullptr;
     C *overflow = (C *) ((char *) workspace + partial_bytes);
-    const int chunk = chain_chunk(steps * segments, ncols > 2 * DL_WAVE ? DL_CHAIN_WAVES_LONG : DL_CHAIN_WAVES);
+    const int chunk = ncols > 2 * DL_WAVE ? chain_chunk_long(steps * segments) : chain_chunk(steps * segments);
     const int64_t blocks = dl_ceil_div(dl_ceil_div(steps, chunk), 4), fix_blocks = dl_ceil_div(n_fix, 4);
     if (blocks > 0x7fffffffLL || fix_blocks > 0x7fffffffLL) return DL_ERR_TOO_LARGE;
     // a few vertices are finished by further workgroups of the same launch; many are cheaper through overflow rows
