@@ -12,11 +12,13 @@ _PLAIN = (torch.nn.Parameter, torch.Tensor)
 _NO_WALK = ([], 0, 0, 0, False, False, False)
 
 
+_is_compiling, _tracing_state = torch.compiler.is_dynamo_compiling, torch._C._get_tracing_state
+
+
 def _in_one_call(x):
     """Whether a native call may take ``x``: a CUDA tensor, not a subclass, of a call that nobody traces (the compiler cannot
     look into a native function; torch.jit would record nothing of it)."""
-    return (type(x) is torch.Tensor and x.is_cuda and not torch.compiler.is_compiling()
-            and torch._C._get_tracing_state() is None)
+    return type(x) is torch.Tensor and x.is_cuda and not _is_compiling() and _tracing_state() is None
 
 
 class LogicLayer(torch.nn.Module):
@@ -268,15 +270,16 @@ class GroupSum(torch.nn.Module):
         if isinstance(x, PackBitsTensor):
             return x.group_sum(self.k)
         assert x.shape[-1] % self.k == 0, (x.shape, self.k)
-        # (k and tau are converted where the kernels take the call alone: the formula below broadcasts a tau per class)
+        if (_in_one_call(x) and type(self.tau) in (float, int) and self.k <= self._HIP_MAX_K
+                and x.shape[-1] <= self._HIP_MAX_OUT_DIM):
+            y = _host.group_sum(x, int(self.k), float(self.tau))            # the case below in one native call
+            if y is not None:
+                return y
+        # (a tau that is a tensor is converted where the kernels take the call alone: the formula below broadcasts it)
         if (x.is_cuda and x.dim() == 2 and x.dtype in (torch.float16, torch.float32, torch.float64)
                 and x.numel() > 0 and x.stride(0) == 1 and x.stride(1) == x.shape[0]
                 and self.k <= self._HIP_MAX_K and x.shape[1] <= self._HIP_MAX_OUT_DIM):
             # the transposed view a 'cuda' LogicLayer returns: sum on the feature-major storage
-            if _in_one_call(x):
-                y = _host.group_sum(x, int(self.k), float(self.tau))
-                if y is not None:
-                    return y
             return GroupSumCudaFunction.apply(x.transpose(0, 1), self.k, float(self.tau))
         return x.reshape(*x.shape[:-1], self.k, x.shape[-1] // self.k).sum(-1) / self.tau
 
