@@ -1843,10 +1843,20 @@ int group_sum_splits(int64_t out_dim, int64_t batch, int64_t k) {
 //   backward_w alone       131 MB 44 / 50, 179 MB 66 / 70, 262 MB 98 / 95, 524 MB 203 / 190, 1 GB 502 / 503
 // (The discretised forward goes by the bytes of x and y: a layer that narrows, 80000 -> 40000 at batch 512, 164 MB and 82 MB,
 // is still better off with both in the cache, three layers 112 / 117 us.)
+// Half and double agree with that table at the same bytes (forward: half 64 MB 34.6 / 33.2, 98 MB 49 / 44, 262 MB 112 / 97, double 65 MB
+// 33.0 / 30.6, 131 MB 61 / 54; one-pass backward: 131 MB 90 / 76 and 86 / 72, 262 MB 174 / 138 and 170 / 136), and so does the forward
+// with given probabilities with the discretised one.  But a whole step of half or double gains by the forward pass only where its
+// backward passes the cache as well, from 80 MB (784 -> 6 x 64000, a captured step: half 51 MB 435 / 443 us, 64 MB 508 / 514, 73 MB
+// 637 / 643, 77 MB 657 / 650, 81 MB 657 / 637, 90 MB 795 / 776; double 51 MB 525 / 532, 76 MB 638 / 646, 81 MB 648 / 630); fp32 is
+// the same either way below that (51 MB 404 / 406 as written and 341 / 343 fused, 65 MB 452 / 451 and 375 / 371, 76 MB 542 / 544 and
+// 464 / 461).  In a trace, where kernels run one by one, the kernel behind one that passes the cache is up to a tenth
+// longer (first layer of 9216 -> 4 x 128000 at batch 1024, backward_w 161 / 173; last layer with GroupSum 210 / 225); the step is
+// shorter all the same (forward alone 2293 / 2201, backward alone 2260 / 2201).
 // Smaller matrices stay in the caches from one kernel to the next; rows that are read several times (a layer much wider
 // than its input, the classes' gradient rows) are read the ordinary way.
 struct PastCache { int64_t from, to; };
-constexpr PastCache DL_PAST_FORWARD = {50000000, INT64_MAX}, DL_PAST_ARGMAX = {280000000, 1400000000},
+constexpr PastCache DL_PAST_FORWARD = {50000000, INT64_MAX}, DL_PAST_FORWARD_HALF_DOUBLE = {80000000, INT64_MAX},
+                    DL_PAST_ARGMAX = {280000000, 1400000000},
                     DL_PAST_BACKWARD = {80000000, 700000000}, DL_PAST_WEIGHTS = {240000000, INT64_MAX};
 
 bool past_cache(PastCache limits, int64_t steps, int64_t in_dim, int64_t row_bytes, int64_t rows_written = 0) {
@@ -1889,7 +1899,7 @@ int forward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron, 
     if (kind != Rows::whole && !(any_rows && kind == Rows::ragged)) return DL_ERR_TOO_LARGE;
     const int64_t nchunks = steps / DL_TRAIN_CHUNK, ncols = dl_ceil_div(batch, V);
     const int64_t row_bytes = batch * (int64_t) sizeof(T);
-    const bool past = probs ? past_cache(DL_PAST_FORWARD, steps, in_dim, row_bytes)
+    const bool past = probs ? past_cache(sizeof(T) == 4 ? DL_PAST_FORWARD : DL_PAST_FORWARD_HALF_DOUBLE, steps, in_dim, row_bytes)
                             : past_cache(DL_PAST_ARGMAX, steps, in_dim, row_bytes, out_dim);
     const T *xp = (const T *) x, *wp = (const T *) w;
     const dim3 block(DL_BLOCK);

@@ -1,6 +1,6 @@
 """Chained training kernels on matrices large enough that their rows are read, and weight gradients and probabilities written,
-past the Infinity Cache (50 MB of input for the forward pass, 80 MB for the one-pass backward, 140 MB for the discretised
-forward, 240 MB for the weight gradient alone): against the kernels that take neurons one by one, which have no such choice.
+past the Infinity Cache (50 MB of input for the forward pass, 80 MB in half and double and for the one-pass backward, 280 MB of
+input and output for the discretised forward, 240 MB for the weight gradient alone): against the kernels that take neurons one by one, which have no such choice.
 Below, at and above a row's last full wave of vectors, whole and ragged rows, and inputs that hold infinities."""
 import pytest
 import torch
@@ -26,7 +26,8 @@ def _same(u, v, dtype, rows=None):
 @pytest.mark.parametrize("dtype,width,batch", [(torch.float32, 26000, 500), (torch.float32, 26000, 512), (torch.float32, 42000, 511),
                                                (torch.float32, 40000, 1024), (torch.float32, 64000, 1000), (torch.float32, 170000, 128),
                                                (torch.float16, 42000, 1001), (torch.float16, 42000, 1024), (torch.float64, 42000, 256),
-                                               (torch.float64, 42000, 255)])
+                                               (torch.float64, 42000, 255), (torch.float16, 40000, 1000), (torch.float16, 40000, 999),
+                                               (torch.float64, 40000, 250), (torch.float64, 40000, 249)])
 def test_rows_read_past_the_cache(ext, dtype, width, batch):
     from difflogic_amd.functional import get_random_connections
     torch.manual_seed(batch)
