@@ -2058,7 +2058,9 @@ int backward_chain_t(const void *x, const int32_t *verts, const int32_t *neuron,
               LOWER ? *lower : none, fix, LOWER ? false : w32)
 #define DL_LAUNCH_BACKWARD_CHAIN_RAG(VV, CPL, RAG, NT)                                                                   \
     do {                                                                                                                 \
-        if (lower && !x) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, RAG, NT);                                               \
+        if (lower && !x) {                           /* (half has been refused: its rows are not recomputed) */          \
+            if constexpr (sizeof(T) != 2) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 2, RAG, NT);                              \
+        }                                                                                                                \
         else if (lower) DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 1, RAG, NT);                                                \
         else DL_LAUNCH_BACKWARD_CHAIN_AS(VV, CPL, 0, RAG, NT);                                                           \
     } while (0)
