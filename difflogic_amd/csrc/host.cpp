@@ -528,7 +528,7 @@ c10::optional<Tensor> count_rows(const Tensor &b, int64_t pad, int64_t k) {
         return c10::nullopt;
     const c10::DeviceGuard guard(b.device());
     Tensor out = at::empty({b.size(1) * 64 - pad, k}, b.options().dtype(at::kInt));
-    check(dl_groupbitsum(b.const_data_ptr(), out.mutable_data_ptr<int32_t>(), b.size(0), b.size(1), 64, (int) pad, (int) k,
+    check(dl_groupbitsum(b.const_data_ptr(), out.mutable_data_ptr<int32_t>(), b.size(0), b.size(1), 64, pad, k,
                          stream_of(b)),
           "groupbitsum");
     return out;

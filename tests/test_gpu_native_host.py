@@ -236,3 +236,14 @@ def test_group_sum_converts_tau_where_the_kernels_take_the_call(dl):
     finally:
         torch.cuda.set_sync_debug_mode("default")
     assert torch.equal(got, want / tau[1])
+
+
+def test_counts_of_rows_padded_by_more_than_31_bits(dl):
+    """pad_len reaches the kernel whole: cut to 32 bits, the kernel would write far more samples than the result has."""
+    words = (1 << 26) + 3
+    b = torch.zeros(2, words, dtype=torch.int64, device="cuda")
+    b[:, :4] = torch.randint(-2 ** 62, 2 ** 62, (2, 4), device="cuda")
+    for samples in (70, 192, 200):
+        got = dl.difflogic_cuda.groupbitsum(b, words * 64 - samples, 1)
+        assert got.shape == (samples, 1)
+        assert torch.equal(got, dl.difflogic_cuda.groupbitsum(b[:, :4].contiguous(), 256 - samples, 1))
