@@ -1731,9 +1731,13 @@ int group_sum_forward_t(const void *x, void *y, void *workspace, int64_t out_dim
     const int64_t gx = dl_ceil_div(kind == Rows::single ? batch : dl_ceil_div(batch, V), DL_WAVE);
     if (gx > 0x7fffffffLL || k > 65535) return DL_ERR_TOO_LARGE;
     const dim3 grid((unsigned) gx, (unsigned) k, (unsigned) splits);
-    // more than the Infinity Cache holds (128000 rows at batch 1024, 524 MB, with eight rows in flight instead of four: 134 -> 90 us
-    // inside the step; 64 and 256 MB are no faster past it)
-    const bool past = out_dim * batch * (int64_t) sizeof(T) >= 400000000;
+    // More than the Infinity Cache holds is read past it: the rows of x that the layer before leaves there stay.  A training layer
+    // with its GroupSum behind it, us with the sum's rows read ordinarily / past the cache: fp32 262 MB 131.5 / 129.8, 311 MB 162 / 157,
+    // 344 MB 203 / 180, 410 MB 260 / 228, 524 MB 319 / 280, 819 MB 524 / 477, 1 GB 652 / 604; half 262 MB 141 / 144, 328 MB 197 / 180,
+    // 524 MB 344 / 301; double 524 MB 308 / 266; whole steps of 784 -> 3 layers, fp32 303 MB 842 / 818, 393 MB 1132 / 1095, half 320 MB
+    // 1104 / 1083.  (In a trace the kernel itself, 128000 rows at batch 1024, with eight rows in flight instead of four as well:
+    // 134 -> 104 us.)
+    const bool past = out_dim * batch * (int64_t) sizeof(T) >= 300000000;
 #define DL_LAUNCH_PARTIAL_AS(VV, RAG, NT)                                                                              \
     DL_LAUNCH((group_sum_partial_kernel<T, VV, RAG, NT>), grid, dim3(DL_BLOCK), 0, s, (const T *) x, (C *) workspace,  \
               per_class, batch, k, rows_per_split)

@@ -1,6 +1,6 @@
 """Chained training kernels on matrices large enough that their rows are read, and weight gradients and probabilities written,
 past the Infinity Cache (50 MB of input for the forward pass, 80 MB in half and double and for the one-pass backward, 280 MB of
-input and output for the discretised forward, 240 MB for the weight gradient alone): against the kernels that take neurons one by one, which have no such choice.
+input and output for the discretised forward, 240 MB for the weight gradient alone, 300 MB of GroupSum's input): against the kernels that take neurons one by one, which have no such choice.
 Below, at and above a row's last full wave of vectors, whole and ragged rows, and inputs that hold infinities."""
 import pytest
 import torch
@@ -78,3 +78,14 @@ def test_infinities_stay_in_their_rows(ext, batch):
     reads = torch.isin(a, hit) | torch.isin(b, hit)
     assert bool(gw[~reads].isfinite().all()) and int(reads.sum()) > 0
     assert torch.equal(gw[~reads], ext.backward_logits(x, a, b, gy, p0)[~reads])
+
+
+@pytest.mark.parametrize("dtype,rows,batch", [(torch.float32, 73240, 1024), (torch.float32, 73250, 1024), (torch.float32, 75000, 1001),
+                                              (torch.float16, 146480, 1024), (torch.float16, 150000, 1024), (torch.float16, 150000, 1001),
+                                              (torch.float64, 36620, 1024), (torch.float64, 37500, 1001)])
+def test_group_sum_past_the_cache(ext, dtype, rows, batch):
+    """Eighths: the sums are exact in fp32 in any order, and rounded once to half."""
+    torch.manual_seed(batch)
+    x = torch.randint(0, 9, (rows, batch), device="cuda", dtype=torch.int8).to(dtype) / 8
+    want = torch.stack([c.double().sum(0) for c in x.view(10, rows // 10, batch)], 1)
+    assert torch.equal(ext.group_sum_forward(x, 10, 1.0), want.to(dtype))
