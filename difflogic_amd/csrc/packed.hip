@@ -2066,8 +2066,8 @@ __device__ __forceinline__ uint32_t fold_gate(uint32_t op, uint32_t sa, uint32_t
 // Gate ids of a layer for packed inference.  Four lanes take a neuron's 16 weights, so a wave reads a contiguous kilobyte (fp32)
 // at once; one lane per neuron read 64 bytes of 64 lines four times.  With `a`: the constants among the layer's input rows
 // are folded in (state_in: 1 all zeros, 2 all ones, 0 varies; null: all vary), and state_out says which of the layer's own
-// outputs are constant.  Bound by latency: 8000 neurons 2.2 us, launch included, 64000 (5 MB) 2.7,
-// 256000 6.5; with a lane per neuron 3.7, 4.1 and 12.4.
+// outputs are constant.  Bound by latency: in a trace of whole calls 8000 neurons take 4.4 us, with a lane per neuron 4.6, and
+// 64000 (5 MB) 4.6, with a lane per neuron 5.6.
 template <typename T, typename C, bool FOLD>
 __global__ __launch_bounds__(DL_BLOCK) void gate_ids_kernel(const T *__restrict__ w, const int64_t *__restrict__ a,
                                                             const int64_t *__restrict__ b, const uint8_t *__restrict__ state_in,
